@@ -125,7 +125,7 @@ int walsh_ternary_unpack(const uint8_t *packed, int64_t rows, int64_t K, int8_t 
  * walsh_hadamard_weight_bytes: size of the kernel weight layout for a shape.
  * walsh_hadamard_prepare: reorders 2-bit packed codes [32, out_o, ceil(in_o/4)]
  *   (walsh_ternary_quantize's `packed`) into that layout.  Call once per
- *   weight version; the layout holds the same bytes, permuted.
+ *   weight version; the layout holds the same codes (2 bits each).
  */
 int64_t walsh_hadamard_weight_bytes(int64_t in_o, int64_t out_o);
 int walsh_hadamard_prepare(const uint8_t *packed, int64_t in_o, int64_t out_o,

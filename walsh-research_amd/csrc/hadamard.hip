@@ -10,7 +10,7 @@
 // transforms run entirely inside the lane's registers (5 butterfly stages on
 // 32 values, no cross-lane traffic).  The per-group contraction
 // y_g[o, t] = sum_i W[g, o, i] xm[t, g, i] is a 16x16 matrix-core product per
-// group with A = W_g (o x i, 2-bit codes expanded through an LDS table) and
+// group with A = W_g (o x i, 2-bit codes expanded in registers) and
 // B = xm^T (i x t, already in the lane layout the instruction wants), so the
 // result lands as 4 consecutive outputs o per lane per group, ready for the
 // output transform and 8/16-byte stores.
@@ -25,27 +25,36 @@ namespace walsh {
 
 // ---------------------------------------------------------------- weights
 
-// Kernel weight layout: [Nt][Kc][64 lanes][32 groups] bytes.  Lane l of tile
-// (nt, c) holds, for each group g, the packed byte with codes
-// W[g, 16nt + l%16, 16c + 4(l/16) .. +3]; that is exactly one byte of the
-// reference packing (4 codes per byte along K), so the layout is a byte
-// permutation.  Rows/columns past out_o/in_o hold 0x55 (four zero codes).
+// Kernel weight layout: [Nt][Kc][64 lanes][8 words].  Word k of lane l of tile
+// (nt, c) holds, for the groups g = 4k .. 4k + 3, the codes of
+// W[g, 16nt + l%16, 16c + 4(l/16) .. +3] in the pair order of code_bits
+// (codes 0, 1 of group 4k + j are pair 2j, codes 2, 3 pair 2j + 1; the
+// second of a pair in the high half).  Rows/columns past out_o/in_o hold
+// zeros.
 __global__ void hadamard_prepare_kernel(const uint8_t *__restrict__ packed, int in_o, int out_o, int Nt,
-                                        int Kc, uint8_t *__restrict__ kw) {
-    const int64_t total = (int64_t)Nt * Kc * 64 * 32;
+                                        int Kc, uint32_t *__restrict__ kw) {
+    const int64_t total = (int64_t)Nt * Kc * 64 * 8;
     const int kp4 = (int)ceil_div(in_o, 4);
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
-        const int g = (int)(e & 31);
-        const int lane = (int)((e >> 5) & 63);
-        const int64_t tc = e >> 11;
+        const int k = (int)(e & 7);
+        const int lane = (int)((e >> 3) & 63);
+        const int64_t tc = e >> 9;
         const int c = (int)(tc % Kc);
         const int nt = (int)(tc / Kc);
         const int o = kNTile * nt + (lane & 15);
         const int i0 = kKChunk * c + 4 * (lane >> 4);
-        uint8_t b = 0x55;
-        if (o < out_o && i0 < in_o) b = packed[((int64_t)g * out_o + o) * kp4 + i0 / 4];
-        kw[e] = b;
+        uint32_t w = 0;
+        if (o < out_o && i0 < in_o) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t b = packed[((int64_t)(4 * k + j) * out_o + o) * kp4 + i0 / 4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    w |= code_bits((b >> (6 - 2 * i)) & 3u) << (14 - 2 * (2 * j + (i >> 1)) + 16 * (i & 1));
+            }
+        }
+        kw[e] = w;
     }
 }
 
@@ -54,7 +63,7 @@ __global__ void hadamard_prepare_kernel(const uint8_t *__restrict__ packed, int 
 // are computed once per tile and reused for every output tile.
 // DENSE: float weights instead of ternary codes (the Hadamard head mixer),
 // as matrix-core A fragments [Nt][Kc][32 g][64 lanes] (bf16x4 or f32x4)
-// copied into LDS in place of the code table.
+// copied into LDS.
 // Per-wave LDS area of the STAGED variant: the tile's 16 rows of 1 KB at a
 // pitch of 1 KB + 16 bytes (16-byte aligned rows for the whole-row
 // accesses).  The 8-byte fragment accesses (row t, bytes 32 g + 8 q) then
@@ -83,8 +92,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
     static_assert(!PIPE1 || (BF16MMA && VEC && KC1 && !DENSE), "PIPE1 shape");
     static_assert(!STAGED || PIPE1, "STAGED is a PIPE1 variant");
     extern __shared__ __align__(16) unsigned char smem[];
-    void *lut = smem;
-    const size_t wbytes = DENSE ? (size_t)a.Nt * a.Kc * 32 * 64 * dense_frag_bytes<BF16MMA>() : lut_bytes<BF16MMA>();
+    const size_t wbytes = DENSE ? (size_t)a.Nt * a.Kc * 32 * 64 * dense_frag_bytes<BF16MMA>() : 0;
     f32x4 *alpha_l = (f32x4 *)(smem + wbytes);
     f32x4 *beta_l = alpha_l + a.Kc * 128;
 
@@ -92,19 +100,6 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
     if constexpr (DENSE) {
         const uint4 *src = (const uint4 *)a.kw;
         for (int e = tid; e < (int)(wbytes / 16); e += kThreads) ((uint4 *)smem)[e] = src[e];
-    } else {
-        const uint32_t byte = (uint32_t)tid;  // kThreads == 256 table entries
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)((byte >> (6 - 2 * j)) & 3u) - 1);
-        if constexpr (BF16MMA) {
-            uint2 e;
-            e.x = pack_bf16x2(val[0], val[1]);
-            e.y = pack_bf16x2(val[2], val[3]);
-            ((uint2 *)lut)[byte] = e;
-        } else {
-            ((f32x4 *)lut)[byte] = f32x4{val[0], val[1], val[2], val[3]};
-        }
     }
     for (int e = tid; e < a.Kc * 128; e += kThreads) {  // e = (c*4 + q)*32 + g
         const int g = e & 31, cq = e >> 5;
@@ -120,7 +115,8 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
         const int o0 = 4 * nq;
         f32x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (o0 + j < a.out_o) ? a.beta[h * a.beta_h + o0 + j] * 0.03125f : 0.f;
+        for (int j = 0; j < 4; ++j)
+            v[j] = (o0 + j < a.out_o) ? a.beta[h * a.beta_h + o0 + j] * (DENSE ? kTransformScale : kCodeScale) : 0.f;
         beta_l[e] = v;
     }
     __syncthreads();
@@ -141,7 +137,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
             contract_dense<BF16MMA>(smem + ((size_t)(nt * a.Kc + c) * 32 * 64 + lane) * dense_frag_bytes<BF16MMA>(),
                                     xm, acc);
         else
-            contract<BF16MMA>(a, nt, c, lane, xm, lut, acc);
+            contract<BF16MMA>(a, nt, c, lane, xm, acc);
     };
 
     if constexpr (PIPE1) {
@@ -214,7 +210,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
                 f32x4 acc[32];
 #pragma unroll
                 for (int g = 0; g < 32; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(a, nt, 0, lane, xm, lut, acc);
+                contract<true>(a, nt, 0, lane, xm, acc);
                 // the next tile's x is requested before any store of this one:
                 // a wait for a load also waits for every memory operation
                 // issued before it, so loads queued behind stores would wait
@@ -240,12 +236,12 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
                 const f32x4 cs = (rope && ok) ? rope_cs(a, row, o0) : f32x4{1.f, 0.f, 1.f, 0.f};
                 auto stores = [&](auto with_rope) {
 #pragma unroll
-                    for (int h0 = 0; h0 < 32; h0 += 4) {
-                        f32x4 b8[4];
+                    for (int h0 = 0; h0 < 32; h0 += 2) {
+                        f32x4 b8[2];
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) b8[j] = bl[h0 + j];
+                        for (int j = 0; j < 2; ++j) b8[j] = bl[h0 + j];
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
+                        for (int j = 0; j < 2; ++j) {
                             f32x4 r = acc[h0 + j] * b8[j];
                             if constexpr (decltype(with_rope)::value) r = rope_apply(r, cs);
                             if constexpr (STAGED) {
@@ -373,10 +369,10 @@ constexpr int64_t kPairMaxTiles = 2048;
 // tiles on: at 32,768 rows one layer takes 21.3 us against the pairs'
 // 22.7 us (20.9 against 22.8 from HBM), at 16,384 rows 16.1 against 15.0.
 constexpr int64_t kPairMaxTilesRows = 1024;
-constexpr size_t kPairLds = 256 * 8 + 2 * 128 * 16 + 2 * 8 * 64 * 16;   // lut, alpha/beta, exchange
+constexpr size_t kPairLds = 2 * 128 * 16 + 2 * 8 * 64 * 16;   // alpha/beta, exchange
 
 template <int HF, bool DENSE>
-__device__ __forceinline__ void pair_tile(const HadArgs &a, int tile, int lane, const uint2 *__restrict__ lut,
+__device__ __forceinline__ void pair_tile(const HadArgs &a, int tile, int lane,
                                           const f32x4 *__restrict__ alpha_l, const f32x4 *__restrict__ beta_l,
                                           f32x4 *__restrict__ xch, __amdgpu_buffer_rsrc_t xr,
                                           __amdgpu_buffer_rsrc_t yr) {
@@ -452,7 +448,7 @@ __device__ __forceinline__ void pair_tile(const HadArgs &a, int tile, int lane, 
         } else {
             const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             const int g = 8 * HF + (s & 7) + 16 * (s >> 3);
-            wa = lut[(wb[g >> 2] >> (8 * (g & 3))) & 0xffu];
+            wa = codes_bf16x4(wb[g >> 2], g & 3);
         }
         acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, wa),
                                                             __builtin_bit_cast(i16x4, xm[s]),
@@ -531,8 +527,8 @@ __device__ __forceinline__ void pair_tile(const HadArgs &a, int tile, int lane, 
 // inputs of groups 16 HF + s; on return acc[u] holds group g_out(u) before
 // beta.
 template <int HF, bool DENSE>
-__device__ __forceinline__ void pair_core(const HadArgs &a, int lane, const uint2 *__restrict__ lut, f32x4 *xch,
-                                          uint4 w0, uint4 w1, f32x4 (&v)[16], f32x4 (&acc)[16]) {
+__device__ __forceinline__ void pair_core(const HadArgs &a, int lane, f32x4 *xch, uint4 w0,
+                                          uint4 w1, f32x4 (&v)[16], f32x4 (&acc)[16]) {
     f32x4 *mine = xch + HF * 8 * 64, *theirs = xch + (1 - HF) * 8 * 64;
 #pragma unroll
     for (int h = 1; h < 16; h <<= 1) {
@@ -578,7 +574,7 @@ __device__ __forceinline__ void pair_core(const HadArgs &a, int lane, const uint
         } else {
             const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
             const int g = 8 * HF + (s & 7) + 16 * (s >> 3);
-            wa = lut[(wb[g >> 2] >> (8 * (g & 3))) & 0xffu];
+            wa = codes_bf16x4(wb[g >> 2], g & 3);
         }
         acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, wa),
                                                             __builtin_bit_cast(i16x4, xm[s]),
@@ -621,7 +617,7 @@ __device__ __forceinline__ void pair_core(const HadArgs &a, int lane, const uint
 
 template <int HF>
 __device__ __forceinline__ void mixproj_tile(const HadArgs &m, const HadArgs &p, int tile, int lane,
-                                             const uint2 *__restrict__ lut, const f32x4 *__restrict__ mbeta_l,
+                                             const f32x4 *__restrict__ mbeta_l,
                                              const f32x4 *__restrict__ palpha_l, const f32x4 *__restrict__ pbeta_l,
                                              f32x4 *xch, __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t yr) {
     const int t = lane & 15, q = lane >> 4;
@@ -643,7 +639,7 @@ __device__ __forceinline__ void mixproj_tile(const HadArgs &m, const HadArgs &p,
             v[s] = f32x4{__uint_as_float(xraw[s].x << 16), __uint_as_float(xraw[s].x & 0xffff0000u),
                          __uint_as_float(xraw[s].y << 16), __uint_as_float(xraw[s].y & 0xffff0000u)};
     }
-    pair_core<HF, true>(m, lane, lut, xch, w0, w1, v, acc);
+    pair_core<HF, true>(m, lane, xch, w0, w1, v, acc);
     // the projection's code bytes (requested here: live through the mixer
     // they would push the kernel past its register budget)
     load_w(p, 0, 0, lane, w0, w1);
@@ -671,7 +667,7 @@ __device__ __forceinline__ void mixproj_tile(const HadArgs &m, const HadArgs &p,
         v[own] = acc[8 * HF + j] * pa[own];
         v[other] = theirs[j * 64 + lane] * pa[other];
     }
-    pair_core<HF, false>(p, lane, lut, xch, w0, w1, v, acc);
+    pair_core<HF, false>(p, lane, xch, w0, w1, v, acc);
     // the projection's beta and the stores of groups g_out(u)
     const int o0 = 4 * q;
     const uint32_t voff = row_ok ? (uint32_t)((int64_t)row * p.ldy * 2) + (uint32_t)o0 * 2 : kOOB;
@@ -684,24 +680,17 @@ __device__ __forceinline__ void mixproj_tile(const HadArgs &m, const HadArgs &p,
     }
 }
 
-constexpr size_t kMixProjLds = 256 * 8 + 3 * 128 * 16 + 2 * 8 * 64 * 16;   // lut, 3 tables, exchange
+constexpr size_t kMixProjLds = 3 * 128 * 16 + 2 * 8 * 64 * 16;   // 3 tables, exchange
 
 // m: the mixer (HadArgs of walsh_head_mixer_fwd), p: the projection (in_o =
 // out_o = 16, its x unused: the mixer's output rows).
 __global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_mixproj_kernel(HadArgs m, HadArgs p) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint2 *lut = (uint2 *)smem;
-    f32x4 *mbeta_l = (f32x4 *)(smem + 256 * 8);   // [4 q][32 h]
+    f32x4 *mbeta_l = (f32x4 *)smem;                // [4 q][32 h]
     f32x4 *palpha_l = mbeta_l + 128;               // [4 q][32 g]
     f32x4 *pbeta_l = palpha_l + 128;               // [4 q][32 h]
     f32x4 *xch = pbeta_l + 128;                    // [2 HF][8][64 lanes]
     const int tid = threadIdx.x;
-    for (int e = tid; e < 256; e += kPairThreads) {
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)(((uint32_t)e >> (6 - 2 * j)) & 3u) - 1);
-        lut[e] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-    }
     {
         const int e = tid;   // (q, g) = (e >> 5, e & 31); kPairThreads == 128 entries
         const int g = e & 31, i0 = 4 * (e >> 5);
@@ -720,9 +709,9 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_mixproj_kernel(
         f32x4 mb, pa, pb;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            mb[j] = __uint_as_float(rm[j]) * 0.03125f;
+            mb[j] = __uint_as_float(rm[j]) * kTransformScale;
             pa[j] = p.alpha ? __uint_as_float(ra[j]) : 1.f;
-            pb[j] = __uint_as_float(rp[j]) * 0.03125f;
+            pb[j] = __uint_as_float(rp[j]) * kCodeScale;
         }
         mbeta_l[e] = mb;
         palpha_l[e] = pa;
@@ -734,8 +723,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_mixproj_kernel(
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(p.y, (uint32_t)((int64_t)m.M * p.ldy * 2));
     const int n_tiles = (int)ceil_div(m.M, kTile);
     for (int tile = (int)blockIdx.x; tile < n_tiles; tile += (int)gridDim.x) {
-        if (hf == 0) mixproj_tile<0>(m, p, tile, lane, lut, mbeta_l, palpha_l, pbeta_l, xch, xr, yr);
-        else mixproj_tile<1>(m, p, tile, lane, lut, mbeta_l, palpha_l, pbeta_l, xch, xr, yr);
+        if (hf == 0) mixproj_tile<0>(m, p, tile, lane, mbeta_l, palpha_l, pbeta_l, xch, xr, yr);
+        else mixproj_tile<1>(m, p, tile, lane, mbeta_l, palpha_l, pbeta_l, xch, xr, yr);
     }
 }
 
@@ -750,10 +739,10 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_mixproj_kernel(
 // chunk loop bitwise.  Every wavefront passes the same barriers (six per tile).
 constexpr int kPairMaxKc = 4;
 constexpr int kKparMaxKc = kPairMaxKc;
-constexpr size_t kpar_lds(int Kc) { return 256 * 8 + (size_t)(Kc + 1) * 128 * 16 + (size_t)Kc * 2 * 8 * 64 * 16; }
+constexpr size_t kpar_lds(int Kc) { return (size_t)(Kc + 1) * 128 * 16 + (size_t)Kc * 2 * 8 * 64 * 16; }
 
 template <int HF>
-__device__ __forceinline__ void kpar_tile(const HadArgs &a, int tile, int pair, int lane, const uint2 *__restrict__ lut,
+__device__ __forceinline__ void kpar_tile(const HadArgs &a, int tile, int pair, int lane,
                                           const f32x4 *__restrict__ alpha_l, const f32x4 *__restrict__ beta_l,
                                           f32x4 *xch_all, __amdgpu_buffer_rsrc_t xr, __amdgpu_buffer_rsrc_t yr) {
     const int t = lane & 15, q = lane >> 4;
@@ -831,7 +820,7 @@ __device__ __forceinline__ void kpar_tile(const HadArgs &a, int tile, int pair, 
             for (int s = 0; s < 16; ++s) {
                 const int g = 8 * HF + (s & 7) + 16 * (s >> 3);
                 acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                    __builtin_bit_cast(i16x4, lut[(wb[g >> 2] >> (8 * (g & 3))) & 0xffu]),
+                    __builtin_bit_cast(i16x4, codes_bf16x4(wb[g >> 2], g & 3)),
                     __builtin_bit_cast(i16x4, xc[s]), acc[s], 0, 0, 0);
             }
         }
@@ -887,17 +876,10 @@ __device__ __forceinline__ void kpar_tile(const HadArgs &a, int tile, int pair, 
 // blockDim.x = 128 * Kc (2 <= Kc <= kKparMaxKc), no RoPE.
 __global__ __launch_bounds__(kPairThreads * kKparMaxKc, 3) void hadamard_pair_kpar_kernel(HadArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint2 *lut = (uint2 *)smem;
-    f32x4 *alpha_l = (f32x4 *)(smem + 256 * 8);   // [Kc][4 q][32 g]
+    f32x4 *alpha_l = (f32x4 *)smem;                // [Kc][4 q][32 g]
     f32x4 *beta_l = alpha_l + a.Kc * 128;          // [4 q][32 h]
     f32x4 *xch = beta_l + 128;                     // [Kc pairs][2 HF][8][64 lanes]
     const int tid = threadIdx.x, nthr = (int)blockDim.x;
-    for (int e = tid; e < 256; e += nthr) {
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)(((uint32_t)e >> (6 - 2 * j)) & 3u) - 1);
-        lut[e] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-    }
     for (int e = tid; e < a.Kc * 128; e += nthr) {   // e = (c*4 + q)*32 + g
         const int g = e & 31, i0 = 4 * (e >> 5);
         f32x4 va;
@@ -909,7 +891,7 @@ __global__ __launch_bounds__(kPairThreads * kKparMaxKc, 3) void hadamard_pair_kp
         const int h = e & 31, o0 = 4 * (e >> 5);
         f32x4 vb;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) vb[j] = (o0 + j < a.out_o) ? a.beta[h * a.beta_h + o0 + j] * 0.03125f : 0.f;
+        for (int j = 0; j < 4; ++j) vb[j] = (o0 + j < a.out_o) ? a.beta[h * a.beta_h + o0 + j] * kCodeScale : 0.f;
         beta_l[e] = vb;
     }
     __syncthreads();
@@ -919,8 +901,8 @@ __global__ __launch_bounds__(kPairThreads * kKparMaxKc, 3) void hadamard_pair_kp
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, (uint32_t)((int64_t)a.M * a.ldy * 2));
     const int n_tiles = (int)ceil_div(a.M, kTile);
     for (int tile = (int)blockIdx.x; tile < n_tiles; tile += (int)gridDim.x) {
-        if (hf == 0) kpar_tile<0>(a, tile, pair, lane, lut, alpha_l, beta_l, xch, xr, yr);
-        else kpar_tile<1>(a, tile, pair, lane, lut, alpha_l, beta_l, xch, xr, yr);
+        if (hf == 0) kpar_tile<0>(a, tile, pair, lane, alpha_l, beta_l, xch, xr, yr);
+        else kpar_tile<1>(a, tile, pair, lane, alpha_l, beta_l, xch, xr, yr);
     }
 }
 
@@ -929,8 +911,7 @@ __global__ __launch_bounds__(kPairThreads * kKparMaxKc, 3) void hadamard_pair_kp
 template <bool DENSE>
 __global__ __launch_bounds__(kPairThreads, DENSE ? 3 : 4) void hadamard_pair_kernel(HadArgsN an) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint2 *lut = (uint2 *)smem;
-    f32x4 *alpha_l = (f32x4 *)(smem + 256 * 8);   // [4 q][32 g]
+    f32x4 *alpha_l = (f32x4 *)smem;                // [4 q][32 g]
     f32x4 *beta_l = alpha_l + 128;                 // [4 q][32 h]
     f32x4 *xch = beta_l + 128;                     // [2 HF][8][64 lanes]
     // (layer, first tile) of this workgroup.  Consecutive workgroups go to
@@ -947,8 +928,8 @@ __global__ __launch_bounds__(kPairThreads, DENSE ? 3 : 4) void hadamard_pair_ker
         const int e = tid;   // (q, g) = (e >> 5, e & 31); kPairThreads == 128 entries
         const int g = e & 31, i0 = 4 * (e >> 5);
         // buffer loads (zero past in_o / out_o) with no branch around them,
-        // converted after the LUT is built: a conversion or branch right
-        // after a load waits for it
+        // converted after all are issued: a conversion or branch right after
+        // a load waits for it
         // (no alpha: a resource of no records, every load out of range)
         uint32_t ra[4], rb[4];
         const __amdgpu_buffer_rsrc_t br = make_rsrc(a.beta, (uint32_t)((31 * a.beta_h + a.out_o) * 4));
@@ -961,17 +942,11 @@ __global__ __launch_bounds__(kPairThreads, DENSE ? 3 : 4) void hadamard_pair_ker
         for (int j = 0; j < 4; ++j)
             rb[j] = __builtin_amdgcn_raw_buffer_load_b32(br, i0 + j < a.out_o ? (uint32_t)(g * a.beta_h + i0 + j) * 4 : kOOB,
                                                          0, 0);
-        for (int c = tid; c < 256; c += kPairThreads) {
-            float val[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) val[j] = (float)((int)(((uint32_t)c >> (6 - 2 * j)) & 3u) - 1);
-            lut[c] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-        }
         f32x4 va, vb;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             va[j] = (i0 + j < a.in_o) ? (a.alpha ? __uint_as_float(ra[j]) : 1.f) : 0.f;
-            vb[j] = (i0 + j < a.out_o) ? __uint_as_float(rb[j]) * 0.03125f : 0.f;
+            vb[j] = (i0 + j < a.out_o) ? __uint_as_float(rb[j]) * (DENSE ? kTransformScale : kCodeScale) : 0.f;
         }
         alpha_l[e] = va;
         beta_l[e] = vb;
@@ -983,8 +958,8 @@ __global__ __launch_bounds__(kPairThreads, DENSE ? 3 : 4) void hadamard_pair_ker
     const int n_tiles = (int)ceil_div(a.M, kTile);
     const int nb = (int)gridDim.x / an.n;
     for (int tile = slot; tile < n_tiles; tile += nb) {
-        if (hf == 0) pair_tile<0, DENSE>(a, tile, lane, lut, alpha_l, beta_l, xch, xr, yr);
-        else pair_tile<1, DENSE>(a, tile, lane, lut, alpha_l, beta_l, xch, xr, yr);
+        if (hf == 0) pair_tile<0, DENSE>(a, tile, lane, alpha_l, beta_l, xch, xr, yr);
+        else pair_tile<1, DENSE>(a, tile, lane, alpha_l, beta_l, xch, xr, yr);
     }
 }
 
@@ -1003,7 +978,7 @@ template <> struct XElem<true> { typedef uint2 type; };
 template <> struct XElem<false> { typedef f32x4 type; };
 
 template <bool BF16MMA> constexpr size_t wide_lds_bytes() {
-    return (size_t)lut_bytes<BF16MMA>() + (size_t)kWideWaves * 128 * 16 +
+    return (size_t)kWideWaves * 128 * 16 +
            (size_t)wide_stage<BF16MMA>() * 32 * 64 * sizeof(typename XElem<BF16MMA>::type);
 }
 
@@ -1020,22 +995,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int S = wide_stage<BF16MMA>();
     typedef typename XElem<BF16MMA>::type XE;
-    void *lut = smem;
-    f32x4 *beta_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());  // [8 local tiles][4][32]
-    XE *xs = (XE *)(beta_l + kWideWaves * 128);             // [S][32 g][64 lanes]
+    f32x4 *beta_l = (f32x4 *)smem;                // [8 local tiles][4][32]
+    XE *xs = (XE *)(beta_l + kWideWaves * 128);   // [S][32 g][64 lanes]
     constexpr uint32_t esz = sizeof(T);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = lane & 15, q = lane >> 4;
-    if (tid < 256) {
-        const uint32_t byte = (uint32_t)tid;
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)((byte >> (6 - 2 * j)) & 3u) - 1);
-        if constexpr (BF16MMA) {
-            ((uint2 *)lut)[byte] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-        } else {
-            ((f32x4 *)lut)[byte] = f32x4{val[0], val[1], val[2], val[3]};
-        }
-    }
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, (uint32_t)((int64_t)a.M * a.ldx * esz));
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, (uint32_t)((int64_t)a.M * a.ldy * esz));
     const int n_tiles = (int)ceil_div(a.M, kTile);
@@ -1046,13 +1009,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
         const bool row_ok = row < a.M;
         const uint32_t xoff = (uint32_t)((int64_t)row * a.ldx * esz);
         const uint32_t yoff = (uint32_t)((int64_t)row * a.ldy * esz);
-        __syncthreads();  // LUT ready / previous item done with beta_l and xs
+        __syncthreads();  // previous item done with beta_l and xs
         for (int e = tid; e < kWideWaves * 128; e += kWideThreads) {
             const int lw = e >> 7, h = e & 31, qq = (e >> 5) & 3;
             const int o0 = kNTile * (nt0 + lw) + 4 * qq;
             f32x4 v;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = (o0 + j < a.out_o) ? a.beta[h * a.out_o + o0 + j] * 0.03125f : 0.f;
+            for (int j = 0; j < 4; ++j) v[j] = (o0 + j < a.out_o) ? a.beta[h * a.out_o + o0 + j] * kCodeScale : 0.f;
             beta_l[e] = v;
         }
         f32x4 acc[32];
@@ -1110,14 +1073,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
                     const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
                     for (int g = 0; g < 32; ++g) {
-                        const uint32_t byte = (wb[g >> 2] >> (8 * (g & 3))) & 0xffu;
                         const XE xg = src[g * 64];
                         if constexpr (BF16MMA) {
-                            const uint2 wa = ((const uint2 *)lut)[byte];
+                            const uint2 wa = codes_bf16x4(wb[g >> 2], g & 3);
                             acc[g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
                                 __builtin_bit_cast(i16x4, wa), __builtin_bit_cast(i16x4, xg), acc[g], 0, 0, 0);
                         } else {
-                            const f32x4 wa = ((const f32x4 *)lut)[byte];
+                            const f32x4 wa = codes_f32x4(wb[g >> 2], g & 3);
 #pragma unroll
                             for (int u = 0; u < 4; ++u)
                                 acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[u], xg[u], acc[g], 0, 0, 0);
@@ -1148,19 +1110,13 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
 //      (the stage's space), which leaves as whole contiguous rows (16 bytes
 //      per lane, 1 KB per wave and store) instead of 32-byte row pieces.
 // The next tile's x is loaded during the last chunk's products and the
-// output phase.  Weight codes are stored 4 per byte in base 3 (byte =
-// sum_j (code_j + 1) 3^j) and expanded through an 81-entry byte -> 4 x bf16
-// table of +-1/32 (the two transforms' 1/sqrt(32)^2, exact in bf16), held in
-// 16 copies, entry-major with one 8-byte copy per lane of a 16-lane group.
-// (A 9-entry table of bf16 pairs in 64 conflict-free copies was measured
-// slower: twice the LDS instructions.)  alpha and beta stay in LDS for the
-// whole launch as fp16 (11-bit significand, 2^-12 relative rounding against
-// the 2^-9 of the bf16 activations): with the 128 KB stage, float32 copies of
-// both would not fit in 160 KB.
-constexpr int kW3Copies = 16;
-constexpr int kW3Entries = 81;
+// output phase.  Weight codes are 8 per group and lane (half a word),
+// expanded in registers (codes_bf16x8); the output multiplies beta by
+// kCodeScale.  alpha and beta stay in LDS for the whole launch as fp16
+// (11-bit significand, 2^-12 relative rounding against the 2^-9 of the bf16
+// activations): with the 128 KB stage, float32 copies of both would not fit
+// in 160 KB.
 constexpr int kW3MaxO = 128;  // in_o and out_o limit
-constexpr size_t kW3LutBytes = (size_t)kW3Entries * kW3Copies * 8;
 constexpr size_t kW3AlphaBytes = (size_t)32 * kW3MaxO * 2;             // [32 g][128 cols] fp16
 constexpr size_t kW3BetaBytes = (size_t)32 * kW3MaxO * 2;              // [8 tiles][32 h][16 o] fp16
 
@@ -1168,41 +1124,37 @@ constexpr int kW3ORow = 32 * kW3MaxO * 2 + 16;                        // output 
 
 static size_t wide3_lds_bytes(int Kc32) {
     const size_t stage = (size_t)Kc32 * 32 * 64 * 16, otile = (size_t)kTile * kW3ORow;
-    return kW3LutBytes + kW3AlphaBytes + kW3BetaBytes + (stage > otile ? stage : otile);
+    return kW3AlphaBytes + kW3BetaBytes + (stage > otile ? stage : otile);
 }
 
-// Base-3 weight layout [Nt][Kc32][64 lanes][32 groups][2] bytes: lane l of
-// (nt, c) holds for group g the bytes of codes
-// W[g, 16nt + l%16, 32c + 8(l/16) + 4h .. +3], h = 0, 1 (40 = four zero codes,
-// used past out_o / in_o).  Packed code 0b11 is never written by the packer;
-// it saturates to +1 here.
+// Weight layout [Nt][Kc32][64 lanes][16 words]: word k of lane l of (nt, c)
+// holds, for the groups g = 2k and 2k + 1, the codes of
+// W[g, 16nt + l%16, 32c + 8(l/16) .. +7] (group 2k + j in pairs 4j .. 4j + 3;
+// zeros past out_o / in_o).
 __global__ void hadamard_prepare3_kernel(const uint8_t *__restrict__ packed, int in_o, int out_o, int Nt, int Kc32,
-                                         uint8_t *__restrict__ kw3) {
-    const int64_t total = (int64_t)Nt * Kc32 * 64 * 64;
+                                         uint32_t *__restrict__ kw3) {
+    const int64_t total = (int64_t)Nt * Kc32 * 64 * 16;
     const int kp4 = (int)ceil_div(in_o, 4);
     for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
          e += (int64_t)gridDim.x * blockDim.x) {
-        const int h = (int)(e & 1);
-        const int g = (int)((e >> 1) & 31);
-        const int lane = (int)((e >> 6) & 63);
-        const int64_t tc = e >> 12;
+        const int k = (int)(e & 15);
+        const int lane = (int)((e >> 4) & 63);
+        const int64_t tc = e >> 10;
         const int c = (int)(tc % Kc32);
         const int nt = (int)(tc / Kc32);
         const int o = kNTile * nt + (lane & 15);
-        const int i0 = 32 * c + 8 * (lane >> 4) + 4 * h;
-        int b = 40;
-        if (o < out_o && i0 < in_o) {
-            const uint32_t p = packed[((int64_t)g * out_o + o) * kp4 + i0 / 4];
-            b = 0;
-            int w3 = 1;
+        uint32_t w = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int d = (int)((p >> (6 - 2 * j)) & 3u);
-                b += (d > 2 ? 2 : d) * w3;
-                w3 *= 3;
+        for (int b8 = 0; b8 < 4; ++b8) {   // group 2k + b8 / 2, columns 4 (b8 % 2) .. +3 of the lane's 8
+            const int i0 = 32 * c + 8 * (lane >> 4) + 4 * (b8 & 1);
+            if (o < out_o && i0 < in_o) {
+                const uint32_t b = packed[((int64_t)(2 * k + (b8 >> 1)) * out_o + o) * kp4 + i0 / 4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    w |= code_bits((b >> (6 - 2 * i)) & 3u) << (14 - 2 * (2 * b8 + (i >> 1)) + 16 * (i & 1));
             }
         }
-        kw3[e] = (uint8_t)b;
+        kw3[e] = w;
     }
 }
 
@@ -1238,31 +1190,20 @@ __device__ __forceinline__ void wide3_transform_x(const u32x2 (&xraw)[32], const
 // layers: strides fixed at compile time), 0 for any other shape.
 // DENSE: dense bf16 weights (the head mixer at head_dim 128) as 16x16x32
 // A fragments [Nt][Kc32][32 g][64 lanes] x 16 bytes, streamed from global
-// memory a few groups ahead of their products, instead of the code table.
+// memory a few groups ahead of their products, instead of codes.
 template <int GS, bool DENSE = false>
 __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide3_kernel(HadArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint2 *lut = (uint2 *)smem;                                          // [81 entries][16 copies]
-    _Float16 *alpha_l = (_Float16 *)(smem + kW3LutBytes);                // [32 g][128 cols]
-    _Float16 *beta_l = (_Float16 *)(smem + kW3LutBytes + kW3AlphaBytes); // [8 tiles][32 h][16 o]
-    uint4 *xs = (uint4 *)(smem + kW3LutBytes + kW3AlphaBytes + kW3BetaBytes);  // [Kc32][32 g][64 lanes]
+    _Float16 *alpha_l = (_Float16 *)smem;                                // [32 g][128 cols]
+    _Float16 *beta_l = (_Float16 *)(smem + kW3AlphaBytes);               // [8 tiles][32 h][16 o]
+    uint4 *xs = (uint4 *)(smem + kW3AlphaBytes + kW3BetaBytes);          // [Kc32][32 g][64 lanes]
     unsigned char *ostage = (unsigned char *)xs;  // after the products: the output tile
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = lane & 15, q = lane >> 4;
-    for (int e = tid; e < (DENSE ? 0 : kW3Entries * kW3Copies); e += kWideThreads) {
-        int r = e / kW3Copies;
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            val[j] = (float)(r % 3 - 1) * 0.03125f;
-            r /= 3;
-        }
-        lut[e] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-    }
     for (int e = tid; e < 32 * kW3MaxO; e += kWideThreads) {
         const int g = e / kW3MaxO, i = e % kW3MaxO;
-        // the two transforms' 1/32 rides on the code table; dense weights
-        // carry no such factor, so it goes on alpha (exact: a power of two)
-        const float a32 = DENSE ? 0.03125f : 1.f;
+        // dense weights: the two transforms' 1/32 goes on alpha (exact: a
+        // power of two); ternary codes: kCodeScale at the output
+        const float a32 = DENSE ? kTransformScale : 1.f;
         alpha_l[e] = (_Float16)(i < a.in_o ? (a.alpha ? a.alpha[g * a.in_o + i] : 1.f) * a32 : 0.f);
         const int o = kNTile * (e >> 9) + (e & 15), h = (e >> 4) & 31;  // e = (nt*32 + h)*16 + o%16
         beta_l[e] = (_Float16)(o < a.out_o ? a.beta[h * a.beta_h + o] : 0.f);
@@ -1271,7 +1212,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide3_kernel(HadArgs
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, (uint32_t)((int64_t)a.M * a.ldy * 2));
     const int n_tiles = (int)ceil_div(a.M, kTile);
     const int Kc32 = (a.in_o + 31) >> 5;
-    const uint2 *lut_l = lut + (lane & 15);
     const uint32_t gstride = (uint32_t)(GS ? GS : a.gsx) * 2;
     // this wave's transform columns and their place in the stage
     const int i0 = 16 * wave + 4 * q;
@@ -1338,13 +1278,11 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide3_kernel(HadArgs
                 const uint4 *xsrc = xs + (size_t)c * 32 * 64 + lane;
 #pragma unroll
                 for (int g = 0; g < 32; ++g) {
-                    const uint32_t word = w[g >> 3][(g >> 1) & 3] >> (16 * (g & 1));
-                    const uint2 lo = lut_l[(word & 0xffu) * kW3Copies];
-                    const uint2 hi = lut_l[((word >> 8) & 0xffu) * kW3Copies];
+                    const uint4 wa = codes_bf16x8(w[g >> 3][(g >> 1) & 3], g & 1);
                     const uint4 xb = xsrc[g * 64];
-                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                        __builtin_bit_cast(bf16x8, uint4{lo.x, lo.y, hi.x, hi.y}), __builtin_bit_cast(bf16x8, xb),
-                        acc[g], 0, 0, 0);
+                    acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wa),
+                                                                     __builtin_bit_cast(bf16x8, xb), acc[g], 0, 0, 0);
+                    if ((g & 7) == 7) __builtin_amdgcn_sched_barrier(0);   // bounds the expansions in flight
                 }
             };
             uint4 w[4];
@@ -1385,7 +1323,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide3_kernel(HadArgs
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const _Float16 *b = (const _Float16 *)&b8[j];
-                    f32x4 r = acc[h0 + j] * f32x4{(float)b[0], (float)b[1], (float)b[2], (float)b[3]};
+                    f32x4 r = acc[h0 + j] * (f32x4{(float)b[0], (float)b[1], (float)b[2], (float)b[3]} *
+                                             (DENSE ? 1.f : kCodeScale));
                     if (rope) r = rope_apply(r, cs);
                     *(uint2 *)(od + (h0 + j) * kW3MaxO * 2) = uint2{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
                 }
@@ -1434,7 +1373,7 @@ constexpr size_t kSplitBetaBytes = (size_t)32 * kNTile * 2;  // [32 h][16 o] fp1
 
 static size_t split3_lds_bytes(int Kc32) {
     const size_t stage = (size_t)Kc32 * 32 * 64 * 16, part = (size_t)32 * 64 * 16;
-    return kW3LutBytes + kW3AlphaBytes + kSplitBetaBytes + (stage > part ? stage : part);
+    return kW3AlphaBytes + kSplitBetaBytes + (stage > part ? stage : part);
 }
 
 // Grid: x = token tile * Nt + output tile, y = layer of `an`.  GS and DENSE
@@ -1443,10 +1382,9 @@ template <int GS, bool DENSE>
 __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArgsN an) {
     extern __shared__ __align__(16) unsigned char smem[];
     const HadArgs a = load_args(an.p[blockIdx.y]);
-    uint2 *lut = (uint2 *)smem;                                           // [81 entries][16 copies]
-    _Float16 *alpha_l = (_Float16 *)(smem + kW3LutBytes);                 // [32 g][128 cols]
-    _Float16 *beta_l = (_Float16 *)(smem + kW3LutBytes + kW3AlphaBytes);  // [32 h][16 o] of this tile
-    uint4 *xs = (uint4 *)(smem + kW3LutBytes + kW3AlphaBytes + kSplitBetaBytes);  // [Kc32][32 g][64 lanes]
+    _Float16 *alpha_l = (_Float16 *)smem;                   // [32 g][128 cols]
+    _Float16 *beta_l = (_Float16 *)(smem + kW3AlphaBytes);  // [32 h][16 o] of this tile
+    uint4 *xs = (uint4 *)(smem + kW3AlphaBytes + kSplitBetaBytes);  // [Kc32][32 g][64 lanes]
     f32x4 *part = (f32x4 *)xs;  // after the products: [32 g][64 lanes]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = lane & 15, q = lane >> 4;
     const int nt = (int)blockIdx.x % a.Nt, tile = (int)blockIdx.x / a.Nt;
@@ -1505,7 +1443,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArg
     // (buffer loads, zero past their ranges, and no arithmetic on the loaded
     // values until they are used: a conversion right after a load would wait
     // for every load before it)
-    const float a32 = DENSE ? 0.03125f : 1.f;  // the dense weights' share of the transforms' 1/32
+    const float a32 = DENSE ? kTransformScale : 1.f;  // the dense weights' share of the transforms' 1/32
     constexpr int kAv = 32 * kW3MaxO / kWideThreads;
     uint32_t avr[kAv];
     {
@@ -1559,16 +1497,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArg
         csr = __builtin_amdgcn_raw_buffer_load_b64(rr, off, 0, 0);
     }
 
-    for (int e = tid; e < (DENSE ? 0 : kW3Entries * kW3Copies); e += kWideThreads) {
-        int r = e / kW3Copies;
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            val[j] = (float)(r % 3 - 1) * 0.03125f;
-            r /= 3;
-        }
-        lut[e] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-    }
 #pragma unroll
     for (int k = 0; k < kAv; ++k) {
         const int i = (tid + k * kWideThreads) % kW3MaxO;
@@ -1617,7 +1545,6 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArg
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const uint4 *xsrc = xs + 4 * wave * 64 + lane;
-    const uint2 *lut_l = lut + (lane & 15);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         if (c < Kc32) {
@@ -1627,10 +1554,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArg
                 if constexpr (DENSE) {
                     wa = wd[c][j];
                 } else {
-                    const uint32_t word = (j < 2 ? wv[c].x : wv[c].y) >> (16 * (j & 1));
-                    const uint2 lo = lut_l[(word & 0xffu) * kW3Copies];
-                    const uint2 hi = lut_l[((word >> 8) & 0xffu) * kW3Copies];
-                    wa = uint4{lo.x, lo.y, hi.x, hi.y};
+                    wa = codes_bf16x8(j < 2 ? wv[c].x : wv[c].y, j & 1);
                 }
                 const uint4 xb = xsrc[(c * 32 + j) * 64];
                 acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wa),
@@ -1658,7 +1582,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_split3_kernel(HadArg
 #pragma unroll
     for (int hi = 0; hi < 16; ++hi) {
         const int h = h0 + hi;
-        float r = (h0 ? v[16 + hi] : v[hi]) * (float)beta_l[h * kNTile + o16];
+        float r = (h0 ? v[16 + hi] : v[hi]) * ((float)beta_l[h * kNTile + o16] * (DENSE ? 1.f : kCodeScale));
         if (rope) {
             // the other element of the pair (lane ^ 1, a DPP quad permutation)
             const float p = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(r), 0xB1, 0xF, 0xF, true));
@@ -1699,28 +1623,13 @@ template <typename T, bool BF16MMA, bool VEC, bool KC1>
 __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_swiglu_kernel(HadArgs g, HadArgs u) {
     extern __shared__ __align__(16) unsigned char smem[];
     typedef typename Stash<BF16MMA>::type SType;
-    void *lut = smem;
-    f32x4 *ag_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());
+    f32x4 *ag_l = (f32x4 *)smem;
     f32x4 *au_l = ag_l + g.Kc * 128;
     f32x4 *bg_l = au_l + g.Kc * 128;
     f32x4 *bu_l = bg_l + g.Nt * 128;
     SType *stash = (SType *)(bu_l + g.Nt * 128);     // [kWaves][32][64]
 
     const int tid = threadIdx.x;
-    {
-        const uint32_t byte = (uint32_t)tid;
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)((byte >> (6 - 2 * j)) & 3u) - 1);
-        if constexpr (BF16MMA) {
-            uint2 e;
-            e.x = pack_bf16x2(val[0], val[1]);
-            e.y = pack_bf16x2(val[2], val[3]);
-            ((uint2 *)lut)[byte] = e;
-        } else {
-            ((f32x4 *)lut)[byte] = f32x4{val[0], val[1], val[2], val[3]};
-        }
-    }
     for (int e = tid; e < g.Kc * 128; e += kThreads) {
         const int gg = e & 31, i0 = 4 * (e >> 5);
         f32x4 va, vb;
@@ -1739,8 +1648,8 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const bool ok = o0 + j < g.out_o;
-            va[j] = ok ? g.beta[h * g.out_o + o0 + j] * 0.03125f : 0.f;
-            vb[j] = ok ? u.beta[h * g.out_o + o0 + j] * 0.03125f : 0.f;
+            va[j] = ok ? g.beta[h * g.out_o + o0 + j] * kCodeScale : 0.f;
+            vb[j] = ok ? u.beta[h * g.out_o + o0 + j] * kCodeScale : 0.f;
         }
         bg_l[e] = va;
         bu_l[e] = vb;
@@ -1775,14 +1684,14 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
             load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, 0, q, ag_l, xm);
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-            contract<BF16MMA>(g, nt, 0, lane, xm, lut, acc);
+            contract<BF16MMA>(g, nt, 0, lane, xm, acc);
         } else {
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int c = 0; c < g.Kc; ++c) {
                 XM<BF16MMA> xm;
                 load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, c, q, ag_l, xm);
-                contract<BF16MMA>(g, nt, c, lane, xm, lut, acc);
+                contract<BF16MMA>(g, nt, c, lane, xm, acc);
             }
         }
         fht32x4(acc);
@@ -1817,14 +1726,14 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
             load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, 0, q, au_l, xm);
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-            contract<BF16MMA>(u, nt, 0, lane, xm, lut, acc);
+            contract<BF16MMA>(u, nt, 0, lane, xm, acc);
         } else {
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int c = 0; c < g.Kc; ++c) {
                 XM<BF16MMA> xm;
                 load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, c, q, au_l, xm);
-                contract<BF16MMA>(u, nt, c, lane, xm, lut, acc);
+                contract<BF16MMA>(u, nt, c, lane, xm, acc);
             }
         }
         fht32x4(acc);
@@ -1901,9 +1810,8 @@ constexpr int kMlpDownWave = 3;
 
 __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, HadArgs u, HadArgs d) {
     extern __shared__ __align__(16) unsigned char smem[];
-    void *lut = smem;
     const int Nt = g.Nt;                                  // hidden tiles = down chunks (2 or 3)
-    f32x4 *ag_l = (f32x4 *)(smem + lut_bytes<true>());   // [1][4][32]
+    f32x4 *ag_l = (f32x4 *)smem;                          // [1][4][32]
     f32x4 *au_l = ag_l + 128;
     f32x4 *bg_l = au_l + 128;                             // [Nt][4][32]
     f32x4 *bu_l = bg_l + Nt * 128;
@@ -1912,13 +1820,6 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
     uint2 *areas = (uint2 *)(bd_l + 128);                 // [3][32][64]
 
     const int tid = threadIdx.x;
-    {
-        const uint32_t byte = (uint32_t)tid;
-        float val[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) val[j] = (float)((int)((byte >> (6 - 2 * j)) & 3u) - 1);
-        ((uint2 *)lut)[byte] = uint2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
-    }
     // alpha / beta of the three layers: every load issued before any
     // conversion (buffer loads, zero past the shapes, no branch around them;
     // a conversion or branch right after a load waits for it)
@@ -1964,7 +1865,7 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
                 const bool ok = i0 + j < g.in_o;
                 va[j] = ok ? __uint_as_float(r1[0][j]) : 0.f;
                 vb[j] = ok ? __uint_as_float(r1[1][j]) : 0.f;
-                vd[j] = i0 + j < d.out_o ? __uint_as_float(r1[2][j]) * 0.03125f : 0.f;
+                vd[j] = i0 + j < d.out_o ? __uint_as_float(r1[2][j]) * kCodeScale : 0.f;
             }
             ag_l[e] = va;
             au_l[e] = vb;
@@ -1978,8 +1879,8 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const bool ok = o0 + j < g.out_o;
-                va[j] = ok ? __uint_as_float(r2[it][0][j]) * 0.03125f : 0.f;
-                vb[j] = ok ? __uint_as_float(r2[it][1][j]) * 0.03125f : 0.f;
+                va[j] = ok ? __uint_as_float(r2[it][0][j]) * kCodeScale : 0.f;
+                vb[j] = ok ? __uint_as_float(r2[it][1][j]) * kCodeScale : 0.f;
                 vd[j] = o0 + j < d.in_o ? __uint_as_float(r2[it][2][j]) : 0.f;  // chunk e / 128, element (h, o0 + j)
             }
             bg_l[e] = va;
@@ -2009,7 +1910,7 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
                 load_transform<uint16_t, true, true>(g, xr, xoff, row_ok, 0, q, ag_l, xm);
 #pragma unroll
                 for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(g, nt, 0, lane, xm, lut, acc);
+                contract<true>(g, nt, 0, lane, xm, acc);
             }
             fht32x4(acc);
             {
@@ -2033,7 +1934,7 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
                 load_transform<uint16_t, true, true>(g, xr, xoff, row_ok, 0, q, au_l, xm);
 #pragma unroll
                 for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(u, nt, 0, lane, xm, lut, acc);
+                contract<true>(u, nt, 0, lane, xm, acc);
             }
             __builtin_amdgcn_sched_barrier(0);
             fht32x4(acc);
@@ -2093,7 +1994,7 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
                 const uint2 *st = areas + c * 32 * 64;
 #pragma unroll
                 for (int h = 0; h < 32; ++h) xm.b[h] = st[h * 64 + lane];
-                contract<true>(d, 0, c, lane, xm, lut, acc);
+                contract<true>(d, 0, c, lane, xm, acc);
             }
             lds_barrier();  // B
             transform_store<uint16_t, true>(d, acc, yr, (uint32_t)((int64_t)row * d.ldy * 2), row_ok, 0, q, bd_l,
@@ -2195,15 +2096,13 @@ __global__ void hadamard_dense_prepare_kernel(const float *__restrict__ w, int i
     }
 }
 
-static size_t hadamard_lds_bytes(bool bf16, int Kc, int Nt) {
-    return (bf16 ? lut_bytes<true>() : lut_bytes<false>()) + (size_t)16 * 128 * (Kc + Nt);
-}
+static size_t hadamard_lds_bytes(int Kc, int Nt) { return (size_t)16 * 128 * (Kc + Nt); }
 
 }  // namespace walsh
 
 using namespace walsh;
 
-// Shapes that also get the base-3 layout of the wide bf16 kernel.
+// Shapes that also get the 32-column layout of the wide bf16 kernel.
 static bool wide3_shape(int64_t in_o, int64_t out_o) {
     return in_o > kKChunk && in_o <= kW3MaxO && out_o <= kW3MaxO;
 }
@@ -2212,7 +2111,7 @@ static int64_t weight_bytes1(int64_t in_o, int64_t out_o) {
     return ceil_div(out_o, kNTile) * ceil_div(in_o, kKChunk) * 64 * 32;
 }
 
-// The first layout, followed by the base-3 one for wide3_shape.
+// The first layout, followed by the 32-column one for wide3_shape.
 WALSH_EXPORT int64_t walsh_hadamard_weight_bytes(int64_t in_o, int64_t out_o) {
     if (in_o <= 0 || out_o <= 0) return 0;
     int64_t n = weight_bytes1(in_o, out_o);
@@ -2227,19 +2126,19 @@ WALSH_EXPORT int walsh_hadamard_prepare(const uint8_t *packed, int64_t in_o, int
         return set_error(WALSH_EINVAL, "walsh_hadamard_prepare: bad shape in_o=%lld out_o=%lld", (long long)in_o,
                          (long long)out_o);
     const int Nt = (int)ceil_div(out_o, kNTile), Kc = (int)ceil_div(in_o, kKChunk);
-    const int64_t total = (int64_t)Nt * Kc * 2048;
+    const int64_t total = (int64_t)Nt * Kc * 512;   // words
     const int block = 256;
     int grid = (int)ceil_div(total, block);
     if (grid > 4096) grid = 4096;
     launch(hadamard_prepare_kernel, dim3(grid), dim3(block), 0, (hipStream_t)stream, packed, (int)in_o,
-                       (int)out_o, Nt, Kc, kweight);
+                       (int)out_o, Nt, Kc, (uint32_t *)kweight);
     if (wide3_shape(in_o, out_o)) {
         const int Kc32 = (int)ceil_div(in_o, 32);
-        const int64_t total3 = (int64_t)Nt * Kc32 * 4096;
+        const int64_t total3 = (int64_t)Nt * Kc32 * 1024;   // words
         int grid3 = (int)ceil_div(total3, block);
         if (grid3 > 4096) grid3 = 4096;
         launch(hadamard_prepare3_kernel, dim3(grid3), dim3(block), 0, (hipStream_t)stream, packed, (int)in_o,
-               (int)out_o, Nt, Kc32, kweight + weight_bytes1(in_o, out_o));
+               (int)out_o, Nt, Kc32, (uint32_t *)(kweight + weight_bytes1(in_o, out_o)));
     }
     return check_hip(hipGetLastError(), "walsh_hadamard_prepare launch");
 }
@@ -2293,14 +2192,15 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
     const int64_t esz = bf16 ? 2 : 4;
     const int Nt = base.Nt, Kc = base.Kc;
     const bool swiglu = ubase != nullptr;
-    size_t lds = hadamard_lds_bytes(bf16, Kc, Nt);
+    size_t lds = hadamard_lds_bytes(Kc, Nt);
     // SwiGLU: the up projection's alpha / beta tables and, per working wave,
     // the gate output (32 groups x 64 lanes x 4 values)
     const size_t stash_wave = (size_t)32 * 64 * (bf16 ? 8 : 16);
     if (swiglu) lds += (size_t)16 * 128 * (Kc + Nt);
-    if (lds + (swiglu ? kWaves * stash_wave : 0) > (size_t)device_info().max_shared_per_block)
+    const size_t limit = device_info().max_shared_per_block - shape_reserve(bf16);
+    if (lds + (swiglu ? kWaves * stash_wave : 0) > limit)
         return set_error(WALSH_ENOTSUP, "%s: in_o=%d out_o=%d need %zu B of LDS", fn, base.in_o, base.out_o,
-                         lds + (swiglu ? kWaves * stash_wave : 0));
+                         lds + (swiglu ? kWaves * stash_wave : 0) + shape_reserve(bf16));
     const size_t valign = bf16 ? 8 : 16;
     const bool vec = (base.gsx % 4 == 0) && (base.ldx % 4 == 0) && ((uintptr_t)base.x % valign == 0) &&
                      (base.gsy % 4 == 0) && (base.ldy % 4 == 0) && ((uintptr_t)base.y % valign == 0);
@@ -2310,7 +2210,7 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
     // several input chunks and output tiles: the workgroup-wide kernel
     const size_t wide_lds = bf16 ? wide_lds_bytes<true>() : wide_lds_bytes<false>();
     const bool wide = !swiglu && vec && Kc >= 2 && Nt >= 4 && wide_lds <= (size_t)device_info().max_shared_per_block;
-    // bf16 with in_o <= 128 and out_o <= 128: the base-3 16x16x32 kernel
+    // bf16 with in_o <= 128 and out_o <= 128: the 16x16x32 kernel
     const size_t wide3_lds = wide3_lds_bytes((base.in_o + 31) / 32);
     const bool wide3 = wide && bf16 && base.kw3 != nullptr && wide3_lds <= (size_t)device_info().max_shared_per_block;
     const int64_t ld = base.ldx > base.ldy ? base.ldx : base.ldy;
@@ -2538,7 +2438,7 @@ static int hadamard_multi(const char *fn, const void *x, int64_t ldx, int64_t M,
         if (ldys[i] > ldy) ldy = ldys[i];
     }
     const bool kc1 = Kc == 1 && (bf16 || Nt == 1);
-    const size_t lds = hadamard_lds_bytes(bf16, Kc, Nt);
+    const size_t lds = hadamard_lds_bytes(Kc, Nt);
     hipStream_t s = (hipStream_t)stream;
     const int64_t ld = ldx > ldy ? ldx : ldy;
     if (bf16 && vec && base[0].kw3 && Kc >= 2 && Nt >= 4 && M <= kSplitRows &&
@@ -2664,7 +2564,7 @@ WALSH_EXPORT int walsh_hadamard_mlp_fwd(const void *x, int64_t ldx, int64_t M, i
     HadArgs ua = had_args(x, ldx, in_o, in_o, hid_o, kw_up, alpha_up, beta_up, nullptr, 0, hid_o);
     HadArgs da = had_args(nullptr, 0, hid_o, hid_o, out_o, kw_down, alpha_down, beta_down, y, ldy, out_o);
     const int Nt = ga.Nt;
-    const size_t lds = lut_bytes<true>() + (size_t)16 * 128 * (2 + 3 * Nt + 1) + (size_t)3 * 32 * 64 * 8;
+    const size_t lds = (size_t)16 * 128 * (2 + 3 * Nt + 1) + (size_t)3 * 32 * 64 * 8;
     if (lds > (size_t)device_info().max_shared_per_block)
         return set_error(WALSH_ENOTSUP, "%s: needs %zu B of LDS", fn, lds);
     const int64_t ld = ldx > ldy ? ldx : ldy;

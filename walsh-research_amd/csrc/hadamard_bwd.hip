@@ -88,21 +88,6 @@ __device__ __forceinline__ void fill_scale(f32x4 *__restrict__ dst, const float 
     }
 }
 
-__device__ __forceinline__ void fill_lut(void *lut, bool bf16, int tid) {
-    const uint32_t byte = (uint32_t)tid;  // 256 threads, 256 entries
-    float val[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) val[j] = (float)((int)((byte >> (6 - 2 * j)) & 3u) - 1);
-    if (bf16) {
-        uint2 e;
-        e.x = pack_bf16x2(val[0], val[1]);
-        e.y = pack_bf16x2(val[2], val[3]);
-        ((uint2 *)lut)[byte] = e;
-    } else {
-        ((f32x4 *)lut)[byte] = f32x4{val[0], val[1], val[2], val[3]};
-    }
-}
-
 // ---------------------------------------------------------------- reduce-epilogue pass
 
 struct BwdRed {
@@ -115,13 +100,11 @@ struct BwdRed {
 
 template <typename T, bool BF16MMA, bool VEC, bool STORE>
 __device__ __forceinline__ void bwd_red_role(const HadArgs &a, const BwdRed &r, int blk, unsigned char *smem) {
-    void *lut = smem;
-    f32x4 *alpha_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());
+    f32x4 *alpha_l = (f32x4 *)smem;
     f32x4 *beta_l = alpha_l + a.Kc * 128;
     const int tid = threadIdx.x;
-    fill_lut(lut, BF16MMA, tid);
     fill_scale(alpha_l, a.alpha, a.in_o, a.Kc, 1.f, tid, kThreads);
-    if (STORE) fill_scale(beta_l, a.beta, a.out_o, a.Nt, 0.03125f, tid, kThreads);
+    if (STORE) fill_scale(beta_l, a.beta, a.out_o, a.Nt, kCodeScale, tid, kThreads);
     __syncthreads();
 
     constexpr uint32_t esz = sizeof(T);
@@ -152,7 +135,7 @@ __device__ __forceinline__ void bwd_red_role(const HadArgs &a, const BwdRed &r, 
         for (int c = 0; c < a.Kc; ++c) {
             XM<BF16MMA> xm;
             load_transform<T, BF16MMA, VEC>(a, xr, xoff, row_ok, c, q, alpha_l, xm);
-            contract<BF16MMA>(a, nt, c, lane, xm, lut, acc);
+            contract<BF16MMA>(a, nt, c, lane, xm, acc);
         }
         fht32x4(acc);
         const uint32_t aoff = (uint32_t)((int64_t)row * r.ld_aux * esz);
@@ -390,7 +373,8 @@ __global__ __launch_bounds__(kSumCols * kSumPhases) void hadamard_bwd_reduce_ker
     double tot = 0.0;
 #pragma unroll
     for (int p = 0; p < kSumPhases; ++p) tot += part[p][cx];
-    const float v = (float)(tot * 0.03125);
+    // dalpha and dbeta come out of the ternary contraction, dW does not
+    const float v = (float)(tot * (kind == 0 ? kTransformScale : kCodeScale));
     if (kind == 0) {
         const int i = (int)(n % r.Ip);
         const int64_t go = n / r.Ip;
@@ -531,13 +515,12 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     float *pw = (float *)((char *)workspace + L.off_w);
     const size_t valign = bf16 ? 8 : 16;
     const int64_t maxlds = device_info().max_shared_per_block;
-    auto lut = [&](void) { return (size_t)(bf16 ? lut_bytes<true>() : lut_bytes<false>()); };
 
     int64_t ia = 0, ib = 0, iw = 0;  // partial rows written so far
-    const size_t lds_red = lut() + (size_t)16 * 128 * (Nt + Kc);
+    const size_t lds_red = (size_t)16 * 128 * (Nt + Kc);
     const size_t lds_dw = (size_t)16 * 128 * (Nt + Kc) + (size_t)32 * 64 * 16;
     const size_t lds = need_w && lds_dw > lds_red ? lds_dw : lds_red;
-    if ((int64_t)lds > maxlds) return set_error(WALSH_ENOTSUP, "%s: shape needs %zu B of LDS", fn, lds);
+    if ((int64_t)(lds_red + shape_reserve(bf16)) > maxlds || (int64_t)lds > maxlds) return set_error(WALSH_ENOTSUP, "%s: shape needs %zu B of LDS", fn, lds);
     for (int64_t r0 = 0; r0 < M; r0 += L.rows_max) {
         const int64_t rows = (M - r0) < L.rows_max ? (M - r0) : L.rows_max;
         const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o);

@@ -45,7 +45,7 @@ struct HadArgs {
     int in_o, out_o, Nt, Kc;
     int gsx, gsy;       // group strides of x / y rows (>= in_o / out_o)
     const uint8_t *kw;
-    const uint8_t *kw3;  // base-3 layout (wide bf16 kernel), or null
+    const uint8_t *kw3;  // 32-column layout (wide bf16 kernel), or null
     const float *alpha;  // [32][in_o]; null: all ones
     const float *beta;   // row h of beta at beta + h * beta_h
     int beta_h;          // out_o, or 0 for one beta row shared by all groups
@@ -126,10 +126,50 @@ template <> struct XM<true> { uint2 b[32]; };
 
 // LDS layout (all 16-byte entries, lane-major so each lane walks its 32
 // groups with immediate offsets):
-//   lut     [256]            code byte -> 4 weights (bf16x4 in 8 B, or f32x4)
 //   alpha_l [Kc][4][32]      alpha[g, 16c+4q .. +3]   (0 past in_o)
-//   beta_l  [Nt][4][32]      beta[h, 16nt+4q .. +3]/32 (0 past out_o)
-template <bool BF16MMA> constexpr int lut_bytes() { return BF16MMA ? 256 * 8 : 256 * 16; }
+//   beta_l  [Nt][4][32]      beta[h, 16nt+4q .. +3] * kCodeScale (0 past out_o)
+
+// ---------------------------------------------------------------- weight codes
+// A ternary weight is stored as the top two bits (sign, exponent's high bit)
+// of the float it stands for: 00 = 0, 01 = +2.0 (0x4000 in bf16, 0x40000000
+// in float32), 11 = -2.0.  A 32-bit word holds 16 codes as 8 pairs, pair p at
+// bits (15 - 2p, 14 - 2p) of both halves, so a shift by 2p and one mask give
+// a register with two bf16 weights: two VALU operations per pair, no table.
+// The factor 2 is a power of two and is taken back with the transforms'
+// 1/32 (kCodeScale), exactly.  The former byte -> 4 x bf16 table in LDS cost
+// a conflicting 8-byte read per lane and 4 weights, a build loop per launch
+// and 2 to 10 KB of LDS.  Measured, outputs bitwise equal: the chunk-loop
+// SwiGLU and down projection at n_embd 768, 6,007 rows 108.3 -> 103.3 us;
+// the launches bound elsewhere (n_embd 4096 linear, 16,384 rows 104.8 ->
+// 104.6 us) keep their time.
+constexpr uint32_t kCodeMask = 0xC000C000u;
+constexpr float kCodeScale = 0.015625f;      // 1/32 of the two transforms, 1/2 of the +-2.0 weights
+constexpr float kTransformScale = 0.03125f;  // the two transforms alone (dense weights)
+
+// LDS that the entry points' shape limits keep free (the size of the code
+// table those limits were set with), so the accepted shapes stay the same.
+__host__ inline size_t shape_reserve(bool bf16) { return bf16 ? 2048 : 4096; }
+
+// Code bits of packed code v (0, 1, 2 for -1, 0, +1; 3 is never written by
+// the packer and counts as +1).
+__host__ __device__ __forceinline__ uint32_t code_bits(uint32_t v) { return v == 0 ? 3u : (v == 1 ? 0u : 1u); }
+
+// 4 weights (pairs 2k, 2k + 1) of a word: one group of a 16-column chunk.
+__device__ __forceinline__ uint2 codes_bf16x4(uint32_t w, int k) {
+    return uint2{(w << (4 * k)) & kCodeMask, (w << (4 * k + 2)) & kCodeMask};
+}
+__device__ __forceinline__ f32x4 codes_f32x4(uint32_t w, int k) {
+    f32x4 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        r[j] = __uint_as_float((w << (4 * k + 2 * (j >> 1) + ((j & 1) ? 0 : 16))) & 0xC0000000u);
+    return r;
+}
+// 8 weights (pairs 4k .. 4k + 3): one group of a 32-column chunk.
+__device__ __forceinline__ uint4 codes_bf16x8(uint32_t w, int k) {
+    return uint4{(w << (8 * k)) & kCodeMask, (w << (8 * k + 2)) & kCodeMask, (w << (8 * k + 4)) & kCodeMask,
+                 (w << (8 * k + 6)) & kCodeMask};
+}
 
 // The lane's 4 columns 16c+4q.. of all 32 groups of its row (zeros past
 // in_o / M).
@@ -180,27 +220,25 @@ __device__ __forceinline__ void load_transform(const HadArgs &a, __amdgpu_buffer
 }
 
 template <bool BF16MMA>
-__device__ __forceinline__ void contract_w(uint4 w0, uint4 w1, const XM<BF16MMA> &xm, const void *__restrict__ lut,
-                                           f32x4 (&acc)[32]) {
+__device__ __forceinline__ void contract_w(uint4 w0, uint4 w1, const XM<BF16MMA> &xm, f32x4 (&acc)[32]) {
     const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
     for (int g = 0; g < 32; ++g) {
-        const uint32_t byte = (wb[g >> 2] >> (8 * (g & 3))) & 0xffu;
         if constexpr (BF16MMA) {
-            const uint2 wa = ((const uint2 *)lut)[byte];
+            const uint2 wa = codes_bf16x4(wb[g >> 2], g & 3);
             acc[g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, wa),
                                                                 __builtin_bit_cast(i16x4, xm.b[g]), acc[g], 0, 0, 0);
         } else {
-            const f32x4 wa = ((const f32x4 *)lut)[byte];
+            const f32x4 wa = codes_f32x4(wb[g >> 2], g & 3);
 #pragma unroll
             for (int s = 0; s < 4; ++s)
                 acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[s], xm.v[g][s], acc[g], 0, 0, 0);
         }
-        if ((g & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+        if ((g & 1) == 1) __builtin_amdgcn_sched_barrier(0);  // no expansion is hoisted
     }
 }
 
-// The lane's 32 code bytes of weight tile (nt, c).
+// The lane's 8 code words of weight tile (nt, c).
 __device__ __forceinline__ void load_w(const HadArgs &a, int nt, int c, int lane, uint4 &w0, uint4 &w1) {
     const uint4 *src = (const uint4 *)(a.kw + (((int64_t)nt * a.Kc + c) * 64 + lane) * 32);
     w0 = src[0];
@@ -209,10 +247,10 @@ __device__ __forceinline__ void load_w(const HadArgs &a, int nt, int c, int lane
 
 template <bool BF16MMA>
 __device__ __forceinline__ void contract(const HadArgs &a, int nt, int c, int lane, const XM<BF16MMA> &xm,
-                                         const void *__restrict__ lut, f32x4 (&acc)[32]) {
+                                         f32x4 (&acc)[32]) {
     uint4 w0, w1;
     load_w(a, nt, c, lane, w0, w1);
-    contract_w<BF16MMA>(w0, w1, xm, lut, acc);
+    contract_w<BF16MMA>(w0, w1, xm, acc);
 }
 
 // Output transform of a 16x16 tile (skipped with FHT = false when the caller
