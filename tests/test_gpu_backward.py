@@ -358,6 +358,48 @@ def test_moe_backward_matches_oracle(C, k, T):
         assert err <= 1e-5 * nb + 1e-6 * G, (n, err, nb)
 
 
+@pytest.mark.parametrize("M,E,k,H,pad", [(1, 16, 1, 128, 0), (16, 1, 1, 128, 0), (17, 2, 2, 64, 1), (33, 4, 2, 48, 3),
+                                         (530, 16, 6, 128, 4), (1100, 2, 1, 128, 0)])
+def test_moe_experts_bwd_tiles(K, M, E, k, H, pad):
+    """walsh_moe_experts_bwd at the edges of its 16-pair tiles (one pair, a
+    full tile, one more, experts without pairs, several tiles per wavefront),
+    hidden sizes on both instantiations and past a tile pair, rows with and
+    without 16-byte alignment, against the float64 formulas on the same
+    codes.  Bar: float32 sums of up to 1,100 products, 1e-5."""
+    g = torch.Generator().manual_seed(M + H)
+    lat = [torch.rand(sh, generator=g) * 2 - 1 for sh in ((E, H, 32), (E, H, 32), (E, 32, H))]
+    qs = [K.ternary_quantize(w.cuda(), codes=True, packed=True) for w in lat]
+    gammas = torch.cat([q["gamma"] for q in qs])
+    W = [q["codes"].double().cpu().reshape(w.shape) * float(q["gamma"]) for q, w in zip(qs, lat)]
+    x = torch.randn(M, 32 * E + pad, generator=g)[:, :32 * E]
+    # small enough that the STE's +-2 clamp leaves the sums alone (clamped, the
+    # largest value left would be 2 and the bar would be on cancelled sums)
+    do = torch.randn(M, 32 * E + pad, generator=g)[:, :32 * E] * 1e-4
+    idx = torch.stack([torch.randperm(E, generator=g)[:k] for _ in range(M)]).sort(-1).values
+    if E > 2:
+        idx = torch.where(idx == E - 1, torch.zeros_like(idx), idx)     # expert E - 1 gets no pair
+        idx = torch.stack([r if len(set(r.tolist())) == k else torch.arange(k) for r in idx])
+    wr = torch.rand(M, k, generator=g)
+    r = K.MoERoute(M, E, k, torch.device("cuda"), dense=False, parts=1)
+    r.topk_idx.copy_(idx)
+    r.topk_w.copy_(wr)
+    r.count_part.copy_(torch.zeros(M, E).scatter_(1, idx, 1.0).sum(0).int().view(1, E))
+    r.probsum_part.zero_()
+    xc = torch.empty(M, 32 * E + pad, device="cuda")[:, :32 * E].copy_(x)
+    dc = torch.empty(M, 32 * E + pad, device="cuda")[:, :32 * E].copy_(do)
+    dx, dpair, (dg, du, dd) = K.moe_experts_bwd(xc, dc, r, K.moe_scatter(r), [q["packed"] for q in qs], gammas, H)
+    leaves = [w.clone().requires_grad_(True) for w in W]
+    x64, w64 = x.double().requires_grad_(True), wr.double().requires_grad_(True)
+    xb = x64.reshape(M, E, 32)
+    o = torch.einsum("meh,edh->med", torch.nn.functional.silu(torch.einsum("med,ehd->meh", xb, leaves[0]))
+                     * torch.einsum("med,ehd->meh", xb, leaves[1]), leaves[2])
+    wd = torch.zeros(M, E, dtype=torch.float64).scatter(1, idx, w64)
+    ref = torch.autograd.grad(((o * wd.unsqueeze(-1)).reshape(M, 32 * E) * do.double()).sum(), [x64, w64] + leaves)
+    ref = list(ref[:2]) + [t.clamp(-2, 2) for t in ref[2:]]
+    for name, a, b in zip(("dx", "dpair", "dgate", "dup", "ddown"), (dx, dpair, dg, du, dd), ref):
+        assert_close(a.cpu().numpy(), b.numpy(), torch.float32, f"experts bwd M={M} E={E} H={H} {name}")
+
+
 def test_moe_checkpointed_backward_equals_plain():
     """Activation checkpointing (non-reentrant, as mHCWalsh's
     gradient_checkpointing uses) recomputes the MoE forward during the

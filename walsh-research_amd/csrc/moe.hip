@@ -23,6 +23,7 @@
 // expert hidden state feeds the down projection without a transpose.
 #include <math.h>
 
+#include "codes.h"
 #include "common.h"
 #include "gemm256.h"
 
@@ -1537,15 +1538,36 @@ __global__ __launch_bounds__(64 * kR1Waves) void moe_decode_kernel(const uint16_
 //   do = dout w;  g = Wg x, u = Wu x, s = silu(g), h = s u, o = Wd h
 //   dw_pair = <dout, o>;  dh = Wd^T do;  dg = dh u silu'(g);  du = dh s
 //   dx = Wg^T dg + Wu^T du;  dWg += dg x^T, dWu += du x^T, dWd += do h^T
-// with W = code * gamma.  A workgroup takes a share of one expert's pairs
-// (S workgroups per expert), two pairs at a time with 128 threads each
-// (thread j owns hidden unit j), the expert's three matrices staged in LDS
-// as float32 and the next pairs' rows prefetched during the current ones;
-// each workgroup writes its weight-gradient sums, which
-// moe_experts_bwd_reduce_kernel adds in workgroup order before the STE clamp.
-constexpr int kEbSlots = 2;
+// with W = code * gamma, all on float32 matrix cores, 16 pairs of one expert
+// at a time.  Operands are arranged so that one 16x16x4 lane layout serves
+// every product (lane (m, q) of a 16-deep operand holds its 4 values at depth
+// 4q .. 4q + 3):
+//   - g, u and dh0 = Wd^T dout as D[pair][hidden] = X W^T: lane (h, q) gets
+//     pairs 4q + j of hidden unit h, which is the layout in which dg, du and
+//     h w enter the weight gradients (depth = the 16 pairs) from registers;
+//   - dx = Wg^T dg + Wu^T du needs dg and du with the hidden units as depth:
+//     one 16x16 transpose each through the wave's LDS area;
+//   - dw_pair = <dout, o> = <dh0, h>: the down product o is not formed.
+// Waves w and w + 4 of a workgroup take the two halves of the hidden units of
+// tile w (96 accumulator registers of weight gradients each, two waves per
+// SIMD, so one's SiLU overlaps the other's products; one wave per tile with
+// all 192 ran 112 us against 607 us for the version before it and is slower
+// than this one); the second half hands its dx and dw_pair sums to the first
+// through LDS.  The codes stay packed in registers and are expanded by shift
+// and mask (codes.h); gamma / 2 goes on the products.  The next tile's rows
+// are requested during the current one's products.
+// The tiles are dealt to the workgroups in proportion to the experts' loads
+// (eb_schedule): routed loads differ by a factor of two and more, and the
+// launch lasts as long as its longest workgroup.
+// Bound by the float32 matrix rate (512 products of 32 clocks per tile) and
+// the SiLU arithmetic.  Measured at 8,192 tokens x 6 of 16 experts, hidden
+// 128: 74 us (607 us for a thread per hidden unit with dot products from
+// LDS).
 constexpr int kEbH = 128;  // hidden units per expert <= 128
-constexpr int kEbThreads = kEbSlots * kEbH;
+constexpr int kEbMaxE = 128;
+static_assert(kEbMaxE >= kMaxE, "experts");
+constexpr int kEbSlots = 4, kEbThreads = 2 * 64 * kEbSlots;  // tiles in flight, two waves each
+constexpr int kEbPitch = 20;  // floats per transposed row: rows 4 apart start 16 banks apart
 struct ExpBwdArgs {
     const float *x;
     int64_t ldx;
@@ -1555,164 +1577,346 @@ struct ExpBwdArgs {
     int64_t ldgx;
     const int *list, *offset;  // pair ids t*k + j grouped by expert (walsh_moe_scatter)
     const float *topk_w;       // [M*k] routing weight of each pair
-    int M, E, k, H, S;
+    int M, E, k, H, W;            // W: workgroups launched
     const uint8_t *pg, *pu, *pd;  // packed codes: gate / up [E][H][8], down [E][32][H/4]
     const float *gammas;          // [3]
     float *dpair;                 // [M*k] gradient of each pair's routing weight
-    float *part;                  // [S][E][3][H*32] per-workgroup weight-gradient sums
+    float *part;                  // [W][3][H*32] per-workgroup weight-gradient sums
+    int vec;                      // rows of x, dout and dx 16-byte aligned
 };
 
-__device__ __forceinline__ float packed_code(const uint8_t *row, int i) {
-    const uint32_t b = row[i >> 2];
-    return (float)((int)((b >> (6 - 2 * (i & 3))) & 3u) - 1);
+__device__ __forceinline__ uint32_t packed_bits(const uint8_t *row, int i) {
+    return code_bits(((uint32_t)row[i >> 2] >> (6 - 2 * (i & 3))) & 3u);
 }
 
-__global__ __launch_bounds__(kEbThreads) void moe_experts_bwd_kernel(ExpBwdArgs a) {
-    __shared__ float wg_l[kEbH][33], wu_l[kEbH][33], wd_l[32][kEbH + 1];
-    __shared__ float xs[kEbSlots][32], os[kEbSlots][32], dos[kEbSlots][32];
-    __shared__ float gs[kEbSlots][kEbH], us[kEbSlots][kEbH], hs[kEbSlots][kEbH];
-    __shared__ float red[kEbSlots][2][32][2];
-    const int e = (int)blockIdx.x / a.S, sp = (int)blockIdx.x % a.S;
-    const int tid = threadIdx.x, slot = tid / kEbH, j = tid % kEbH;
-    const int H = a.H, k = a.k;
-    {
-        const float g0 = a.gammas[0], g1 = a.gammas[1], g2 = a.gammas[2];
-        for (int i = tid; i < H * 32; i += kEbThreads) {
-            const int h = i >> 5, d = i & 31;
-            wg_l[h][d] = packed_code(a.pg + ((int64_t)e * H + h) * 8, d) * g0;
-            wu_l[h][d] = packed_code(a.pu + ((int64_t)e * H + h) * 8, d) * g1;
-            wd_l[d][h] = packed_code(a.pd + ((int64_t)e * 32 + d) * (H / 4), h) * g2;
+__device__ __forceinline__ f32x4 eb_mma(f32x4 x, f32x4 y, f32x4 c) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) c = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], y[s], c, 0, 0, 0);
+    return c;
+}
+
+__device__ __forceinline__ float eb_row_sum16(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));
+    return v;
+}
+
+// Deals the experts' 16-pair tiles to W workgroups: expert e gets
+// ceil(tiles_e / T) consecutive workgroups of T tiles each (T a multiple of
+// kEbSlots, such that they fit), starting at start[e]; start[E] of them in
+// all.  Every thread of the workgroup calls it; start and tmp are LDS.
+// Returns T.
+__device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int *start, int *tmp) {
+    const int tid = threadIdx.x;
+    int tiles = 0;
+    if (tid < 128) {
+        tiles = tid < E ? (offset[tid + 1] - offset[tid] + 15) / 16 : 0;
+        int sum = tiles, top = tiles;
+        for (int s = 32; s > 0; s >>= 1) {
+            sum += __shfl_xor(sum, s, 64);
+            top = max(top, __shfl_xor(top, s, 64));
+        }
+        if ((tid & 63) == 0) {
+            tmp[tid >> 6] = sum;
+            tmp[2 + (tid >> 6)] = top;
         }
     }
-    const int p0 = a.offset[e], p1 = a.offset[e + 1];
-    const int per = (p1 - p0 + a.S - 1) / a.S;
-    const int b0 = p0 + sp * per, b1 = min(p1, b0 + per);
-    const int iters = b1 > b0 ? (b1 - b0 + kEbSlots - 1) / kEbSlots : 0;
-    float agw[32], auw[32], adw[32];
-#pragma unroll
-    for (int d = 0; d < 32; ++d) agw[d] = auw[d] = adw[d] = 0.f;
-    // the slot's next pair: id, weight and (threads j < 32) element j of its
-    // x and dout rows, loaded one iteration ahead
-    int npid = -1;
-    float nw = 0.f, nx = 0.f, nd = 0.f;
-    auto fetch = [&](int it) {
-        const int p = b0 + it * kEbSlots + slot;
-        npid = (it < iters && p < b1) ? a.list[p] : -1;
-        if (npid >= 0) {
-            const int64_t t = npid / k;
-            nw = a.topk_w[npid];
-            if (j < 32) {
-                nx = a.x[t * a.ldx + 32 * e + j];
-                nd = a.dout[t * a.ldd + 32 * e + j];
-            }
+    __syncthreads();
+    const int total = tmp[0] + tmp[1], top = max(tmp[2], tmp[3]);
+    int T = W > E ? (total + W - E - 1) / (W - E) : top;
+    T = max(kEbSlots, (T + kEbSlots - 1) / kEbSlots * kEbSlots);
+    __syncthreads();
+    if (tid < 128) {
+        int v = (tiles + T - 1) / T;
+        for (int s = 1; s < 64; s <<= 1) {
+            const int o = __shfl_up(v, s, 64);
+            if ((tid & 63) >= s) v += o;
         }
+        if (tid == 63) tmp[0] = v;
+        start[tid + 1] = v;
+    }
+    __syncthreads();
+    if (tid >= 64 && tid < 128) start[tid + 1] += tmp[0];
+    if (tid == 0) start[0] = 0;
+    __syncthreads();
+    return T;
+}
+
+// NHT: hidden tiles of 16 held (H <= 16 NHT; units past H have zero codes).
+template <int NHT>
+__global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdArgs a) {
+    constexpr int NH = NHT / 2;    // hidden tiles of one wave
+    constexpr int NW = NHT / 2;    // code words of one matrix: 2 tiles x 2 depth chunks each
+    constexpr int HW = NW / 2;     // of them, one wave's
+    // [matrix form][word][lane]: gate, up as [h][d]; down^T as [h][d]; gate^T, up^T as [d][h]
+    __shared__ uint32_t words[5][NW][64];
+    __shared__ __align__(16) f32x4 sums[3][NHT][2][64];
+    __shared__ int start[kEbMaxE + 1], tmp[4];
+    // per wave the transposes, per tile in flight the second half's dx and
+    // dw_pair (two buffers)
+    struct Work {
+        float tr[2 * kEbSlots][2][16 * kEbPitch];
+        f32x4 dx[2][kEbSlots][2][64];
+        float pw[2][kEbSlots][16];
     };
-    fetch(0);
-    for (int it = 0; it < iters; ++it) {
-        const int pid = npid;
-        const float w = nw;
-        if (j < 32) {
-            xs[slot][j] = nx;
-            os[slot][j] = nd;
-            dos[slot][j] = nd * w;
+    __shared__ __align__(16) Work work;
+    const int T = eb_schedule(a.offset, a.E, a.W, start, tmp);
+    const int wg = (int)blockIdx.x;
+    if (wg >= start[a.E]) return;   // workgroup-uniform
+    int e = 0;
+    {
+        int hi = a.E - 1;   // the expert with start[e] <= wg < start[e + 1]
+        while (e < hi) {
+            const int mid = (e + hi + 1) >> 1;
+            if (start[mid] <= wg) e = mid;
+            else hi = mid - 1;
         }
-        fetch(it + 1);
-        __syncthreads();  // rows in LDS (and, on the first pass, the matrices)
-        if (pid >= 0 && j < H) {
-            float g = 0.f, u = 0.f, dh = 0.f;
+    }
+    e = __builtin_amdgcn_readfirstlane(e);
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), slot = wave & (kEbSlots - 1), half = wave / kEbSlots;
+    const int H = a.H, k = a.k;
+    // the expert's packed bytes through LDS (the gathers below read single
+    // bytes, from memory a chain of round trips)
+    uint8_t *bytes = (uint8_t *)&sums[0][0][0][0];   // gate [H][8], up [H][8], down [32][H/4]
+    for (int i = tid; i < 8 * H; i += kEbThreads) {
+        const uint8_t b0 = a.pg[(int64_t)e * H * 8 + i], b1 = a.pu[(int64_t)e * H * 8 + i],
+                      b2 = a.pd[(int64_t)e * H * 8 + i];
+        bytes[i] = b0;
+        bytes[8 * H + i] = b1;
+        bytes[16 * H + i] = b2;
+    }
+    __syncthreads();
+    for (int i = tid; i < 5 * NW * 64; i += kEbThreads) {
+        const int l = i & 63, w = (i >> 6) % NW, m = i / (64 * NW), lm = l & 15, lq = l >> 4;
+        uint32_t v = 0;
 #pragma unroll
-            for (int d = 0; d < 32; ++d) {
-                const float xv = xs[slot][d];
-                g += wg_l[j][d] * xv;
-                u += wu_l[j][d] * xv;
-                dh += wd_l[d][j] * dos[slot][d];
-            }
-            const float sg = 1.0f / (1.0f + expf(-g));
-            const float sv = g * sg, dsil = sg * (1.0f + g * (1.0f - sg));
-            const float hv = sv * u, dg = dh * u * dsil, du = dh * sv;
+        for (int g = 0; g < 4; ++g) {   // hidden tile 2w + g / 2, depth chunk (or column tile) g % 2
 #pragma unroll
-            for (int d = 0; d < 32; ++d) {
-                const float xv = xs[slot][d];
-                agw[d] += dg * xv;
-                auw[d] += du * xv;
-                adw[d] += dos[slot][d] * hv;
-            }
-            gs[slot][j] = dg;
-            us[slot][j] = du;
-            hs[slot][j] = hv;
-        }
-        __syncthreads();
-        {
-            // thread (d = j % 32, q = j / 32) sums hidden units [32q, 32q + 32)
-            const int d = j & 31, q = j >> 5;
-            float vx = 0.f, vo = 0.f;
-            if (pid >= 0) {
-                const int h1 = min(H, 32 * q + 32);
-                for (int h = 32 * q; h < h1; ++h) {
-                    vx += gs[slot][h] * wg_l[h][d] + us[slot][h] * wu_l[h][d];
-                    vo += hs[slot][h] * wd_l[d][h];
+            for (int c = 0; c < 4; ++c) {
+                const int hA = 16 * (2 * w + (g >> 1)) + lm, dA = 16 * (g & 1) + 4 * lq + c;   // forms 0, 1, 2
+                const int hB = 16 * (2 * w + (g >> 1)) + 4 * lq + c, dB = 16 * (g & 1) + lm;   // forms 3, 4
+                const int h = m < 3 ? hA : hB, d = m < 3 ? dA : dB;
+                if (h < H) {
+                    const uint32_t b = m == 2 ? packed_bits(bytes + 16 * H + d * (H / 4), h)
+                                              : packed_bits(bytes + (m == 0 || m == 3 ? 0 : 8 * H) + h * 8, d);
+                    v |= b << (14 - 2 * (2 * g + (c >> 1)) + 16 * (c & 1));
                 }
             }
-            vx += __shfl_xor(vx, 32, 64);  // q and q ^ 1 share a wave
-            vo += __shfl_xor(vo, 32, 64);
-            if ((j & 63) < 32) {
-                red[slot][j >> 6][d][0] = vx;
-                red[slot][j >> 6][d][1] = vo;
+        }
+        words[m][w][l] = v;
+    }
+    const float gg = 0.5f * a.gammas[0], gu = 0.5f * a.gammas[1], gd = 0.5f * a.gammas[2];
+    const int p1 = a.offset[e + 1], b0 = a.offset[e] + 16 * T * (wg - start[e]), b1 = min(p1, b0 + 16 * T);
+    __syncthreads();
+    uint32_t cw[5][HW];
+#pragma unroll
+    for (int m = 0; m < 5; ++m)
+#pragma unroll
+        for (int w = 0; w < HW; ++w) cw[m][w] = words[m][half * HW + w][lane];
+
+    f32x4 ag[NH][2], au[NH][2], ad[NH][2];
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) ag[i][c] = au[i][c] = ad[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // the pair of lane n of the tile at b (-1: none)
+    auto pair_of = [&](int b) { return b + n < b1 ? a.list[b + n] : -1; };
+    auto row4 = [&](const float *base, int64_t ld, int pid, int d0) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (pid >= 0) {
+            const float *p = base + (int64_t)(pid / k) * ld + 32 * e + d0;
+            if (a.vec) v = *(const f32x4 *)p;
+            else v = f32x4{p[0], p[1], p[2], p[3]};
+        }
+        return v;
+    };
+    // one tile's operands: rows with the pair as lane (x4, d4: chunk c holds
+    // columns 16c + 4q ..) and with the column as lane (xt, dt: chunk c,
+    // pairs 4q ..), the weights of pairs 4q ..
+    struct Rows {
+        f32x4 x4[2], d4[2], xt[2], dt[2], w;
+    };
+    auto fetch = [&](int pid) {
+        Rows r;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            r.x4[c] = row4(a.x, a.ldx, pid, 16 * c + 4 * q);
+            r.d4[c] = row4(a.dout, a.ldd, pid, 16 * c + 4 * q);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int ps = __shfl(pid, 4 * q + s, 64);
+            const int64_t tok = ps < 0 ? 0 : ps / k;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                r.xt[c][s] = ps < 0 ? 0.f : a.x[tok * a.ldx + 32 * e + 16 * c + n];
+                r.dt[c][s] = ps < 0 ? 0.f : a.dout[tok * a.ldd + 32 * e + 16 * c + n];
+            }
+            r.w[s] = ps < 0 ? 0.f : a.topk_w[ps];
+        }
+        return r;
+    };
+
+    float *tg = work.tr[wave][0], *tu = work.tr[wave][1];
+    int pid = pair_of(b0 + 16 * slot);
+    Rows r = fetch(pid);
+    // every wave of the workgroup runs every iteration (the barriers below);
+    // a slot past the last tile has no pairs and adds zeros
+    int it = 0;
+    for (int bt = b0; bt < b1; bt += 16 * kEbSlots, ++it) {
+        const int next_pid = pair_of(bt + 16 * (kEbSlots + slot));
+        f32x4 dx[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+        f32x4 pw = {0.f, 0.f, 0.f, 0.f};
+        const Rows cur = r;
+#pragma unroll
+        for (int nt = 0; nt < NH; ++nt) {
+            // opaque copies: the expansions stay here instead of being hoisted
+            // out of the tile loop (160 registers)
+            uint32_t w5[5];
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                w5[m] = cw[m][nt >> 1];
+                asm volatile("" : "+v"(w5[m]));
+            }
+            f32x4 g = {0.f, 0.f, 0.f, 0.f}, u = g, dh = g;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int kk = 2 * (nt & 1) + c;
+                g = eb_mma(cur.x4[c], codes_f32x4(w5[0], kk), g);
+                u = eb_mma(cur.x4[c], codes_f32x4(w5[1], kk), u);
+                dh = eb_mma(cur.d4[c], codes_f32x4(w5[2], kk), dh);
+            }
+            // the next tile's rows once this one's x and dout by pair are used
+            if (nt == NH - 1) r = fetch(next_pid);
+            f32x4 hw, dg, du;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float gv = gg * g[j], uv = gu * u[j], dv = gd * dh[j];
+                const float sg = 1.0f / (1.0f + expf(-gv));
+                const float sv = gv * sg, dsil = sg * (1.0f + gv * (1.0f - sg));
+                const float hv = sv * uv, dw = dv * cur.w[j];
+                pw[j] += dv * hv;
+                hw[j] = hv * cur.w[j];
+                dg[j] = dw * uv * dsil;
+                du[j] = dw * sv;
+            }
+            // dg, du with the hidden units as depth: row h of the area holds
+            // its 16 pairs
+            *(f32x4 *)(tg + n * kEbPitch + 4 * q) = dg * gg;
+            *(f32x4 *)(tu + n * kEbPitch + 4 * q) = du * gu;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                ag[nt][c] = eb_mma(dg, cur.xt[c], ag[nt][c]);
+                au[nt][c] = eb_mma(du, cur.xt[c], au[nt][c]);
+                ad[nt][c] = eb_mma(hw, cur.dt[c], ad[nt][c]);
+            }
+            wave_lds_fence();
+            f32x4 bg, bu;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                bg[j] = tg[(4 * q + j) * kEbPitch + n];
+                bu[j] = tu[(4 * q + j) * kEbPitch + n];
+            }
+            wave_lds_fence();
+#pragma unroll
+            for (int mt = 0; mt < 2; ++mt) {
+                const int kk = 2 * (nt & 1) + mt;
+                dx[mt] = eb_mma(codes_f32x4(w5[3], kk), bg, dx[mt]);
+                dx[mt] = eb_mma(codes_f32x4(w5[4], kk), bu, dx[mt]);
             }
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) pw[j] = eb_row_sum16(pw[j]);
+        // the second half's sums to the first (two buffers, so one barrier
+        // per iteration orders both the hand-over and the reuse)
+        f32x4 *hdx = &work.dx[it & 1][slot][0][lane];
+        float *hpw = work.pw[it & 1][slot];
+        if (half) {
+            hdx[0] = dx[0];
+            hdx[64] = dx[1];
+            if (n == 0) *(f32x4 *)(hpw + 4 * q) = pw;
+        }
+        lds_barrier();
+        if (!half) {
+            if (pid >= 0) {
+                float *p = a.dx + (int64_t)(pid / k) * a.ldgx + 32 * e;
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) {
+                    float *pm = p + 16 * mt + 4 * q;
+                    const f32x4 v = dx[mt] + hdx[64 * mt];
+                    if (a.vec) {
+                        *(f32x4 *)pm = v;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) pm[j] = v[j];
+                    }
+                }
+            }
+            const f32x4 pv = pw + *(const f32x4 *)(hpw + 4 * q);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int ps = __shfl(pid, 4 * q + j, 64);
+                if (n == 0 && ps >= 0) a.dpair[ps] = pv[j];
+            }
+        }
+        pid = next_pid;
+    }
+    // the waves' sums in wave order (the two halves hold different units)
+    for (int w = 0; w < kEbSlots; ++w) {
+        if (slot == w) {
+#pragma unroll
+            for (int i = 0; i < NH; ++i)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int nt = half * NH + i;
+                    sums[0][nt][c][lane] = w ? sums[0][nt][c][lane] + ag[i][c] : ag[i][c];
+                    sums[1][nt][c][lane] = w ? sums[1][nt][c][lane] + au[i][c] : au[i][c];
+                    sums[2][nt][c][lane] = w ? sums[2][nt][c][lane] + ad[i][c] : ad[i][c];
+                }
+        }
         __syncthreads();
-        if (pid >= 0 && j < 32) {
-            const float vx = red[slot][0][j][0] + red[slot][1][j][0];
-            const float vo = red[slot][0][j][1] + red[slot][1][j][1];
-            a.dx[(int64_t)(pid / k) * a.ldgx + 32 * e + j] = vx;
-            float pw = os[slot][j] * vo;
-#pragma unroll
-            for (int off = 16; off > 0; off >>= 1) pw += __shfl_xor(pw, off, 64);
-            if (j == 0) a.dpair[pid] = pw;
-        }
     }
-    // the two slots' sums meet in LDS (the matrices are no longer needed)
-    __syncthreads();
-    if (slot == 1 && j < H) {
+    float *dst = a.part + (int64_t)wg * 3 * H * 32;
+    const f32x4 *sl = &sums[0][0][0][0];
+    for (int i = tid; i < 3 * NHT * 2 * 64; i += kEbThreads) {
+        const int l = i & 63, c = (i >> 6) & 1, nt = (i >> 7) % NHT, m = i / (128 * NHT);
+        const int h = 16 * nt + 4 * (l >> 4), d = 16 * c + (l & 15);
+        if (h >= H) continue;
+        const f32x4 v = sl[i];
+        float *o = dst + (int64_t)m * H * 32;
 #pragma unroll
-        for (int d = 0; d < 32; ++d) {
-            wg_l[j][d] = agw[d];
-            wu_l[j][d] = auw[d];
-            wd_l[d][j] = adw[d];
-        }
-    }
-    __syncthreads();
-    if (slot == 0 && j < H) {
-        float *dst = a.part + ((int64_t)sp * a.E + e) * 3 * H * 32;
-#pragma unroll
-        for (int d = 0; d < 32; ++d) {
-            dst[j * 32 + d] = agw[d] + wg_l[j][d];
-            dst[H * 32 + j * 32 + d] = auw[d] + wu_l[j][d];
-            dst[2 * H * 32 + d * H + j] = adw[d] + wd_l[d][j];
-        }
+        for (int j = 0; j < 4; ++j) o[m == 2 ? d * H + h + j : (h + j) * 32 + d] = v[j];
     }
 }
 
-// Weight gradients: the per-workgroup sums added in workgroup order, then
-// clamp(., -2, 2) (the MoE STE); gate / up [E][H][32], down [E][32][H].
-__global__ __launch_bounds__(256) void moe_experts_bwd_reduce_kernel(const float *__restrict__ part, int S, int E,
+// Weight gradients: the sums of the expert's workgroups added in workgroup
+// order, then clamp(., -2, 2) (the MoE STE); gate / up [E][H][32], down
+// [E][32][H].  Grid: x = blocks of 256 values, y = expert.
+__global__ __launch_bounds__(256) void moe_experts_bwd_reduce_kernel(const float *__restrict__ part,
+                                                                     const int *__restrict__ offset, int W, int E,
                                                                      int H, float *__restrict__ dg,
                                                                      float *__restrict__ du, float *__restrict__ dd) {
-    const int64_t per = 3LL * H * 32, n = (int64_t)E * per;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int e = (int)(i / per), r = (int)(i % per);
-        float v = 0.f;
-        for (int sp = 0; sp < S; ++sp) v += part[((int64_t)sp * E + e) * per + r];
-        v = fminf(fmaxf(v, -2.f), 2.f);
-        const int kind = r / (H * 32), rr = r % (H * 32);
-        float *dst = kind == 0 ? dg : (kind == 1 ? du : dd);
-        if (dst) dst[(int64_t)e * H * 32 + rr] = v;
-    }
+    __shared__ int start[kEbMaxE + 1], tmp[4];
+    eb_schedule(offset, E, W, start, tmp);
+    const int per = 3 * H * 32, e = (int)blockIdx.y, r = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (r >= per) return;
+    float v = 0.f;
+    for (int wg = start[e]; wg < start[e + 1]; ++wg) v += part[(int64_t)wg * per + r];
+    v = fminf(fmaxf(v, -2.f), 2.f);
+    const int kind = r / (H * 32), rr = r % (H * 32);
+    float *dst = kind == 0 ? dg : (kind == 1 ? du : dd);
+    if (dst) dst[(int64_t)e * H * 32 + rr] = v;
 }
 
-static int experts_bwd_splits(int64_t E) {
-    int64_t S = ceil_div(2 * (int64_t)device_info().cu_count, E);
-    return (int)(S < 1 ? 1 : (S > 16 ? 16 : S));
+// Workgroups of the backward launch: one per CU (its registers allow one),
+// and twice the experts at least, so that eb_schedule has room to deal.
+static int experts_bwd_groups(int64_t E) {
+    const int64_t cu = device_info().cu_count;
+    return (int)(cu > 2 * E ? cu : 2 * E);
 }
 
 static int route_out_check(const char *fn, int64_t M, int64_t E, int64_t k, const int *topk_idx, const float *topk_w,
@@ -1916,7 +2120,7 @@ WALSH_EXPORT int walsh_moe_decode_fwd(const void *x, int64_t ldx, int64_t M, int
 
 WALSH_EXPORT int64_t walsh_moe_experts_bwd_workspace_bytes(int64_t E, int64_t H) {
     if (E < 1 || E > kMaxE || H < 16 || H > kEbH) return 0;
-    return (int64_t)experts_bwd_splits(E) * E * 3 * H * 32 * 4;
+    return (int64_t)experts_bwd_groups(E) * 3 * H * 32 * 4;
 }
 
 WALSH_EXPORT int walsh_moe_experts_bwd(const float *x, int64_t ldx, const float *dout, int64_t ldd, int64_t M,
@@ -1937,7 +2141,7 @@ WALSH_EXPORT int walsh_moe_experts_bwd(const float *x, int64_t ldx, const float 
         return set_error(WALSH_EINVAL, "%s: workspace of %lld bytes, needs %lld", fn, (long long)work_bytes,
                          (long long)walsh_moe_experts_bwd_workspace_bytes(E, H));
     hipStream_t s = (hipStream_t)stream;
-    const int S = experts_bwd_splits(E);
+    const int W = experts_bwd_groups(E);
     ExpBwdArgs a;
     a.x = x;
     a.ldx = ldx;
@@ -1952,20 +2156,21 @@ WALSH_EXPORT int walsh_moe_experts_bwd(const float *x, int64_t ldx, const float 
     a.E = (int)E;
     a.k = (int)k;
     a.H = (int)H;
-    a.S = S;
+    a.W = W;
     a.pg = gate_packed;
     a.pu = up_packed;
     a.pd = down_packed;
     a.gammas = gammas;
     a.dpair = d_pair_w;
     a.part = (float *)work;
-    launch(moe_experts_bwd_kernel, dim3((unsigned)(E * S)), dim3(kEbThreads), 0, s, a);
+    a.vec = ldx % 4 == 0 && ldd % 4 == 0 && ldgx % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)dout % 16 == 0 &&
+            (uintptr_t)dx % 16 == 0;
+    if (H <= 64) launch(moe_experts_bwd_kernel<4>, dim3((unsigned)W), dim3(kEbThreads), 0, s, a);
+    else launch(moe_experts_bwd_kernel<8>, dim3((unsigned)W), dim3(kEbThreads), 0, s, a);
     int rc = check_hip(hipGetLastError(), fn);
     if (rc) return rc;
-    int64_t grid = ceil_div(E * 3 * H * 32, 256);
-    if (grid > 4096) grid = 4096;
-    launch(moe_experts_bwd_reduce_kernel, dim3((unsigned)grid), dim3(256), 0, s, (const float *)work, S, (int)E,
-           (int)H, dgate, dup, ddown);
+    launch(moe_experts_bwd_reduce_kernel, dim3((unsigned)ceil_div(3 * H * 32, 256), (unsigned)E), dim3(256), 0, s,
+           (const float *)work, offset, W, (int)E, (int)H, dgate, dup, ddown);
     return check_hip(hipGetLastError(), fn);
 }
 
