@@ -235,6 +235,25 @@ def test_sinkhorn_bwd_vs_oracle(K, n):
     assert_close(dh, ref, torch.float32, f"sinkhorn bwd n={n}")
 
 
+@pytest.mark.parametrize("n,batch,n_iter", [(4, 1, 20), (4, 16, 1), (3, 17, 20), (1, 70, 3), (2, 33, 60), (4, 5, 100)])
+def test_sinkhorn_quad_forms(K, n, batch, n_iter):
+    """Forward and backward of the four-lane Sinkhorn kernels (n <= 4): one
+    matrix, full and ragged groups of 16, fewer streams than lanes, one and
+    many iterations (100 takes the kernel that recomputes its states)."""
+    from oracle import mhc as omhc
+    rng = np.random.default_rng(n * 100 + batch)
+    h = rng.normal(0, 1.0, (batch, n, n)).astype(np.float32)
+    g = rng.normal(0, 1, (batch, n, n)).astype(np.float32)
+    m = K.sinkhorn(torch.from_numpy(h).cuda(), n_iter=n_iter).cpu().numpy()
+    assert_close(m, omhc.sinkhorn(h.astype(np.float64), n_iter), torch.float32, f"sinkhorn n={n}")
+    dh = K.sinkhorn_bwd(torch.from_numpy(h).cuda(), torch.from_numpy(g).cuda(), n_iter=n_iter).cpu().numpy()
+    ref = omhc.sinkhorn_bwd(h.astype(np.float64), g.astype(np.float64), n_iter)
+    if n == 1:   # the exact gradient is O(eps)
+        assert np.abs(ref).max() < 1e-6 and np.abs(dh).max() < 1e-6
+        return
+    assert_close(dh, ref, torch.float32, f"sinkhorn bwd n={n} n_iter={n_iter}")
+
+
 def test_sinkhorn_function_autograd():
     from oracle import mhc as omhc
     from src.model.mhc import SinkhornKnopp
