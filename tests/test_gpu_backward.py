@@ -521,6 +521,34 @@ def test_hadamard_bwd_group_padded(K, in_o, gsx, out_o, gsy, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,C,M,off", [(4, 8, 5, 0), (4, 520, 9, 0), (2, 1032, 3, 0), (4, 512, 6, 4), (4, 516, 3, 0)])
+def test_stream_mixing_bwd_row_forms(K, n, C, M, off, dtype):
+    """The backward of the stream mixing over the row forms of its kernels:
+    rows of whole 16-byte pieces (8 bf16 columns per lane) shorter, longer
+    and not a multiple of a wavefront's span, 8-byte aligned rows (``off``
+    elements into a buffer) and widths that are not a multiple of 8."""
+    g = torch.Generator().manual_seed(n * 100 + C + off)
+
+    def dev(*shape):
+        t = torch.randn(*shape, generator=g).to(dtype)
+        buf = torch.empty(t.numel() + off, dtype=dtype, device="cuda")
+        return t, buf[off:].view(shape).copy_(t)
+    (x, xc), (out, oc), (gli, gc), (gnew, nc) = dev(M, n, C), dev(M, C), dev(M, C), dev(M, n, C)
+    hp, hr, hq = torch.rand(M, 1, n, generator=g), torch.rand(M, n, n, generator=g), 2 * torch.rand(M, 1, n, generator=g)
+    dx1, dhp = K.mhc_aggregate_bwd(xc, hp.cuda(), gc)
+    dx2, dout, dhr, dhq = K.mhc_post_bwd(xc, oc, hr.cuda(), hq.cuda(), nc)
+    x64, o64, gl64, gn64 = (t.double() for t in (x, out, gli, gnew))
+    ref = [(dx1, hp.double().transpose(1, 2) * gl64.unsqueeze(1), "dx (aggregate)"),
+           (dhp.reshape(M, n), (x64 * gl64.unsqueeze(1)).sum(-1), "dh_pre"),
+           (dx2, torch.matmul(hr.double().transpose(1, 2), gn64), "dx (update)"),
+           (dout, torch.matmul(hq.double(), gn64).squeeze(1), "d_out"),
+           (dhr, torch.matmul(gn64, x64.transpose(1, 2).contiguous()), "dh_res"),
+           (dhq.reshape(M, n), (gn64 * o64.unsqueeze(1)).sum(-1), "dh_post")]
+    for a, b, what in ref:
+        assert_close(a.float().cpu().numpy(), b.numpy(), dtype, f"{what} n={n} C={C} off={off}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("n,C", [(4, 512), (3, 44), (1, 260)])
 def test_stream_mixing_bwd(K, n, C, dtype):
     """walsh_mhc_aggregate_fwd/_bwd and walsh_mhc_post_bwd against float64

@@ -7,6 +7,7 @@
 //   walsh_mhc_post_fwd  x_new = H_res @ x + H_post^T (x) out (mhc.py:366-381)
 //
 // Stream tensors are [M tokens][n streams][C] (row stride ldx >= n*C).
+#include <initializer_list>
 #include <type_traits>
 
 #include "common.h"
@@ -317,15 +318,57 @@ __global__ __launch_bounds__(kSkThreads) void sinkhorn_bwd_quad_kernel(const flo
 // ---------------------------------------------------------------- stream mixing for training
 // Dense rows: x / dx / dnew [M][n][C], li / dli / out / dout [M][C] (one
 // dtype T), h_pre / h_post [M][n], h_res [M][n][n] float32.  One wavefront
-// per token; lane l covers columns 4l + 256k; sums over the C columns are
-// per-lane partials reduced across the wavefront with xor shuffles.
+// per token; lane l covers W columns from W l + 64 W k (W = 8 for bf16 rows
+// of whole 16-byte pieces, 4 otherwise); sums over the C columns are
+// per-lane partials reduced across the wavefront by mix_reduce.
 constexpr int kMixWaves = 4;
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+template <typename T, int W> struct MixRow;   // W consecutive columns as loaded
+template <typename T> struct MixRow<T, 4> {
+    f32x4 v;
+    __device__ __forceinline__ void load(const T *p) { v = load4(p); }
+    __device__ __forceinline__ f32x4 get(int) const { return v; }
+};
+template <> struct MixRow<uint16_t, 8> {
+    u32x4 v;
+    __device__ __forceinline__ void load(const uint16_t *p) { v = *(const u32x4 *)p; }
+    __device__ __forceinline__ f32x4 get(int h) const {
+        const uint32_t a = h ? v.z : v.x, b = h ? v.w : v.y;
+        return f32x4{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), __uint_as_float(b << 16),
+                     __uint_as_float(b & 0xffff0000u)};
+    }
+};
+template <typename T, int W> __device__ __forceinline__ void mix_store(T *p, const f32x4 (&v)[W / 4]) {
+    if constexpr (W == 8)
+        *(u32x4 *)p = u32x4{pack_bf16x2(v[0].x, v[0].y), pack_bf16x2(v[0].z, v[0].w), pack_bf16x2(v[1].x, v[1].y),
+                            pack_bf16x2(v[1].z, v[1].w)};
+    else
+        store4(p, v[0]);
 }
+
+__device__ __forceinline__ float dot4(const f32x4 &a, const f32x4 &b) {
+    return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
+}
+
+// Sums of the 4 values v over the wavefront: afterwards every lane of row
+// rho (16 lanes) holds the sum of v[mix_index(rho)].  The half and row
+// swaps of gfx950 add two values at a time (two instructions each), then the
+// row's 16 lanes are added by rotations: 10 instructions for 4 sums, where 4
+// butterflies through ds_bpermute took 24 LDS round trips.
+__device__ __forceinline__ float mix_reduce(float v0, float v1, float v2, float v3) {
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    const u2 a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v0), __float_as_uint(v1), false, false);
+    const u2 b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v2), __float_as_uint(v3), false, false);
+    const float s0 = __uint_as_float(a.x) + __uint_as_float(a.y), s1 = __uint_as_float(b.x) + __uint_as_float(b.y);
+    const u2 c = __builtin_amdgcn_permlane16_swap(__float_as_uint(s0), __float_as_uint(s1), false, false);
+    float t = __uint_as_float(c.x) + __uint_as_float(c.y);
+    t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x128, 0xf, 0xf, false));
+    t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x124, 0xf, 0xf, false));
+    t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x122, 0xf, 0xf, false));
+    t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x121, 0xf, 0xf, false));
+    return t;
+}
+__device__ __forceinline__ int mix_index(int row) { return ((row & 1) << 1) | (row >> 1); }
 
 template <typename T>
 __global__ __launch_bounds__(64 * kMixWaves) void mhc_agg_fwd_kernel(const T *__restrict__ x,
@@ -346,49 +389,63 @@ __global__ __launch_bounds__(64 * kMixWaves) void mhc_agg_fwd_kernel(const T *__
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * kMixWaves) void mhc_agg_bwd_kernel(const T *__restrict__ x,
+template <typename T, int W>
+__global__ __launch_bounds__(64 * kMixWaves, 4) void mhc_agg_bwd_kernel(const T *__restrict__ x,
                                                                      const float *__restrict__ h_pre,
                                                                      const T *__restrict__ dli, T *__restrict__ dx,
                                                                      float *__restrict__ dh_pre, int64_t M, int n,
                                                                      int C) {
     const int lane = threadIdx.x & 63;
-    for (int64_t t = (int64_t)blockIdx.x * kMixWaves + (threadIdx.x >> 6); t < M; t += (int64_t)gridDim.x * kMixWaves) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int64_t t = (int64_t)blockIdx.x * kMixWaves + wave; t < M; t += (int64_t)gridDim.x * kMixWaves) {
         float hp[kMaxStreams], dh[kMaxStreams];
 #pragma unroll
         for (int s = 0; s < kMaxStreams; ++s) {
             hp[s] = s < n ? h_pre[t * n + s] : 0.f;
             dh[s] = 0.f;
         }
-        for (int c = 4 * lane; c < C; c += 256) {
-            const f32x4 g = load4(dli + t * C + c);
+#pragma unroll 1
+        for (int c = W * lane; c < C; c += 64 * W) {
+            MixRow<T, W> gr, xr[kMaxStreams];
+            gr.load(dli + t * C + c);
+#pragma unroll
+            for (int s = 0; s < kMaxStreams; ++s)
+                if (s < n) xr[s].load(x + (t * n + s) * C + c);
 #pragma unroll
             for (int s = 0; s < kMaxStreams; ++s) {
                 if (s >= n) continue;
-                const f32x4 xv = load4(x + (t * n + s) * C + c);
-                dh[s] += g[0] * xv[0] + g[1] * xv[1] + g[2] * xv[2] + g[3] * xv[3];
-                store4(dx + (t * n + s) * C + c, hp[s] * g);
+                f32x4 d[W / 4];
+#pragma unroll
+                for (int h = 0; h < W / 4; ++h) {
+                    dh[s] += dot4(gr.get(h), xr[s].get(h));
+                    d[h] = hp[s] * gr.get(h);
+                }
+                mix_store<T, W>(dx + (t * n + s) * C + c, d);
             }
         }
-#pragma unroll
-        for (int s = 0; s < kMaxStreams; ++s) {
-            if (s >= n) continue;
-            const float v = wave_sum(dh[s]);
-            if (lane == 0) dh_pre[t * n + s] = v;
-        }
+        const float v = mix_reduce(dh[0], dh[1], dh[2], dh[3]);
+        const int s = mix_index(lane >> 4);
+        if ((lane & 15) == 0 && s < n) dh_pre[t * n + s] = v;
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * kMixWaves) void mhc_post_bwd_kernel(const T *__restrict__ x, const T *__restrict__ out,
+// N: the number of streams, or 0 for n <= 4 at run time.  The token of a
+// wavefront is made scalar, so the mixing matrices sit in scalar registers and
+// four wavefronts fit a SIMD (two at 208 registers before).
+// HBM bound: 117 MB at 8,192 tokens x 4 streams x 512 bf16 columns: 23 us
+// with 16-byte accesses and mix_reduce; 65 us (1.8 TB/s) with 8-byte
+// accesses and 20 butterflies through LDS per token.
+template <typename T, int W, int N>
+__global__ __launch_bounds__(64 * kMixWaves, 4) void mhc_post_bwd_kernel(const T *__restrict__ x, const T *__restrict__ out,
                                                                       const float *__restrict__ h_res,
                                                                       const float *__restrict__ h_post,
                                                                       const T *__restrict__ dnew, T *__restrict__ dx,
                                                                       T *__restrict__ dout, float *__restrict__ dh_res,
-                                                                      float *__restrict__ dh_post, int64_t M, int n,
+                                                                      float *__restrict__ dh_post, int64_t M, int nr,
                                                                       int C) {
-    const int lane = threadIdx.x & 63;
-    for (int64_t t = (int64_t)blockIdx.x * kMixWaves + (threadIdx.x >> 6); t < M; t += (int64_t)gridDim.x * kMixWaves) {
+    const int lane = threadIdx.x & 63, n = N ? N : nr;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (int64_t t = (int64_t)blockIdx.x * kMixWaves + wave; t < M; t += (int64_t)gridDim.x * kMixWaves) {
         float hr[kMaxStreams][kMaxStreams], hq[kMaxStreams];
         float dr[kMaxStreams][kMaxStreams], dq[kMaxStreams];
 #pragma unroll
@@ -401,45 +458,52 @@ __global__ __launch_bounds__(64 * kMixWaves) void mhc_post_bwd_kernel(const T *_
                 dr[i][s] = 0.f;
             }
         }
-        for (int c = 4 * lane; c < C; c += 256) {
-            f32x4 g[kMaxStreams], xv[kMaxStreams];
+#pragma unroll 1
+        for (int c = W * lane; c < C; c += 64 * W) {
+            MixRow<T, W> gr[kMaxStreams], xr[kMaxStreams], o;
 #pragma unroll
             for (int i = 0; i < kMaxStreams; ++i) {
-                g[i] = i < n ? load4(dnew + (t * n + i) * C + c) : f32x4{0.f, 0.f, 0.f, 0.f};
-                xv[i] = i < n ? load4(x + (t * n + i) * C + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+                if (i >= n) continue;
+                gr[i].load(dnew + (t * n + i) * C + c);
+                xr[i].load(x + (t * n + i) * C + c);
             }
-            const f32x4 o = load4(out + t * C + c);
-            f32x4 go = f32x4{0.f, 0.f, 0.f, 0.f};
+            o.load(out + t * C + c);
+            f32x4 go[W / 4], d[kMaxStreams][W / 4];
 #pragma unroll
-            for (int i = 0; i < kMaxStreams; ++i) {
-                go += hq[i] * g[i];
-                dq[i] += g[i][0] * o[0] + g[i][1] * o[1] + g[i][2] * o[2] + g[i][3] * o[3];
+            for (int h = 0; h < W / 4; ++h) {
+                go[h] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < kMaxStreams; ++s)
-                    dr[i][s] += g[i][0] * xv[s][0] + g[i][1] * xv[s][1] + g[i][2] * xv[s][2] + g[i][3] * xv[s][3];
+                for (int s = 0; s < kMaxStreams; ++s) d[s][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 ov = o.get(h);
+#pragma unroll
+                for (int i = 0; i < kMaxStreams; ++i) {
+                    if (i >= n) continue;
+                    const f32x4 g = gr[i].get(h);
+                    go[h] += hq[i] * g;
+                    dq[i] += dot4(g, ov);
+#pragma unroll
+                    for (int s = 0; s < kMaxStreams; ++s) {
+                        if (s >= n) continue;
+                        dr[i][s] += dot4(g, xr[s].get(h));
+                        d[s][h] += hr[i][s] * g;
+                    }
+                }
             }
-            store4(dout + t * C + c, go);
+            mix_store<T, W>(dout + t * C + c, go);
 #pragma unroll
-            for (int s = 0; s < kMaxStreams; ++s) {
-                if (s >= n) continue;
-                f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int i = 0; i < kMaxStreams; ++i) d += hr[i][s] * g[i];
-                store4(dx + (t * n + s) * C + c, d);
-            }
+            for (int s = 0; s < kMaxStreams; ++s)
+                if (s < n) mix_store<T, W>(dx + (t * n + s) * C + c, d[s]);
         }
+        const int s = mix_index(lane >> 4);
+        const bool wr = (lane & 15) == 0 && s < n;
 #pragma unroll
         for (int i = 0; i < kMaxStreams; ++i) {
             if (i >= n) continue;
-            const float vq = wave_sum(dq[i]);
-            if (lane == 0) dh_post[t * n + i] = vq;
-#pragma unroll
-            for (int s = 0; s < kMaxStreams; ++s) {
-                if (s >= n) continue;
-                const float v = wave_sum(dr[i][s]);
-                if (lane == 0) dh_res[(t * n + i) * n + s] = v;
-            }
+            const float v = mix_reduce(dr[i][0], dr[i][1], dr[i][2], dr[i][3]);
+            if (wr) dh_res[(t * n + i) * n + s] = v;
         }
+        const float vq = mix_reduce(dq[0], dq[1], dq[2], dq[3]);
+        if (wr) dh_post[t * n + s] = vq;
     }
 }
 
@@ -2115,6 +2179,13 @@ static int mix_check(const char *fn, int64_t M, int64_t n, int64_t C, int dtype)
     return WALSH_OK;
 }
 
+// bf16 rows in whole 16-byte pieces: 8 columns per lane and access
+static bool mix_wide(std::initializer_list<const void *> rows, int64_t C) {
+    bool ok = C % 8 == 0;
+    for (const void *p : rows) ok = ok && (uintptr_t)p % 16 == 0;
+    return ok;
+}
+
 static dim3 mix_grid(int64_t M) {
     int64_t g = ceil_div(M, kMixWaves);
     const int64_t cap = (int64_t)device_info().cu_count * 16;
@@ -2145,10 +2216,11 @@ WALSH_EXPORT int walsh_mhc_aggregate_bwd(const void *x, const float *h_pre, cons
     if (M == 0) return WALSH_OK;
     if (!x || !h_pre || !d_layer_in || !dx || !dh_pre) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
     if (dtype == WALSH_BF16)
-        launch(mhc_agg_bwd_kernel<uint16_t>, mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream,
-               (const uint16_t *)x, h_pre, (const uint16_t *)d_layer_in, (uint16_t *)dx, dh_pre, M, (int)n, (int)C);
+        launch((mix_wide({x, d_layer_in, dx}, C) ? mhc_agg_bwd_kernel<uint16_t, 8> : mhc_agg_bwd_kernel<uint16_t, 4>),
+               mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream, (const uint16_t *)x, h_pre,
+               (const uint16_t *)d_layer_in, (uint16_t *)dx, dh_pre, M, (int)n, (int)C);
     else
-        launch(mhc_agg_bwd_kernel<float>, mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream, (const float *)x,
+        launch((mhc_agg_bwd_kernel<float, 4>), mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream, (const float *)x,
                h_pre, (const float *)d_layer_in, (float *)dx, dh_pre, M, (int)n, (int)C);
     return check_hip(hipGetLastError(), fn);
 }
@@ -2162,13 +2234,19 @@ WALSH_EXPORT int walsh_mhc_post_bwd(const void *x, const void *out, const float 
     if (M == 0) return WALSH_OK;
     if (!x || !out || !h_res || !h_post || !d_new || !dx || !d_out || !dh_res || !dh_post)
         return set_error(WALSH_EINVAL, "%s: null pointer", fn);
-    if (dtype == WALSH_BF16)
-        launch(mhc_post_bwd_kernel<uint16_t>, mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream,
-               (const uint16_t *)x, (const uint16_t *)out, h_res, h_post, (const uint16_t *)d_new, (uint16_t *)dx,
-               (uint16_t *)d_out, dh_res, dh_post, M, (int)n, (int)C);
-    else
-        launch(mhc_post_bwd_kernel<float>, mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream, (const float *)x,
-               (const float *)out, h_res, h_post, (const float *)d_new, (float *)dx, (float *)d_out, dh_res, dh_post,
-               M, (int)n, (int)C);
+#define WALSH_POST_BWD(T, W, N)                                                                                   \
+    launch((mhc_post_bwd_kernel<T, W, N>), mix_grid(M), dim3(64 * kMixWaves), 0, (hipStream_t)stream, (const T *)x, \
+           (const T *)out, h_res, h_post, (const T *)d_new, (T *)dx, (T *)d_out, dh_res, dh_post, M, (int)n, (int)C)
+    const bool wide = mix_wide({x, out, d_new, dx, d_out}, C);
+    if (dtype == WALSH_BF16) {
+        if (wide && n == 4) WALSH_POST_BWD(uint16_t, 8, 4);
+        else if (wide) WALSH_POST_BWD(uint16_t, 8, 0);
+        else WALSH_POST_BWD(uint16_t, 4, 0);
+    } else if (n == 4) {
+        WALSH_POST_BWD(float, 4, 4);
+    } else {
+        WALSH_POST_BWD(float, 4, 0);
+    }
+#undef WALSH_POST_BWD
     return check_hip(hipGetLastError(), fn);
 }
