@@ -75,6 +75,31 @@ def test_hadamard_bwd_vs_oracle(K, in_o, out_o, M, dtype):
         assert_close(got.cpu().numpy(), r, dtype, f"{name} {in_o}x{out_o} M={M}")
 
 
+@pytest.mark.parametrize("in_o,out_o,M", [(16, 16, 1), (16, 16, 16), (4, 16, 17), (16, 20, 33), (36, 4, 1030), (64, 48, 95),
+                                          (16, 44, 4000), (128, 16, 31)])
+def test_hadamard_bwd_pairs_equal_general(K, in_o, out_o, M):
+    """bf16 rows in 8-byte pieces run on wavefront pairs, unaligned rows on
+    the general kernel: the input gradient is equal bitwise (same products,
+    transforms and roundings), the sums over the rows differ in grouping only
+    (float32 sums of the same products: 1e-5), and both meet the oracle.  One
+    row, full and ragged tiles, several chunks and output tiles, several
+    tiles per workgroup."""
+    c = make_case(K, M, in_o, out_o, torch.bfloat16, seed=in_o + 131 * out_o + M)
+    rest = (in_o, out_o, c["kw"], c["kwt"], c["alpha"].cuda(), c["beta"].cuda())
+
+    def odd(t):   # the same rows one element off 8-byte alignment
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+    pair = K.hadamard_linear_bwd(c["x"].cuda(), c["gy"].cuda(), *rest, latent=c["lc"])
+    general = K.hadamard_linear_bwd(odd(c["x"]), odd(c["gy"]), *rest, latent=c["lc"])
+    assert torch.equal(pair[0], general[0])
+    ref = ohad.hadamard_linear_bwd_f64(c["x"].double().numpy(), c["codes"], c["alpha"].double().numpy(),
+                                       c["beta"].double().numpy(), c["gy"].double().numpy(),
+                                       latent=c["latent"].double().numpy())
+    for name, a, b, r in zip(("gx", "dalpha", "dbeta", "dweight"), pair, general, ref):
+        assert_close(a.float().cpu().numpy(), b.double().cpu().numpy(), torch.float32, f"{name} pair vs general")
+        assert_close(a.float().cpu().numpy(), r, torch.bfloat16, f"{name} {in_o}x{out_o} M={M}")
+
+
 def test_hadamard_bwd_partial_outputs_and_determinism(K):
     c = make_case(K, 500, 16, 16, torch.bfloat16, seed=9)
     args = (c["x"].cuda(), c["gy"].cuda(), 16, 16, c["kw"], c["kwt"], c["alpha"].cuda(), c["beta"].cuda())

@@ -356,7 +356,6 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1 && VEC) ? 2 : 1) void had
 // and stage 16 pairs slots u and u + 8 locally.
 // Several layers on the same input rows (q, k, v): workgroup b runs layer
 // b % n over tiles b / n, b / n + G / n, ... as hadamard_fwdn_kernel does.
-constexpr int kPairThreads = 128;
 // Above this many 16-row tiles per layer the one-wavefront kernel (its next
 // tile's loads in flight during the current one's output) is faster once the
 // rows come from HBM rather than the Infinity Cache: 65,536 bf16 rows from
@@ -527,36 +526,9 @@ __device__ __forceinline__ void pair_tile(const HadArgs &a, int tile, int lane,
 // inputs of groups 16 HF + s; on return acc[u] holds group g_out(u) before
 // beta.
 template <int HF, bool DENSE>
-__device__ __forceinline__ void pair_core(const HadArgs &a, int lane, f32x4 *xch, uint4 w0,
-                                          uint4 w1, f32x4 (&v)[16], f32x4 (&acc)[16]) {
-    f32x4 *mine = xch + HF * 8 * 64, *theirs = xch + (1 - HF) * 8 * 64;
-#pragma unroll
-    for (int h = 1; h < 16; h <<= 1) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            if (s & h) continue;
-            const f32x4 x0 = v[s], x1 = v[s + h];
-            v[s] = x0 + x1;
-            v[s + h] = x0 - x1;
-        }
-    }
-    lds_barrier();   // the partner is done reading the previous exchange
-#pragma unroll
-    for (int j = 0; j < 8; ++j) mine[j * 64 + lane] = v[HF ? j : j + 8];
-    lds_barrier();
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const f32x4 other = theirs[j * 64 + lane];
-        if (HF == 0) {
-            const f32x4 x0 = v[j], x1 = other;
-            v[j] = x0 + x1;
-            v[j + 8] = x0 - x1;
-        } else {
-            const f32x4 x0 = other, x1 = v[j + 8];
-            v[j] = x0 + x1;
-            v[j + 8] = x0 - x1;
-        }
-    }
+__device__ __forceinline__ void pair_core(const HadArgs &a, int lane, f32x4 *xch, uint4 w0, uint4 w1, f32x4 (&v)[16],
+                                          f32x4 (&acc)[16]) {
+    pair_in<HF>(v, xch, lane);
     u32x2 xm[16];
 #pragma unroll
     for (int s = 0; s < 16; ++s) xm[s] = u32x2{pack_bf16x2(v[s].x, v[s].y), pack_bf16x2(v[s].z, v[s].w)};
@@ -564,7 +536,7 @@ __device__ __forceinline__ void pair_core(const HadArgs &a, int lane, f32x4 *xch
     if constexpr (DENSE) {
         const uint2 *wf = (const uint2 *)a.kw;   // [32 g][64 lanes] bf16x4
 #pragma unroll
-        for (int s = 0; s < 16; ++s) wd[s] = wf[(8 * HF + (s & 7) + 16 * (s >> 3)) * 64 + lane];
+        for (int s = 0; s < 16; ++s) wd[s] = wf[pair_gin<HF>(s) * 64 + lane];
     }
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
@@ -573,46 +545,14 @@ __device__ __forceinline__ void pair_core(const HadArgs &a, int lane, f32x4 *xch
             wa = wd[s];
         } else {
             const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-            const int g = 8 * HF + (s & 7) + 16 * (s >> 3);
+            const int g = pair_gin<HF>(s);
             wa = codes_bf16x4(wb[g >> 2], g & 3);
         }
         acc[s] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, wa),
                                                             __builtin_bit_cast(i16x4, xm[s]),
                                                             f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     }
-#pragma unroll
-    for (int h = 1; h < 8; h <<= 1) {
-#pragma unroll
-        for (int s = 0; s < 16; ++s) {
-            if (s & h) continue;
-            const f32x4 x0 = acc[s], x1 = acc[s + h];
-            acc[s] = x0 + x1;
-            acc[s + h] = x0 - x1;
-        }
-    }
-    lds_barrier();   // the partner is done reading the input exchange
-#pragma unroll
-    for (int p = 0; p < 8; ++p) {
-        const int snd = (p & 3) + 4 * (1 - HF) + 8 * (p >> 2);
-        mine[p * 64 + lane] = acc[snd];
-    }
-    lds_barrier();
-#pragma unroll
-    for (int p = 0; p < 8; ++p) {
-        const int kept = (p & 3) + 4 * HF + 8 * (p >> 2);
-        const int lo = kept & ~4, hi = kept | 4;
-        const f32x4 other = theirs[p * 64 + lane];
-        const f32x4 x0 = HF == 0 ? acc[kept] : other;
-        const f32x4 x1 = HF == 0 ? other : acc[kept];
-        acc[lo] = x0 + x1;
-        acc[hi] = x0 - x1;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const f32x4 x0 = acc[u], x1 = acc[u + 8];
-        acc[u] = x0 + x1;
-        acc[u + 8] = x0 - x1;
-    }
+    pair_out<HF>(acc, xch, lane);
 }
 
 template <int HF>

@@ -17,7 +17,9 @@
 // Every product above is H0 ... H0 / 32, so the kernels run unnormalised
 // transforms and the reduction applies the 1/32.
 //
-// Kernel: hadamard_bwd_kernel, one launch with three workgroup roles.
+// Kernel: hadamard_bwd_kernel (float32, and bf16 rows without 8-byte
+// alignment) or hadamard_bwd_pair_kernel (bf16), one launch with three
+// workgroup roles.
 //   dW role: per (token range, output tile, input chunk), H0(beta .* gy) and
 //     H0(alpha .* x) in the forward lane layout (lane = token, 4 columns),
 //     turned into token-major fragments by a matrix-core product with the
@@ -86,6 +88,22 @@ __device__ __forceinline__ void fill_scale(f32x4 *__restrict__ dst, const float 
         for (int j = 0; j < 4; ++j) v[j] = (i0 + j < n) ? (s ? s[g * n + i0 + j] : 1.f) * mul : 0.f;
         dst[e] = v;
     }
+}
+
+// One chunk of such a table (128 threads, 128 entries): entry q*32 + g holds
+// s[g][16c + 4q .. +3]; buffer loads with no branch around them.
+__device__ __forceinline__ void fill_scale_chunk(f32x4 *__restrict__ dst, const float *__restrict__ s, int n, int c,
+                                                 float mul, int tid) {
+    const int g = tid & 31, i0 = kKChunk * c + 4 * (tid >> 5);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(s, s ? (uint32_t)(32 * n * 4) : 0u);
+    uint32_t raw[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        raw[j] = __builtin_amdgcn_raw_buffer_load_b32(r, i0 + j < n ? (uint32_t)(g * n + i0 + j) * 4 : kOOB, 0, 0);
+    f32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = i0 + j < n ? (s ? __uint_as_float(raw[j]) : 1.f) * mul : 0.f;
+    dst[tid] = v;
 }
 
 // ---------------------------------------------------------------- reduce-epilogue pass
@@ -319,6 +337,182 @@ __global__ __launch_bounds__(kThreads, 1) void hadamard_bwd_kernel(BwdJob j) {
     bwd_red_role<T, BF16MMA, VEC, false>(j.b, j.rb, blk - j.nA, smem);
 }
 
+// ---------------------------------------------------------------- bf16: wavefront pairs
+// The same three roles for bf16 rows in 8-byte pieces, each workgroup a
+// pair of wavefronts that splits a 16-token tile by group (hadamard_core.h):
+// 64 accumulator registers instead of 128 for the sums and 64 for the
+// products, so two wavefronts fit a SIMD and a role's rows spread over twice
+// the wavefronts.  One wavefront per tile with 512 registers left a single
+// wavefront per SIMD with nothing to cover its loads and its 32-deep
+// transforms.  dx is bitwise the one-wavefront kernel's; the sums over rows
+// group differently.  A role's tile range per workgroup follows from
+// pair_plan.  Latency bound at small row counts.  Measured (kernel alone):
+// 512 -> 512 features, 8,192 rows 64 -> 34 us, 32,768 rows 103 -> 65 us; whole
+// calls (with the reduction) 512 -> 1408 at 8,192 rows 126 -> 53 us, 1024 -> 1024
+// at 16,384 rows 163 -> 108 us, 4096 -> 4096 at 4,096 rows 417 -> 429 us.
+__device__ __forceinline__ void pair_scale(f32x4 (&v)[16], const u32x2 (&raw)[16], const f32x4 *al) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        v[k] = bf16x4_f32(raw[k]) * al[k];
+        if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // bounds the scale reads in flight
+    }
+}
+
+template <int HF, bool STORE>
+__device__ __forceinline__ void pair_red_role(const HadArgs &a, const BwdRed &r, int blk, int lane, unsigned char *smem) {
+    const f32x4 *alpha_l = (const f32x4 *)smem;          // [Kc][4][32]
+    const f32x4 *beta_l = alpha_l + a.Kc * 128;          // [4][32] of this output tile
+    f32x4 *xch = (f32x4 *)beta_l + 128;
+    const int t = lane & 15, q = lane >> 4;
+    const int nt = blk % a.Nt, s = blk / a.Nt;
+    const int n_tiles = (int)ceil_div(a.M, kTile);
+    const int t0 = s * r.tps, t1 = min(t0 + r.tps, n_tiles);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, x_bytes(a, 2));
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, STORE ? (uint32_t)((int64_t)a.M * a.ldy * 2) : 0u);
+    const __amdgpu_buffer_rsrc_t ar = make_rsrc(r.aux, (uint32_t)((int64_t)a.M * r.ld_aux * 2));
+    const int o0 = kNTile * nt + 4 * q;
+    const uint32_t gsx = (uint32_t)a.gsx * 2, gsa = (uint32_t)r.gs_aux * 2, gsy = (uint32_t)a.gsy * 2;
+    f32x4 red[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) red[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tile = t0; tile < t1; ++tile) {
+        const int row = tile * kTile + t;
+        const bool row_ok = row < a.M;
+        f32x4 acc[16];
+        auto chunk = [&](int c, auto first) {
+            const int i0 = kKChunk * c + 4 * q;
+            u32x2 raw[16];
+            pair_load<HF>(xr, row_ok && i0 < a.in_o ? x_row_off(a, row, 2) + (uint32_t)i0 * 2 : kOOB, gsx, raw);
+            uint4 w0, w1;
+            load_w(a, nt, c, lane, w0, w1);
+            f32x4 v[16];
+            pair_scale(v, raw, alpha_l + (c * 4 + q) * 32 + 16 * HF);
+            pair_in<HF>(v, xch, lane);
+            const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int g = pair_gin<HF>(k);
+                const u32x2 xm = {pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)};
+                acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    __builtin_bit_cast(i16x4, codes_bf16x4(wb[g >> 2], g & 3)), __builtin_bit_cast(i16x4, xm),
+                    decltype(first)::value ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[k], 0, 0, 0);
+                if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        chunk(0, std::true_type{});
+        for (int c = 1; c < a.Kc; ++c) chunk(c, std::false_type{});
+        // the auxiliary rows, behind the output transform
+        const uint32_t ao = row_ok && o0 < a.out_o ? (uint32_t)((int64_t)row * r.ld_aux * 2) + (uint32_t)o0 * 2 : kOOB;
+        u32x2 aux[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            aux[u] = __builtin_amdgcn_raw_buffer_load_b64(ar, ao, (uint32_t)pair_gout<HF>(u) * gsa, 0);
+        pair_out<HF>(acc, xch, lane);
+        const uint32_t yo = row_ok && o0 < a.out_o ? (uint32_t)((int64_t)row * a.ldy * 2) + (uint32_t)o0 * 2 : kOOB;
+        const f32x4 *bl = beta_l + q * 32;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int h = pair_gout<HF>(u);
+            red[u] += acc[u] * bf16x4_f32(aux[u]);
+            if constexpr (STORE) Buf4<uint16_t>::store(acc[u] * bl[h], yr, yo, (uint32_t)h * gsy);
+            if ((u & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    const int W = a.Nt * kNTile;
+    float *dst = r.part + (int64_t)s * 32 * W + o0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        f32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = row_sum16(red[u][j]);
+        if (t == 0) *(f32x4 *)(dst + (int64_t)pair_gout<HF>(u) * W) = v;
+    }
+}
+
+template <int HF>
+__device__ __forceinline__ void pair_dw_role(const HadArgs &ax, const HadArgs &ag, const BwdDW &d, int blk, int lane,
+                                             unsigned char *smem) {
+    const f32x4 *alpha_l = (const f32x4 *)smem;          // [4][32] of this input chunk
+    const f32x4 *beta_l = alpha_l + 128;                 // [4][32] of this output tile
+    f32x4 *xch = (f32x4 *)beta_l + 128;
+    const int t = lane & 15, q = lane >> 4;
+    const int Kc = ax.Kc, Nt = ag.Kc;
+    const int c = blk % Kc, nt = (blk / Kc) % Nt, s = blk / (Kc * Nt);
+    const int n_tiles = (int)ceil_div(ax.M, kTile);
+    const int t0 = s * d.tps, t1 = min(t0 + d.tps, n_tiles);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(ax.x, x_bytes(ax, 2));
+    const __amdgpu_buffer_rsrc_t gr = make_rsrc(ag.x, x_bytes(ag, 2));
+    const int i0 = kKChunk * c + 4 * q, o0 = kNTile * nt + 4 * q;
+    const uint32_t gsx = (uint32_t)ax.gsx * 2, gsg = (uint32_t)ag.gsx * 2;
+    // identity B fragment: lane (n, kq) holds I[4kq + j][n]
+    uint2 id_b;
+    id_b.x = (4 * q + 0 == t ? 0x3f80u : 0u) | (4 * q + 1 == t ? 0x3f800000u : 0u);
+    id_b.y = (4 * q + 2 == t ? 0x3f80u : 0u) | (4 * q + 3 == t ? 0x3f800000u : 0u);
+    f32x4 dw[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) dw[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int tile = t0; tile < t1; ++tile) {
+        const int row = tile * kTile + t;
+        const bool row_ok = row < ax.M;
+        u32x2 rg[16], rx[16];
+        pair_load<HF>(gr, row_ok && o0 < ag.in_o ? x_row_off(ag, row, 2) + (uint32_t)o0 * 2 : kOOB, gsg, rg);
+        pair_load<HF>(xr, row_ok && i0 < ax.in_o ? x_row_off(ax, row, 2) + (uint32_t)i0 * 2 : kOOB, gsx, rx);
+        f32x4 v[16];
+        pair_scale(v, rg, beta_l + q * 32 + 16 * HF);
+        pair_in<HF>(v, xch, lane);
+        uint2 gt[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            gt[k] = transpose_bf16(uint2{pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)}, id_b);
+        pair_scale(v, rx, alpha_l + q * 32 + 16 * HF);
+        pair_in<HF>(v, xch, lane);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const uint2 xt = transpose_bf16(uint2{pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)}, id_b);
+            dw[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, gt[k]),
+                                                               __builtin_bit_cast(i16x4, xt), dw[k], 0, 0, 0);
+        }
+    }
+    // lane (n, mq) of group g holds dW_g[o = 16nt + 4mq + j][i = 16c + n]
+    const int Op = Nt * kNTile, Ip = Kc * kKChunk;
+    float *dst = d.part + (int64_t)s * 32 * Op * Ip + kKChunk * c + t;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dst[((int64_t)pair_gin<HF>(k) * Op + o0 + j) * Ip] = dw[k][j];
+}
+
+template <bool STORE>
+__global__ __launch_bounds__(kPairThreads, 2) void hadamard_bwd_pair_kernel(BwdJob j) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, hf = tid >> 6, lane = tid & 63;
+    int blk = blockIdx.x;
+    f32x4 *tab = (f32x4 *)smem;
+    if (blk < j.nW) {
+        const int c = blk % j.wx.Kc, nt = (blk / j.wx.Kc) % j.wg.Kc;
+        fill_scale_chunk(tab, j.wx.alpha, j.wx.in_o, c, 1.f, tid);
+        fill_scale_chunk(tab + 128, j.wg.alpha, j.wg.in_o, nt, 1.f, tid);
+        __syncthreads();
+        if (hf == 0) pair_dw_role<0>(j.wx, j.wg, j.dw, blk, lane, smem);
+        else pair_dw_role<1>(j.wx, j.wg, j.dw, blk, lane, smem);
+        return;
+    }
+    blk -= j.nW;
+    const bool first = blk < j.nA;
+    if (!first) blk -= j.nA;
+    const HadArgs &a = first ? j.a : j.b;
+    for (int c = 0; c < a.Kc; ++c) fill_scale_chunk(tab + c * 128, a.alpha, a.in_o, c, 1.f, tid);
+    if (STORE && first) fill_scale_chunk(tab + a.Kc * 128, a.beta, a.out_o, blk % a.Nt, kCodeScale, tid);
+    __syncthreads();
+    if (first) {
+        if (hf == 0) pair_red_role<0, STORE>(j.a, j.ra, blk, lane, smem);
+        else pair_red_role<1, STORE>(j.a, j.ra, blk, lane, smem);
+    } else {
+        if (hf == 0) pair_red_role<0, false>(j.b, j.rb, blk, lane, smem);
+        else pair_red_role<1, false>(j.b, j.rb, blk, lane, smem);
+    }
+}
+
 // ---------------------------------------------------------------- final reduction
 
 struct BwdSum {
@@ -331,8 +525,11 @@ struct BwdSum {
     float *da, *db, *dw;  // null: not wanted
 };
 
-constexpr int kSumCols = 64;     // partial columns per workgroup
-constexpr int kSumPhases = 16;   // partial rows summed in parallel, s = phase mod 16
+// 32 columns x 32 rows in flight: a layer of 16x16 groups has 8,192 dW columns
+// (256 workgroups), and each thread's loads are independent (unrolled); 64 x
+// 16 left half the CUs idle (512 partial rows: 10.8 -> 5.3 us).
+constexpr int kSumCols = 32;     // partial columns per workgroup
+constexpr int kSumPhases = 32;   // partial rows summed in parallel, s = phase mod 32
 
 __host__ __device__ inline int64_t sum_blocks(const BwdSum &r, int64_t *bw, int64_t *ba) {
     *bw = r.dw ? ceil_div((int64_t)32 * r.Op * r.Ip, kSumCols) : 0;
@@ -342,8 +539,8 @@ __host__ __device__ inline int64_t sum_blocks(const BwdSum &r, int64_t *bw, int6
 }
 
 // Column sums of the partial arrays P[S][N] (each partial row contiguous):
-// thread (column, phase) sums rows phase, phase + 16, ... in order, then
-// phase 0 adds the 16 phase sums in order; then the 1/32, the output
+// thread (column, phase) sums rows phase, phase + 32, ... in order, then
+// phase 0 adds the 32 phase sums in order; then the 1/32, the output
 // mapping (padded columns dropped) and the STE mask.
 __global__ __launch_bounds__(kSumCols * kSumPhases) void hadamard_bwd_reduce_kernel(BwdSum r) {
     __shared__ double part[kSumPhases][kSumCols];
@@ -365,8 +562,10 @@ __global__ __launch_bounds__(kSumCols * kSumPhases) void hadamard_bwd_reduce_ker
     const int cx = threadIdx.x % kSumCols, ph = threadIdx.x / kSumCols;
     const int64_t n = blk * kSumCols + cx;
     double acc = 0.0;
-    if (n < N)
+    if (n < N) {
+#pragma unroll 8
         for (int s = ph; s < S; s += kSumPhases) acc += (double)P[(int64_t)s * N + n];
+    }
     part[ph][cx] = acc;
     __syncthreads();
     if (ph != 0 || n >= N) return;
@@ -413,9 +612,28 @@ static int split_count(int n_tiles, int per_split_min, int64_t target, int *tps)
     return (int)ceil_div(n_tiles, *tps);
 }
 
-static BwdChunk plan_chunk(int64_t rows, int in_o, int out_o) {
+// Pair kernel: the workgroups that are resident at once (two wavefronts per
+// SIMD, a pair per workgroup) take equal shares of the roles' tile steps: a
+// step is one input chunk of a tile's transform (a dW step two, x and gy).
+// At least two tiles per dW workgroup: each writes 32 KB of partial sums.
+static BwdChunk pair_plan(int n_tiles, int Nt, int Kc) {
+    const int64_t T = n_tiles, slots = (int64_t)device_info().cu_count * 4;
+    const int64_t U = ceil_div(2 * T * Nt * Kc + 2 * T * Nt * Kc, slots);
+    auto split = [&](int64_t tps, int *out_tps) {
+        *out_tps = (int)(tps < 1 ? 1 : tps);
+        return (int)ceil_div(T, *out_tps);
+    };
+    BwdChunk p;
+    p.Sa = split(U / Nt, &p.tpa);   // dx / dalpha: Nt chunks per tile
+    p.Sb = split(U / Kc, &p.tpb);
+    p.Sw = split(U / 2 < 2 ? 2 : U / 2, &p.tpw);
+    return p;
+}
+
+static BwdChunk plan_chunk(int64_t rows, int in_o, int out_o, bool pair) {
     const int n_tiles = (int)ceil_div(rows, kTile);
     const int Nt = (int)ceil_div(out_o, kNTile), Kc = (int)ceil_div(in_o, kKChunk);
+    if (pair) return pair_plan(n_tiles, Nt, Kc);
     const int64_t waves = (int64_t)device_info().cu_count;  // per red role
     BwdChunk p;
     p.Sa = split_count(n_tiles, 1, ceil_div(waves, Kc), &p.tpa);  // transposed layer: Kc output tiles
@@ -430,7 +648,7 @@ struct BwdLayout {
     int64_t off_b, off_w, bytes;        // byte offsets of the dbeta / dW partials, total
 };
 
-static BwdLayout plan(int64_t M, int64_t in_o, int64_t out_o, int64_t ld, int64_t esz) {
+static BwdLayout plan(int64_t M, int64_t in_o, int64_t out_o, int64_t ld, int64_t esz, bool pair) {
     BwdLayout L{};
     int64_t rows_max = (int64_t)kMaxBufferBytes / (ld * esz);
     rows_max = rows_max / kTile * kTile;
@@ -441,7 +659,7 @@ static BwdLayout plan(int64_t M, int64_t in_o, int64_t out_o, int64_t ld, int64_
     L.rows_max = balanced_rows(M, rows_max, kTile);
     for (int64_t r0 = 0; r0 < M; r0 += L.rows_max) {
         const int64_t rows = (M - r0) < L.rows_max ? (M - r0) : L.rows_max;
-        const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o);
+        const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o, pair);
         L.Sa += p.Sa;
         L.Sb += p.Sb;
         L.Sw += p.Sw;
@@ -476,7 +694,19 @@ WALSH_EXPORT int64_t walsh_hadamard_bwd_workspace_bytes(int64_t M, int64_t in_o,
     if (M <= 0 || in_o <= 0 || out_o <= 0 || in_o > 65536 || out_o > 65536) return 0;
     const int64_t esz = dtype == WALSH_BF16 ? 2 : 4;
     const int64_t ld = 32 * (in_o > out_o ? in_o : out_o);
-    return plan(M, in_o, out_o, ld, esz).bytes;
+    const int64_t general = plan(M, in_o, out_o, ld, esz, false).bytes;
+    if (dtype != WALSH_BF16) return general;
+    // The pair kernel's need is bounded by the resident workgroups, not only
+    // by this shape's own split: callers size the workspace with padded group
+    // counts, whose split differs.  With U = ceil(4 T Nt Kc / slots) and the
+    // tile counts of pair_plan, Sw Nt Kc <= 0.625 slots + Nt Kc, Sa Kc <=
+    // slots / 2 + Kc and Sb Nt <= slots / 2 + Nt per row chunk.
+    const BwdLayout L = plan(M, in_o, out_o, ld, esz, true);
+    if (L.rows_max == 0) return general;
+    const int64_t slots = (int64_t)device_info().cu_count * 4, Nt = ceil_div(out_o, kNTile), Kc = ceil_div(in_o, kKChunk);
+    const int64_t bound = (5 * slots / 8 + 1 + Nt * Kc) * 32 * 1024 + (slots + 2 + Nt + Kc) * 32 * 16 * 4 + 1024;
+    const int64_t pair = ceil_div(M, L.rows_max) * bound;
+    return pair > general ? pair : general;
 }
 
 WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_t gsx, const void *gy, int64_t ldg,
@@ -502,7 +732,12 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     int64_t ld = ldx > ldg ? ldx : ldg;
     if (gx && ldgx > ld) ld = ldgx;
     // the workspace query assumes dense rows; strided rows may need more chunks
-    const BwdLayout L = plan(M, in_o, out_o, ld, esz);
+    const size_t valign = bf16 ? 8 : 16;
+    const bool vec = gsy % 4 == 0 && gsx % 4 == 0 && ldx % 4 == 0 && ldg % 4 == 0 && (!gx || ldgx % 4 == 0) &&
+                     (uintptr_t)gy % valign == 0 && (uintptr_t)x % valign == 0 && (!gx || (uintptr_t)gx % valign == 0);
+    // bf16 rows in 8-byte pieces: wavefront pairs
+    const bool pair = bf16 && vec;
+    const BwdLayout L = plan(M, in_o, out_o, ld, esz, pair);
     if (M > 0 && L.rows_max == 0) return set_error(WALSH_ENOTSUP, "%s: row stride too large", fn);
     if (M > 0 && (!workspace || workspace_bytes < L.bytes))
         return set_error(WALSH_EINVAL, "%s: workspace of %lld bytes < %lld needed", fn, (long long)workspace_bytes,
@@ -513,7 +748,6 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     float *pa = (float *)workspace;
     float *pb = (float *)((char *)workspace + L.off_b);
     float *pw = (float *)((char *)workspace + L.off_w);
-    const size_t valign = bf16 ? 8 : 16;
     const int64_t maxlds = device_info().max_shared_per_block;
 
     int64_t ia = 0, ib = 0, iw = 0;  // partial rows written so far
@@ -523,7 +757,7 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     if ((int64_t)(lds_red + shape_reserve(bf16)) > maxlds || (int64_t)lds > maxlds) return set_error(WALSH_ENOTSUP, "%s: shape needs %zu B of LDS", fn, lds);
     for (int64_t r0 = 0; r0 < M; r0 += L.rows_max) {
         const int64_t rows = (M - r0) < L.rows_max ? (M - r0) : L.rows_max;
-        const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o);
+        const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o, pair);
         const char *xc = (const char *)x + r0 * ldx * esz;
         const char *gc = (const char *)gy + r0 * ldg * esz;
         char *gxc = gx ? (char *)gx + r0 * ldgx * esz : nullptr;
@@ -546,14 +780,14 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
         j.a.gsx = (int)gsy; j.a.gsy = (int)gsx; j.a.kw = kweight_t; j.a.alpha = beta; j.a.beta = alpha;
         j.a.beta_h = (int)in_o; j.a.y = gxc; j.a.ldy = gx ? ldgx : 0;
         j.ra = BwdRed{xc, ldx, (int)gsx, pa + ia * 32 * Ap, p.Sa, p.tpa};
-        j.nA = need_a ? (int)ceil_div((int64_t)p.Sa * Kc, kWaves) : 0;
+        j.nA = need_a ? (pair ? p.Sa * Kc : (int)ceil_div((int64_t)p.Sa * Kc, kWaves)) : 0;
         // the layer on x without beta or store, aux = gy (dbeta)
         base(j.b);
         j.b.x = xc; j.b.ldx = ldx; j.b.in_o = (int)in_o; j.b.out_o = (int)out_o; j.b.Nt = Nt; j.b.Kc = Kc;
         j.b.gsx = (int)gsx; j.b.gsy = (int)gsy; j.b.kw = kweight; j.b.alpha = alpha; j.b.beta = nullptr;
         j.b.beta_h = 0; j.b.y = nullptr; j.b.ldy = 0;
         j.rb = BwdRed{gc, ldg, (int)gsy, pb + ib * 32 * Bp, p.Sb, p.tpb};
-        j.nB = need_b ? (int)ceil_div((int64_t)p.Sb * Nt, kWaves) : 0;
+        j.nB = need_b ? (pair ? p.Sb * Nt : (int)ceil_div((int64_t)p.Sb * Nt, kWaves)) : 0;
         // x and gy as transform inputs (dW)
         base(j.wx);
         j.wx.x = xc; j.wx.ldx = ldx; j.wx.in_o = (int)in_o; j.wx.Kc = Kc; j.wx.gsx = (int)gsx; j.wx.alpha = alpha;
@@ -561,14 +795,14 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
         j.wg.x = gc; j.wg.ldx = ldg; j.wg.in_o = (int)out_o; j.wg.Kc = Nt; j.wg.gsx = (int)gsy; j.wg.alpha = beta;
         j.dw = BwdDW{pw + iw * 32 * (int64_t)Bp * Ap, p.Sw, p.tpw};
         j.nW = need_w ? p.Sw * Nt * Kc : 0;
-        const bool vec = gsy % 4 == 0 && gsx % 4 == 0 && ldx % 4 == 0 && ldg % 4 == 0 &&
-                         (!gx || ldgx % 4 == 0) && (uintptr_t)gc % valign == 0 && (uintptr_t)xc % valign == 0 &&
-                         (!gx || (uintptr_t)gxc % valign == 0);
         const dim3 G((unsigned)(j.nW + j.nA + j.nB)), B(kThreads);
 #define WALSH_BWD(T, MMA, V, ST) launch((hadamard_bwd_kernel<T, MMA, V, ST>), G, B, lds, s, j)
-        if (bf16) {
-            if (vec) { if (gx) WALSH_BWD(uint16_t, true, true, true); else WALSH_BWD(uint16_t, true, true, false); }
-            else     { if (gx) WALSH_BWD(uint16_t, true, false, true); else WALSH_BWD(uint16_t, true, false, false); }
+        if (pair) {
+            const size_t plds = (size_t)16 * 128 * ((Nt > Kc ? Nt : Kc) + 1) + kPairXch;
+            if (gx) launch(hadamard_bwd_pair_kernel<true>, G, dim3(kPairThreads), plds, s, j);
+            else launch(hadamard_bwd_pair_kernel<false>, G, dim3(kPairThreads), plds, s, j);
+        } else if (bf16) {
+            if (gx) WALSH_BWD(uint16_t, true, false, true); else WALSH_BWD(uint16_t, true, false, false);
         } else {
             if (vec) { if (gx) WALSH_BWD(float, false, true, true); else WALSH_BWD(float, false, true, false); }
             else     { if (gx) WALSH_BWD(float, false, false, true); else WALSH_BWD(float, false, false, false); }

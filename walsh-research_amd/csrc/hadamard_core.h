@@ -280,4 +280,93 @@ __device__ __forceinline__ void contract_dense(const unsigned char *__restrict__
     }
 }
 
+// ---------------------------------------------------------------- wavefront pairs
+// A 16-token tile split over a pair of wavefronts by group (HF = 0, 1): a
+// wavefront holds 16 groups, slot s of the input = group 16 HF + s.  The
+// exchange area xch is [2 HF][8][64 lanes] f32x4.  Both wavefronts run the
+// same barriers.
+constexpr int kPairThreads = 128;
+constexpr size_t kPairXch = (size_t)2 * 8 * 64 * 16;
+
+// group of slot s after the input transform, of slot u after the output one
+template <int HF> constexpr int pair_gin(int s) { return 8 * HF + (s & 7) + 16 * (s >> 3); }
+template <int HF> constexpr int pair_gout(int u) { return (u & 3) + 4 * HF + 8 * ((u >> 2) & 1) + 16 * (u >> 3); }
+
+// Input transform: stages 1..8 within the wavefront, 16 across the pair (each
+// sends the 8 slots the other needs and keeps both results of its pairs).
+template <int HF>
+__device__ __forceinline__ void pair_in(f32x4 (&v)[16], f32x4 *xch, int lane) {
+    f32x4 *mine = xch + HF * 8 * 64, *theirs = xch + (1 - HF) * 8 * 64;
+#pragma unroll
+    for (int h = 1; h < 16; h <<= 1) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            if (s & h) continue;
+            const f32x4 x0 = v[s], x1 = v[s + h];
+            v[s] = x0 + x1;
+            v[s + h] = x0 - x1;
+        }
+    }
+    lds_barrier();   // the partner is done reading the previous exchange
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mine[j * 64 + lane] = v[HF ? j : j + 8];
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const f32x4 other = theirs[j * 64 + lane];
+        const f32x4 x0 = HF == 0 ? v[j] : other, x1 = HF == 0 ? other : v[j + 8];
+        v[j] = x0 + x1;
+        v[j + 8] = x0 - x1;
+    }
+}
+
+// Output transform: stages 1, 2, 4 within the slots, 8 across the pair, 16
+// within the slots.
+template <int HF>
+__device__ __forceinline__ void pair_out(f32x4 (&acc)[16], f32x4 *xch, int lane) {
+    f32x4 *mine = xch + HF * 8 * 64, *theirs = xch + (1 - HF) * 8 * 64;
+#pragma unroll
+    for (int h = 1; h < 8; h <<= 1) {
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            if (s & h) continue;
+            const f32x4 x0 = acc[s], x1 = acc[s + h];
+            acc[s] = x0 + x1;
+            acc[s + h] = x0 - x1;
+        }
+    }
+    lds_barrier();   // the partner is done reading the input exchange
+#pragma unroll
+    for (int p = 0; p < 8; ++p) mine[p * 64 + lane] = acc[(p & 3) + 4 * (1 - HF) + 8 * (p >> 2)];
+    lds_barrier();
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+        const int kept = (p & 3) + 4 * HF + 8 * (p >> 2);
+        const int lo = kept & ~4, hi = kept | 4;
+        const f32x4 other = theirs[p * 64 + lane];
+        const f32x4 x0 = HF == 0 ? acc[kept] : other;   // group with bit 3 clear
+        const f32x4 x1 = HF == 0 ? other : acc[kept];   // its partner + 8
+        acc[lo] = x0 + x1;
+        acc[hi] = x0 - x1;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const f32x4 x0 = acc[u], x1 = acc[u + 8];
+        acc[u] = x0 + x1;
+        acc[u + 8] = x0 - x1;
+    }
+}
+
+// The lane's 4 columns c4.. of groups 16 HF + s of its row, raw bf16 (zeros
+// past the row / column limits: off is kOOB).
+template <int HF>
+__device__ __forceinline__ void pair_load(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t gstride, u32x2 (&raw)[16]) {
+#pragma unroll
+    for (int s = 0; s < 16; ++s) raw[s] = __builtin_amdgcn_raw_buffer_load_b64(r, off, (uint32_t)(16 * HF + s) * gstride, 0);
+}
+__device__ __forceinline__ f32x4 bf16x4_f32(u32x2 u) {
+    return f32x4{__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u), __uint_as_float(u.y << 16),
+                 __uint_as_float(u.y & 0xffff0000u)};
+}
+
 }  // namespace walsh
