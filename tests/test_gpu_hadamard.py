@@ -186,6 +186,26 @@ def test_hadamard_wide_bf16(K, in_o, out_o, M):
     assert_close(y, ref, torch.bfloat16, f"wide in_o={in_o} out_o={out_o} M={M}")
 
 
+@pytest.mark.parametrize("M,pad", [(257, 0), (272, 8), (4105, 0)])
+def test_hadamard_wide_whole_rows_equal_general(K, M, pad):
+    """The 128x128 bf16 kernel moves 16-byte aligned rows of 4,096 contiguous
+    values whole; rows off that alignment or with a stride that is not a
+    multiple of 8 take the 8-byte loads.  Same arithmetic: equal bitwise, on
+    ragged last tiles, padded strides and several tiles per workgroup."""
+    g = torch.Generator().manual_seed(M)
+    codes = torch.randint(-1, 2, (32, 128, 128), generator=g).numpy().astype(np.int8)
+    kw = _prepare(K, codes)
+    alpha, beta = (1 + 0.5 * torch.randn(32, 128, generator=g)).cuda(), (0.1 * torch.randn(32, 128, generator=g)).cuda()
+    x = torch.randn(M, 4096, generator=g).to(torch.bfloat16)
+
+    def rows(stride, off):
+        buf = torch.zeros(M * stride + off, dtype=torch.bfloat16, device="cuda")
+        return buf[off:off + M * stride].view(M, stride)[:, :4096].copy_(x)
+    whole = K.hadamard_linear(rows(4096 + pad, 0), 128, 128, kw, alpha, beta)
+    assert torch.equal(whole, K.hadamard_linear(rows(4096, 4), 128, 128, kw, alpha, beta))
+    assert torch.equal(whole, K.hadamard_linear(rows(4096 + 4, 0), 128, 128, kw, alpha, beta))
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 1000])
 def test_hadamard_linear_row_tails(K, M):
     rng = np.random.default_rng(M)
