@@ -206,6 +206,48 @@ def test_hadamard_wide_whole_rows_equal_general(K, M, pad):
     assert torch.equal(whole, K.hadamard_linear(rows(4096 + 4, 0), 128, 128, kw, alpha, beta))
 
 
+@pytest.mark.parametrize("in_o,out_o,M", [(24, 24, 1), (24, 20, 17), (64, 24, 127), (80, 36, 16), (8, 24, 8192), (16, 64, 8193),
+                                          (24, 16, 4096), (24, 8, 4112), (48, 12, 5000), (16, 16, 16384), (4, 4, 40)])
+def test_hadamard_pair_linear_equals_general(K, in_o, out_o, M):
+    """bf16 layers of a few chunks and output tiles on wavefront pairs, across
+    the dispatch's row counts, ragged widths and tiles: bitwise the general
+    kernel's rows (taken by rows one element off 8-byte alignment), with and
+    without RoPE, and padded group strides."""
+    g = torch.Generator().manual_seed(in_o * 100 + out_o + M)
+    codes = torch.randint(-1, 2, (32, out_o, in_o), generator=g).numpy().astype(np.int8)
+    kw = _prepare(K, codes)
+    alpha, beta = (1 + 0.5 * torch.randn(32, in_o, generator=g)).cuda(), (0.1 * torch.randn(32, out_o, generator=g)).cuda()
+    x = torch.randn(M, 32 * in_o, generator=g).to(torch.bfloat16).cuda()
+
+    def off(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+    y = K.hadamard_linear(x, in_o, out_o, kw, alpha, beta)
+    assert torch.equal(y, K.hadamard_linear(off(x), in_o, out_o, kw, alpha, beta))
+    pad = torch.full((M, 32, in_o + 4), 7.0, dtype=torch.bfloat16, device="cuda")
+    pad[..., :in_o] = x.view(M, 32, in_o)
+    z = K.hadamard_linear(pad.view(M, -1), in_o, out_o, kw, alpha, beta, gsx=in_o + 4, gsy=out_o + 4)
+    assert torch.equal(z.view(M, 32, out_o + 4)[..., :out_o], y.view(M, 32, out_o))
+    ref = ohad.hadamard_linear_f64(x[:64].double().cpu().numpy(), codes, alpha.double().cpu().numpy(),
+                                   beta.double().cpu().numpy())
+    assert_close(y[:64].float().cpu().numpy(), ref, torch.bfloat16, f"pair linear {in_o}x{out_o} M={M}")
+
+
+@pytest.mark.parametrize("in_o,hid_o,M", [(8, 24, 33), (16, 44, 1), (24, 64, 500), (32, 88, 130), (80, 20, 17)])
+def test_hadamard_pair_swiglu_equals_general(K, in_o, hid_o, M):
+    """The SwiGLU on wavefront pairs is bitwise the general kernel's (rows one
+    element off 8-byte alignment): one and five input chunks, ragged output
+    tiles and rows, every output tile of a token tile."""
+    g = torch.Generator().manual_seed(in_o + hid_o + M)
+    layers = []
+    for _ in range(2):
+        codes = torch.randint(-1, 2, (32, hid_o, in_o), generator=g).numpy().astype(np.int8)
+        layers.append((_prepare(K, codes), (1 + 0.5 * torch.randn(32, in_o, generator=g)).cuda(),
+                       (0.3 * torch.randn(32, hid_o, generator=g)).cuda()))
+    x = torch.randn(M, 32 * in_o, generator=g).to(torch.bfloat16).cuda()
+    xo = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view(x.shape).copy_(x)
+    assert torch.equal(K.hadamard_swiglu(x, in_o, hid_o, *layers), K.hadamard_swiglu(xo, in_o, hid_o, *layers))
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 1000])
 def test_hadamard_linear_row_tails(K, M):
     rng = np.random.default_rng(M)

@@ -2015,6 +2015,155 @@ __global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, Ha
     }
 }
 
+// ---------------------------------------------------------------- pairs, several chunks or output tiles
+// bf16 linear and SwiGLU on wavefront pairs for layers of a few 16-wide
+// input chunks and output tiles (n_embd 768 and 1024): a workgroup is one
+// pair and one (token tile, output tile), the chunks in order through one
+// accumulator chain, so results equal hadamard_fwd_kernel's and
+// hadamard_swiglu_kernel's bitwise.  Those hold a whole tile per wavefront
+// (350 registers: one wavefront per SIMD, a 32-deep chain per chunk); a
+// pair halves both and two or three pairs cover each other's latencies.
+// The gate result of the SwiGLU stays in registers as bf16 (both
+// projections leave the same groups in a lane), so there is no stash.
+// Latency bound.  6,007 rows, n_embd 768: SwiGLU 60 -> 44 us, down projection
+// 42 -> 23 us; n_embd 1024: SwiGLU 97 -> 63 us.
+template <int HF>
+__device__ __forceinline__ void pair_linear_item(const HadArgs &a, int tile, int nt, int lane, unsigned char *smem) {
+    const f32x4 *alpha_l = (const f32x4 *)smem;          // [Kc][4][32]
+    const f32x4 *beta_l = alpha_l + a.Kc * 128;          // [4][32] of this output tile
+    f32x4 *xch = (f32x4 *)beta_l + 128;
+    const int t = lane & 15, q = lane >> 4;
+    const int row = tile * kTile + t;
+    const bool row_ok = row < a.M;
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, x_bytes(a, 2));
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, (uint32_t)((int64_t)a.M * a.ldy * 2));
+    f32x4 acc[16];
+    pair_contract<HF>(a, xr, row_ok ? x_row_off(a, row, 2) : 0u, row_ok, nt, lane, alpha_l, xch, acc);
+    pair_out<HF>(acc, xch, lane);
+    const int o0 = kNTile * nt + 4 * q;
+    const bool ok = row_ok && o0 < a.out_o;
+    const uint32_t yo = ok ? (uint32_t)((int64_t)row * a.ldy * 2) + (uint32_t)o0 * 2 : kOOB;
+    const uint32_t gsy = (uint32_t)a.gsy * 2;
+    const f32x4 *bl = beta_l + q * 32;
+    if (a.rope) {
+        const f32x4 cs = ok ? rope_cs(a, row, o0) : f32x4{1.f, 0.f, 1.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int h = pair_gout<HF>(u);
+            Buf4<uint16_t>::store(rope_apply(acc[u] * bl[h], cs), yr, yo, (uint32_t)h * gsy);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int h = pair_gout<HF>(u);
+            Buf4<uint16_t>::store(acc[u] * bl[h], yr, yo, (uint32_t)h * gsy);
+        }
+    }
+}
+
+__global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_linear_kernel(HadArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    int tile, nt;
+    pair_item((int)blockIdx.x, (int)ceil_div(a.M, kTile), a.Nt, tile, nt);
+    f32x4 *tab = (f32x4 *)smem;
+    for (int c = 0; c < a.Kc; ++c) fill_scale_chunk(tab + c * 128, a.alpha, a.in_o, a.in_o, c, 1.f, tid);
+    fill_scale_chunk(tab + a.Kc * 128, a.beta, a.out_o, a.beta_h, nt, kCodeScale, tid);
+    __syncthreads();
+    if (tid < 64) pair_linear_item<0>(a, tile, nt, lane, smem);
+    else pair_linear_item<1>(a, tile, nt, lane, smem);
+}
+
+template <int HF>
+__device__ __forceinline__ void pair_swiglu_item(const HadArgs &g, const HadArgs &u, int tile, int nt, int lane,
+                                                 unsigned char *smem) {
+    const f32x4 *ag_l = (const f32x4 *)smem;             // [Kc][4][32]
+    const f32x4 *au_l = ag_l + g.Kc * 128;
+    const f32x4 *bg_l = au_l + g.Kc * 128;               // [4][32] of this output tile
+    const f32x4 *bu_l = bg_l + 128;
+    f32x4 *xch = (f32x4 *)bu_l + 128;
+    const int t = lane & 15, q = lane >> 4;
+    const int row = tile * kTile + t;
+    const bool row_ok = row < g.M;
+    const uint32_t xo = row_ok ? (uint32_t)((int64_t)row * g.ldx * 2) : 0u;
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.ldx * 2));
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(g.y, (uint32_t)((int64_t)g.M * g.ldy * 2));
+    f32x4 acc[16];
+    pair_contract<HF>(g, xr, xo, row_ok, nt, lane, ag_l, xch, acc);
+    pair_out<HF>(acc, xch, lane);
+    u32x2 gate[16];   // bf16, as the gate projection's own result would be
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const f32x4 v = acc[k] * bg_l[q * 32 + pair_gout<HF>(k)];
+        gate[k] = u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
+        // opaque: packed here, not where it is used (64 registers until then)
+        asm volatile("" : "+v"(gate[k].x), "+v"(gate[k].y));
+        if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    // opaque: the rows are loaded again (from the caches) instead of being
+    // kept through the gate projection
+    uint32_t xo2 = xo;
+    asm volatile("" : "+v"(xo2)::"memory");
+    __builtin_amdgcn_sched_barrier(0);
+    pair_contract<HF>(u, xr, xo2, row_ok, nt, lane, au_l, xch, acc);
+    pair_out<HF>(acc, xch, lane);
+    const int o0 = kNTile * nt + 4 * q;
+    const uint32_t yo = row_ok && o0 < g.out_o ? (uint32_t)((int64_t)row * g.ldy * 2) + (uint32_t)o0 * 2 : kOOB;
+    const uint32_t gsy = (uint32_t)g.gsy * 2;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const int h = pair_gout<HF>(k);
+        const f32x4 uv = acc[k] * bu_l[q * 32 + h], gv = bf16x4_f32(gate[k]);
+        f32x4 hv;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hv[j] = silu_fast(gv[j]) * uv[j];
+        Buf4<uint16_t>::store(hv, yr, yo, (uint32_t)h * gsy);
+        if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+__global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_swiglu_kernel(HadArgs g, HadArgs u) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    int tile, nt;
+    pair_item((int)blockIdx.x, (int)ceil_div(g.M, kTile), g.Nt, tile, nt);
+    f32x4 *tab = (f32x4 *)smem;
+    for (int c = 0; c < g.Kc; ++c) {
+        fill_scale_chunk(tab + c * 128, g.alpha, g.in_o, g.in_o, c, 1.f, tid);
+        fill_scale_chunk(tab + (g.Kc + c) * 128, u.alpha, g.in_o, g.in_o, c, 1.f, tid);
+    }
+    fill_scale_chunk(tab + 2 * g.Kc * 128, g.beta, g.out_o, g.out_o, nt, kCodeScale, tid);
+    fill_scale_chunk(tab + (2 * g.Kc + 1) * 128, u.beta, g.out_o, g.out_o, nt, kCodeScale, tid);
+    __syncthreads();
+    if (tid < 64) pair_swiglu_item<0>(g, u, tile, nt, lane, smem);
+    else pair_swiglu_item<1>(g, u, tile, nt, lane, smem);
+}
+
+// Input chunks up to which the pair kernels hold their tables beside the
+// exchange area with four workgroups per CU.
+constexpr int kPairLinMaxKc = 5;
+
+// Linear layers that hadamard_pair_linear_kernel takes (bf16, 8-byte pieces,
+// not the wide kernel's shapes).  Measured us, other kernel -> this one, at
+// 64 / 1,024 / 6,007 / 16,384 / 65,536 rows, in_o -> out_o:
+//   several chunks and output tiles, always:  24 -> 24  19.5 19.8 23.2 34.5 114
+//     -> 7.8 8.1 13.5 31.5 100;  64 -> 24  33.1 33.6 41.6 94.4 -> 12.7 13.5 23.1 58.0
+//   one chunk, several output tiles: the other kernel transforms a tile once
+//     for all of them and wins once the chip is full:  16 -> 24  10.3 10.6 13.7
+//     21.1 63.3 -> 6.0 6.3 10.8 23.5 75.6;  16 -> 64  16.0 16.7 20.8 38.3 -> 6.1 6.7
+//     18.7 40.8
+//   several chunks, one output tile: the chunk-parallel kernel has the
+//     shorter chain while its pairs fit, and at four chunks keeps it longer:
+//     24 -> 16  7.6 7.8 11.7 18.4 61.1 -> 7.8 8.0 11.1 17.7 55.7;  64 -> 16  11.0
+//     11.5 21.6 42.6 -> 12.7 13.3 18.2 46.3
+//   one of each: 16 -> 16  6.4 6.6 9.7 14.9 34.9 -> 6.0 6.1 8.9 14.3 45.2
+static bool pair_linear_shape(int Kc, int Nt, int64_t tiles) {
+    if (Kc > kPairLinMaxKc) return false;
+    if (Kc == 1) return tiles <= (Nt == 1 ? kPairMaxTilesRows : 512);
+    if (Nt == 1) return Kc <= 3 && tiles > 256;
+    return true;
+}
+
 // ---------------------------------------------------------------- standalone FHT
 // Normalised (or not) fast Walsh-Hadamard transform of rows of length
 // N = 2^logN (fht_cuda.py:281-309): rows staged in LDS, log2(N) butterfly
@@ -2266,7 +2415,14 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
         }
         if (grid > cap) grid = cap;
         const dim3 G((unsigned)grid), B(kThreads);
-        if (swiglu) {
+        if (swiglu && bf16 && vec && Kc <= kPairLinMaxKc) {
+            HadArgs ua = *ubase;
+            ua.x = a.x;
+            ua.y = a.y;
+            ua.M = a.M;
+            launch(hadamard_pair_swiglu_kernel, dim3((unsigned)(ceil_div(rows, kTile) * Nt)), dim3(kPairThreads),
+                   (size_t)16 * 128 * (2 * Kc + 2) + kPairXch, s, a, ua);
+        } else if (swiglu) {
             HadArgs ua = *ubase;
             ua.x = a.x;
             ua.y = a.y;
@@ -2276,13 +2432,16 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
 #define WALSH_SW_LAUNCH(T, MMA, V, K1) launch((hadamard_swiglu_kernel<T, MMA, V, K1>), G, B, sw_lds, s, a, ua)
             const bool one = Kc == 1;
             if (bf16) {
-                if (vec) { if (one) WALSH_SW_LAUNCH(uint16_t, true, true, true); else WALSH_SW_LAUNCH(uint16_t, true, true, false); }
+                if (vec) WALSH_SW_LAUNCH(uint16_t, true, true, false);   // more than kPairLinMaxKc chunks
                 else     { if (one) WALSH_SW_LAUNCH(uint16_t, true, false, true); else WALSH_SW_LAUNCH(uint16_t, true, false, false); }
             } else {
                 if (vec) { if (one) WALSH_SW_LAUNCH(float, false, true, true); else WALSH_SW_LAUNCH(float, false, true, false); }
                 else     { if (one) WALSH_SW_LAUNCH(float, false, false, true); else WALSH_SW_LAUNCH(float, false, false, false); }
             }
 #undef WALSH_SW_LAUNCH
+        } else if (bf16 && vec && !wide3 && pair_linear_shape(Kc, Nt, ceil_div(rows, kTile))) {
+            launch(hadamard_pair_linear_kernel, dim3((unsigned)(ceil_div(rows, kTile) * Nt)), dim3(kPairThreads),
+                   (size_t)16 * 128 * (Kc + 1) + kPairXch, s, a);
         } else if (wide3 && rows <= kSplitRows) {
             HadArgsN an;
             an.n = 1;

@@ -90,22 +90,6 @@ __device__ __forceinline__ void fill_scale(f32x4 *__restrict__ dst, const float 
     }
 }
 
-// One chunk of such a table (128 threads, 128 entries): entry q*32 + g holds
-// s[g][16c + 4q .. +3]; buffer loads with no branch around them.
-__device__ __forceinline__ void fill_scale_chunk(f32x4 *__restrict__ dst, const float *__restrict__ s, int n, int c,
-                                                 float mul, int tid) {
-    const int g = tid & 31, i0 = kKChunk * c + 4 * (tid >> 5);
-    const __amdgpu_buffer_rsrc_t r = make_rsrc(s, s ? (uint32_t)(32 * n * 4) : 0u);
-    uint32_t raw[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        raw[j] = __builtin_amdgcn_raw_buffer_load_b32(r, i0 + j < n ? (uint32_t)(g * n + i0 + j) * 4 : kOOB, 0, 0);
-    f32x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = i0 + j < n ? (s ? __uint_as_float(raw[j]) : 1.f) * mul : 0.f;
-    dst[tid] = v;
-}
-
 // ---------------------------------------------------------------- reduce-epilogue pass
 
 struct BwdRed {
@@ -350,14 +334,6 @@ __global__ __launch_bounds__(kThreads, 1) void hadamard_bwd_kernel(BwdJob j) {
 // 512 -> 512 features, 8,192 rows 64 -> 34 us, 32,768 rows 103 -> 65 us; whole
 // calls (with the reduction) 512 -> 1408 at 8,192 rows 126 -> 53 us, 1024 -> 1024
 // at 16,384 rows 163 -> 108 us, 4096 -> 4096 at 4,096 rows 417 -> 429 us.
-__device__ __forceinline__ void pair_scale(f32x4 (&v)[16], const u32x2 (&raw)[16], const f32x4 *al) {
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-        v[k] = bf16x4_f32(raw[k]) * al[k];
-        if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // bounds the scale reads in flight
-    }
-}
-
 template <int HF, bool STORE>
 __device__ __forceinline__ void pair_red_role(const HadArgs &a, const BwdRed &r, int blk, int lane, unsigned char *smem) {
     const f32x4 *alpha_l = (const f32x4 *)smem;          // [Kc][4][32]
@@ -371,7 +347,7 @@ __device__ __forceinline__ void pair_red_role(const HadArgs &a, const BwdRed &r,
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, STORE ? (uint32_t)((int64_t)a.M * a.ldy * 2) : 0u);
     const __amdgpu_buffer_rsrc_t ar = make_rsrc(r.aux, (uint32_t)((int64_t)a.M * r.ld_aux * 2));
     const int o0 = kNTile * nt + 4 * q;
-    const uint32_t gsx = (uint32_t)a.gsx * 2, gsa = (uint32_t)r.gs_aux * 2, gsy = (uint32_t)a.gsy * 2;
+    const uint32_t gsa = (uint32_t)r.gs_aux * 2, gsy = (uint32_t)a.gsy * 2;
     f32x4 red[16];
 #pragma unroll
     for (int u = 0; u < 16; ++u) red[u] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -379,28 +355,7 @@ __device__ __forceinline__ void pair_red_role(const HadArgs &a, const BwdRed &r,
         const int row = tile * kTile + t;
         const bool row_ok = row < a.M;
         f32x4 acc[16];
-        auto chunk = [&](int c, auto first) {
-            const int i0 = kKChunk * c + 4 * q;
-            u32x2 raw[16];
-            pair_load<HF>(xr, row_ok && i0 < a.in_o ? x_row_off(a, row, 2) + (uint32_t)i0 * 2 : kOOB, gsx, raw);
-            uint4 w0, w1;
-            load_w(a, nt, c, lane, w0, w1);
-            f32x4 v[16];
-            pair_scale(v, raw, alpha_l + (c * 4 + q) * 32 + 16 * HF);
-            pair_in<HF>(v, xch, lane);
-            const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                const int g = pair_gin<HF>(k);
-                const u32x2 xm = {pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)};
-                acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                    __builtin_bit_cast(i16x4, codes_bf16x4(wb[g >> 2], g & 3)), __builtin_bit_cast(i16x4, xm),
-                    decltype(first)::value ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[k], 0, 0, 0);
-                if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        chunk(0, std::true_type{});
-        for (int c = 1; c < a.Kc; ++c) chunk(c, std::false_type{});
+        pair_contract<HF>(a, xr, row_ok ? x_row_off(a, row, 2) : 0u, row_ok, nt, lane, alpha_l, xch, acc);
         // the auxiliary rows, behind the output transform
         const uint32_t ao = row_ok && o0 < a.out_o ? (uint32_t)((int64_t)row * r.ld_aux * 2) + (uint32_t)o0 * 2 : kOOB;
         u32x2 aux[16];
@@ -490,8 +445,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_bwd_pair_kernel(BwdJ
     f32x4 *tab = (f32x4 *)smem;
     if (blk < j.nW) {
         const int c = blk % j.wx.Kc, nt = (blk / j.wx.Kc) % j.wg.Kc;
-        fill_scale_chunk(tab, j.wx.alpha, j.wx.in_o, c, 1.f, tid);
-        fill_scale_chunk(tab + 128, j.wg.alpha, j.wg.in_o, nt, 1.f, tid);
+        fill_scale_chunk(tab, j.wx.alpha, j.wx.in_o, j.wx.in_o, c, 1.f, tid);
+        fill_scale_chunk(tab + 128, j.wg.alpha, j.wg.in_o, j.wg.in_o, nt, 1.f, tid);
         __syncthreads();
         if (hf == 0) pair_dw_role<0>(j.wx, j.wg, j.dw, blk, lane, smem);
         else pair_dw_role<1>(j.wx, j.wg, j.dw, blk, lane, smem);
@@ -501,8 +456,8 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_bwd_pair_kernel(BwdJ
     const bool first = blk < j.nA;
     if (!first) blk -= j.nA;
     const HadArgs &a = first ? j.a : j.b;
-    for (int c = 0; c < a.Kc; ++c) fill_scale_chunk(tab + c * 128, a.alpha, a.in_o, c, 1.f, tid);
-    if (STORE && first) fill_scale_chunk(tab + a.Kc * 128, a.beta, a.out_o, blk % a.Nt, kCodeScale, tid);
+    for (int c = 0; c < a.Kc; ++c) fill_scale_chunk(tab + c * 128, a.alpha, a.in_o, a.in_o, c, 1.f, tid);
+    if (STORE && first) fill_scale_chunk(tab + a.Kc * 128, a.beta, a.out_o, a.out_o, blk % a.Nt, kCodeScale, tid);
     __syncthreads();
     if (first) {
         if (hf == 0) pair_red_role<0, STORE>(j.a, j.ra, blk, lane, smem);

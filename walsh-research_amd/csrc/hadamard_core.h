@@ -369,4 +369,72 @@ __device__ __forceinline__ f32x4 bf16x4_f32(u32x2 u) {
                  __uint_as_float(u.y & 0xffff0000u)};
 }
 
+
+// v = raw * alpha for the lane's 16 groups (al[k]: group 16 HF + k).
+__device__ __forceinline__ void pair_scale(f32x4 (&v)[16], const u32x2 (&raw)[16], const f32x4 *al) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        v[k] = bf16x4_f32(raw[k]) * al[k];
+        if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // bounds the scale reads in flight
+    }
+}
+
+// Output tile nt of the layer on the lane's row, before the output transform:
+// acc[k] of group pair_gin(k), summed over the input chunks in order.
+// alpha_l: [Kc][4][32] scales in LDS.
+template <int HF>
+__device__ __forceinline__ void pair_contract(const HadArgs &a, __amdgpu_buffer_rsrc_t xr, uint32_t row_off, bool row_ok,
+                                              int nt, int lane, const f32x4 *alpha_l, f32x4 *xch, f32x4 (&acc)[16]) {
+    const int q = lane >> 4;
+    auto chunk = [&](int c, auto first) {
+        const int i0 = kKChunk * c + 4 * q;
+        u32x2 raw[16];
+        pair_load<HF>(xr, row_ok && i0 < a.in_o ? row_off + (uint32_t)i0 * 2 : kOOB, (uint32_t)a.gsx * 2, raw);
+        uint4 w0, w1;
+        load_w(a, nt, c, lane, w0, w1);
+        f32x4 v[16];
+        pair_scale(v, raw, alpha_l + (c * 4 + q) * 32 + 16 * HF);
+        pair_in<HF>(v, xch, lane);
+        const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int g = pair_gin<HF>(k);
+            const u32x2 xm = {pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)};
+            acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                __builtin_bit_cast(i16x4, codes_bf16x4(wb[g >> 2], g & 3)), __builtin_bit_cast(i16x4, xm),
+                decltype(first)::value ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[k], 0, 0, 0);
+            if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    chunk(0, std::true_type{});
+    for (int c = 1; c < a.Kc; ++c) chunk(c, std::false_type{});
+}
+
+// One chunk of a scale table (128 threads, 128 entries): entry q*32 + g holds
+// s[g][16c + 4q .. +3] * mul, rows of s at a stride of ld (zeros past n, ones
+// * mul if s is null); buffer loads with no branch around them.
+__device__ __forceinline__ void fill_scale_chunk(f32x4 *__restrict__ dst, const float *__restrict__ s, int n, int ld,
+                                                 int c, float mul, int tid) {
+    const int g = tid & 31, i0 = kKChunk * c + 4 * (tid >> 5);
+    const __amdgpu_buffer_rsrc_t r = make_rsrc(s, s ? (uint32_t)((31 * ld + n) * 4) : 0u);
+    uint32_t raw[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        raw[j] = __builtin_amdgcn_raw_buffer_load_b32(r, i0 + j < n ? (uint32_t)(g * ld + i0 + j) * 4 : kOOB, 0, 0);
+    f32x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = i0 + j < n ? (s ? __uint_as_float(raw[j]) : 1.f) * mul : 0.f;
+    dst[tid] = v;
+}
+
+// (tile, output tile) of workgroup b in a launch of n_tiles * Nt workgroups:
+// consecutive workgroups go to the 8 XCDs in turn, so the Nt output tiles of
+// a token tile sit 8 apart and read its rows from one L2 (a last partial
+// group of 8 Nt keeps b / Nt, b % Nt).
+__device__ __forceinline__ void pair_item(int b, int n_tiles, int Nt, int &tile, int &nt) {
+    const int full = n_tiles / 8 * 8 * Nt;
+    nt = b < full ? (b / 8) % Nt : b % Nt;
+    tile = b < full ? (b / (8 * Nt)) * 8 + b % 8 : b / Nt;
+}
+
 }  // namespace walsh

@@ -168,7 +168,15 @@ def _whole_rows(in_o, out_o, ldx, dt, ptr):
 def _pair_shape(rows, in_o, out_o, dt, vec, rope=False, whole_rows=False):
     """The pair kernel the library dispatches for this shape, or None."""
     limit = PAIR_MAX_TILES_ROWS if whole_rows else PAIR_MAX_TILES
-    if dt != torch.bfloat16 or not vec or out_o > 16 or (rows + 15) // 16 > limit:
+    tiles, kc, nt = (rows + 15) // 16, (in_o + 15) // 16, (out_o + 15) // 16
+    if dt != torch.bfloat16 or not vec:
+        return None
+    if kc > 1 and nt >= 4 and in_o <= 128 and out_o <= 128:
+        return None
+    if kc <= 5 and (tiles <= (PAIR_MAX_TILES_ROWS if nt == 1 else 512) if kc == 1 else
+                    kc <= 3 and tiles > 256 if nt == 1 else True):
+        return "hadamard_pair_linear_kernel"
+    if out_o > 16 or tiles > limit:
         return None
     if in_o <= 16:
         return "hadamard_pair_kernel"
@@ -181,7 +189,8 @@ def _had_meta(rows, in_o, out_o, dt, vec, kc1, swiglu=False, rope=False, whole_r
     esz = 2 if dt == torch.bfloat16 else 4
     tag = "bf16" if dt == torch.bfloat16 else "f32"
     if swiglu:
-        kname = "hadamard_swiglu_kernel<%s,%s>" % (tag, "vec" if vec else "scalar")
+        kname = "hadamard_pair_swiglu_kernel<bf16>" if dt == torch.bfloat16 and vec and in_o <= 80 else \
+            "hadamard_swiglu_kernel<%s,%s>" % (tag, "vec" if vec else "scalar")
         nbytes = rows * 32 * (in_o + out_o) * esz + 2 * 32 * out_o * ((in_o + 3) // 4) + 8 * 32 * (in_o + out_o)
         flops = rows * 2 * (2 * 32 * in_o * out_o + 10 * 32 * (in_o + out_o)) + rows * 32 * out_o * 4
     else:
@@ -340,9 +349,10 @@ def hadamard_linear_multi(x: torch.Tensor, in_o: int, out_o: int, layers, freqs_
     kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt, True, in_o <= 16)
     nbytes = rows * 32 * (in_o + n * out_o) * x.element_size()
     whole = _whole_rows(in_o, out_o, ldx, dt, xv.data_ptr()) and all(o is None for o in outs)
-    kname = ("hadamard_pair_kernel<bf16,x%d>" % n) \
-        if _pair_shape(rows, in_o, out_o, dt, True, whole_rows=whole) == "hadamard_pair_kernel" \
-        else "hadamard_fwdn_kernel<%s,x%d%s>" % ("bf16" if dt == torch.bfloat16 else "f32", n, ",rows" if whole else "")
+    pair = dt == torch.bfloat16 and in_o <= 16 and out_o <= 16 and \
+        (rows + 15) // 16 <= (PAIR_MAX_TILES_ROWS if whole else PAIR_MAX_TILES)
+    kname = ("hadamard_pair_kernel<bf16,x%d>" % n) if pair else \
+        "hadamard_fwdn_kernel<%s,x%d%s>" % ("bf16" if dt == torch.bfloat16 else "f32", n, ",rows" if whole else "")
     rope_args = (0 if table is None else table.data_ptr(), T, head_dim or 4, mask, _hip.dtype_code(dt),
                  _hip.stream(x.device))
     if all(o is None for o in outs):
