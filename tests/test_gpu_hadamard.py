@@ -358,6 +358,16 @@ def test_hadamard_mlp_equals_swiglu_then_down(K, M, in_o, hid_o):
     assert_close(y[torch.from_numpy(rows).cuda()].float().cpu().numpy(), ref, torch.bfloat16, f"mlp M={M}")
 
 
+@pytest.mark.parametrize("M,in_o,hid_o", [(16 * 257 + 16, 16, 43), (16 * 258 + 1, 4, 33), (16 * 256, 8, 48), (17, 4, 17),
+                                          (16 * 768 + 16 * 8 + 5, 16, 32)])
+def test_hadamard_mlp_tile_pairs(K, M, in_o, hid_o):
+    """The fused MLP where a workgroup takes two token tiles side by side
+    (three hidden tiles, more token tiles than CUs): even and odd counts and a
+    last tile of one row, the largest launch below it, and two hidden tiles
+    past one round of workgroups.  Same bitwise comparison and oracle."""
+    test_hadamard_mlp_equals_swiglu_then_down(K, M, in_o, hid_o)
+
+
 def test_launch_timer_records_kernel_time(K):
     """walsh_timing_*: every entry-point call inside LaunchTimer gets its
     kernel's own duration (hipExtLaunchKernelGGL events)."""

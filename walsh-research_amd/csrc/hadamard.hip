@@ -1796,225 +1796,6 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
     }
 }
 
-// ---------------------------------------------------------------- fused MLP
-// down(silu(gate(x)) * up(x)) (SwiGLUMLP.forward, chassis.py:498-504) in one
-// launch, for bf16 rows with in_o <= 16 (n_embd 512), a hidden width of two
-// or three 16-wide tiles (16 < hid_o <= 48) and a down projection with
-// out_o <= 16.  A workgroup takes one 16-token tile at a time:
-//   - wave nt < Nt runs the SwiGLU item of hidden tile nt as
-//     hadamard_swiglu_kernel does (gate into its LDS area, up, silu(g) u),
-//     rounds the hidden values to bf16 as that kernel's store does, and runs
-//     the down projection's input transform of chunk nt on them in
-//     registers: hidden tile nt's columns 16 nt + 4q .. +3 are exactly
-//     chunk nt's in the lane layout load_transform reads, so nothing is
-//     rearranged.  The transformed chunk (bf16, 16 KB) replaces the gate
-//     stash in the wave's area;
-//   - after a barrier wave 3 contracts the chunks in order into one
-//     accumulator chain (the one-wavefront chunk loop's order) and, after a
-//     second barrier that frees the areas for the next tile, runs the output
-//     transform, beta and the stores, overlapping the next tile's items.
-// The hidden activation never leaves the CU, and the output equals
-// walsh_hadamard_swiglu_fwd followed by the down projection bitwise.
-constexpr int kMlpDownWave = 3;
-
-__global__ __launch_bounds__(kThreads, 2) void hadamard_mlp_kernel(HadArgs g, HadArgs u, HadArgs d) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int Nt = g.Nt;                                  // hidden tiles = down chunks (2 or 3)
-    f32x4 *ag_l = (f32x4 *)smem;                          // [1][4][32]
-    f32x4 *au_l = ag_l + 128;
-    f32x4 *bg_l = au_l + 128;                             // [Nt][4][32]
-    f32x4 *bu_l = bg_l + Nt * 128;
-    f32x4 *ad_l = bu_l + Nt * 128;                        // [Nt][4][32] down alpha per chunk
-    f32x4 *bd_l = ad_l + Nt * 128;                        // [1][4][32]
-    uint2 *areas = (uint2 *)(bd_l + 128);                 // [3][32][64]
-
-    const int tid = threadIdx.x;
-    // alpha / beta of the three layers: every load issued before any
-    // conversion (buffer loads, zero past the shapes, no branch around them;
-    // a conversion or branch right after a load waits for it)
-    {
-        const __amdgpu_buffer_rsrc_t gar = make_rsrc(g.alpha, (uint32_t)(32 * g.in_o * 4));
-        const __amdgpu_buffer_rsrc_t uar = make_rsrc(u.alpha, (uint32_t)(32 * g.in_o * 4));
-        const __amdgpu_buffer_rsrc_t dbr = make_rsrc(d.beta, (uint32_t)((31 * d.beta_h + d.out_o) * 4));
-        const __amdgpu_buffer_rsrc_t gbr = make_rsrc(g.beta, (uint32_t)(32 * g.out_o * 4));
-        const __amdgpu_buffer_rsrc_t ubr = make_rsrc(u.beta, (uint32_t)(32 * g.out_o * 4));
-        const __amdgpu_buffer_rsrc_t dar = make_rsrc(d.alpha, (uint32_t)(32 * d.in_o * 4));
-        constexpr int kIt = (3 * 128 + kThreads - 1) / kThreads;   // Nt <= 3
-        uint32_t r1[3][4], r2[kIt][3][4];
-        {
-            const int e = tid, gg = e & 31, i0 = 4 * (e >> 5);
-            const bool live = e < 128;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool ok = live && i0 + j < g.in_o, okd = live && i0 + j < d.out_o;
-                r1[0][j] = __builtin_amdgcn_raw_buffer_load_b32(gar, ok ? (uint32_t)(gg * g.in_o + i0 + j) * 4 : kOOB, 0, 0);
-                r1[1][j] = __builtin_amdgcn_raw_buffer_load_b32(uar, ok ? (uint32_t)(gg * g.in_o + i0 + j) * 4 : kOOB, 0, 0);
-                r1[2][j] = __builtin_amdgcn_raw_buffer_load_b32(
-                    dbr, okd ? (uint32_t)(gg * d.beta_h + i0 + j) * 4 : kOOB, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int it = 0; it < kIt; ++it) {
-            const int e = tid + it * kThreads, h = e & 31, o0 = 4 * (e >> 5);
-            const bool live = e < Nt * 128;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool ok = live && o0 + j < g.out_o, okd = live && o0 + j < d.in_o;
-                r2[it][0][j] = __builtin_amdgcn_raw_buffer_load_b32(gbr, ok ? (uint32_t)(h * g.out_o + o0 + j) * 4 : kOOB, 0, 0);
-                r2[it][1][j] = __builtin_amdgcn_raw_buffer_load_b32(ubr, ok ? (uint32_t)(h * g.out_o + o0 + j) * 4 : kOOB, 0, 0);
-                r2[it][2][j] = __builtin_amdgcn_raw_buffer_load_b32(
-                    dar, okd ? (uint32_t)(h * d.in_o + o0 + j) * 4 : kOOB, 0, 0);
-            }
-        }
-        if (tid < 128) {
-            const int e = tid, i0 = 4 * (e >> 5);
-            f32x4 va, vb, vd;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool ok = i0 + j < g.in_o;
-                va[j] = ok ? __uint_as_float(r1[0][j]) : 0.f;
-                vb[j] = ok ? __uint_as_float(r1[1][j]) : 0.f;
-                vd[j] = i0 + j < d.out_o ? __uint_as_float(r1[2][j]) * kCodeScale : 0.f;
-            }
-            ag_l[e] = va;
-            au_l[e] = vb;
-            bd_l[e] = vd;
-        }
-#pragma unroll
-        for (int it = 0; it < kIt; ++it) {
-            const int e = tid + it * kThreads, o0 = 4 * (e >> 5);
-            if (e >= Nt * 128) continue;
-            f32x4 va, vb, vd;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool ok = o0 + j < g.out_o;
-                va[j] = ok ? __uint_as_float(r2[it][0][j]) * kCodeScale : 0.f;
-                vb[j] = ok ? __uint_as_float(r2[it][1][j]) * kCodeScale : 0.f;
-                vd[j] = o0 + j < d.in_o ? __uint_as_float(r2[it][2][j]) : 0.f;  // chunk e / 128, element (h, o0 + j)
-            }
-            bg_l[e] = va;
-            bu_l[e] = vb;
-            ad_l[e] = vd;
-        }
-    }
-    __syncthreads();
-
-    const int lane = tid & 63;
-    // logical wave: the down wave rotates over the SIMDs with the workgroup
-    const int wave = ((tid >> 6) - (int)blockIdx.x) & (kWaves - 1);
-    const int t = lane & 15, q = lane >> 4;
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.ldx * 2));
-    const __amdgpu_buffer_rsrc_t yr = make_rsrc(d.y, (uint32_t)((int64_t)d.M * d.ldy * 2));
-    const int n_tiles = (int)ceil_div(g.M, kTile);
-    for (int tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int row = tile * kTile + t;
-        const bool row_ok = row < g.M;
-        if (wave < Nt) {
-            const int nt = wave;
-            uint2 *st = areas + wave * 32 * 64;
-            const uint32_t xoff = (uint32_t)((int64_t)row * g.ldx * 2);
-            f32x4 acc[32];
-            {   // gate, into the area
-                XM<true> xm;
-                load_transform<uint16_t, true, true>(g, xr, xoff, row_ok, 0, q, ag_l, xm);
-#pragma unroll
-                for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(g, nt, 0, lane, xm, acc);
-            }
-            fht32x4(acc);
-            {
-                const f32x4 *bl = bg_l + (nt * 4 + q) * 32;
-#pragma unroll
-                for (int h0 = 0; h0 < 32; h0 += 4) {
-                    f32x4 b4[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) b4[j] = bl[h0 + j];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const f32x4 v = acc[h0 + j] * b4[j];
-                        st[(h0 + j) * 64 + lane] = uint2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            {   // up
-                XM<true> xm;
-                load_transform<uint16_t, true, true>(g, xr, xoff, row_ok, 0, q, au_l, xm);
-#pragma unroll
-                for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(u, nt, 0, lane, xm, acc);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            fht32x4(acc);
-            __builtin_amdgcn_sched_barrier(0);
-            // h = bf16(silu(g) u) (the SwiGLU kernel's stored value), then
-            // the down projection's alpha for chunk nt (zero past hid_o, so
-            // those columns contribute zeros, as the down projection's
-            // out-of-range loads do)
-            {
-                const f32x4 *bl = bu_l + (nt * 4 + q) * 32;
-                const f32x4 *al = ad_l + (nt * 4 + q) * 32;
-#pragma unroll
-                for (int h0 = 0; h0 < 32; h0 += 4) {
-                    f32x4 b4[4], a4[4];
-                    uint2 e4[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        b4[j] = bl[h0 + j];
-                        a4[j] = al[h0 + j];
-                        e4[j] = st[(h0 + j) * 64 + lane];
-                    }
-#pragma unroll
-                    for (int j4 = 0; j4 < 4; ++j4) {
-                        const int h = h0 + j4;
-                        const f32x4 uv = acc[h] * b4[j4];
-                        const uint2 e = e4[j4];
-                        const f32x4 gv{__uint_as_float(e.x << 16), __uint_as_float(e.x & 0xffff0000u),
-                                       __uint_as_float(e.y << 16), __uint_as_float(e.y & 0xffff0000u)};
-                        f32x4 hv;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) hv[j] = silu_fast(gv[j]) * uv[j];
-                        const uint32_t p0 = pack_bf16x2(hv.x, hv.y), p1 = pack_bf16x2(hv.z, hv.w);
-                        const f32x4 hb{__uint_as_float(p0 << 16), __uint_as_float(p0 & 0xffff0000u),
-                                       __uint_as_float(p1 << 16), __uint_as_float(p1 & 0xffff0000u)};
-                        acc[h] = hb * a4[j4];
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-            fht32x4(acc);
-            __builtin_amdgcn_sched_barrier(0);
-            // the transformed chunk replaces the gate stash (this wave's own
-            // area: its reads above are done, LDS operations run in order)
-            wave_lds_fence();
-#pragma unroll
-            for (int h = 0; h < 32; ++h)
-                st[h * 64 + lane] = uint2{pack_bf16x2(acc[h].x, acc[h].y), pack_bf16x2(acc[h].z, acc[h].w)};
-            lds_barrier();  // A: the chunks are in the areas
-            lds_barrier();  // B: the down wave has read them
-        } else if (wave == kMlpDownWave) {
-            lds_barrier();  // A
-            f32x4 acc[32];
-#pragma unroll
-            for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-            for (int c = 0; c < Nt; ++c) {
-                XM<true> xm;
-                const uint2 *st = areas + c * 32 * 64;
-#pragma unroll
-                for (int h = 0; h < 32; ++h) xm.b[h] = st[h * 64 + lane];
-                contract<true>(d, 0, c, lane, xm, acc);
-            }
-            lds_barrier();  // B
-            transform_store<uint16_t, true>(d, acc, yr, (uint32_t)((int64_t)row * d.ldy * 2), row_ok, 0, q, bd_l,
-                                            row);
-        } else {
-            lds_barrier();  // A
-            lds_barrier();  // B
-        }
-    }
-}
-
 // ---------------------------------------------------------------- pairs, several chunks or output tiles
 // bf16 linear and SwiGLU on wavefront pairs for layers of a few 16-wide
 // input chunks and output tiles (n_embd 768 and 1024): a workgroup is one
@@ -2137,6 +1918,208 @@ __global__ __launch_bounds__(kPairThreads, 2) void hadamard_pair_swiglu_kernel(H
     __syncthreads();
     if (tid < 64) pair_swiglu_item<0>(g, u, tile, nt, lane, smem);
     else pair_swiglu_item<1>(g, u, tile, nt, lane, smem);
+}
+
+// down(silu(gate(x)) * up(x)) (SwiGLUMLP.forward, chassis.py:498-504) in one
+// launch, for bf16 rows with in_o <= 16 (n_embd 512), a hidden width of two
+// or three 16-wide tiles (16 < hid_o <= 48) and a down projection with
+// out_o <= 16.  A 16-token tile is worked on by one wavefront pair per hidden
+// tile:
+//   - pair 0 transforms the rows with the gate's alpha and pair 1 with the
+//     up's, and every pair takes both results (bf16) from their exchange
+//     areas;
+//   - pair nt contracts both with hidden tile nt and forms silu(g) u, rounded
+//     to bf16 as the SwiGLU kernels store it; that is the down projection's
+//     input chunk nt, so the pair hands the 8 slots of the other half to its
+//     partner and runs the down projection's input transform;
+//   - pairs 1 .. leave their transformed chunk in their exchange areas, pair 0
+//     contracts the chunks in order through one accumulator chain and runs
+//     the output transform and the stores.
+// The hidden activation never leaves the CU, and the output equals
+// walsh_hadamard_swiglu_fwd followed by the down projection bitwise.  Every
+// wavefront passes the same 16 barriers per tile.
+// The vector ALU bounds it once each SIMD has its three wavefronts (164
+// registers), the chain of five transforms below that.  Against one wavefront
+// per hidden tile plus one for the down projection, in us per launch:
+//   16 -> 43 -> 16, 1,024 / 8,192 / 65,536 rows: 24.8 / 36.0 / 230 to 17.1 /
+//   26.4 / 166; 8 -> 22 -> 8: 21.2 / 28.7 / 194 to 13.6 / 18.9 / 98.
+// Each pair transforming the rows for itself: 22.5 / 35.5 / 241 and 16.1 /
+// 21.4 / 112.
+constexpr int kMlpMaxNt = 3;
+constexpr size_t mlp_lds(int Nt, int P) { return (size_t)16 * 128 * (3 + 3 * Nt) + (size_t)P * Nt * kPairXch; }
+
+template <int HF>
+__device__ __forceinline__ void mlp_tile(const HadArgs &g, const HadArgs &u, const HadArgs &d, int tile, int nt, int lane,
+                                         const f32x4 *tab, f32x4 *xch_all, __amdgpu_buffer_rsrc_t xr,
+                                         __amdgpu_buffer_rsrc_t yr) {
+    const int Nt = g.Nt;
+    const f32x4 *bd_l = tab + 256;   // tab: the gate's alpha, then the up's
+    const f32x4 *bg_l = tab + (3 + nt) * 128, *bu_l = tab + (3 + Nt + nt) * 128, *ad_l = tab + (3 + 2 * Nt + nt) * 128;
+    f32x4 *xch = xch_all + nt * 2 * 8 * 64;
+    const int t = lane & 15, q = lane >> 4;
+    const int row = tile * kTile + t;
+    const bool row_ok = row < g.M;
+    u32x2 *mine = (u32x2 *)(xch + HF * 8 * 64), *theirs = (u32x2 *)(xch + (1 - HF) * 8 * 64);
+    // pair 0 transforms the rows for the gate, pair 1 for the up projection;
+    // every pair takes both from their exchange areas
+    u32x2 xg[16], xu[16];
+    if (nt < 2) {
+        u32x2 raw[16];
+        pair_load<HF>(xr, row_ok && 4 * q < g.in_o ? (uint32_t)((int64_t)row * g.ldx * 2) + (uint32_t)q * 8 : kOOB,
+                      (uint32_t)g.gsx * 2, raw);
+        f32x4 v[16];
+        pair_scale(v, raw, tab + nt * 128 + q * 32 + 16 * HF);
+        pair_in<HF>(v, xch, lane);
+        lds_barrier();   // the partner has read the exchange
+#pragma unroll
+        for (int k = 0; k < 16; ++k) mine[k * 64 + lane] = u32x2{pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)};
+    } else {
+        lds_barrier();   // the three above
+        lds_barrier();
+        lds_barrier();
+    }
+    uint4 wg0, wg1, wu0, wu1;
+    load_w(g, nt, 0, lane, wg0, wg1);
+    load_w(u, nt, 0, lane, wu0, wu1);
+    lds_barrier();
+    {
+        const u32x2 *in = (const u32x2 *)(xch_all + HF * 8 * 64);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) xg[k] = in[k * 64 + lane];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) xu[k] = in[(16 * 64 + 16 * 64) + k * 64 + lane];
+    }
+    auto contract1 = [&](const uint4 &w0, const uint4 &w1, const u32x2 (&x)[16], f32x4 (&acc)[16]) {
+        const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int gr = pair_gin<HF>(k);
+            acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                __builtin_bit_cast(i16x4, codes_bf16x4(wb[gr >> 2], gr & 3)), __builtin_bit_cast(i16x4, x[k]),
+                f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+    };
+    u32x2 hb[16];   // the gate's, then the hidden values, as bf16
+    {
+        f32x4 acc[16];
+        contract1(wg0, wg1, xg, acc);
+        pair_out<HF>(acc, xch, lane);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const f32x4 v = acc[k] * bg_l[q * 32 + pair_gout<HF>(k)];
+            hb[k] = u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
+            asm volatile("" : "+v"(hb[k].x), "+v"(hb[k].y));   // packed here, not where it is used
+            if ((k & 3) == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        contract1(wu0, wu1, xu, acc);
+        pair_out<HF>(acc, xch, lane);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const f32x4 uv = acc[k] * bu_l[q * 32 + pair_gout<HF>(k)], gv = bf16x4_f32(hb[k]);
+            f32x4 hv;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) hv[j] = silu_fast(gv[j]) * uv[j];
+            hb[k] = u32x2{pack_bf16x2(hv.x, hv.y), pack_bf16x2(hv.z, hv.w)};
+            asm volatile("" : "+v"(hb[k].x), "+v"(hb[k].y));
+            if ((k & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // to the down projection's input layout (groups 16 HF + s): slots with
+    // u >> 3 == HF hold groups of this half, the others go to the partner
+    lds_barrier();   // the partner is done reading the output exchange
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mine[j * 64 + lane] = hb[8 * (1 - HF) + j];
+    lds_barrier();
+    u32x2 xm[16];
+    {
+        f32x4 v[16];
+        const f32x4 *al = ad_l + q * 32 + 16 * HF;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int own = (j & 3) + 4 * HF + 8 * ((j >> 2) & 1);
+            const int other = (j & 3) + 4 * (1 - HF) + 8 * ((j >> 2) & 1);
+            v[own] = bf16x4_f32(hb[8 * HF + j]) * al[own];
+            v[other] = bf16x4_f32(theirs[j * 64 + lane]) * al[other];
+            if ((j & 1) == 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        pair_in<HF>(v, xch, lane);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) xm[k] = u32x2{pack_bf16x2(v[k].x, v[k].y), pack_bf16x2(v[k].z, v[k].w)};
+    }
+    lds_barrier();   // the partner has read this wavefront's exchange slots
+    if (nt > 0) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) mine[k * 64 + lane] = xm[k];   // 16 x 64 x 8 bytes: the wavefront's half
+    }
+    lds_barrier();   // the chunks are in the areas
+    if (nt > 0) {
+        lds_barrier();   // pair 0's output exchange
+        lds_barrier();
+        return;
+    }
+    f32x4 acc[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < Nt; ++c) {
+        uint4 w0, w1;
+        load_w(d, 0, c, lane, w0, w1);
+        const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+        if (c > 0) {
+            const u32x2 *in = (const u32x2 *)(xch_all + c * 2 * 8 * 64 + HF * 8 * 64);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) xm[k] = in[k * 64 + lane];
+        }
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int gr = pair_gin<HF>(k);
+            acc[k] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                __builtin_bit_cast(i16x4, codes_bf16x4(wb[gr >> 2], gr & 3)), __builtin_bit_cast(i16x4, xm[k]), acc[k], 0,
+                0, 0);
+        }
+    }
+    pair_out<HF>(acc, xch, lane);
+    const int o0 = 4 * q;
+    const uint32_t yo = row_ok && o0 < d.out_o ? (uint32_t)((int64_t)row * d.ldy * 2) + (uint32_t)o0 * 2 : kOOB;
+    const uint32_t gsy = (uint32_t)d.gsy * 2;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        const int h = pair_gout<HF>(k);
+        Buf4<uint16_t>::store(acc[k] * bd_l[q * 32 + h], yr, yo, (uint32_t)h * gsy);
+    }
+}
+
+// blockDim.x = 128 * Nt * P: P token tiles side by side.
+__global__ __launch_bounds__(kPairThreads * kMlpMaxNt * 2, 3) void hadamard_mlp_kernel(HadArgs g, HadArgs u, HadArgs d) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int Nt = g.Nt, tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), pair = wave >> 1, hf = wave & 1;
+    const int P = (int)blockDim.x / (kPairThreads * Nt), sub = pair / Nt, nt = pair - sub * Nt;
+    // tables: gate alpha, up alpha, down beta, then per hidden tile the
+    // gate's beta, the up's beta and the down's alpha; pair nt fills its own
+    // and pairs 0, 1, .. the common ones
+    f32x4 *tab = (f32x4 *)smem;
+    f32x4 *xch = tab + (3 + 3 * Nt) * 128 + sub * Nt * (int)(kPairXch / 16);
+    if (sub == 0) {
+        const int pt = tid & (kPairThreads - 1);
+        fill_scale_chunk(tab + (3 + nt) * 128, g.beta, g.out_o, g.out_o, nt, kCodeScale, pt);
+        fill_scale_chunk(tab + (3 + Nt + nt) * 128, u.beta, g.out_o, g.out_o, nt, kCodeScale, pt);
+        fill_scale_chunk(tab + (3 + 2 * Nt + nt) * 128, d.alpha, d.in_o, d.in_o, nt, 1.f, pt);
+        for (int k = nt; k < 3; k += Nt) {
+            if (k == 0) fill_scale_chunk(tab, g.alpha, g.in_o, g.in_o, 0, 1.f, pt);
+            else if (k == 1) fill_scale_chunk(tab + 128, u.alpha, g.in_o, g.in_o, 0, 1.f, pt);
+            else fill_scale_chunk(tab + 256, d.beta, d.out_o, d.beta_h, 0, kCodeScale, pt);
+        }
+    }
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(g.x, (uint32_t)((int64_t)g.M * g.ldx * 2));
+    const __amdgpu_buffer_rsrc_t yr = make_rsrc(d.y, (uint32_t)((int64_t)d.M * d.ldy * 2));
+    const int n_tiles = (int)ceil_div(g.M, kTile);
+    // a tile past the last (odd counts) has no valid row: it loads zeros and
+    // stores nothing, and keeps the barriers
+    for (int tile0 = blockIdx.x * P; tile0 < n_tiles; tile0 += gridDim.x * P) {
+        if (hf == 0) mlp_tile<0>(g, u, d, tile0 + sub, nt, lane, tab, xch, xr, yr);
+        else mlp_tile<1>(g, u, d, tile0 + sub, nt, lane, tab, xch, xr, yr);
+    }
 }
 
 // Input chunks up to which the pair kernels hold their tables beside the
@@ -2734,12 +2717,13 @@ WALSH_EXPORT int walsh_hadamard_mlp_fwd(const void *x, int64_t ldx, int64_t M, i
     HadArgs ua = had_args(x, ldx, in_o, in_o, hid_o, kw_up, alpha_up, beta_up, nullptr, 0, hid_o);
     HadArgs da = had_args(nullptr, 0, hid_o, hid_o, out_o, kw_down, alpha_down, beta_down, y, ldy, out_o);
     const int Nt = ga.Nt;
-    const size_t lds = (size_t)16 * 128 * (2 + 3 * Nt + 1) + (size_t)3 * 32 * 64 * 8;
+    const size_t lds = mlp_lds(Nt, 1);
     if (lds > (size_t)device_info().max_shared_per_block)
         return set_error(WALSH_ENOTSUP, "%s: needs %zu B of LDS", fn, lds);
     const int64_t ld = ldx > ldy ? ldx : ldy;
     const int64_t rows_max = (int64_t)kMaxBufferBytes / (ld * 2) / kTile * kTile;
-    const int64_t resident = (int64_t)device_info().cu_count * 2;
+    const int64_t cus = device_info().cu_count;
+    const bool two = lds * 2 <= (size_t)device_info().max_shared_per_block;
     hipStream_t s = (hipStream_t)stream;
     for (int64_t r0 = 0; r0 < M; r0 += rows_max) {
         const int64_t rows = (M - r0) < rows_max ? (M - r0) : rows_max;
@@ -2747,9 +2731,16 @@ WALSH_EXPORT int walsh_hadamard_mlp_fwd(const void *x, int64_t ldx, int64_t M, i
         g.x = u.x = (const char *)x + r0 * ldx * 2;
         d.y = (char *)y + r0 * ldy * 2;
         g.M = u.M = d.M = (int)rows;
-        int64_t grid = ceil_div(rows, kTile);
+        // Two hidden tiles: three workgroups of four wavefronts fill a CU.
+        // Three: a second workgroup of six is not placed beside the first
+        // (8,192 rows took 44 us, 4,096 rows 23), so beyond one tile per CU a
+        // workgroup of twelve takes two tiles.
+        const int64_t tiles = ceil_div(rows, kTile);
+        const int P = Nt == kMlpMaxNt && tiles > cus && two ? 2 : 1;
+        const int64_t resident = Nt == kMlpMaxNt ? cus : 3 * cus;
+        int64_t grid = ceil_div(tiles, P);
         if (grid > resident) grid = resident;
-        launch(hadamard_mlp_kernel, dim3((unsigned)grid), dim3(kThreads), (uint32_t)lds, s, g, u, d);
+        launch(hadamard_mlp_kernel, dim3((unsigned)grid), dim3(kPairThreads * Nt * P), (uint32_t)mlp_lds(Nt, P), s, g, u, d);
         const int rc = check_hip(hipGetLastError(), fn);
         if (rc) return rc;
     }
