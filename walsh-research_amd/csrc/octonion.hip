@@ -204,7 +204,15 @@ __global__ void octonion_expand_t_kernel(const uint8_t *__restrict__ packed, int
 }
 
 // dW and dbeta from C.  Threads [0, 8*out_o*in_o) take one dW element each;
-// workgroups past that take one dbeta[n] each (256 threads, fixed-order tree).
+// workgroups past that take one dbeta[n] each (256 threads, fixed-order tree),
+// a thread's pieces being 4 consecutive m of one (i, j): one byte of codes and
+// one 16-byte load of C where rows allow it.  ONE: a single C (no partials).
+// The chain of loads bounds it, so a thread requests kFoldBatch pieces (8
+// values of a dW element) before it uses the first: 1024 -> 1024 features took
+// 23 us with one load at a time, now 6.
+constexpr int kFoldBatch = 4;
+
+template <bool ONE>
 __global__ __launch_bounds__(256) void octonion_fold_kernel(const float *__restrict__ C, int64_t ldc, int Sc,
                                                             int64_t cstride, const uint8_t *__restrict__ packed,
                                                             int in_o, int out_o, const float *__restrict__ beta,
@@ -218,12 +226,20 @@ __global__ __launch_bounds__(256) void octonion_fold_kernel(const float *__restr
         const int64_t wn = e / in_o;
         const int n = (int)(wn % out_o), w = (int)(wn / out_o);
         double acc = 0.0;
-        for (int i = 0; i < 8; ++i) {
-            const int j = i ^ w;
-            const int64_t off = (int64_t)(i * out_o + n) * ldc + (int64_t)j * in_o + m;
-            double c = 0.0;
-            for (int s = 0; s < Sc; ++s) c += (double)C[s * cstride + off];
-            acc += kOctSign[i][j] * c;
+        if constexpr (ONE) {
+            float c[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) c[i] = C[(int64_t)(i * out_o + n) * ldc + (int64_t)(i ^ w) * in_o + m];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc += kOctSign[i][i ^ w] * (double)c[i];
+        } else {
+            for (int i = 0; i < 8; ++i) {
+                const int j = i ^ w;
+                const int64_t off = (int64_t)(i * out_o + n) * ldc + (int64_t)j * in_o + m;
+                double c = 0.0;
+                for (int s = 0; s < Sc; ++s) c += (double)C[s * cstride + off];
+                acc += kOctSign[i][j] * c;
+            }
         }
         float v = (float)(acc * (double)beta[n]);
         if (latent) {
@@ -236,16 +252,47 @@ __global__ __launch_bounds__(256) void octonion_fold_kernel(const float *__restr
     if (!db) return;
     __shared__ double part[256];
     const int n = (int)blockIdx.x - dw_blocks;
+    const bool vec = in_o % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+    const int pieces = 64 * kp4;   // e = (i*8 + j)*kp4 + m/4
     double acc = 0.0;
-    for (int e = threadIdx.x; e < 64 * in_o; e += blockDim.x) {  // e = (i*8 + j)*in_o + m
-        const int m = e % in_o, ij = e / in_o, i = ij >> 3, j = ij & 7;
-        const uint32_t byte = packed[((int64_t)(i ^ j) * out_o + n) * kp4 + m / 4];
-        const int code = (int)((byte >> (6 - 2 * (m & 3))) & 3u) - 1;
-        if (!code) continue;
-        const int64_t off = (int64_t)(i * out_o + n) * ldc + (int64_t)j * in_o + m;
-        double c = 0.0;
-        for (int s = 0; s < Sc; ++s) c += (double)C[s * cstride + off];
-        acc += (double)(kOctSign[i][j] * code) * c;
+    for (int e0 = threadIdx.x; e0 < pieces; e0 += 256 * kFoldBatch) {
+        uint32_t codes[kFoldBatch];
+        double sg[kFoldBatch];
+        float c[kFoldBatch][4];
+        int64_t off[kFoldBatch];
+        int left[kFoldBatch];
+#pragma unroll
+        for (int b = 0; b < kFoldBatch; ++b) {
+            const int e = e0 + 256 * b;
+            const bool live = e < pieces;
+            const int ij = live ? e / kp4 : 0, mq = live ? e - ij * kp4 : 0, i = ij >> 3, j = ij & 7;
+            codes[b] = packed[((int64_t)(i ^ j) * out_o + n) * kp4 + mq];
+            sg[b] = kOctSign[i][j];
+            off[b] = (int64_t)(i * out_o + n) * ldc + (int64_t)j * in_o + 4 * mq;
+            left[b] = live ? in_o - 4 * mq : 0;
+            if constexpr (ONE) {
+                if (vec) {
+                    const f32x4 v = *(const f32x4 *)(C + off[b]);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) c[b][k] = v[k];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) c[b][k] = C[off[b] + (k < left[b] ? k : 0)];
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < kFoldBatch; ++b)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int code = (int)((codes[b] >> (6 - 2 * k)) & 3u) - 1;
+                if (!code || k >= left[b]) continue;
+                double cv = 0.0;
+                if constexpr (ONE) cv = (double)c[b][k];
+                else
+                    for (int s = 0; s < Sc; ++s) cv += (double)C[s * cstride + off[b] + k];
+                acc += (sg[b] * code) * cv;
+            }
     }
     part[threadIdx.x] = acc;
     __syncthreads();
@@ -290,8 +337,9 @@ WALSH_EXPORT int walsh_octonion_bwd_fold(const float *C, int64_t ldc, int64_t n_
     const int dw_blocks = dweight ? (int)ceil_div(nw, 256) : 0;
     const int64_t grid = dw_blocks + (dbeta ? out_o : 0);
     if (grid == 0) return WALSH_OK;
-    launch(octonion_fold_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, C, ldc, (int)n_parts,
-           part_stride, packed, (int)in_o, (int)out_o, beta, latent, dweight, dbeta, dw_blocks);
+    launch(n_parts == 1 ? octonion_fold_kernel<true> : octonion_fold_kernel<false>, dim3((unsigned)grid), dim3(256), 0,
+           (hipStream_t)stream, C, ldc, (int)n_parts, part_stride, packed, (int)in_o, (int)out_o, beta, latent, dweight,
+           dbeta, dw_blocks);
     return check_hip(hipGetLastError(), "walsh_octonion_bwd_fold launch");
 }
 
@@ -353,7 +401,8 @@ __global__ __launch_bounds__(256) void octonion_transpose_kernel(const T *__rest
     }
 }
 
-// C = the split-K partial sums added in split order (float32).
+// C = the split-K partial sums added in split order (float32).  Bound by
+// reading them: 16 parts of 4 MB in 14 us, 4.9 TB/s.
 __global__ __launch_bounds__(256) void octonion_sum_parts_kernel(const float *__restrict__ parts, int S,
                                                                  int64_t stride, int64_t n, float *__restrict__ C) {
     for (int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; e < n;
@@ -364,8 +413,13 @@ __global__ __launch_bounds__(256) void octonion_sum_parts_kernel(const float *__
     }
 }
 
-// split-K plan: about two work items per CU, splits of whole K stages and at
-// least 4 stages each
+// split-K plan, splits of whole K stages and at least 4 stages each.  float32:
+// about two work items per CU.  bf16 (a persistent workgroup per CU): the
+// count that makes the rounds of items times their stages (1.6 us each, the
+// matrix cores' rate) plus the partial sums' way through memory (written,
+// then read again: 0.1 us per 256 x 256 item) least.  1,024 -> 1,024 features
+// at 16,384 tokens: 16 splits, product and sum 45 and 14 us; 32 (two items per
+// CU) 57 and 26.
 static void octonion_dw_plan(int64_t M, int64_t in_o, int64_t out_o, bool bf16, int64_t *S, int64_t *kspan,
                              int64_t *Mp) {
     const int64_t N8o = 8 * out_o, N8i = 8 * in_o;
@@ -375,6 +429,18 @@ static void octonion_dw_plan(int64_t M, int64_t in_o, int64_t out_o, bool bf16, 
     const int64_t smax = ceil_div(M, 4 * stage);
     if (s > smax) s = smax;
     if (s < 1) s = 1;
+    if (bf16) {
+        int64_t best = 1, least = INT64_MAX;
+        for (int64_t c = 1; c <= s; ++c) {
+            const int64_t stages = ceil_div(ceil_div(M, c), stage), n = ceil_div(M, stages * stage);
+            const int64_t t = ceil_div(tiles * n, device_info().cu_count) * stages * 16 + (n > 1 ? n * tiles : 0);
+            if (t < least) {
+                least = t;
+                best = c;
+            }
+        }
+        s = best;
+    }
     *kspan = ceil_div(ceil_div(M, s), stage) * stage;
     *S = ceil_div(M, *kspan);
     *Mp = ceil_div(M, 8) * 8;
