@@ -242,6 +242,71 @@ def test_octonion_module_autograd(dtype, cls):
     assert_close(layer.beta.grad.cpu().numpy(), ref[2], dtype_bar, f"oct {cls} beta.grad")
 
 
+@pytest.mark.parametrize("n_parts", [1, 3])
+@pytest.mark.parametrize("in_o,out_o,pad", [(1, 1, 0), (6, 2, 0), (16, 3, 3), (64, 2, 4), (68, 2, 1), (130, 3, 2)])
+def test_octonion_fold_pieces(K, in_o, out_o, pad, n_parts):
+    """The fold's pieces of 4 codes at widths that leave remainders, fill a
+    batch exactly (64) and pass it, with row strides that allow 16-byte loads
+    of C or not, one C or several partial ones, against float64 (the kernel
+    adds in float64 and rounds once: half a float32 unit of the result, plus
+    float64 rounding of the terms)."""
+    from src.model import _hip
+    from src.model.constants import SIGN_TABLE
+    gen = torch.Generator().manual_seed(in_o + out_o)
+    ldc = 8 * in_o + pad
+    C = torch.randn(n_parts, 8 * out_o, ldc, generator=gen).cuda()
+    q = K.ternary_quantize((torch.rand(8, out_o, in_o, generator=gen) * 4 - 2).cuda(), codes=True, packed=True)
+    beta = torch.randn(out_o, generator=gen).cuda()
+    dw = torch.empty(8, out_o, in_o, device="cuda")
+    db = torch.empty(out_o, device="cuda")
+    _hip.call("walsh_octonion_bwd_fold", C.data_ptr(), ldc, n_parts, 8 * out_o * ldc, q["packed"].data_ptr(), in_o,
+              out_o, beta.data_ptr(), 0, dw.data_ptr(), db.data_ptr(), _hip.stream(C.device))
+    torch.cuda.synchronize()
+    c = C.double().cpu().numpy().sum(0)[:, :8 * in_o].reshape(8, out_o, 8, in_o)
+    codes, b = q["codes"].cpu().numpy().astype(np.float64), beta.double().cpu().numpy()
+    rw, rb, aw, ab = (np.zeros((8, out_o, in_o)), np.zeros(out_o), np.zeros((8, out_o, in_o)), np.zeros(out_o))
+    for i in range(8):
+        for j in range(8):
+            t = SIGN_TABLE[i][j] * c[i, :, j]
+            rw[i ^ j] += t
+            rb += (codes[i ^ j] * t).sum(1)
+            aw[i ^ j] += abs(t)
+            ab += abs(t).sum(1)
+    rw, aw = rw * b[:, None], aw * abs(b)[:, None]
+    assert (abs(dw.double().cpu().numpy() - rw) <= 2.0 ** -24 * abs(rw) + 2.0 ** -44 * aw).all()
+    assert (abs(db.double().cpu().numpy() - rb) <= 2.0 ** -24 * abs(rb) + 2.0 ** -40 * ab).all()
+
+
+def test_octonion_parts_gradient_forms(K):
+    """The output parts' gradients side by side in one buffer (a concatenated
+    output: read in place), in eight buffers, in one buffer in another order,
+    expanded, and with parts left out: each equals the gradient of the rows."""
+    from src.model.octonion import OctonionFusedLinear
+    torch.manual_seed(5)
+    layer = OctonionFusedLinear(64, 128).cuda()
+    x = torch.randn(3, 7, 64, device="cuda", requires_grad=True)
+    g = torch.randn(3, 7, 128, device="cuda")
+    g0 = torch.cat([t if k in (1, 6) else torch.zeros_like(t) for k, t in enumerate(g.split(16, -1))], -1)
+
+    def grads(loss):
+        return torch.autograd.grad(loss, (x, layer.weight, layer.beta))
+
+    def parts():
+        return layer(x.split(8, -1))
+
+    cases = {
+        "cat": ((torch.cat(parts(), -1) * g).sum(), g),
+        "separate": (sum((y * t).sum() for y, t in zip(parts(), g.split(16, -1))), g),
+        "permuted": ((torch.cat(parts()[::-1], -1) * torch.cat(g.split(16, -1)[::-1], -1)).sum(), g),
+        "expanded": (sum(y.sum() for y in parts()), torch.ones_like(g)),
+        "left out": (sum((y * t).sum() for y, t in list(zip(parts(), g.split(16, -1)))[1::5]), g0),
+    }
+    for name, (loss, rows) in cases.items():
+        ref = grads((layer.forward_full(x) * rows).sum())
+        for a, b in zip(grads(loss), ref):
+            assert torch.equal(a, b), name
+
+
 # ---------------------------------------------------------------- Sinkhorn
 
 @pytest.mark.parametrize("n", [1, 2, 4, 7])
