@@ -748,6 +748,20 @@ int walsh_chanmod_bwd(const void *gy, int64_t ldg, const void *x, int64_t ldx, i
                       void *gx, int64_t ldgx, float *dscale, float *dshift, int dtype, void *workspace,
                       int64_t workspace_bytes, void *stream);
 
+/* walsh_rmsnorm_fwd / _bwd: RMSNorm of training (chassis.py:96-106) on
+ *   contiguous bf16 rows x [M, C] with a float weight w [C]:
+ *     rstd[t] = rsqrt(mean(x[t]^2) + eps);  y = bf16(x rstd) w   (float32)
+ *     g = bf16(gy w);  gx = bf16(rstd g - x rstd^3 mean(g x))     (bf16)
+ *     gw = sum over rows of gy bf16(x rstd)       (fixed order: deterministic)
+ *   M >= 1, C a multiple of 4 up to 2048.  gx or gw may be null; gw needs
+ *   work of walsh_rmsnorm_bwd_workspace_bytes(M, C) bytes.  x and gx 8-byte,
+ *   the float arrays 16-byte aligned. */
+int walsh_rmsnorm_fwd(const void *x, const float *w, int64_t M, int64_t C, float eps, float *y, float *rstd,
+                      void *stream);
+int64_t walsh_rmsnorm_bwd_workspace_bytes(int64_t M, int64_t C);
+int walsh_rmsnorm_bwd(const void *x, const float *w, const float *rstd, const float *gy, int64_t M, int64_t C, void *gx,
+                      float *gw, void *work, int64_t work_bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,111 @@
+"""RMSNorm of training on the HIP kernels against float64 and the
+element-by-element form (chassis.py:96-106)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _plain(norm, x):
+    return norm._norm(x.float()).type_as(x) * norm.weight
+
+
+@pytest.mark.parametrize("rows,C", [(1, 4), (3, 252), (9, 256), (33, 260), (1000, 512), (4099, 516), (77, 1024),
+                                    (8200, 1028), (130, 2048)])
+def test_rmsnorm_kernels(rows, C):
+    """Pieces of 256 columns with and without a remainder, row counts below,
+    at and past one pass of the workgroups.  The forward rounds to bf16 once:
+    2^-8 of the value (half a unit, and half again where the factor's float32
+    error moves the rounding).  gx is rounded to bf16 twice, the first time in
+    each term of a sum over C; gw sums rows of values with one bf16 rounding."""
+    from src.model.chassis import RMSNorm
+    gen = torch.Generator(device="cuda").manual_seed(rows + C)
+    norm = RMSNorm(C).cuda()
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5, generator=gen)
+    x = (torch.randn(rows, C, device="cuda", generator=gen) * 3).bfloat16().requires_grad_(True)
+    g = torch.randn(rows, C, device="cuda", generator=gen)
+    assert norm._fused(x)
+    y = norm(x)
+    assert y.dtype == torch.float32
+    gx, gw = torch.autograd.grad(y, (x, norm.weight), g)
+    xd, wd = x.detach().double().requires_grad_(True), norm.weight.detach().double().requires_grad_(True)
+    yd = xd * torch.rsqrt(xd.pow(2).mean(-1, keepdim=True) + norm.eps) * wd
+    rx, rw = torch.autograd.grad(yd, (xd, wd), g.double())
+    xn = (yd / wd).detach()
+    r = (xn / xd.detach()).abs().nan_to_num().amax(-1, keepdim=True)
+    gn = (g.double() * wd).abs().detach()
+    assert ((y - yd).abs() <= 2.0 ** -8 * yd.abs() + 1e-30).all()
+    lim = 2.0 ** -8 * (rx.abs() + r * (gn + xn.abs() * (gn * xn.abs()).mean(-1, keepdim=True))) + 1e-30
+    assert ((gx - rx).abs() <= lim).all()
+    assert ((gw - rw).abs() <= 2.0 ** -8 * (g.double() * xn).abs().sum(0) + 1e-30).all()
+    # no less exact than the element-by-element form
+    px, pw = torch.autograd.grad(_plain(norm, x), (x, norm.weight), g)
+    assert (gx - rx).norm() <= 1.02 * (px - rx).norm() + 1e-30 and (gw - rw).norm() <= 1.02 * (pw - rw).norm() + 1e-6 * rw.norm()
+
+
+def test_rmsnorm_forms():
+    """What training may do around the kernels: strided and expanded rows, x
+    changed before the backward, one gradient only, a differentiated backward,
+    and the forms that keep the plain path."""
+    from src.model.chassis import RMSNorm
+    torch.manual_seed(3)
+    norm = RMSNorm(64).cuda()
+    with torch.no_grad():
+        norm.weight.uniform_(0.5, 1.5)
+    base = torch.randn(6, 5, 128, device="cuda").bfloat16()
+
+    def close(a, b):
+        for u, v in zip(a, b):
+            u, v = u.detach(), v.detach()
+            assert torch.allclose(u.float(), v.float(), rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.float().abs().max()))
+
+    for x in (base[..., 32:96], base[:, :1, :64].expand(6, 5, 64), base[0, 0, :64], base[..., 1:65].transpose(0, 1)):
+        x = x.detach().requires_grad_(True)
+        g = torch.randn(x.shape, device="cuda")
+        close(torch.autograd.grad(norm(x), (x, norm.weight), g), torch.autograd.grad(_plain(norm, x), (x, norm.weight), g))
+        close(torch.autograd.grad(norm(x), (norm.weight,), g), torch.autograd.grad(_plain(norm, x), (norm.weight,), g))
+        close((norm(x.detach()),), (_plain(norm, x.detach()),))
+    x = base[..., :64].detach().requires_grad_(True)
+    t = x * 1.0
+    y, ref = norm(t), _plain(norm, t * 1.0)
+    t.mul_(2.0)
+    close(torch.autograd.grad(y.sum(), (x, norm.weight), retain_graph=True),
+          torch.autograd.grad(ref.sum(), (x, norm.weight)))
+    second = []
+    for f in (norm, lambda v: _plain(norm, v)):
+        gx, = torch.autograd.grad(f(x).square().sum(), x, create_graph=True)
+        second.append(torch.autograd.grad(gx.float().square().sum(), (x, norm.weight)))
+    close(*second)
+    assert norm._fused(x)
+    with torch.no_grad():
+        assert not norm._fused(x)
+    assert not norm._fused(x.float()) and not norm._fused(x[:0]) and not norm._fused(x.cpu())
+    with torch.autograd.forward_ad.dual_level():
+        assert not norm._fused(x)
+    torch.func.vmap(lambda v: norm(v))(x.detach())
+
+
+def test_rmsnorm_kernels_capture():
+    """Both kernels recorded in a graph, replayed with new inputs and eager
+    work in between: equal to the eager results."""
+    from src.model import kernels
+    x, g = torch.randn(300, 64, device="cuda").bfloat16(), torch.randn(300, 64, device="cuda")
+    w = torch.rand(64, device="cuda") + 0.5
+
+    def step():
+        y, rstd = kernels.rmsnorm(x, w, 1e-6)
+        return (y, rstd) + kernels.rmsnorm_bwd(x, w, rstd, g)
+
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for k in range(3):
+        x.copy_(torch.randn(300, 64, device="cuda"))
+        g.normal_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, step()):
+            assert torch.equal(a, b), k

@@ -68,6 +68,39 @@ def get_head_mixer(config: WalshConfig, head_dim: int):
     return OctonionHeadMixerFused(head_dim)
 
 
+def _plain_eager() -> bool:
+    """No transform, trace or dispatch mode that has to see each operation."""
+    return (torch.autograd.forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch.utils._python_dispatch._get_current_dispatch_mode() is None)
+
+
+class RMSNormFunction(torch.autograd.Function):
+    """RMSNorm of bf16 rows with a float32 weight on the HIP kernels; the
+    values and roundings of the element-by-element form, which a backward that
+    is itself differentiated falls back to."""
+
+    @staticmethod
+    def forward(ctx, x, w, eps):
+        y, rstd = kernels.rmsnorm(x, w, eps)
+        ctx.eps = eps
+        ctx.save_for_backward(x, w, rstd)
+        return y
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, w, rstd = ctx.saved_tensors
+        need = ctx.needs_input_grad[:2]
+        if torch.is_grad_enabled():
+            y = RMSNorm.normalised(x.float(), ctx.eps).type_as(x) * w
+            ins = [t for t, n in zip((x, w), need) if n]
+            got = iter(torch.autograd.grad(y, ins, gy, create_graph=True))
+            gx, gw = (next(got) if n else None for n in need)
+        else:
+            gx, gw = kernels.rmsnorm_bwd(x, w, rstd, gy, need)
+        return gx, gw, None
+
+
 class RMSNorm(nn.Module):
     """x * rsqrt(mean(x^2) + eps) * weight, computed in float32 (chassis.py:96-106)."""
 
@@ -76,10 +109,26 @@ class RMSNorm(nn.Module):
         self.eps = eps
         self.weight = nn.Parameter(torch.ones(dim))
 
+    @staticmethod
+    def normalised(x, eps):
+        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps)
+
     def _norm(self, x):
-        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.eps)
+        return self.normalised(x, self.eps)
+
+    def _fused(self, x):
+        """Training on bf16 rows: one kernel forward and two backward."""
+        w = self.weight
+        return (x.is_cuda and x.dtype == torch.bfloat16 and torch.is_grad_enabled()
+                and (x.requires_grad or w.requires_grad) and x.dim() > 0 and x.numel() > 0
+                and type(x) is torch.Tensor and type(w) is nn.Parameter and w.device == x.device
+                and w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and w.shape == x.shape[-1:] and x.shape[-1] % 4 == 0 and x.shape[-1] <= 2048 and _plain_eager())
 
     def forward(self, x):
+        if self._fused(x):
+            # a copy, as x.float() is: x may be changed before the backward
+            return RMSNormFunction.apply(x.clone(memory_format=torch.contiguous_format), self.weight, self.eps)
         return self._norm(x.float()).type_as(x) * self.weight
 
 

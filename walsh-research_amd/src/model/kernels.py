@@ -772,6 +772,37 @@ def octonion_linear_bwd(x: torch.Tensor, gy: torch.Tensor, in_o: int, out_o: int
     return gx, dw, db
 
 
+# ------------------------------------------------------------------ RMSNorm (training)
+
+def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float):
+    """bf16(x rsqrt(mean(x^2) + eps)) * w in float32 and the float32 factors
+    per row; x contiguous bf16 [..., C], w float32 [C], C % 4 == 0, C <= 2048."""
+    _hip.require_device(x, "input")
+    assert x.dtype == torch.bfloat16 and x.is_contiguous() and w.dtype == torch.float32 and w.is_contiguous()
+    C = x.shape[-1]
+    M = x.numel() // C
+    y = torch.empty(x.shape, device=x.device, dtype=torch.float32)
+    rstd = torch.empty(M, device=x.device, dtype=torch.float32)
+    _hip.call("walsh_rmsnorm_fwd", x.data_ptr(), w.data_ptr(), M, C, eps, y.data_ptr(), rstd.data_ptr(),
+              _hip.stream(x.device), kernel="rmsnorm_fwd_kernel", nbytes=M * C * 6, flops=4 * M * C)
+    return y, rstd
+
+
+def rmsnorm_bwd(x: torch.Tensor, w: torch.Tensor, rstd: torch.Tensor, gy: torch.Tensor, need=(True, True)):
+    """(gx, gw) of rmsnorm; entries not requested in ``need`` are None."""
+    C = x.shape[-1]
+    M = x.numel() // C
+    gy = gy.contiguous()
+    gx = torch.empty_like(x) if need[0] else None
+    gw = torch.empty_like(w) if need[1] else None
+    nws = _hip.lib().walsh_rmsnorm_bwd_workspace_bytes(M, C) if need[1] else 0
+    ws = torch.empty(nws, device=x.device, dtype=torch.uint8) if need[1] else None
+    ptr = lambda t: 0 if t is None else t.data_ptr()  # noqa: E731
+    _hip.call("walsh_rmsnorm_bwd", x.data_ptr(), w.data_ptr(), rstd.data_ptr(), gy.data_ptr(), M, C, ptr(gx), ptr(gw),
+              ptr(ws), nws, _hip.stream(x.device), kernel="rmsnorm_bwd_kernel", nbytes=M * C * 8, flops=10 * M * C)
+    return gx, gw
+
+
 # ------------------------------------------------------------------ decode attention
 
 DECODE_HEAD_DIMS = (16, 32, 64, 128)
