@@ -277,36 +277,6 @@ def test_octonion_fold_pieces(K, in_o, out_o, pad, n_parts):
     assert (abs(db.double().cpu().numpy() - rb) <= 2.0 ** -24 * abs(rb) + 2.0 ** -40 * ab).all()
 
 
-def test_octonion_parts_gradient_forms(K):
-    """The output parts' gradients side by side in one buffer (a concatenated
-    output: read in place), in eight buffers, in one buffer in another order,
-    expanded, and with parts left out: each equals the gradient of the rows."""
-    from src.model.octonion import OctonionFusedLinear
-    torch.manual_seed(5)
-    layer = OctonionFusedLinear(64, 128).cuda()
-    x = torch.randn(3, 7, 64, device="cuda", requires_grad=True)
-    g = torch.randn(3, 7, 128, device="cuda")
-    g0 = torch.cat([t if k in (1, 6) else torch.zeros_like(t) for k, t in enumerate(g.split(16, -1))], -1)
-
-    def grads(loss):
-        return torch.autograd.grad(loss, (x, layer.weight, layer.beta))
-
-    def parts():
-        return layer(x.split(8, -1))
-
-    cases = {
-        "cat": ((torch.cat(parts(), -1) * g).sum(), g),
-        "separate": (sum((y * t).sum() for y, t in zip(parts(), g.split(16, -1))), g),
-        "permuted": ((torch.cat(parts()[::-1], -1) * torch.cat(g.split(16, -1)[::-1], -1)).sum(), g),
-        "expanded": (sum(y.sum() for y in parts()), torch.ones_like(g)),
-        "left out": (sum((y * t).sum() for y, t in list(zip(parts(), g.split(16, -1)))[1::5]), g0),
-    }
-    for name, (loss, rows) in cases.items():
-        ref = grads((layer.forward_full(x) * rows).sum())
-        for a, b in zip(grads(loss), ref):
-            assert torch.equal(a, b), name
-
-
 # ---------------------------------------------------------------- Sinkhorn
 
 @pytest.mark.parametrize("n", [1, 2, 4, 7])

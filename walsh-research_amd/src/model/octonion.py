@@ -20,31 +20,7 @@ from .hadamard import pack_ternary_weights, unpack_ternary_weights  # noqa: F401
 def _parts_to_rows(x_parts, in_o):
     assert len(x_parts) == 8, f"Expected 8 parts, got {len(x_parts)}"
     x = adjacent_parts_view(x_parts, in_o)
-    if x is not None:
-        return x
-    if _one_buffer(x_parts) and all(p.is_cuda for p in x_parts):
-        return _JoinParts.apply(in_o, *x_parts)
-    return torch.cat(x_parts, dim=-1)
-
-
-def _one_buffer(parts):
-    return all(type(p) is torch.Tensor for p in parts) and len({p.untyped_storage().data_ptr() for p in parts}) == 1
-
-
-class _JoinParts(torch.autograd.Function):
-    """torch.cat(parts, -1) of tracked parts; parts that lie side by side in
-    one buffer are copied as whole rows (16,384 rows of 8 x 128 bf16: 33 us
-    part by part, 13 us as rows)."""
-
-    @staticmethod
-    def forward(ctx, width, *parts):
-        ctx.width = width
-        x = adjacent_parts_view(parts, width)
-        return torch.cat(parts, dim=-1) if x is None else x.clone(memory_format=torch.contiguous_format)
-
-    @staticmethod
-    def backward(ctx, g):
-        return (None, *g.split(ctx.width, dim=-1))
+    return torch.cat(x_parts, dim=-1) if x is None else x
 
 
 def _prepared(cache: WeightCache, w_ternary_src, packed_fn, in_o, out_o, dtype):
@@ -79,34 +55,27 @@ class OctonionLinearFunction(torch.autograd.Function):
     of physics.quantize_ternary (physics.py:48-50).  ``fused``: the forward
     is the reference GPU module's (bf16 operands, the product rounded to
     bf16, times beta in float32: a float32 result); the roundings pass the
-    gradient straight through.  ``parts``: the 8 output parts (views of one
-    buffer) instead of the rows.  Their gradients are then read in place
-    where they lie side by side in one buffer, as those of a concatenated
-    output do; splitting the rows outside would add a pass that joins them."""
+    gradient straight through."""
 
     @staticmethod
-    def forward(ctx, x, weight, beta, layer, fused, parts=False):
+    def forward(ctx, x, weight, beta, layer, fused):
         if fused:
             y = kernels.octonion_fused_linear(x, layer.in_o, layer.out_o, layer.block_matrix(torch.bfloat16), beta)
         else:
             y = kernels.octonion_linear(x, layer.in_o, layer.out_o, layer.block_matrix(x.dtype), beta)
         ctx.layer = layer
         ctx.save_for_backward(x, weight, beta)
-        return tuple(y.split(layer.out_o, dim=-1)) if parts else y
+        return y
 
     @staticmethod
-    def backward(ctx, *gys):
+    def backward(ctx, gy):
         x, weight, beta = ctx.saved_tensors
         layer = ctx.layer
-        nx, nw, nb = ctx.needs_input_grad[:3]
-        gy = gys[0]
-        if len(gys) > 1:
-            gy = adjacent_parts_view(gys, layer.out_o) if _one_buffer(gys) else None
-            gy = torch.cat(gys, dim=-1) if gy is None else gy
+        nx, nw, nb, _, _ = ctx.needs_input_grad
         packed = layer.ternary_state()[1]
         gx, dw, db = kernels.octonion_linear_bwd(x, gy.to(x.dtype).contiguous(), layer.in_o, layer.out_o, packed,
                                                  beta, latent=weight, need=(nx, nw, nb))
-        return gx, dw, db, None, None, None
+        return gx, dw, db, None, None
 
 
 class _OctonionTernaryBase(nn.Module):
@@ -155,17 +124,11 @@ class OctonionFusedLinear(_OctonionTernaryBase):
 
     def forward_full(self, x: torch.Tensor) -> torch.Tensor:
         """Rows x [..., 8*in_o] (parts side by side) -> float32 [..., 8*out_o]."""
-        return self._apply_rows(x, False)
-
-    def _apply_rows(self, x: torch.Tensor, parts: bool):
         xb = x if x.dtype == torch.bfloat16 else x.to(torch.bfloat16)
         if self._tracked(x):
-            return OctonionLinearFunction.apply(xb, self.weight, self.beta, self, True, parts)
-        y = kernels.octonion_fused_linear(xb, self.in_o, self.out_o, self.block_matrix(torch.bfloat16), self.beta)
-        return tuple(y.split(self.out_o, dim=-1)) if parts else y
-
-    def forward(self, x_parts):
-        return self._apply_rows(_parts_to_rows(x_parts, self.in_o), True)
+            return OctonionLinearFunction.apply(xb, self.weight, self.beta, self, True)
+        return kernels.octonion_fused_linear(xb, self.in_o, self.out_o, self.block_matrix(torch.bfloat16),
+                                             self.beta)
 
 
 class OctonionTernaryLinearRef(_OctonionTernaryBase):
