@@ -109,3 +109,52 @@ def test_rmsnorm_kernels_capture():
         torch.cuda.synchronize()
         for a, b in zip(out, step()):
             assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 8), (15, 24, 128), (17, 16, 136), (129, 24, 2048), (1000, 17, 264),
+                                   (8193, 24, 2048), (300, 32, 16384), (40000, 3, 1024)])
+def test_mhc_dphi(M, N, K):
+    """Row counts around the 16-token step and the splits, projection rows
+    below, at and above 16, column blocks with a remainder, against float64.
+    Products of bf16 values are exact in float32; each of the at most M sums
+    rounds once, the errors of a fixed-order sum adding up like its square
+    root (2^-24 sqrt(M), taken 8 times over) of the terms' magnitudes."""
+    from src.model import kernels
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    g = torch.randn(M, N, device="cuda", generator=gen).bfloat16()
+    x = torch.randn(M, K, device="cuda", generator=gen).bfloat16()
+    out = kernels.mhc_dphi(g, x)
+    gt = g.double().t().contiguous()
+    ref, mag = gt @ x.double(), gt.abs() @ x.double().abs()
+    assert ((out - ref).abs() <= 8 * 2.0 ** -24 * max(1, M) ** 0.5 * mag).all()
+
+
+def test_phi_function_forms():
+    """The mappings' projection under autograd: values as F.linear's, gx the
+    same, dphi as exact or more; a differentiated backward; other types and
+    transforms keep F.linear."""
+    import torch.nn.functional as F
+    from src.model.mhc import PhiFunction
+    torch.manual_seed(1)
+    x = torch.randn(3, 50, 256, device="cuda").bfloat16().requires_grad_(True)
+    phi = torch.randn(24, 256, device="cuda").requires_grad_(True)
+    rows = phi * 1.0
+    g = torch.randn(3, 50, 24, device="cuda").bfloat16()
+    assert PhiFunction.takes(x, rows)
+    y, ref = PhiFunction.apply(x, rows), F.linear(x, rows.to(x.dtype))
+    assert torch.equal(y, ref)
+    (gx, gp), (rx, rp) = (torch.autograd.grad(v, (x, phi), g, retain_graph=True) for v in (y, ref))
+    exact = g.double().reshape(-1, 24).t() @ x.detach().double().reshape(-1, 256)
+    assert torch.equal(gx, rx) and gp.dtype == torch.float32
+    assert (gp - exact).norm() <= (rp - exact).norm()
+    second = []
+    for f in (PhiFunction.apply, lambda a, b: F.linear(a, b.to(a.dtype))):
+        a, b = torch.autograd.grad(f(x, phi * 1.0).float().square().sum(), (x, phi), create_graph=True)
+        second.append(torch.autograd.grad(a.float().square().sum() + b.square().sum(), (x, phi)))
+    for u, v in zip(*second):
+        assert torch.allclose(u.float(), v.float(), rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.abs().max()))
+    assert not PhiFunction.takes(x.float(), rows) and not PhiFunction.takes(x[..., :255], rows[:, :255])
+    with torch.autograd.forward_ad.dual_level():
+        assert not PhiFunction.takes(x, rows)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not PhiFunction.takes(x, rows)

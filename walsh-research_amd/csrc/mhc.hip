@@ -350,6 +350,101 @@ __device__ __forceinline__ float dot4(const f32x4 &a, const f32x4 &b) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
 
+// ---------------------------------------------------------------- gradient of the stream projection
+// dphi[r][k] = sum_t g[t][r] x[t][k] for N <= 32 projection rows and wide
+// rows x (n C columns): a wavefront takes 128 columns and a range of tokens,
+// 16 tokens per step.  A lane loads 8 columns of 4 tokens (16 bytes each) and
+// pairs them up by token for the 16x16x16 MFMA (column 8m + j of the block is
+// column m of product j), so the rows are read once, whole, and never laid
+// out again.  The four wavefronts of a workgroup add up in LDS, the
+// workgroups' partial sums in a second kernel, in a fixed order, in float32.
+// Bound by reading x: 8,192 x 2,048 with 24 rows 12 us and 5 us for the sum;
+// the library's product of 32 workgroups took 64 us and rounded to bf16.
+constexpr int kDphiCols = 128, kDphiWaves = 4;
+
+__global__ __launch_bounds__(64 * kDphiWaves) void mhc_dphi_kernel(const uint16_t *__restrict__ g,
+                                                                   const uint16_t *__restrict__ x, int M, int N, int K,
+                                                                   int span, float *__restrict__ parts) {
+    __shared__ f32x4 sum[kDphiWaves - 1][16][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m = lane & 15, q = lane >> 4;
+    const int c = blockIdx.x * kDphiCols + 8 * m;
+    const int lo = (blockIdx.y * kDphiWaves + wave) * span, hi = min(M, lo + span);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)((int64_t)M * K * 2));
+    const __amdgpu_buffer_rsrc_t gr = make_rsrc(g, (uint32_t)((int64_t)M * N * 2));
+    f32x4 acc[2][8];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[h][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    u32x4 xv[4];
+    uint32_t gv[2][4];
+    auto request = [&](int t0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + 4 * q + i;
+            xv[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, t < hi && c < K ? (uint32_t)(((int64_t)t * K + c) * 2) : kOOB,
+                                                          0, 0);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                gv[h][i] = __builtin_amdgcn_raw_buffer_load_b16(
+                    gr, t < hi && 16 * h + m < N ? (uint32_t)(((int64_t)t * N + 16 * h + m) * 2) : kOOB, 0, 0);
+        }
+    };
+    request(lo);
+    for (int t0 = lo; t0 < hi; t0 += 16) {
+        u32x4 xc[4];
+        u32x2 a[2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xc[i] = xv[i];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            a[h] = u32x2{(gv[h][0] & 0xffffu) | (gv[h][1] << 16), (gv[h][2] & 0xffffu) | (gv[h][3] << 16)};
+        request(t0 + 16);   // past the range: zeros, no access
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;   // high or low halves of two words
+            const u32x2 b = {__builtin_amdgcn_perm(xc[1][j >> 1], xc[0][j >> 1], sel),
+                             __builtin_amdgcn_perm(xc[3][j >> 1], xc[2][j >> 1], sel)};
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                acc[h][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, a[h]),
+                                                                      __builtin_bit_cast(i16x4, b), acc[h][j], 0, 0, 0);
+        }
+    }
+    if (wave > 0) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[wave - 1][e][lane] = acc[e >> 3][e & 7];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int w = 0; w < kDphiWaves - 1; ++w) acc[e >> 3][e & 7] += sum[w][e][lane];
+    if (c >= K) return;
+    float *dst = parts + (int64_t)blockIdx.y * N * K + c;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 16 * h + 4 * q + i;
+            if (r >= N) continue;
+            *(f32x4 *)(dst + (int64_t)r * K) = f32x4{acc[h][0][i], acc[h][1][i], acc[h][2][i], acc[h][3][i]};
+            *(f32x4 *)(dst + (int64_t)r * K + 4) = f32x4{acc[h][4][i], acc[h][5][i], acc[h][6][i], acc[h][7][i]};
+        }
+}
+
+__global__ __launch_bounds__(256) void mhc_dphi_sum_kernel(const float *__restrict__ parts, int S, int64_t n,
+                                                           float *__restrict__ dphi) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= n) return;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int sp = 0; sp < S; ++sp) acc += parts[sp * n + e];
+    dphi[e] = acc;
+}
+
 // Sums of the 4 values v over the wavefront: afterwards every lane of row
 // rho (16 lanes) holds the sum of v[mix_index(rho)].  The half and row
 // swaps of gfx950 add two values at a time (two instructions each), then the
@@ -1726,6 +1821,47 @@ __global__ __launch_bounds__(256) void mhc_post_kernel(const T *__restrict__ x, 
 }  // namespace walsh
 
 using namespace walsh;
+
+// Token ranges: two workgroups per CU over the column blocks, at least 32
+// tokens per wavefront, whole 16-token steps.
+static void dphi_plan(int64_t M, int64_t K, int64_t *S, int64_t *span) {
+    const int64_t blocks = ceil_div(K, kDphiCols);
+    int64_t sp = ceil_div(2 * (int64_t)device_info().cu_count, blocks);
+    const int64_t most = ceil_div(M, 32 * kDphiWaves);
+    if (sp > most) sp = most;
+    *span = ceil_div(ceil_div(M, sp * kDphiWaves), 16) * 16;
+    *S = ceil_div(M, *span * kDphiWaves);
+}
+
+WALSH_EXPORT int64_t walsh_mhc_dphi_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    if (M < 1 || N < 1 || K < 1) return 0;
+    int64_t S, span;
+    dphi_plan(M, K, &S, &span);
+    return S * N * K * 4;
+}
+
+WALSH_EXPORT int walsh_mhc_dphi(const void *g, const void *x, int64_t M, int64_t N, int64_t K, float *dphi, void *work,
+                                int64_t work_bytes, void *stream) {
+    const char *fn = "walsh_mhc_dphi";
+    if (!g || !x || !dphi || !work) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
+    if (M < 1 || N < 1 || N > 32 || K < 8 || K % 8 || M * (K > N ? K : N) * 2 > (int64_t)kMaxBufferBytes)
+        return set_error(WALSH_ENOTSUP, "%s: needs N <= 32, K a multiple of 8, operands below 2^31 bytes (M=%lld N=%lld "
+                         "K=%lld)", fn, (long long)M, (long long)N, (long long)K);
+    if ((uintptr_t)x % 16 || (uintptr_t)g % 2 || (uintptr_t)work % 16 ||
+        work_bytes < walsh_mhc_dphi_workspace_bytes(M, N, K))
+        return set_error(WALSH_EINVAL, "%s: x and a workspace of %lld bytes 16-byte aligned, needs %lld", fn,
+                         (long long)work_bytes, (long long)walsh_mhc_dphi_workspace_bytes(M, N, K));
+    int64_t S, span;
+    dphi_plan(M, K, &S, &span);
+    hipStream_t s = (hipStream_t)stream;
+    launch(mhc_dphi_kernel, dim3((unsigned)ceil_div(K, kDphiCols), (unsigned)S), dim3(64 * kDphiWaves), 0, s,
+           (const uint16_t *)g, (const uint16_t *)x, (int)M, (int)N, (int)K, (int)span, (float *)work);
+    const int rc = check_hip(hipGetLastError(), fn);
+    if (rc) return rc;
+    launch(mhc_dphi_sum_kernel, dim3((unsigned)ceil_div(N * K, 256)), dim3(256), 0, s, (const float *)work, (int)S, N * K,
+           dphi);
+    return check_hip(hipGetLastError(), fn);
+}
 
 WALSH_EXPORT int walsh_sinkhorn_fwd(const float *h, int64_t batch, int64_t n, int64_t n_iter, float eps, float *out,
                                     void *stream) {

@@ -82,6 +82,13 @@ def cached_linear(mod: torch.nn.Linear, x: torch.Tensor, cache: WeightCache) -> 
     return torch.nn.functional.linear(x, cast[0], cast[1] if len(cast) > 1 else None)
 
 
+def plain_eager() -> bool:
+    """No transform, trace or dispatch mode that has to see each operation."""
+    return (torch.autograd.forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch.utils._python_dispatch._get_current_dispatch_mode() is None)
+
+
 def adjacent_parts_view(parts, width: int):
     """If ``parts`` are equal-shape slices laid side by side along the last
     dim of one tensor (what ``x.split(width, -1)`` returns), return the

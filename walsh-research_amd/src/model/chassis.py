@@ -22,7 +22,7 @@ from .hadamard import HadamardLinearFunction
 from .hadamard import HadamardHeadMixer, HadamardHeadMixerFused
 from .octonion import OctonionHeadMixerFused, OctonionTernaryLinear
 from . import kernels
-from ._common import WeightCache, act_dtype, cached_linear
+from ._common import WeightCache, act_dtype, cached_linear, plain_eager
 
 _HADAMARD_AVAILABLE = True
 _HADAMARD_HEAD_MIXER_AVAILABLE = True
@@ -66,13 +66,6 @@ def get_head_mixer(config: WalshConfig, head_dim: int):
     if config.n_head % 8 != 0:
         raise ValueError(f"Octonion head_mixing requires n_head % 8 == 0, got {config.n_head}")
     return OctonionHeadMixerFused(head_dim)
-
-
-def _plain_eager() -> bool:
-    """No transform, trace or dispatch mode that has to see each operation."""
-    return (torch.autograd.forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active()
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and torch.utils._python_dispatch._get_current_dispatch_mode() is None)
 
 
 class RMSNormFunction(torch.autograd.Function):
@@ -123,7 +116,7 @@ class RMSNorm(nn.Module):
                 and (x.requires_grad or w.requires_grad) and x.dim() > 0 and x.numel() > 0
                 and type(x) is torch.Tensor and type(w) is nn.Parameter and w.device == x.device
                 and w.dtype == torch.float32 and w.is_contiguous() and w.data_ptr() % 16 == 0
-                and w.shape == x.shape[-1:] and x.shape[-1] % 4 == 0 and x.shape[-1] <= 2048 and _plain_eager())
+                and w.shape == x.shape[-1:] and x.shape[-1] % 4 == 0 and x.shape[-1] <= 2048 and plain_eager())
 
     def forward(self, x):
         if self._fused(x):

@@ -211,7 +211,7 @@ def rope_supported(x: torch.Tensor, out_o: int, head_dim: int) -> bool:
 
 
 # The bf16 Hadamard kernels for in_o > 16 and out_o > 48 (n_embd 4096: the
-# base-3 wide kernel and its decode-sized split) keep alpha and beta in LDS as
+# wide kernel and its decode-sized split) keep alpha and beta in LDS as
 # float16 for the whole launch.  float16 overflows above 65504 and rounds
 # non-zeros below 2^-24 (its smallest subnormal) to zero or to a value 100%
 # off; in between, its absolute error stays below 2^-25 (relative 2^-11 from
@@ -770,6 +770,22 @@ def octonion_linear_bwd(x: torch.Tensor, gy: torch.Tensor, in_o: int, out_o: int
                       kernel="octonion_bwd_params<%s>" % ("bf16" if dt == torch.bfloat16 else "f32"),
                       nbytes=2 * M * 8 * (in_o + out_o) * esz, flops=2 * M * 64 * in_o * out_o)
     return gx, dw, db
+
+
+# ------------------------------------------------------------------ stream projection (training)
+
+def mhc_dphi(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """g^T x in float32: g [M, N <= 32], x [M, K], contiguous bf16, K % 8 == 0."""
+    _hip.require_device(x, "input")
+    M, N = g.shape
+    K = x.shape[1]
+    assert x.shape[0] == M and g.dtype == x.dtype == torch.bfloat16 and g.is_contiguous() and x.is_contiguous()
+    out = torch.empty(N, K, device=x.device, dtype=torch.float32)
+    nws = _hip.lib().walsh_mhc_dphi_workspace_bytes(M, N, K)
+    ws = torch.empty(nws, device=x.device, dtype=torch.uint8)
+    _hip.call("walsh_mhc_dphi", g.data_ptr(), x.data_ptr(), M, N, K, out.data_ptr(), ws.data_ptr(), nws,
+              _hip.stream(x.device), kernel="mhc_dphi_kernel", nbytes=2 * M * (K + N), flops=2 * M * N * K)
+    return out
 
 
 # ------------------------------------------------------------------ RMSNorm (training)
