@@ -762,13 +762,14 @@ int64_t walsh_rmsnorm_bwd_workspace_bytes(int64_t M, int64_t C);
 int walsh_rmsnorm_bwd(const void *x, const float *w, const float *rstd, const float *gy, int64_t M, int64_t C, void *gx,
                       float *gw, void *work, int64_t work_bytes, void *stream);
 
-/* walsh_mhc_dphi: gradient of the stream mappings' projection d = x phi^T
- *   (mhc.py:283-318): dphi [N, K] = sum over the M rows of g [M, N] (x) x
- *   [M, K], contiguous bf16 rows, float32 sums in a fixed order.  N <= 32, K a
+/* walsh_linear_wgrad: weight gradient of a Linear without bias (the stream
+ *   mappings' projection, mhc.py:283-318; the MoE router, moe.py:383-416):
+ *   dw [N, K] = sum over the M rows of g [M, N] (x) x [M, K], contiguous bf16
+ *   rows, float32 sums in a fixed order.  N <= 1024, K a
  *   multiple of 8, x 16-byte aligned; work of
- *   walsh_mhc_dphi_workspace_bytes(M, N, K) bytes, 16-byte aligned. */
-int64_t walsh_mhc_dphi_workspace_bytes(int64_t M, int64_t N, int64_t K);
-int walsh_mhc_dphi(const void *g, const void *x, int64_t M, int64_t N, int64_t K, float *dphi, void *work,
+ *   walsh_linear_wgrad_workspace_bytes(M, N, K) bytes, 16-byte aligned. */
+int64_t walsh_linear_wgrad_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int walsh_linear_wgrad(const void *g, const void *x, int64_t M, int64_t N, int64_t K, float *dw, void *work,
                    int64_t work_bytes, void *stream);
 
 #ifdef __cplusplus

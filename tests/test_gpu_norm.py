@@ -112,8 +112,9 @@ def test_rmsnorm_kernels_capture():
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (15, 24, 128), (17, 16, 136), (129, 24, 2048), (1000, 17, 264),
-                                   (8193, 24, 2048), (300, 32, 16384), (40000, 3, 1024)])
-def test_mhc_dphi(M, N, K):
+                                   (8193, 24, 2048), (300, 32, 16384), (40000, 3, 1024), (515, 33, 136),
+                                   (8192, 128, 512), (700, 1000, 264)])
+def test_linear_wgrad(M, N, K):
     """Row counts around the 16-token step and the splits, projection rows
     below, at and above 16, column blocks with a remainder, against float64.
     Products of bf16 values are exact in float32; each of the at most M sums
@@ -123,38 +124,68 @@ def test_mhc_dphi(M, N, K):
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     g = torch.randn(M, N, device="cuda", generator=gen).bfloat16()
     x = torch.randn(M, K, device="cuda", generator=gen).bfloat16()
-    out = kernels.mhc_dphi(g, x)
+    out = kernels.linear_wgrad(g, x)
     gt = g.double().t().contiguous()
     ref, mag = gt @ x.double(), gt.abs() @ x.double().abs()
     assert ((out - ref).abs() <= 8 * 2.0 ** -24 * max(1, M) ** 0.5 * mag).all()
 
 
-def test_phi_function_forms():
+def test_few_rows_linear_forms():
     """The mappings' projection under autograd: values as F.linear's, gx the
     same, dphi as exact or more; a differentiated backward; other types and
     transforms keep F.linear."""
     import torch.nn.functional as F
-    from src.model.mhc import PhiFunction
+    from src.model.linear import FewRowsLinear
     torch.manual_seed(1)
     x = torch.randn(3, 50, 256, device="cuda").bfloat16().requires_grad_(True)
     phi = torch.randn(24, 256, device="cuda").requires_grad_(True)
     rows = phi * 1.0
     g = torch.randn(3, 50, 24, device="cuda").bfloat16()
-    assert PhiFunction.takes(x, rows)
-    y, ref = PhiFunction.apply(x, rows), F.linear(x, rows.to(x.dtype))
+    assert FewRowsLinear.takes(x, rows)
+    y, ref = FewRowsLinear.apply(x, rows), F.linear(x, rows.to(x.dtype))
     assert torch.equal(y, ref)
     (gx, gp), (rx, rp) = (torch.autograd.grad(v, (x, phi), g, retain_graph=True) for v in (y, ref))
     exact = g.double().reshape(-1, 24).t() @ x.detach().double().reshape(-1, 256)
     assert torch.equal(gx, rx) and gp.dtype == torch.float32
     assert (gp - exact).norm() <= (rp - exact).norm()
     second = []
-    for f in (PhiFunction.apply, lambda a, b: F.linear(a, b.to(a.dtype))):
+    for f in (FewRowsLinear.apply, lambda a, b: F.linear(a, b.to(a.dtype))):
         a, b = torch.autograd.grad(f(x, phi * 1.0).float().square().sum(), (x, phi), create_graph=True)
         second.append(torch.autograd.grad(a.float().square().sum() + b.square().sum(), (x, phi)))
     for u, v in zip(*second):
         assert torch.allclose(u.float(), v.float(), rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.abs().max()))
-    assert not PhiFunction.takes(x.float(), rows) and not PhiFunction.takes(x[..., :255], rows[:, :255])
+    assert not FewRowsLinear.takes(x.float(), rows) and not FewRowsLinear.takes(x[..., :255], rows[:, :255])
     with torch.autograd.forward_ad.dual_level():
-        assert not PhiFunction.takes(x, rows)
+        assert not FewRowsLinear.takes(x, rows)
     with torch.autocast("cuda", dtype=torch.float16):
-        assert not PhiFunction.takes(x, rows)
+        assert not FewRowsLinear.takes(x, rows)
+
+
+def test_router_linears_under_hooks():
+    """The router's Linears on the kernel and as modules (a hook on one of
+    them keeps the module calls): the same logits and equally exact weight
+    gradients."""
+    from src.model.moe import HadamardRouter
+    torch.manual_seed(2)
+    r = HadamardRouter(256, 8).cuda()
+    x = torch.randn(4, 100, 256, device="cuda").bfloat16().requires_grad_(True)
+    g = torch.randn(4, 100, 8, device="cuda").bfloat16()
+    outs, seen = [], []
+    for hooked in (False, True):
+        h = r.gate[2].register_forward_hook(lambda *a: seen.append(1)) if hooked else None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = r._gate_autograd(x)
+        outs.append((y,) + torch.autograd.grad(y, (x, r.gate[0].weight, r.gate[2].weight), g))
+        if h is not None:
+            h.remove()
+    assert seen == [1]
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    for a, b in zip(outs[0][2:], outs[1][2:]):
+        assert (a - b).abs().max() <= 2.0 ** -8 * b.abs().max()
+    try:
+        plain = r.gate(x)
+    except RuntimeError:
+        plain = None
+    if plain is None:   # bf16 rows without autocast stay refused
+        with pytest.raises(RuntimeError):
+            r._gate_autograd(x)

@@ -350,26 +350,27 @@ __device__ __forceinline__ float dot4(const f32x4 &a, const f32x4 &b) {
     return a[0] * b[0] + a[1] * b[1] + a[2] * b[2] + a[3] * b[3];
 }
 
-// ---------------------------------------------------------------- gradient of the stream projection
-// dphi[r][k] = sum_t g[t][r] x[t][k] for N <= 32 projection rows and wide
-// rows x (n C columns): a wavefront takes 128 columns and a range of tokens,
-// 16 tokens per step.  A lane loads 8 columns of 4 tokens (16 bytes each) and
+// ---------------------------------------------------------------- weight gradient of a Linear
+// dw[r][k] = sum_t g[t][r] x[t][k] for a Linear with few weights and many
+// tokens (the stream mappings' phi, the MoE router): a wavefront takes 32
+// rows r, 128 columns and a range of tokens, 16 tokens per step.  A lane loads 8 columns of 4 tokens (16 bytes each) and
 // pairs them up by token for the 16x16x16 MFMA (column 8m + j of the block is
 // column m of product j), so the rows are read once, whole, and never laid
 // out again.  The four wavefronts of a workgroup add up in LDS, the
 // workgroups' partial sums in a second kernel, in a fixed order, in float32.
 // Bound by reading x: 8,192 x 2,048 with 24 rows 12 us and 5 us for the sum;
 // the library's product of 32 workgroups took 64 us and rounded to bf16.
-constexpr int kDphiCols = 128, kDphiWaves = 4;
+// 128 rows of 512 columns: 15 us in all, 65 (8 workgroups).
+constexpr int kWgradCols = 128, kWgradWaves = 4;
 
-__global__ __launch_bounds__(64 * kDphiWaves) void mhc_dphi_kernel(const uint16_t *__restrict__ g,
+__global__ __launch_bounds__(64 * kWgradWaves) void linear_wgrad_kernel(const uint16_t *__restrict__ g,
                                                                    const uint16_t *__restrict__ x, int M, int N, int K,
                                                                    int span, float *__restrict__ parts) {
-    __shared__ f32x4 sum[kDphiWaves - 1][16][64];
+    __shared__ f32x4 sum[kWgradWaves - 1][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m = lane & 15, q = lane >> 4;
-    const int c = blockIdx.x * kDphiCols + 8 * m;
-    const int lo = (blockIdx.y * kDphiWaves + wave) * span, hi = min(M, lo + span);
+    const int c = blockIdx.x * kWgradCols + 8 * m, n0 = 32 * blockIdx.z;
+    const int lo = (blockIdx.y * kWgradWaves + wave) * span, hi = min(M, lo + span);
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)((int64_t)M * K * 2));
     const __amdgpu_buffer_rsrc_t gr = make_rsrc(g, (uint32_t)((int64_t)M * N * 2));
     f32x4 acc[2][8];
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(64 * kDphiWaves) void mhc_dphi_kernel(const uint16_
 #pragma unroll
             for (int h = 0; h < 2; ++h)
                 gv[h][i] = __builtin_amdgcn_raw_buffer_load_b16(
-                    gr, t < hi && 16 * h + m < N ? (uint32_t)(((int64_t)t * N + 16 * h + m) * 2) : kOOB, 0, 0);
+                    gr, t < hi && n0 + 16 * h + m < N ? (uint32_t)(((int64_t)t * N + n0 + 16 * h + m) * 2) : kOOB, 0, 0);
         }
     };
     request(lo);
@@ -421,28 +422,28 @@ __global__ __launch_bounds__(64 * kDphiWaves) void mhc_dphi_kernel(const uint16_
 #pragma unroll
     for (int e = 0; e < 16; ++e)
 #pragma unroll
-        for (int w = 0; w < kDphiWaves - 1; ++w) acc[e >> 3][e & 7] += sum[w][e][lane];
+        for (int w = 0; w < kWgradWaves - 1; ++w) acc[e >> 3][e & 7] += sum[w][e][lane];
     if (c >= K) return;
     float *dst = parts + (int64_t)blockIdx.y * N * K + c;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int r = 16 * h + 4 * q + i;
+            const int r = n0 + 16 * h + 4 * q + i;
             if (r >= N) continue;
             *(f32x4 *)(dst + (int64_t)r * K) = f32x4{acc[h][0][i], acc[h][1][i], acc[h][2][i], acc[h][3][i]};
             *(f32x4 *)(dst + (int64_t)r * K + 4) = f32x4{acc[h][4][i], acc[h][5][i], acc[h][6][i], acc[h][7][i]};
         }
 }
 
-__global__ __launch_bounds__(256) void mhc_dphi_sum_kernel(const float *__restrict__ parts, int S, int64_t n,
-                                                           float *__restrict__ dphi) {
+__global__ __launch_bounds__(256) void linear_wgrad_sum_kernel(const float *__restrict__ parts, int S, int64_t n,
+                                                           float *__restrict__ dw) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= n) return;
     float acc = 0.f;
 #pragma unroll 8
     for (int sp = 0; sp < S; ++sp) acc += parts[sp * n + e];
-    dphi[e] = acc;
+    dw[e] = acc;
 }
 
 // Sums of the 4 values v over the wavefront: afterwards every lane of row
@@ -1822,44 +1823,44 @@ __global__ __launch_bounds__(256) void mhc_post_kernel(const T *__restrict__ x, 
 
 using namespace walsh;
 
-// Token ranges: two workgroups per CU over the column blocks, at least 32
+// Token ranges: two workgroups per CU over the blocks of dw, at least 32
 // tokens per wavefront, whole 16-token steps.
-static void dphi_plan(int64_t M, int64_t K, int64_t *S, int64_t *span) {
-    const int64_t blocks = ceil_div(K, kDphiCols);
+static void wgrad_plan(int64_t M, int64_t N, int64_t K, int64_t *S, int64_t *span) {
+    const int64_t blocks = ceil_div(K, kWgradCols) * ceil_div(N, 32);
     int64_t sp = ceil_div(2 * (int64_t)device_info().cu_count, blocks);
-    const int64_t most = ceil_div(M, 32 * kDphiWaves);
+    const int64_t most = ceil_div(M, 32 * kWgradWaves);
     if (sp > most) sp = most;
-    *span = ceil_div(ceil_div(M, sp * kDphiWaves), 16) * 16;
-    *S = ceil_div(M, *span * kDphiWaves);
+    *span = ceil_div(ceil_div(M, sp * kWgradWaves), 16) * 16;
+    *S = ceil_div(M, *span * kWgradWaves);
 }
 
-WALSH_EXPORT int64_t walsh_mhc_dphi_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+WALSH_EXPORT int64_t walsh_linear_wgrad_workspace_bytes(int64_t M, int64_t N, int64_t K) {
     if (M < 1 || N < 1 || K < 1) return 0;
     int64_t S, span;
-    dphi_plan(M, K, &S, &span);
+    wgrad_plan(M, N, K, &S, &span);
     return S * N * K * 4;
 }
 
-WALSH_EXPORT int walsh_mhc_dphi(const void *g, const void *x, int64_t M, int64_t N, int64_t K, float *dphi, void *work,
+WALSH_EXPORT int walsh_linear_wgrad(const void *g, const void *x, int64_t M, int64_t N, int64_t K, float *dw, void *work,
                                 int64_t work_bytes, void *stream) {
-    const char *fn = "walsh_mhc_dphi";
-    if (!g || !x || !dphi || !work) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
-    if (M < 1 || N < 1 || N > 32 || K < 8 || K % 8 || M * (K > N ? K : N) * 2 > (int64_t)kMaxBufferBytes)
-        return set_error(WALSH_ENOTSUP, "%s: needs N <= 32, K a multiple of 8, operands below 2^31 bytes (M=%lld N=%lld "
+    const char *fn = "walsh_linear_wgrad";
+    if (!g || !x || !dw || !work) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
+    if (M < 1 || N < 1 || N > 1024 || K < 8 || K % 8 || M * (K > N ? K : N) * 2 > (int64_t)kMaxBufferBytes)
+        return set_error(WALSH_ENOTSUP, "%s: needs N <= 1024, K a multiple of 8, operands below 2^31 bytes (M=%lld N=%lld "
                          "K=%lld)", fn, (long long)M, (long long)N, (long long)K);
     if ((uintptr_t)x % 16 || (uintptr_t)g % 2 || (uintptr_t)work % 16 ||
-        work_bytes < walsh_mhc_dphi_workspace_bytes(M, N, K))
+        work_bytes < walsh_linear_wgrad_workspace_bytes(M, N, K))
         return set_error(WALSH_EINVAL, "%s: x and a workspace of %lld bytes 16-byte aligned, needs %lld", fn,
-                         (long long)work_bytes, (long long)walsh_mhc_dphi_workspace_bytes(M, N, K));
+                         (long long)work_bytes, (long long)walsh_linear_wgrad_workspace_bytes(M, N, K));
     int64_t S, span;
-    dphi_plan(M, K, &S, &span);
+    wgrad_plan(M, N, K, &S, &span);
     hipStream_t s = (hipStream_t)stream;
-    launch(mhc_dphi_kernel, dim3((unsigned)ceil_div(K, kDphiCols), (unsigned)S), dim3(64 * kDphiWaves), 0, s,
+    launch(linear_wgrad_kernel, dim3((unsigned)ceil_div(K, kWgradCols), (unsigned)S, (unsigned)ceil_div(N, 32)), dim3(64 * kWgradWaves), 0, s,
            (const uint16_t *)g, (const uint16_t *)x, (int)M, (int)N, (int)K, (int)span, (float *)work);
     const int rc = check_hip(hipGetLastError(), fn);
     if (rc) return rc;
-    launch(mhc_dphi_sum_kernel, dim3((unsigned)ceil_div(N * K, 256)), dim3(256), 0, s, (const float *)work, (int)S, N * K,
-           dphi);
+    launch(linear_wgrad_sum_kernel, dim3((unsigned)ceil_div(N * K, 256)), dim3(256), 0, s, (const float *)work, (int)S, N * K,
+           dw);
     return check_hip(hipGetLastError(), fn);
 }
 

@@ -80,8 +80,8 @@ SIGNATURES = {
                                ctypes.c_float, _P, _I64, _P, _P, _I, _P, _I64, _P]),
     "walsh_prefill_attention": (_I, [_P, _I64, _I64, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64,
                                      ctypes.c_float, _P, _I64, _I64, _I64, _I, _P]),
-    "walsh_mhc_dphi_workspace_bytes": (_I64, [_I64, _I64, _I64]),
-    "walsh_mhc_dphi": (_I, [_P, _P, _I64, _I64, _I64, _P, _P, _I64, _P]),
+    "walsh_linear_wgrad_workspace_bytes": (_I64, [_I64, _I64, _I64]),
+    "walsh_linear_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "walsh_rmsnorm_fwd": (_I, [_P, _P, _I64, _I64, ctypes.c_float, _P, _P, _P]),
     "walsh_rmsnorm_bwd_workspace_bytes": (_I64, [_I64, _I64]),
     "walsh_rmsnorm_bwd": (_I, [_P, _P, _P, _P, _I64, _I64, _P, _P, _P, _I64, _P]),

@@ -772,19 +772,19 @@ def octonion_linear_bwd(x: torch.Tensor, gy: torch.Tensor, in_o: int, out_o: int
     return gx, dw, db
 
 
-# ------------------------------------------------------------------ stream projection (training)
+# ------------------------------------------------------------------ small Linears (training)
 
-def mhc_dphi(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """g^T x in float32: g [M, N <= 32], x [M, K], contiguous bf16, K % 8 == 0."""
+def linear_wgrad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """g^T x in float32: g [M, N <= 1024], x [M, K], contiguous bf16, K % 8 == 0."""
     _hip.require_device(x, "input")
     M, N = g.shape
     K = x.shape[1]
     assert x.shape[0] == M and g.dtype == x.dtype == torch.bfloat16 and g.is_contiguous() and x.is_contiguous()
     out = torch.empty(N, K, device=x.device, dtype=torch.float32)
-    nws = _hip.lib().walsh_mhc_dphi_workspace_bytes(M, N, K)
+    nws = _hip.lib().walsh_linear_wgrad_workspace_bytes(M, N, K)
     ws = torch.empty(nws, device=x.device, dtype=torch.uint8)
-    _hip.call("walsh_mhc_dphi", g.data_ptr(), x.data_ptr(), M, N, K, out.data_ptr(), ws.data_ptr(), nws,
-              _hip.stream(x.device), kernel="mhc_dphi_kernel", nbytes=2 * M * (K + N), flops=2 * M * N * K)
+    _hip.call("walsh_linear_wgrad", g.data_ptr(), x.data_ptr(), M, N, K, out.data_ptr(), ws.data_ptr(), nws,
+              _hip.stream(x.device), kernel="linear_wgrad_kernel", nbytes=2 * M * (K + N), flops=2 * M * N * K)
     return out
 
 

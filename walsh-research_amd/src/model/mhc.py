@@ -13,7 +13,8 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import kernels
-from ._common import WeightCache, act_dtype, cached_linear, invalidate_weight_caches, plain_eager
+from .linear import FewRowsLinear
+from ._common import WeightCache, act_dtype, cached_linear, invalidate_weight_caches
 
 _MAX_STREAMS = 4
 
@@ -195,37 +196,6 @@ def materialize(x):
     return x.materialize() if isinstance(x, PendingUpdate) else x
 
 
-class PhiFunction(torch.autograd.Function):
-    """F.linear(xn, phi.to(bf16)) of bf16 rows with the mappings' float32 rows
-    phi; dphi on the HIP kernel (float32, not rounded to bf16 on the way)."""
-
-    @staticmethod
-    def takes(xn, phi) -> bool:
-        K = xn.shape[-1]
-        return (xn.is_cuda and xn.dtype == torch.bfloat16 and phi.dtype == torch.float32 and phi.device == xn.device
-                and type(xn) is torch.Tensor and type(phi) is torch.Tensor and xn.numel() > 0 and xn.is_contiguous()
-                and xn.data_ptr() % 16 == 0 and phi.shape[0] <= 32 and K % 8 == 0 and xn.numel() * 2 < 2 ** 31
-                and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
-                and plain_eager())
-
-    @staticmethod
-    def forward(ctx, xn, phi):
-        w = phi.to(xn.dtype)
-        ctx.save_for_backward(xn, phi, w)
-        return F.linear(xn, w)
-
-    @staticmethod
-    def backward(ctx, gd):
-        xn, phi, w = ctx.saved_tensors
-        nx, nw = ctx.needs_input_grad
-        g2, x2 = gd.reshape(-1, gd.shape[-1]), xn.reshape(-1, xn.shape[-1])
-        if torch.is_grad_enabled():   # differentiated itself: as F.linear's
-            gx = (g2 @ phi.to(xn.dtype)).view(xn.shape) if nx else None
-            return gx, (g2.t() @ x2).to(phi.dtype) if nw else None
-        gx = (g2 @ w).view(xn.shape) if nx else None
-        return gx, kernels.mhc_dphi(g2.contiguous(), x2) if nw else None
-
-
 class mHCResidualStream(nn.Module):
     """x_{l+1} = H_res @ x_l + H_post^T F(H_pre @ x_l) (mhc.py:321-381)."""
 
@@ -288,8 +258,8 @@ class mHCResidualStream(nn.Module):
         B, T, n, C = x.shape
         xn = F.rms_norm(x.reshape(B, T, n * C), (n * C,))
         phi = torch.cat([self.H_pre.phi.weight, self.H_post.phi.weight, self.H_res.phi.weight], 0)
-        if PhiFunction.takes(xn, phi):
-            d = PhiFunction.apply(xn, phi)
+        if FewRowsLinear.takes(xn, phi):
+            d = FewRowsLinear.apply(xn, phi)
         else:
             d = F.linear(xn, phi.to(xn.dtype))
         d_pre, d_post, d_res = d.split([n, n, n * n], dim=-1)

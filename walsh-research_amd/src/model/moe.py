@@ -31,6 +31,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import kernels
+from .linear import FewRowsLinear
 from ._common import WeightCache, act_dtype, tracked_dtype
 
 # A fused router keeps W1 in each wavefront's working set; beyond this width
@@ -289,11 +290,27 @@ class HadamardRouter(nn.Module):
             _zero_unselected(y2d, r)
         return r
 
+    def _gate_autograd(self, x: torch.Tensor) -> torch.Tensor:
+        """self.gate(x); under bf16 autocast its Linears take their weight
+        gradients on the HIP kernel, unless the modules were changed or carry
+        hooks that have to see the calls."""
+        mods = (self.gate, *self.gate)
+        l1, act, l2 = self.gate if len(self.gate) == 3 else (None, None, None)
+        if (x.is_cuda and torch.is_autocast_enabled("cuda") and type(l1) is nn.Linear and type(l2) is nn.Linear
+                and type(act) is nn.SiLU and not act.inplace and l1.bias is None and l2.bias is None
+                and not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                            for m in mods)
+                and not torch.nn.modules.module._has_any_global_hook()
+                and FewRowsLinear.takes(x, l1.weight)):
+            h = act(FewRowsLinear.apply(x, l1.weight))
+            return FewRowsLinear.apply(h, l2.weight) if FewRowsLinear.takes(h, l2.weight) else l2(h)
+        return self.gate(x)
+
     def route_autograd(self, x: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """moe.py:418-447 as differentiable operations (training): the router
         MLP, softmax, top-k mask and the renormalised weights; the gradient
         reaches the router through the probabilities of the selected experts."""
-        logits = self.gate(x)
+        logits = self._gate_autograd(x)
         probs = F.softmax(logits, dim=-1)
         _, idx = probs.topk(self.top_k, dim=-1)
         mask = torch.zeros_like(probs).scatter_(-1, idx, 1.0)
