@@ -206,6 +206,25 @@ def test_hadamard_wide_whole_rows_equal_general(K, M, pad):
     assert torch.equal(whole, K.hadamard_linear(rows(4096 + 4, 0), 128, 128, kw, alpha, beta))
 
 
+@pytest.mark.parametrize("M", [16384 + 1, 16384 + 16, 20007])
+def test_hadamard_whole_rows_store_only_their_rows(K, M):
+    """16x16 layers of 512-value rows beyond the wavefront pairs' row count move
+    whole rows on both sides: rows past M are neither read (NaN there) nor
+    written (guard rows behind the output)."""
+    from src.model import _hip
+    g = torch.Generator().manual_seed(M)
+    kw = _prepare(K, torch.randint(-1, 2, (32, 16, 16), generator=g).numpy().astype(np.int8))
+    alpha, beta = (1 + 0.5 * torch.randn(32, 16, generator=g)).cuda(), (0.1 * torch.randn(32, 16, generator=g)).cuda()
+    x = torch.full((M + 16, 512), float("nan"), dtype=torch.bfloat16, device="cuda")
+    x[:M] = torch.randn(M, 512, generator=g).to(torch.bfloat16).cuda()
+    y = torch.full((M + 16, 512), 7.0, dtype=torch.bfloat16, device="cuda")
+    _hip.call("walsh_hadamard_linear_ex_fwd", x.data_ptr(), 512, 16, M, 16, 16, kw.data_ptr(), alpha.data_ptr(),
+              beta.data_ptr(), y.data_ptr(), 512, 16, _hip.dtype_code(x.dtype), _hip.stream(x.device))
+    assert torch.all(y[M:] == 7.0)
+    pieces = torch.cat([K.hadamard_linear(p, 16, 16, kw, alpha, beta) for p in x[:M].split(4096)])   # pairs
+    assert torch.equal(y[:M], pieces)
+
+
 @pytest.mark.parametrize("in_o,out_o,M", [(24, 24, 1), (24, 20, 17), (64, 24, 127), (80, 36, 16), (8, 24, 8192), (16, 64, 8193),
                                           (24, 16, 4096), (24, 8, 4112), (48, 12, 5000), (16, 16, 16384), (4, 4, 40)])
 def test_hadamard_pair_linear_equals_general(K, in_o, out_o, M):

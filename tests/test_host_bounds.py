@@ -5,6 +5,10 @@ rows).  An operand holding fewer elements than the kernel would address is
 rejected on the host, before any launch.  (The Hadamard backward reads and
 writes its rows through bounds-checked buffer resources and checks its
 workspace size in walsh_hadamard_linear_ex_bwd.)"""
+import glob
+import os
+import re
+
 import pytest
 import torch
 
@@ -69,3 +73,35 @@ def test_half_range_check_of_wide_kernel_scales():
         p.mul_(1e5)
     with pytest.raises(ValueError):
         K.check_half_range("beta", p)
+
+
+def _calls(text, name):
+    """Argument lists of the calls of ``name`` (a pattern), split at top level."""
+    for m in re.finditer(name + r"\(", text):
+        args, depth, start = [], 1, m.end()
+        for i in range(m.end(), len(text)):
+            depth += (text[i] in "([{") - (text[i] in ")]}")
+            if depth == 0 or (depth == 1 and text[i] == ","):
+                args.append(" ".join(text[start:i].split()))
+                start = i + 1
+            if depth == 0:
+                break
+        yield args
+
+
+def test_buffer_scalar_offsets_lie_in_range():
+    """The range check of a buffer access covers its vector offset only, so a
+    scalar offset neither is the out-of-range marker nor depends on a row that
+    may lie past the last one: it is a constant, a group's or stream's stride
+    multiple, or the clamped half of row_offsets."""
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "walsh-research_amd", "csrc")
+    seen = 0
+    for path in sorted(glob.glob(os.path.join(csrc, "*.h")) + glob.glob(os.path.join(csrc, "*.hip"))):
+        text = open(path).read()
+        for name, at in ((r"raw_buffer_load_\w+", 2), (r"raw_buffer_store_\w+", 3), (r"buffer_load_lds", 4),
+                         (r"Buf4<\w+>::load1?", 2), (r"Buf4<\w+>::store1?", 3)):
+            for args in _calls(text, name):
+                seen += 1
+                bad = re.search(r"\bkOOB\b|\b(?:row|orow|tile|tok|tok0|tl|r0)\b", args[at])
+                assert not bad, f"{os.path.basename(path)}: {args}"
+    assert seen > 80

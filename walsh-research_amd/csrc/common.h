@@ -135,9 +135,20 @@ inline int64_t balanced_rows(int64_t M, int64_t rows_max, int64_t align) {
 // ---------------------------------------------------------------- buffer access
 // Raw buffer resources (gfx9 descriptor word 3 = 0x00020000).  A lane whose
 // byte offset is >= the buffer size reads zeros and its stores are dropped,
-// which replaces per-lane branches for tails.  kOOB is such an offset.
+// which replaces per-lane branches for tails.  kOOB is such an offset.  The
+// check covers the vector offset only: a scalar offset has to lie inside the
+// buffer by itself (row_offsets for rows that may not exist).
 constexpr uint32_t kOOB = 0x80000000u;
 constexpr uint32_t kMaxBufferBytes = 0x7fffffffu;
+
+// Offsets of a lane's bytes at voff of the row that starts at byte soff, for a
+// row index that the whole wavefront shares; a row that is not ok is dropped.
+struct RowOffsets {
+    uint32_t v, s;
+};
+__device__ __forceinline__ RowOffsets row_offsets(bool ok, uint32_t voff, uint32_t soff) {
+    return RowOffsets{ok ? voff : kOOB, ok ? soff : 0u};
+}
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);

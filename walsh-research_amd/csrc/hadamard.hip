@@ -164,8 +164,8 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
 #pragma unroll
             for (int i = 0; i < kTile; ++i) {
                 const int r = tl * kTile + i;
-                xrow[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)lane * 16,
-                                                                (tl < n_tiles && r < a.M) ? (uint32_t)r * 1024u : kOOB, 0);
+                const RowOffsets o = row_offsets(tl < n_tiles && r < a.M, (uint32_t)lane * 16, (uint32_t)r * 1024u);
+                xrow[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, o.v, o.s, 0);
             }
         };
         if constexpr (STAGED) {
@@ -259,16 +259,16 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
                 if (rope) stores(std::true_type{});
                 else stores(std::false_type{});
                 if constexpr (STAGED) {
-                    // whole output rows out of the area (rows past M fall
-                    // outside the buffer and are dropped)
+                    // whole output rows out of the area (rows past M are
+                    // dropped)
                     wave_lds_fence();
                     auto store_rows = [&](auto aux) {
 #pragma unroll
                         for (int i = 0; i < kTile; ++i) {
                             const u32x4 v = *(const u32x4 *)(area + i * kStagePitch + lane * 16);
-                            __builtin_amdgcn_raw_buffer_store_b128(v, yr, (uint32_t)lane * 16,
-                                                                   (uint32_t)(tile * kTile + i) * 1024u,
-                                                                   decltype(aux)::value);
+                            const int r = tile * kTile + i;
+                            const RowOffsets o = row_offsets(r < a.M, (uint32_t)lane * 16, (uint32_t)r * 1024u);
+                            __builtin_amdgcn_raw_buffer_store_b128(v, yr, o.v, o.s, decltype(aux)::value);
                         }
                     };
                     // cache policy 2: non-temporal
@@ -1183,8 +1183,8 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide3_kernel(HadArgs
 #pragma unroll
             for (int i = decltype(R0)::value; i < decltype(R1)::value; ++i) {
                 const int row = tl * kTile + i;
-                xrow[i] = __builtin_amdgcn_raw_buffer_load_b128(
-                    xr, (uint32_t)tid * 16, row < a.M ? (uint32_t)((int64_t)row * a.ldx * 2) : kOOB, 0);
+                const RowOffsets o = row_offsets(row < a.M, (uint32_t)tid * 16, (uint32_t)((int64_t)row * a.ldx * 2));
+                xrow[i] = __builtin_amdgcn_raw_buffer_load_b128(xr, o.v, o.s, 0);
             }
         }
     };
