@@ -1,0 +1,96 @@
+"""What autograd may do around the training functions that stand in for chains
+of torch operations, on the CPU: their kernels are replaced by stand-ins of
+the same contract, which read their operands by address as the kernels do."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from src.model import kernels
+from src.model.chassis import RMSNorm, RMSNormFunction
+
+
+def _floats(ptr, n):
+    return torch.from_numpy(np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(ctypes.c_float)), (n,)).copy())
+
+
+def _bf16(ptr, n):
+    raw = np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(ctypes.c_int16)), (n,)).copy()
+    return torch.from_numpy(raw).view(torch.bfloat16)
+
+
+def _store(ptr, t):
+    if ptr:
+        ctypes.memmove(ptr, t.contiguous().data_ptr(), t.numel() * t.element_size())
+
+
+class _Lib:
+    def __getattr__(self, name):
+        return lambda *a: 64
+
+
+def _call(name, *a, **kw):
+    """walsh_rmsnorm_fwd / _bwd on host memory, with their alignment checks."""
+    x, w, M, C = (a[0], a[1], a[2], a[3]) if name == "walsh_rmsnorm_fwd" else (a[0], a[1], a[4], a[5])
+    assert x % 8 == 0 and w % 16 == 0
+    xf, wf = _bf16(x, M * C).view(M, C).float(), _floats(w, C) if w else None
+    if name == "walsh_rmsnorm_fwd":
+        r = torch.rsqrt(xf.pow(2).mean(-1) + a[4])
+        _store(a[5], (xf * r[:, None]).bfloat16().float() * wf)
+        _store(a[6], r)
+        return
+    assert name == "walsh_rmsnorm_bwd" and a[3] % 16 == 0 and a[6] % 8 == 0
+    r, gy = _floats(a[2], M)[:, None], _floats(a[3], M * C).view(M, C)
+    if a[6]:
+        g = (gy * wf).bfloat16().float()
+        _store(a[6], (g * r - xf * r.pow(3) * (g * xf).mean(-1, keepdim=True)).bfloat16())
+    _store(a[7], (gy * (xf * r).bfloat16().float()).sum(0))
+
+
+@pytest.fixture
+def norm(monkeypatch):
+    """(fused, plain) RMSNorm of one weight on bf16 rows of 8 columns."""
+    monkeypatch.setattr(kernels._hip, "call", _call)
+    monkeypatch.setattr(kernels._hip, "lib", lambda: _Lib())
+    monkeypatch.setattr(kernels._hip, "stream", lambda d: 0)
+    monkeypatch.setattr(kernels._hip, "require_device", lambda t, what="": None)
+    torch.manual_seed(0)
+    m = RMSNorm(8)
+    with torch.no_grad():
+        m.weight.uniform_(0.5, 1.5)
+    return m, lambda x: RMSNormFunction.apply(x.clone(), m.weight, m.eps), lambda x: m(x)
+
+
+def _close(a, b):
+    for u, v in zip(a, b):
+        assert torch.allclose(u.float(), v.float(), rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.float().abs().max()))
+
+
+def _rows(n=5):
+    return torch.randn(n, 8).bfloat16().requires_grad_(True)
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+def test_rmsnorm_gradient_at_any_offset(norm, rows):
+    """A gradient that arrives as a contiguous view 12 bytes past an aligned
+    address (the norm's output flattened behind three other values)."""
+    m, fused, plain = norm
+    x, head, g = _rows(rows), torch.zeros(3), torch.randn(3 + rows * 8)
+    close = [torch.autograd.grad(torch.cat([head, f(x).reshape(-1)]), (x, m.weight), g) for f in (fused, plain)]
+    _close(*close)
+
+
+def test_rmsnorm_saved_tensor_hooks(norm):
+    """Hooks that give the saved rows back in another layout or off alignment."""
+    m, fused, plain = norm
+    x, g = _rows(), torch.randn(5, 8)
+    ref = torch.autograd.grad(plain(x), (x, m.weight), g)
+
+    def shifted(t):
+        return torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)
+    for pack, unpack in ((lambda t: t.t().contiguous() if t.dim() == 2 else t,
+                          lambda t: t.t() if t.dim() == 2 else t), (lambda t: t, shifted)):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = fused(x)
+        _close(torch.autograd.grad(y, (x, m.weight), g), ref)

@@ -790,6 +790,13 @@ def linear_wgrad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 # ------------------------------------------------------------------ RMSNorm (training)
 
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous and 16-byte aligned: itself, or a copy (a gradient may
+    be a view at any offset, a saved tensor whatever its hook returns)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float):
     """bf16(x rsqrt(mean(x^2) + eps)) * w in float32 and the float32 factors
     per row; x contiguous bf16 [..., C], w float32 [C], C % 4 == 0, C <= 2048."""
@@ -808,7 +815,7 @@ def rmsnorm_bwd(x: torch.Tensor, w: torch.Tensor, rstd: torch.Tensor, gy: torch.
     """(gx, gw) of rmsnorm; entries not requested in ``need`` are None."""
     C = x.shape[-1]
     M = x.numel() // C
-    gy = gy.contiguous()
+    x, w, rstd, gy = (_rows16(t) for t in (x, w, rstd, gy))
     gx = torch.empty_like(x) if need[0] else None
     gw = torch.empty_like(w) if need[1] else None
     nws = _hip.lib().walsh_rmsnorm_bwd_workspace_bytes(M, C) if need[1] else 0
