@@ -6,9 +6,11 @@ import ctypes
 import numpy as np
 import pytest
 import torch
+import torch.nn.functional as F
 
 from src.model import kernels
 from src.model.chassis import RMSNorm, RMSNormFunction
+from src.model.linear import FewRowsLinear
 
 
 def _floats(ptr, n):
@@ -64,7 +66,8 @@ def norm(monkeypatch):
 
 def _close(a, b):
     for u, v in zip(a, b):
-        assert torch.allclose(u.float(), v.float(), rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.float().abs().max()))
+        u, v = u.detach().float(), v.detach().float()
+        assert torch.allclose(u, v, rtol=2.0 ** -6, atol=2.0 ** -7 * float(v.abs().max()))
 
 
 def _rows(n=5):
@@ -94,3 +97,53 @@ def test_rmsnorm_saved_tensor_hooks(norm):
         with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
             y = fused(x)
         _close(torch.autograd.grad(y, (x, m.weight), g), ref)
+
+
+def _linear(w):
+    return lambda x: FewRowsLinear.apply(x, w), lambda x: F.linear(x, w.to(x.dtype))
+
+
+@pytest.fixture
+def wgrad(monkeypatch):
+    def call(name, g, x, M, N, K, dw, *rest, **kw):
+        assert name == "walsh_linear_wgrad" and x % 16 == 0
+        _store(dw, _bf16(g, M * N).view(M, N).float().t() @ _bf16(x, M * K).view(M, K).float())
+    monkeypatch.setattr(kernels._hip, "call", call)
+    monkeypatch.setattr(kernels._hip, "lib", lambda: _Lib())
+    monkeypatch.setattr(kernels._hip, "stream", lambda d: 0)
+    monkeypatch.setattr(kernels._hip, "require_device", lambda t, what="": None)
+    torch.manual_seed(1)
+    return torch.randn(6, 8).requires_grad_(True)
+
+
+def test_few_rows_linear_weight_updated_before_backward(wgrad):
+    """Two forwards before an optimizer step, or a step between a forward and
+    its backward: the gradients belong to the weight of the forward."""
+    w = wgrad
+    x, g = _rows(), torch.randn(5, 6).bfloat16()
+    got = []
+    for f in _linear(w):
+        y = f(x)
+        before = w.detach().clone()
+        with torch.no_grad():
+            w.mul_(-3.0)
+        got.append((y,) + torch.autograd.grad(y, (x, w), g))
+        with torch.no_grad():
+            w.copy_(before)
+    _close(*got)
+    second = []
+    for f in _linear(w):
+        gx, gw = torch.autograd.grad(f(x).float().square().sum(), (x, w), create_graph=True)
+        second.append(torch.autograd.grad(gx.float().square().sum() + gw.square().sum(), (x, w)))
+    _close(*second)
+
+
+def test_few_rows_linear_saved_tensor_hooks(wgrad):
+    x, g = _rows(), torch.randn(5, 6).bfloat16()
+    f, plain = _linear(wgrad)
+    ref = torch.autograd.grad(plain(x), (x, wgrad), g)
+    for pack, unpack in ((lambda t: t.t().contiguous(), lambda t: t.t()),
+                         (lambda t: t, lambda t: torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape))):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            y = f(x)
+        _close(torch.autograd.grad(y, (x, wgrad), g), ref)

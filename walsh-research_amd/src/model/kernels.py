@@ -774,12 +774,20 @@ def octonion_linear_bwd(x: torch.Tensor, gy: torch.Tensor, in_o: int, out_o: int
 
 # ------------------------------------------------------------------ small Linears (training)
 
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous and 16-byte aligned: itself, or a copy (a gradient may
+    be a view at any offset, a saved tensor whatever its hook returns)."""
+    t = t.contiguous()
+    return t.clone() if t.data_ptr() % 16 else t
+
+
 def linear_wgrad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """g^T x in float32: g [M, N <= 1024], x [M, K], contiguous bf16, K % 8 == 0."""
+    """g^T x in float32: g [M, N <= 1024], x [M, K], bf16, K % 8 == 0."""
     _hip.require_device(x, "input")
     M, N = g.shape
     K = x.shape[1]
-    assert x.shape[0] == M and g.dtype == x.dtype == torch.bfloat16 and g.is_contiguous() and x.is_contiguous()
+    assert x.shape[0] == M and g.dtype == x.dtype == torch.bfloat16
+    g, x = g.contiguous(), _rows16(x)
     out = torch.empty(N, K, device=x.device, dtype=torch.float32)
     nws = _hip.lib().walsh_linear_wgrad_workspace_bytes(M, N, K)
     ws = torch.empty(nws, device=x.device, dtype=torch.uint8)
@@ -789,13 +797,6 @@ def linear_wgrad(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
 
 
 # ------------------------------------------------------------------ RMSNorm (training)
-
-def _rows16(t: torch.Tensor) -> torch.Tensor:
-    """``t`` contiguous and 16-byte aligned: itself, or a copy (a gradient may
-    be a view at any offset, a saved tensor whatever its hook returns)."""
-    t = t.contiguous()
-    return t.clone() if t.data_ptr() % 16 else t
-
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float):
     """bf16(x rsqrt(mean(x^2) + eps)) * w in float32 and the float32 factors

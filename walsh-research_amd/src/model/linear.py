@@ -15,7 +15,29 @@ from ._common import plain_eager
 MAX_WEIGHTS = 400 * 1024
 
 
-class FewRowsLinear(torch.autograd.Function):
+class _FewRowsLinearFunction(torch.autograd.Function):
+    """F.linear(x, wb) for wb = w.to(bf16) of a float32 weight w: the plain
+    backward gives w its gradient in float32, one that is itself
+    differentiated gives wb its own, as F.linear's.  Of the weights only wb is
+    saved, so w may change between the forward and its backward."""
+
+    @staticmethod
+    def forward(ctx, x, w, wb):
+        ctx.save_for_backward(x, wb)
+        return F.linear(x, wb)
+
+    @staticmethod
+    def backward(ctx, gy):
+        x, wb = ctx.saved_tensors
+        nx, nw, _ = ctx.needs_input_grad
+        g2, x2 = gy.reshape(-1, gy.shape[-1]), x.reshape(-1, x.shape[-1])
+        gx = (g2 @ wb).view(x.shape) if nx else None
+        if torch.is_grad_enabled():
+            return gx, None, g2.t() @ x2 if nw else None
+        return gx, kernels.linear_wgrad(g2, x2) if nw else None, None
+
+
+class FewRowsLinear:
     """F.linear(x, w.to(bf16)) of bf16 rows with a float32 weight w; dw on the
     HIP kernel (float32, not rounded to bf16 on the way)."""
 
@@ -30,18 +52,5 @@ class FewRowsLinear(torch.autograd.Function):
                 and plain_eager())
 
     @staticmethod
-    def forward(ctx, x, w):
-        wb = w.to(x.dtype)
-        ctx.save_for_backward(x, w, wb)
-        return F.linear(x, wb)
-
-    @staticmethod
-    def backward(ctx, gy):
-        x, w, wb = ctx.saved_tensors
-        nx, nw = ctx.needs_input_grad
-        g2, x2 = gy.reshape(-1, gy.shape[-1]), x.reshape(-1, x.shape[-1])
-        if torch.is_grad_enabled():   # differentiated itself: as F.linear's
-            gx = (g2 @ w.to(x.dtype)).view(x.shape) if nx else None
-            return gx, (g2.t() @ x2).to(w.dtype) if nw else None
-        gx = (g2 @ wb).view(x.shape) if nx else None
-        return gx, kernels.linear_wgrad(g2.contiguous(), x2) if nw else None
+    def apply(x, w):
+        return _FewRowsLinearFunction.apply(x, w, w.to(x.dtype))
