@@ -753,9 +753,9 @@ int walsh_chanmod_bwd(const void *gy, int64_t ldg, const void *x, int64_t ldx, i
  *     rstd[t] = rsqrt(mean(x[t]^2) + eps);  y = bf16(x rstd) w   (float32)
  *     g = bf16(gy w);  gx = bf16(rstd g - x rstd^3 mean(g x))     (bf16)
  *     gw = sum over rows of gy bf16(x rstd)       (fixed order: deterministic)
- *   M >= 1, C a multiple of 4 up to 2048.  gx or gw may be null; gw needs
- *   work of walsh_rmsnorm_bwd_workspace_bytes(M, C) bytes.  x and gx 8-byte,
- *   the float arrays 16-byte aligned. */
+ *   M >= 1, C a multiple of 4 up to 2048.  gx (then w too) or gw may be null;
+ *   gw needs work of walsh_rmsnorm_bwd_workspace_bytes(M, C) bytes.  x and gx
+ *   8-byte, the float arrays 16-byte aligned. */
 int walsh_rmsnorm_fwd(const void *x, const float *w, int64_t M, int64_t C, float eps, float *y, float *rstd,
                       void *stream);
 int64_t walsh_rmsnorm_bwd_workspace_bytes(int64_t M, int64_t C);

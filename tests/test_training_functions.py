@@ -147,3 +147,31 @@ def test_few_rows_linear_saved_tensor_hooks(wgrad):
         with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
             y = f(x)
         _close(torch.autograd.grad(y, (x, wgrad), g), ref)
+
+
+def test_rmsnorm_gain_updated_before_backward(norm):
+    """Rows without a gradient: the gain's own gradient does not depend on it,
+    and it may change between the forward and the backward."""
+    m, fused, plain = norm
+    x, g = _rows().detach(), torch.randn(5, 8)
+    got = []
+    for f in (fused, plain):
+        y = f(x)
+        with torch.no_grad():
+            m.weight.mul_(2.0)
+        got.append(torch.autograd.grad(y, (m.weight,), g))
+    _close(*got)
+
+
+@pytest.mark.parametrize("wrt", [(0, 1), (0,), (1,)])
+def test_rmsnorm_differentiated_backward(norm, wrt):
+    m, fused, plain = norm
+    x = _rows()
+    ins = [(x, m.weight)[i] for i in wrt]
+    if 0 not in wrt:
+        x = x.detach()
+    got = []
+    for f in (fused, plain):
+        first = torch.autograd.grad(f(x).pow(3).sum(), ins, create_graph=True)
+        got.append(first + torch.autograd.grad(sum(v.float().square().sum() for v in first), ins))
+    _close(*got)

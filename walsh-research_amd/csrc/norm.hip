@@ -73,7 +73,7 @@ __global__ __launch_bounds__(64 * kNormWaves) void rmsnorm_bwd_kernel(const uint
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         const int c = 256 * k + 4 * lane;
-        wv[k] = c < C ? load4(w + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+        wv[k] = gx && c < C ? load4(w + c) : f32x4{0.f, 0.f, 0.f, 0.f};
         gw[k] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     for (int64_t t = (int64_t)blockIdx.x * kNormWaves + wave; t < M; t += (int64_t)gridDim.x * kNormWaves) {
@@ -178,7 +178,7 @@ WALSH_EXPORT int64_t walsh_rmsnorm_bwd_workspace_bytes(int64_t M, int64_t C) {
 WALSH_EXPORT int walsh_rmsnorm_bwd(const void *x, const float *w, const float *rstd, const float *gy, int64_t M,
                                    int64_t C, void *gx, float *gw, void *work, int64_t work_bytes, void *stream) {
     const char *fn = "walsh_rmsnorm_bwd";
-    if (!x || !w || !rstd || !gy || (gw && !work)) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
+    if (!x || (gx && !w) || !rstd || !gy || (gw && !work)) return set_error(WALSH_EINVAL, "%s: null pointer", fn);
     int rc = norm_check(fn, M, C, x, w, gy);
     if (rc) return rc;
     if (!gx && !gw) return WALSH_OK;

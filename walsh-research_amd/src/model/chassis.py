@@ -71,26 +71,31 @@ def get_head_mixer(config: WalshConfig, head_dim: int):
 class RMSNormFunction(torch.autograd.Function):
     """RMSNorm of bf16 rows with a float32 weight on the HIP kernels; the
     values and roundings of the element-by-element form, which a backward that
-    is itself differentiated falls back to."""
+    is itself differentiated falls back to.  The weight is saved only where
+    the rows' gradient needs it, so elsewhere it may change before the
+    backward, as in that form."""
 
     @staticmethod
     def forward(ctx, x, w, eps):
         y, rstd = kernels.rmsnorm(x, w, eps)
         ctx.eps = eps
-        ctx.save_for_backward(x, w, rstd)
+        ctx.save_for_backward(x, w if ctx.needs_input_grad[0] else None, rstd)
         return y
 
     @staticmethod
     def backward(ctx, gy):
         x, w, rstd = ctx.saved_tensors
         need = ctx.needs_input_grad[:2]
-        if torch.is_grad_enabled():
-            y = RMSNorm.normalised(x.float(), ctx.eps).type_as(x) * w
-            ins = [t for t, n in zip((x, w), need) if n]
-            got = iter(torch.autograd.grad(y, ins, gy, create_graph=True))
-            gx, gw = (next(got) if n else None for n in need)
-        else:
-            gx, gw = kernels.rmsnorm_bwd(x, w, rstd, gy, need)
+        if not torch.is_grad_enabled():
+            return *kernels.rmsnorm_bwd(x, w, rstd, gy, need), None
+        xf = x.float()
+        r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)
+        gx = gw = None
+        if need[0]:
+            g = (gy * w).type_as(x).float()
+            gx = (g * r - xf * r.pow(3) * (g * xf).mean(-1, keepdim=True)).type_as(x)
+        if need[1]:
+            gw = (gy * (xf * r).type_as(x)).reshape(-1, x.shape[-1]).sum(0)
         return gx, gw, None
 
 

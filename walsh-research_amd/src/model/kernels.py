@@ -813,16 +813,18 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float):
 
 
 def rmsnorm_bwd(x: torch.Tensor, w: torch.Tensor, rstd: torch.Tensor, gy: torch.Tensor, need=(True, True)):
-    """(gx, gw) of rmsnorm; entries not requested in ``need`` are None."""
+    """(gx, gw) of rmsnorm; entries not requested in ``need`` are None (gw alone
+    does not use ``w``, which may then be None)."""
     C = x.shape[-1]
     M = x.numel() // C
-    x, w, rstd, gy = (_rows16(t) for t in (x, w, rstd, gy))
+    x, rstd, gy = (_rows16(t) for t in (x, rstd, gy))
+    w = _rows16(w) if need[0] else None
     gx = torch.empty_like(x) if need[0] else None
-    gw = torch.empty_like(w) if need[1] else None
+    gw = torch.empty(C, device=x.device, dtype=torch.float32) if need[1] else None
     nws = _hip.lib().walsh_rmsnorm_bwd_workspace_bytes(M, C) if need[1] else 0
     ws = torch.empty(nws, device=x.device, dtype=torch.uint8) if need[1] else None
     ptr = lambda t: 0 if t is None else t.data_ptr()  # noqa: E731
-    _hip.call("walsh_rmsnorm_bwd", x.data_ptr(), w.data_ptr(), rstd.data_ptr(), gy.data_ptr(), M, C, ptr(gx), ptr(gw),
+    _hip.call("walsh_rmsnorm_bwd", x.data_ptr(), ptr(w), rstd.data_ptr(), gy.data_ptr(), M, C, ptr(gx), ptr(gw),
               ptr(ws), nws, _hip.stream(x.device), kernel="rmsnorm_bwd_kernel", nbytes=M * C * 8, flops=10 * M * C)
     return gx, gw
 
