@@ -175,3 +175,39 @@ def test_rmsnorm_differentiated_backward(norm, wrt):
         first = torch.autograd.grad(f(x).pow(3).sum(), ins, create_graph=True)
         got.append(first + torch.autograd.grad(sum(v.float().square().sum() for v in first), ins))
     _close(*got)
+
+
+def _batched(y, ins, gs):
+    return torch.autograd.grad(y, ins, gs, is_grads_batched=True)
+
+
+def test_rmsnorm_batched_gradients(norm):
+    m, fused, plain = norm
+    x, gs = _rows(), torch.randn(3, 5, 8)
+    _close(_batched(fused(x), (x, m.weight), gs), _batched(plain(x), (x, m.weight), gs))
+    jac = [torch.autograd.functional.jacobian(f, x.detach(), vectorize=True) for f in (fused, plain)]
+    _close(*([j] for j in jac))
+
+
+def test_few_rows_linear_batched_gradients(wgrad):
+    x, gs = _rows(), torch.randn(3, 5, 6).bfloat16()
+    f, plain = _linear(wgrad)
+    _close(_batched(f(x), (x, wgrad), gs), _batched(plain(x), (x, wgrad), gs))
+
+
+def test_backward_under_a_dispatch_mode(norm):
+    """A mode around the backward alone sees its operations, and a functional
+    transform of a whole step keeps the plain form's values."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    m, fused, plain = norm
+    x, g = _rows(), torch.randn(5, 8)
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+    seen, y = [], fused(x)
+    with Seen():
+        got = torch.autograd.grad(y, (x, m.weight), g)
+    assert len(seen) > 5
+    _close(got, torch.autograd.grad(plain(x), (x, m.weight), g))

@@ -89,6 +89,15 @@ def plain_eager() -> bool:
             and torch.utils._python_dispatch._get_current_dispatch_mode() is None)
 
 
+def first_order(gy: torch.Tensor) -> bool:
+    """Whether a backward may run kernels on the gradient ``gy``: it is not
+    differentiated itself, and neither a transform (batched gradients, a
+    vectorised Jacobian) nor a mode has to see its operations."""
+    f = torch._C._functorch
+    return (not torch.is_grad_enabled() and type(gy) is torch.Tensor and not f.is_legacy_batchedtensor(gy)
+            and not f.is_functorch_wrapped_tensor(gy) and plain_eager())
+
+
 def adjacent_parts_view(parts, width: int):
     """If ``parts`` are equal-shape slices laid side by side along the last
     dim of one tensor (what ``x.split(width, -1)`` returns), return the

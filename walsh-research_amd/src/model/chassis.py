@@ -22,7 +22,7 @@ from .hadamard import HadamardLinearFunction
 from .hadamard import HadamardHeadMixer, HadamardHeadMixerFused
 from .octonion import OctonionHeadMixerFused, OctonionTernaryLinear
 from . import kernels
-from ._common import WeightCache, act_dtype, cached_linear, plain_eager
+from ._common import WeightCache, act_dtype, cached_linear, first_order, plain_eager
 
 _HADAMARD_AVAILABLE = True
 _HADAMARD_HEAD_MIXER_AVAILABLE = True
@@ -71,7 +71,7 @@ def get_head_mixer(config: WalshConfig, head_dim: int):
 class RMSNormFunction(torch.autograd.Function):
     """RMSNorm of bf16 rows with a float32 weight on the HIP kernels; the
     values and roundings of the element-by-element form, which a backward that
-    is itself differentiated falls back to.  The weight is saved only where
+    is itself differentiated or batched falls back to.  The weight is saved only where
     the rows' gradient needs it, so elsewhere it may change before the
     backward, as in that form."""
 
@@ -86,7 +86,7 @@ class RMSNormFunction(torch.autograd.Function):
     def backward(ctx, gy):
         x, w, rstd = ctx.saved_tensors
         need = ctx.needs_input_grad[:2]
-        if not torch.is_grad_enabled():
+        if first_order(gy):
             return *kernels.rmsnorm_bwd(x, w, rstd, gy, need), None
         xf = x.float()
         r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)

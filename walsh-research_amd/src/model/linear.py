@@ -4,7 +4,7 @@ import torch
 import torch.nn.functional as F
 
 from . import kernels
-from ._common import plain_eager
+from ._common import first_order, plain_eager
 
 # N * K up to which the weight gradient runs on the HIP kernel: the library
 # gives a product with a small output few workgroups.  Kernel against library
@@ -17,8 +17,8 @@ MAX_WEIGHTS = 400 * 1024
 
 class _FewRowsLinearFunction(torch.autograd.Function):
     """F.linear(x, wb) for wb = w.to(bf16) of a float32 weight w: the plain
-    backward gives w its gradient in float32, one that is itself
-    differentiated gives wb its own, as F.linear's.  Of the weights only wb is
+    backward gives w its gradient in float32, one that is itself differentiated
+    or batched gives wb its own, as F.linear's.  Of the weights only wb is
     saved, so w may change between the forward and its backward."""
 
     @staticmethod
@@ -32,7 +32,7 @@ class _FewRowsLinearFunction(torch.autograd.Function):
         nx, nw, _ = ctx.needs_input_grad
         g2, x2 = gy.reshape(-1, gy.shape[-1]), x.reshape(-1, x.shape[-1])
         gx = (g2 @ wb).view(x.shape) if nx else None
-        if torch.is_grad_enabled():
+        if not first_order(gy):
             return gx, None, g2.t() @ x2 if nw else None
         return gx, kernels.linear_wgrad(g2, x2) if nw else None, None
 
