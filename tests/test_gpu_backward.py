@@ -100,6 +100,27 @@ def test_hadamard_bwd_pairs_equal_general(K, in_o, out_o, M):
         assert_close(a.float().cpu().numpy(), r, torch.bfloat16, f"{name} {in_o}x{out_o} M={M}")
 
 
+@pytest.mark.parametrize("in_o,out_o", [(71 * 16, 16), (72 * 16, 4), (4, 75 * 16), (75 * 16, 20)])
+def test_hadamard_bwd_very_wide_without_weight_gradient(K, in_o, out_o):
+    """Frozen weights lower the general kernel's LDS need below that of the
+    wavefront pairs (from 72 chunks or tiles of one side on): such layers stay
+    accepted, rows aligned or not, with the same input gradient."""
+    c = make_case(K, 33, in_o, out_o, torch.bfloat16, seed=in_o + out_o)
+    rest = (in_o, out_o, c["kw"], c["kwt"], c["alpha"].cuda(), c["beta"].cuda())
+
+    def odd(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+    need = (True, True, True, False)
+    got = K.hadamard_linear_bwd(c["x"].cuda(), c["gy"].cuda(), *rest, need=need)
+    other = K.hadamard_linear_bwd(odd(c["x"]), odd(c["gy"]), *rest, need=need)
+    assert torch.equal(got[0], other[0]) and got[3] is None
+    ref = ohad.hadamard_linear_bwd_f64(c["x"].double().numpy(), c["codes"], c["alpha"].double().numpy(),
+                                       c["beta"].double().numpy(), c["gy"].double().numpy(),
+                                       latent=c["latent"].double().numpy())
+    for name, a, r in zip(("gx", "dalpha", "dbeta"), got, ref):
+        assert_close(a.float().cpu().numpy(), r, torch.bfloat16, f"{name} {in_o}x{out_o}")
+
+
 def test_hadamard_bwd_partial_outputs_and_determinism(K):
     c = make_case(K, 500, 16, 16, torch.bfloat16, seed=9)
     args = (c["x"].cuda(), c["gy"].cuda(), 16, 16, c["kw"], c["kwt"], c["alpha"].cuda(), c["beta"].cuda())

@@ -17,9 +17,9 @@
 // Every product above is H0 ... H0 / 32, so the kernels run unnormalised
 // transforms and the reduction applies the 1/32.
 //
-// Kernel: hadamard_bwd_kernel (float32, and bf16 rows without 8-byte
-// alignment) or hadamard_bwd_pair_kernel (bf16), one launch with three
-// workgroup roles.
+// Kernel: hadamard_bwd_kernel or, for bf16 rows in 8-byte pieces whose tables
+// fit its LDS, hadamard_bwd_pair_kernel: one launch with three workgroup
+// roles.
 //   dW role: per (token range, output tile, input chunk), H0(beta .* gy) and
 //     H0(alpha .* x) in the forward lane layout (lane = token, 4 columns),
 //     turned into token-major fragments by a matrix-core product with the
@@ -567,6 +567,11 @@ static int split_count(int n_tiles, int per_split_min, int64_t target, int *tps)
     return (int)ceil_div(n_tiles, *tps);
 }
 
+// LDS of the pair kernel: the larger side's scales, one tile of the other's,
+// the exchange area.  A very wide layer that asks for no weight gradient fits
+// the one-wavefront kernel (16 * 128 * (Nt + Kc)) and not this one.
+static size_t pair_lds(int Nt, int Kc) { return (size_t)16 * 128 * ((Nt > Kc ? Nt : Kc) + 1) + kPairXch; }
+
 // Pair kernel: the workgroups that are resident at once (two wavefronts per
 // SIMD, a pair per workgroup) take equal shares of the roles' tile steps: a
 // step is one input chunk of a tile's transform (a dW step two, x and gy).
@@ -690,26 +695,27 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     const size_t valign = bf16 ? 8 : 16;
     const bool vec = gsy % 4 == 0 && gsx % 4 == 0 && ldx % 4 == 0 && ldg % 4 == 0 && (!gx || ldgx % 4 == 0) &&
                      (uintptr_t)gy % valign == 0 && (uintptr_t)x % valign == 0 && (!gx || (uintptr_t)gx % valign == 0);
+    const int Nt = (int)ceil_div(out_o, kNTile), Kc = (int)ceil_div(in_o, kKChunk);
+    const int64_t maxlds = device_info().max_shared_per_block;
     // bf16 rows in 8-byte pieces: wavefront pairs
-    const bool pair = bf16 && vec;
+    const bool pair = bf16 && vec && (int64_t)pair_lds(Nt, Kc) <= maxlds;
     const BwdLayout L = plan(M, in_o, out_o, ld, esz, pair);
     if (M > 0 && L.rows_max == 0) return set_error(WALSH_ENOTSUP, "%s: row stride too large", fn);
     if (M > 0 && (!workspace || workspace_bytes < L.bytes))
         return set_error(WALSH_EINVAL, "%s: workspace of %lld bytes < %lld needed", fn, (long long)workspace_bytes,
                          (long long)L.bytes);
     hipStream_t s = (hipStream_t)stream;
-    const int Nt = (int)ceil_div(out_o, kNTile), Kc = (int)ceil_div(in_o, kKChunk);
     const int Ap = Kc * kKChunk, Bp = Nt * kNTile;
     float *pa = (float *)workspace;
     float *pb = (float *)((char *)workspace + L.off_b);
     float *pw = (float *)((char *)workspace + L.off_w);
-    const int64_t maxlds = device_info().max_shared_per_block;
 
     int64_t ia = 0, ib = 0, iw = 0;  // partial rows written so far
     const size_t lds_red = (size_t)16 * 128 * (Nt + Kc);
     const size_t lds_dw = (size_t)16 * 128 * (Nt + Kc) + (size_t)32 * 64 * 16;
     const size_t lds = need_w && lds_dw > lds_red ? lds_dw : lds_red;
-    if ((int64_t)(lds_red + shape_reserve(bf16)) > maxlds || (int64_t)lds > maxlds) return set_error(WALSH_ENOTSUP, "%s: shape needs %zu B of LDS", fn, lds);
+    if ((int64_t)(lds_red + shape_reserve(bf16)) > maxlds || (int64_t)lds > maxlds)
+        return set_error(WALSH_ENOTSUP, "%s: shape needs %zu B of LDS", fn, lds);
     for (int64_t r0 = 0; r0 < M; r0 += L.rows_max) {
         const int64_t rows = (M - r0) < L.rows_max ? (M - r0) : L.rows_max;
         const BwdChunk p = plan_chunk(rows, (int)in_o, (int)out_o, pair);
@@ -753,11 +759,12 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
         const dim3 G((unsigned)(j.nW + j.nA + j.nB)), B(kThreads);
 #define WALSH_BWD(T, MMA, V, ST) launch((hadamard_bwd_kernel<T, MMA, V, ST>), G, B, lds, s, j)
         if (pair) {
-            const size_t plds = (size_t)16 * 128 * ((Nt > Kc ? Nt : Kc) + 1) + kPairXch;
+            const size_t plds = pair_lds(Nt, Kc);
             if (gx) launch(hadamard_bwd_pair_kernel<true>, G, dim3(kPairThreads), plds, s, j);
             else launch(hadamard_bwd_pair_kernel<false>, G, dim3(kPairThreads), plds, s, j);
         } else if (bf16) {
-            if (gx) WALSH_BWD(uint16_t, true, false, true); else WALSH_BWD(uint16_t, true, false, false);
+            if (vec) { if (gx) WALSH_BWD(uint16_t, true, true, true); else WALSH_BWD(uint16_t, true, true, false); }
+            else     { if (gx) WALSH_BWD(uint16_t, true, false, true); else WALSH_BWD(uint16_t, true, false, false); }
         } else {
             if (vec) { if (gx) WALSH_BWD(float, false, true, true); else WALSH_BWD(float, false, true, false); }
             else     { if (gx) WALSH_BWD(float, false, false, true); else WALSH_BWD(float, false, false, false); }
