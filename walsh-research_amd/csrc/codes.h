@@ -11,12 +11,12 @@ namespace walsh {
 // bits (15 - 2p, 14 - 2p) of both halves, so a shift by 2p and one mask give
 // a register with two bf16 weights: two VALU operations per pair, no table.
 // The factor 2 is a power of two and is taken back with the transforms'
-// 1/32 (kCodeScale), exactly.  The former byte -> 4 x bf16 table in LDS cost
-// a conflicting 8-byte read per lane and 4 weights, a build loop per launch
-// and 2 to 10 KB of LDS.  Measured, outputs bitwise equal: the chunk-loop
-// SwiGLU and down projection at n_embd 768, 6,007 rows 108.3 -> 103.3 us;
-// the launches bound elsewhere (n_embd 4096 linear, 16,384 rows 104.8 ->
-// 104.6 us) keep their time.
+// 1/32 (kCodeScale), exactly, but float32 sums reach infinity one power of two
+// earlier than with +-1 weights (six in hadamard_wide3_kernel, whose table held
+// +-1/32).  A byte -> 4 x bf16 table in LDS costs a conflicting 8-byte read per
+// lane and 4 weights, a build loop per launch and 2 to 10 KB of LDS that the
+// wavefront pairs need for themselves.  By itself the change is small: general
+// bf16 kernel, 64 -> 64 columns per group at 8,192 rows 292 -> 286 us.
 constexpr uint32_t kCodeMask = 0xC000C000u;
 constexpr float kCodeScale = 0.015625f;      // 1/32 of the two transforms, 1/2 of the +-2.0 weights
 constexpr float kTransformScale = 0.03125f;  // the two transforms alone (dense weights)
@@ -35,6 +35,25 @@ __device__ __forceinline__ f32x4 codes_f32x4(uint32_t w, int k) {
     for (int j = 0; j < 4; ++j)
         r[j] = __uint_as_float((w << (4 * k + 2 * (j >> 1) + ((j & 1) ? 0 : 16))) & 0xC0000000u);
     return r;
+}
+// float32 kernels of the Hadamard layers: a table of the four weights in a byte
+// of a word (entry b, element i: the code at bits 7 - 2i, 6 - 2i).  The float32
+// products share the VALU's issue, so two operations for each weight's register
+// lengthened the launches by 2 to 18% (512 -> 512 features, 16 rows 10.7 ->
+// 11.2 us; 2,048 -> 2,048, 16,384 rows 162 -> 184; backward of 4,096 -> 4,096 at
+// 1,024 rows 166 -> 190); one 16-byte LDS read gives four.
+constexpr int kCodeLut = 256;
+__device__ __forceinline__ f32x4 code_lut_entry(uint32_t byte) {
+    return f32x4{__uint_as_float((byte << 24) & 0xC0000000u), __uint_as_float((byte << 26) & 0xC0000000u),
+                 __uint_as_float((byte << 28) & 0xC0000000u), __uint_as_float((byte << 30) & 0xC0000000u)};
+}
+// The weights of groups 2m and 2m + 1 of a 16-column chunk's word: its bytes
+// hold the first and third (lower half) and the second and fourth (upper half)
+// of both.
+__device__ __forceinline__ void codes_f32x8(const f32x4 *__restrict__ lut, uint32_t w, int m, f32x4 &w0, f32x4 &w1) {
+    const f32x4 lo = lut[(w >> (8 - 8 * m)) & 0xffu], hi = lut[(w >> (24 - 8 * m)) & 0xffu];
+    w0 = f32x4{lo[0], hi[0], lo[1], hi[1]};
+    w1 = f32x4{lo[2], hi[2], lo[3], hi[3]};
 }
 // 8 weights (pairs 4k .. 4k + 3): one group of a 32-column chunk.
 __device__ __forceinline__ uint4 codes_bf16x8(uint32_t w, int k) {

@@ -92,7 +92,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
     static_assert(!PIPE1 || (BF16MMA && VEC && KC1 && !DENSE), "PIPE1 shape");
     static_assert(!STAGED || PIPE1, "STAGED is a PIPE1 variant");
     extern __shared__ __align__(16) unsigned char smem[];
-    const size_t wbytes = DENSE ? (size_t)a.Nt * a.Kc * 32 * 64 * dense_frag_bytes<BF16MMA>() : 0;
+    const size_t wbytes = DENSE ? (size_t)a.Nt * a.Kc * 32 * 64 * dense_frag_bytes<BF16MMA>() : lut_bytes<BF16MMA>();
     f32x4 *alpha_l = (f32x4 *)(smem + wbytes);
     f32x4 *beta_l = alpha_l + a.Kc * 128;
 
@@ -100,6 +100,8 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
     if constexpr (DENSE) {
         const uint4 *src = (const uint4 *)a.kw;
         for (int e = tid; e < (int)(wbytes / 16); e += kThreads) ((uint4 *)smem)[e] = src[e];
+    } else {
+        fill_lut<BF16MMA>(smem, tid);
     }
     for (int e = tid; e < a.Kc * 128; e += kThreads) {  // e = (c*4 + q)*32 + g
         const int g = e & 31, cq = e >> 5;
@@ -137,7 +139,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
             contract_dense<BF16MMA>(smem + ((size_t)(nt * a.Kc + c) * 32 * 64 + lane) * dense_frag_bytes<BF16MMA>(),
                                     xm, acc);
         else
-            contract<BF16MMA>(a, nt, c, lane, xm, acc);
+            contract<BF16MMA>(a, nt, c, lane, xm, smem, acc);
     };
 
     if constexpr (PIPE1) {
@@ -210,7 +212,7 @@ __device__ __forceinline__ void hadamard_fwd_body(const HadArgs &a, int blk, int
                 f32x4 acc[32];
 #pragma unroll
                 for (int g = 0; g < 32; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-                contract<true>(a, nt, 0, lane, xm, acc);
+                contract<true>(a, nt, 0, lane, xm, smem, acc);
                 // the next tile's x is requested before any store of this one:
                 // a wait for a load also waits for every memory operation
                 // issued before it, so loads queued behind stores would wait
@@ -918,7 +920,7 @@ template <> struct XElem<true> { typedef uint2 type; };
 template <> struct XElem<false> { typedef f32x4 type; };
 
 template <bool BF16MMA> constexpr size_t wide_lds_bytes() {
-    return (size_t)kWideWaves * 128 * 16 +
+    return lut_bytes<BF16MMA>() + (size_t)kWideWaves * 128 * 16 +
            (size_t)wide_stage<BF16MMA>() * 32 * 64 * sizeof(typename XElem<BF16MMA>::type);
 }
 
@@ -935,10 +937,11 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int S = wide_stage<BF16MMA>();
     typedef typename XElem<BF16MMA>::type XE;
-    f32x4 *beta_l = (f32x4 *)smem;                // [8 local tiles][4][32]
-    XE *xs = (XE *)(beta_l + kWideWaves * 128);   // [S][32 g][64 lanes]
+    f32x4 *beta_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());   // [8 local tiles][4][32]
+    XE *xs = (XE *)(beta_l + kWideWaves * 128);               // [S][32 g][64 lanes]
     constexpr uint32_t esz = sizeof(T);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, t = lane & 15, q = lane >> 4;
+    fill_lut<BF16MMA>(smem, tid);
     const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, (uint32_t)((int64_t)a.M * a.ldx * esz));
     const __amdgpu_buffer_rsrc_t yr = make_rsrc(a.y, (uint32_t)((int64_t)a.M * a.ldy * esz));
     const int n_tiles = (int)ceil_div(a.M, kTile);
@@ -949,7 +952,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
         const bool row_ok = row < a.M;
         const uint32_t xoff = (uint32_t)((int64_t)row * a.ldx * esz);
         const uint32_t yoff = (uint32_t)((int64_t)row * a.ldy * esz);
-        __syncthreads();  // previous item done with beta_l and xs
+        __syncthreads();  // table ready / previous item done with beta_l and xs
         for (int e = tid; e < kWideWaves * 128; e += kWideThreads) {
             const int lw = e >> 7, h = e & 31, qq = (e >> 5) & 3;
             const int o0 = kNTile * (nt0 + lw) + 4 * qq;
@@ -1012,19 +1015,23 @@ __global__ __launch_bounds__(kWideThreads, 1) void hadamard_wide_kernel(HadArgs 
                     const XE *src = xs + (size_t)j * 32 * 64 + lane;
                     const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-                    for (int g = 0; g < 32; ++g) {
-                        const XE xg = src[g * 64];
-                        if constexpr (BF16MMA) {
-                            const uint2 wa = codes_bf16x4(wb[g >> 2], g & 3);
-                            acc[g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
-                                __builtin_bit_cast(i16x4, wa), __builtin_bit_cast(i16x4, xg), acc[g], 0, 0, 0);
-                        } else {
-                            const f32x4 wa = codes_f32x4(wb[g >> 2], g & 3);
+                    for (int g = 0; g < 32; g += 2) {
+                        f32x4 wf[2];
+                        if constexpr (!BF16MMA) codes_f32x8((const f32x4 *)smem, wb[g >> 2], (g >> 1) & 1, wf[0], wf[1]);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[u], xg[u], acc[g], 0, 0, 0);
+                        for (int h = 0; h < 2; ++h) {
+                            const XE xg = src[(g + h) * 64];
+                            if constexpr (BF16MMA) {
+                                const uint2 wa = codes_bf16x4(wb[g >> 2], (g + h) & 3);
+                                acc[g + h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                                    __builtin_bit_cast(i16x4, wa), __builtin_bit_cast(i16x4, xg), acc[g + h], 0, 0, 0);
+                            } else {
+#pragma unroll
+                                for (int u = 0; u < 4; ++u)
+                                    acc[g + h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[h][u], xg[u], acc[g + h], 0, 0, 0);
+                            }
                         }
-                        if ((g & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+                        if ((g & 6) == 6) __builtin_amdgcn_sched_barrier(0);
                     }
                     w0 = n0;
                     w1 = n1;
@@ -1632,13 +1639,14 @@ template <typename T, bool BF16MMA, bool VEC, bool KC1>
 __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_swiglu_kernel(HadArgs g, HadArgs u) {
     extern __shared__ __align__(16) unsigned char smem[];
     typedef typename Stash<BF16MMA>::type SType;
-    f32x4 *ag_l = (f32x4 *)smem;
+    f32x4 *ag_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());
     f32x4 *au_l = ag_l + g.Kc * 128;
     f32x4 *bg_l = au_l + g.Kc * 128;
     f32x4 *bu_l = bg_l + g.Nt * 128;
     SType *stash = (SType *)(bu_l + g.Nt * 128);     // [kWaves][32][64]
 
     const int tid = threadIdx.x;
+    fill_lut<BF16MMA>(smem, tid);
     for (int e = tid; e < g.Kc * 128; e += kThreads) {
         const int gg = e & 31, i0 = 4 * (e >> 5);
         f32x4 va, vb;
@@ -1693,14 +1701,14 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
             load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, 0, q, ag_l, xm);
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-            contract<BF16MMA>(g, nt, 0, lane, xm, acc);
+            contract<BF16MMA>(g, nt, 0, lane, xm, smem, acc);
         } else {
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int c = 0; c < g.Kc; ++c) {
                 XM<BF16MMA> xm;
                 load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, c, q, ag_l, xm);
-                contract<BF16MMA>(g, nt, c, lane, xm, acc);
+                contract<BF16MMA>(g, nt, c, lane, xm, smem, acc);
             }
         }
         fht32x4(acc);
@@ -1735,14 +1743,14 @@ __global__ __launch_bounds__(kThreads, (BF16MMA && KC1) ? 2 : 1) void hadamard_s
             load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, 0, q, au_l, xm);
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-            contract<BF16MMA>(u, nt, 0, lane, xm, acc);
+            contract<BF16MMA>(u, nt, 0, lane, xm, smem, acc);
         } else {
 #pragma unroll
             for (int k = 0; k < 32; ++k) acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
             for (int c = 0; c < g.Kc; ++c) {
                 XM<BF16MMA> xm;
                 load_transform<T, BF16MMA, VEC>(g, xr, xoff, row_ok, c, q, au_l, xm);
-                contract<BF16MMA>(u, nt, c, lane, xm, acc);
+                contract<BF16MMA>(u, nt, c, lane, xm, smem, acc);
             }
         }
         fht32x4(acc);
@@ -2237,7 +2245,9 @@ __global__ void hadamard_dense_prepare_kernel(const float *__restrict__ w, int i
     }
 }
 
-static size_t hadamard_lds_bytes(int Kc, int Nt) { return (size_t)16 * 128 * (Kc + Nt); }
+static size_t hadamard_lds_bytes(bool bf16, int Kc, int Nt) {
+    return (bf16 ? lut_bytes<true>() : lut_bytes<false>()) + (size_t)16 * 128 * (Kc + Nt);
+}
 
 }  // namespace walsh
 
@@ -2333,7 +2343,7 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
     const int64_t esz = bf16 ? 2 : 4;
     const int Nt = base.Nt, Kc = base.Kc;
     const bool swiglu = ubase != nullptr;
-    size_t lds = hadamard_lds_bytes(Kc, Nt);
+    size_t lds = hadamard_lds_bytes(bf16, Kc, Nt);
     // SwiGLU: the up projection's alpha / beta tables and, per working wave,
     // the gate output (32 groups x 64 lanes x 4 values)
     const size_t stash_wave = (size_t)32 * 64 * (bf16 ? 8 : 16);
@@ -2591,7 +2601,7 @@ static int hadamard_multi(const char *fn, const void *x, int64_t ldx, int64_t M,
         if (ldys[i] > ldy) ldy = ldys[i];
     }
     const bool kc1 = Kc == 1 && (bf16 || Nt == 1);
-    const size_t lds = hadamard_lds_bytes(Kc, Nt);
+    const size_t lds = hadamard_lds_bytes(bf16, Kc, Nt);
     hipStream_t s = (hipStream_t)stream;
     const int64_t ld = ldx > ldy ? ldx : ldy;
     if (bf16 && vec && base[0].kw3 && Kc >= 2 && Nt >= 4 && M <= kSplitRows &&

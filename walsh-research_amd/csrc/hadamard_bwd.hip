@@ -102,9 +102,10 @@ struct BwdRed {
 
 template <typename T, bool BF16MMA, bool VEC, bool STORE>
 __device__ __forceinline__ void bwd_red_role(const HadArgs &a, const BwdRed &r, int blk, unsigned char *smem) {
-    f32x4 *alpha_l = (f32x4 *)smem;
+    f32x4 *alpha_l = (f32x4 *)(smem + lut_bytes<BF16MMA>());
     f32x4 *beta_l = alpha_l + a.Kc * 128;
     const int tid = threadIdx.x;
+    fill_lut<BF16MMA>(smem, tid);
     fill_scale(alpha_l, a.alpha, a.in_o, a.Kc, 1.f, tid, kThreads);
     if (STORE) fill_scale(beta_l, a.beta, a.out_o, a.Nt, kCodeScale, tid, kThreads);
     __syncthreads();
@@ -137,7 +138,7 @@ __device__ __forceinline__ void bwd_red_role(const HadArgs &a, const BwdRed &r, 
         for (int c = 0; c < a.Kc; ++c) {
             XM<BF16MMA> xm;
             load_transform<T, BF16MMA, VEC>(a, xr, xoff, row_ok, c, q, alpha_l, xm);
-            contract<BF16MMA>(a, nt, c, lane, xm, acc);
+            contract<BF16MMA>(a, nt, c, lane, xm, smem, acc);
         }
         fht32x4(acc);
         const uint32_t aoff = (uint32_t)((int64_t)row * r.ld_aux * esz);
@@ -711,7 +712,7 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     float *pw = (float *)((char *)workspace + L.off_w);
 
     int64_t ia = 0, ib = 0, iw = 0;  // partial rows written so far
-    const size_t lds_red = (size_t)16 * 128 * (Nt + Kc);
+    const size_t lds_red = (bf16 ? lut_bytes<true>() : lut_bytes<false>()) + (size_t)16 * 128 * (Nt + Kc);
     const size_t lds_dw = (size_t)16 * 128 * (Nt + Kc) + (size_t)32 * 64 * 16;
     const size_t lds = need_w && lds_dw > lds_red ? lds_dw : lds_red;
     if ((int64_t)(lds_red + shape_reserve(bf16)) > maxlds || (int64_t)lds > maxlds)

@@ -127,12 +127,21 @@ template <> struct XM<true> { uint2 b[32]; };
 
 // LDS layout (all 16-byte entries, lane-major so each lane walks its 32
 // groups with immediate offsets):
+//   lut     [256]            float32 only: codes.h
 //   alpha_l [Kc][4][32]      alpha[g, 16c+4q .. +3]   (0 past in_o)
 //   beta_l  [Nt][4][32]      beta[h, 16nt+4q .. +3] * kCodeScale (0 past out_o)
 
+template <bool BF16MMA> constexpr size_t lut_bytes() { return BF16MMA ? 0 : kCodeLut * 16; }
+
 // LDS that the entry points' shape limits keep free (the size of the code
 // table those limits were set with), so the accepted shapes stay the same.
-__host__ inline size_t shape_reserve(bool bf16) { return bf16 ? 2048 : 4096; }
+__host__ inline size_t shape_reserve(bool bf16) { return bf16 ? 2048 : 0; }
+
+template <bool BF16MMA> __device__ __forceinline__ void fill_lut(void *lut, int tid) {
+    if constexpr (!BF16MMA) {
+        if (tid < kCodeLut) ((f32x4 *)lut)[tid] = code_lut_entry((uint32_t)tid);
+    }
+}
 
 // The lane's 4 columns 16c+4q.. of all 32 groups of its row (zeros past
 // in_o / M).
@@ -183,21 +192,32 @@ __device__ __forceinline__ void load_transform(const HadArgs &a, __amdgpu_buffer
 }
 
 template <bool BF16MMA>
-__device__ __forceinline__ void contract_w(uint4 w0, uint4 w1, const XM<BF16MMA> &xm, f32x4 (&acc)[32]) {
+__device__ __forceinline__ void contract_w(uint4 w0, uint4 w1, const XM<BF16MMA> &xm, const void *__restrict__ lut,
+                                           f32x4 (&acc)[32]) {
     const uint32_t wb[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    [[maybe_unused]] f32x4 wn[2];
+    if constexpr (!BF16MMA) codes_f32x8((const f32x4 *)lut, wb[0], 0, wn[0], wn[1]);
 #pragma unroll
-    for (int g = 0; g < 32; ++g) {
+    for (int g = 0; g < 32; g += 2) {
         if constexpr (BF16MMA) {
-            const uint2 wa = codes_bf16x4(wb[g >> 2], g & 3);
-            acc[g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(i16x4, wa),
-                                                                __builtin_bit_cast(i16x4, xm.b[g]), acc[g], 0, 0, 0);
-        } else {
-            const f32x4 wa = codes_f32x4(wb[g >> 2], g & 3);
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[s], xm.v[g][s], acc[g], 0, 0, 0);
+            for (int h = g; h < g + 2; ++h) {
+                const uint2 wa = codes_bf16x4(wb[h >> 2], h & 3);
+                acc[h] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(
+                    __builtin_bit_cast(i16x4, wa), __builtin_bit_cast(i16x4, xm.b[h]), acc[h], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // no expansion is hoisted
+        } else {
+            // the next two groups' table reads in front of these products
+            const f32x4 wa[2] = {wn[0], wn[1]};
+            if (g < 30) codes_f32x8((const f32x4 *)lut, wb[(g + 2) >> 2], ((g + 2) >> 1) & 1, wn[0], wn[1]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    acc[g + h] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[h][s], xm.v[g + h][s], acc[g + h], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if ((g & 1) == 1) __builtin_amdgcn_sched_barrier(0);  // no expansion is hoisted
     }
 }
 
@@ -210,10 +230,10 @@ __device__ __forceinline__ void load_w(const HadArgs &a, int nt, int c, int lane
 
 template <bool BF16MMA>
 __device__ __forceinline__ void contract(const HadArgs &a, int nt, int c, int lane, const XM<BF16MMA> &xm,
-                                         f32x4 (&acc)[32]) {
+                                         const void *__restrict__ lut, f32x4 (&acc)[32]) {
     uint4 w0, w1;
     load_w(a, nt, c, lane, w0, w1);
-    contract_w<BF16MMA>(w0, w1, xm, acc);
+    contract_w<BF16MMA>(w0, w1, xm, lut, acc);
 }
 
 // Output transform of a 16x16 tile (skipped with FHT = false when the caller
