@@ -481,11 +481,14 @@ struct BwdSum {
     float *da, *db, *dw;  // null: not wanted
 };
 
-// 32 columns x 32 rows in flight: a layer of 16x16 groups has 8,192 dW columns
-// (256 workgroups), and each thread's loads are independent (unrolled); 64 x
-// 16 left half the CUs idle (512 partial rows: 10.8 -> 5.3 us).
-constexpr int kSumCols = 32;     // partial columns per workgroup
-constexpr int kSumPhases = 32;   // partial rows summed in parallel, s = phase mod 32
+// Each thread's loads are independent (unrolled).  32 columns x 32 rows per
+// workgroup launch twice the workgroups, most of whose phases have no row once
+// a layer is wide: whole backward calls at 16 / 1,024 / 16,384 rows with 64 x 16
+// against 32 x 32, in us: 128 -> 128 groups' columns 46 / 137 / 1,790 to 66 / 156 /
+// 1,808, 32 -> 88 25 / 41 / 390 to 29 / 45 / 398, 16 -> 16 (512 partial rows of 8,192
+// columns) 11.5 / 17 / 42 to 11.9 / 17 / 42.
+constexpr int kSumCols = 64;     // partial columns per workgroup
+constexpr int kSumPhases = 16;   // partial rows summed in parallel, s = phase mod 16
 
 __host__ __device__ inline int64_t sum_blocks(const BwdSum &r, int64_t *bw, int64_t *ba) {
     *bw = r.dw ? ceil_div((int64_t)32 * r.Op * r.Ip, kSumCols) : 0;
@@ -495,8 +498,8 @@ __host__ __device__ inline int64_t sum_blocks(const BwdSum &r, int64_t *bw, int6
 }
 
 // Column sums of the partial arrays P[S][N] (each partial row contiguous):
-// thread (column, phase) sums rows phase, phase + 32, ... in order, then
-// phase 0 adds the 32 phase sums in order; then the 1/32, the output
+// thread (column, phase) sums rows phase, phase + 16, ... in order, then
+// phase 0 adds the 16 phase sums in order; then the 1/32, the output
 // mapping (padded columns dropped) and the STE mask.
 __global__ __launch_bounds__(kSumCols * kSumPhases) void hadamard_bwd_reduce_kernel(BwdSum r) {
     __shared__ double part[kSumPhases][kSumCols];
