@@ -100,6 +100,25 @@ def test_hadamard_bwd_pairs_equal_general(K, in_o, out_o, M):
         assert_close(a.float().cpu().numpy(), r, torch.bfloat16, f"{name} {in_o}x{out_o} M={M}")
 
 
+@pytest.mark.parametrize("in_o,out_o,M", [(128, 64, 4080), (128, 64, 4096), (128, 128, 2048), (116, 64, 4100),
+                                          (64, 64, 4095), (60, 64, 4096), (64, 128, 2048), (256, 128, 4081)])
+def test_hadamard_bwd_routes_of_wide_layers_agree(K, in_o, out_o, M):
+    """Layers on both sides of the line between the wavefront pairs and the
+    one-wavefront kernel: the input gradient bitwise that of unaligned rows
+    (always the latter, element by element), the sums over the rows as
+    float32 sums of the same products in another grouping (1e-5)."""
+    c = make_case(K, M, in_o, out_o, torch.bfloat16, seed=in_o + out_o + M)
+    rest = (in_o, out_o, c["kw"], c["kwt"], c["alpha"].cuda(), c["beta"].cuda())
+
+    def odd(t):
+        return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+    got = K.hadamard_linear_bwd(c["x"].cuda(), c["gy"].cuda(), *rest, latent=c["lc"])
+    other = K.hadamard_linear_bwd(odd(c["x"]), odd(c["gy"]), *rest, latent=c["lc"])
+    assert torch.equal(got[0], other[0])
+    for name, a, b in zip(("dalpha", "dbeta", "dweight"), got[1:], other[1:]):
+        assert_close(a.cpu().numpy(), b.double().cpu().numpy(), torch.float32, f"{name} {in_o}x{out_o} M={M}")
+
+
 @pytest.mark.parametrize("in_o,out_o", [(71 * 16, 16), (72 * 16, 4), (4, 75 * 16), (75 * 16, 20)])
 def test_hadamard_bwd_very_wide_without_weight_gradient(K, in_o, out_o):
     """Frozen weights lower the general kernel's LDS need below that of the

@@ -334,7 +334,7 @@ __global__ __launch_bounds__(kThreads, 1) void hadamard_bwd_kernel(BwdJob j) {
 // pair_plan.  Latency bound at small row counts.  Measured (kernel alone):
 // 512 -> 512 features, 8,192 rows 64 -> 34 us, 32,768 rows 103 -> 65 us; whole
 // calls (with the reduction) 512 -> 1408 at 8,192 rows 126 -> 53 us, 1024 -> 1024
-// at 16,384 rows 163 -> 108 us, 4096 -> 4096 at 4,096 rows 417 -> 429 us.
+// at 16,384 rows 163 -> 108 us (one_wave_faster: the layers left to the other).
 template <int HF, bool STORE>
 __device__ __forceinline__ void pair_red_role(const HadArgs &a, const BwdRed &r, int blk, int lane, unsigned char *smem) {
     const f32x4 *alpha_l = (const f32x4 *)smem;          // [Kc][4][32]
@@ -606,6 +606,24 @@ static BwdChunk plan_chunk(int64_t rows, int in_o, int out_o, bool pair) {
     return p;
 }
 
+// Where the one-wavefront kernel is the faster one: many tiles of layers whose
+// work its four-wavefront workgroups divide evenly into one round.  It spends
+// fewer LDS exchanges per transform there; elsewhere its rounds do not come
+// out even, or too few wavefronts hide its loads.  Whole calls in us, that
+// kernel -> pairs, in_o -> out_o at 2,048 / 8,192 / 32,768 rows:  128 -> 128  237
+// 797 3,380 -> 230 861 3,800;  120 -> 64  131 435 1,808 -> 132 505 2,115;  256 -> 128
+// at 2,048 / 8,192 / 16,384  403 1,449 2,910 -> 411 1,637 3,463;  64 -> 64 at 4,096 /
+// 8,192 / 32,768  133 252 1,075 -> 157 260 1,032, but 60 -> 60  132 248 994 -> 123 231 944.
+// Others at 8,192:  64 -> 128  503 -> 508, 100 -> 100  1,118 -> 906, 192 -> 192  2,901
+// -> 2,031, 32 -> 32  85 -> 64.
+static bool one_wave_faster(int64_t M, int in_o, int out_o) {
+    const int64_t T = ceil_div(M, kTile), Nt = ceil_div(out_o, kNTile), Kc = ceil_div(in_o, kKChunk);
+    if (Nt < 4 || Nt % 4 || Kc % 4 || Kc < Nt || T * Nt < 128 * (Kc > 8 ? Kc : 8)) return false;
+    if (Kc < 8 && (in_o % kKChunk || out_o % kNTile || T > 1536)) return false;
+    const BwdChunk p = plan_chunk(M, in_o, out_o, false);
+    return p.Sw * Nt * Kc + ceil_div(p.Sa * Kc, kWaves) + ceil_div(p.Sb * Nt, kWaves) <= device_info().cu_count;
+}
+
 struct BwdLayout {
     int64_t rows_max;
     int64_t Sa, Sb, Sw;                 // total partial rows over all chunks
@@ -702,7 +720,7 @@ WALSH_EXPORT int walsh_hadamard_linear_ex_bwd(const void *x, int64_t ldx, int64_
     const int Nt = (int)ceil_div(out_o, kNTile), Kc = (int)ceil_div(in_o, kKChunk);
     const int64_t maxlds = device_info().max_shared_per_block;
     // bf16 rows in 8-byte pieces: wavefront pairs
-    const bool pair = bf16 && vec && (int64_t)pair_lds(Nt, Kc) <= maxlds;
+    const bool pair = bf16 && vec && (int64_t)pair_lds(Nt, Kc) <= maxlds && !one_wave_faster(M, (int)in_o, (int)out_o);
     const BwdLayout L = plan(M, in_o, out_o, ld, esz, pair);
     if (M > 0 && L.rows_max == 0) return set_error(WALSH_ENOTSUP, "%s: row stride too large", fn);
     if (M > 0 && (!workspace || workspace_bytes < L.bytes))
