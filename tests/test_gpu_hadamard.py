@@ -172,8 +172,8 @@ def test_hadamard_linear_shapes(K, dtype, in_o, out_o):
 @pytest.mark.parametrize("in_o,out_o,M", [(128, 128, 1), (128, 128, 17), (128, 128, 4200), (64, 64, 300),
                                           (100, 128, 77), (128, 68, 77), (36, 64, 77), (128, 112, 33)])
 def test_hadamard_wide_bf16(K, in_o, out_o, M):
-    # bf16 layers with 16 < in_o <= 128 and 64 <= out_o <= 128 run the base-3
-    # 16x16x32 kernel: partial 32-column chunks (in_o 100, 36), a partial last
+    # bf16 layers with 16 < in_o <= 128 and 64 <= out_o <= 128 run the 16x16x32
+    # kernel: partial 32-column chunks (in_o 100, 36), a partial last
     # output tile (68), fewer than 8 output tiles (112, 64), and more 16-row
     # tiles than workgroups (4200 rows)
     rng = np.random.default_rng(in_o * 7 + out_o + M)
@@ -230,8 +230,8 @@ def test_hadamard_whole_rows_store_only_their_rows(K, M):
 def test_hadamard_pair_linear_equals_general(K, in_o, out_o, M):
     """bf16 layers of a few chunks and output tiles on wavefront pairs, across
     the dispatch's row counts, ragged widths and tiles: bitwise the general
-    kernel's rows (taken by rows one element off 8-byte alignment), with and
-    without RoPE, and padded group strides."""
+    kernel's rows (taken by rows one element off 8-byte alignment), and padded
+    group strides."""
     g = torch.Generator().manual_seed(in_o * 100 + out_o + M)
     codes = torch.randint(-1, 2, (32, out_o, in_o), generator=g).numpy().astype(np.int8)
     kw = _prepare(K, codes)
@@ -249,6 +249,59 @@ def test_hadamard_pair_linear_equals_general(K, in_o, out_o, M):
     ref = ohad.hadamard_linear_f64(x[:64].double().cpu().numpy(), codes, alpha.double().cpu().numpy(),
                                    beta.double().cpu().numpy())
     assert_close(y[:64].float().cpu().numpy(), ref, torch.bfloat16, f"pair linear {in_o}x{out_o} M={M}")
+
+
+def _off(t):
+    """The same values one element off 8-byte alignment (the general kernels)."""
+    return torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape).copy_(t)
+
+
+def _layer(K, in_o, out_o, g, scale=0.1):
+    kw = _prepare(K, torch.randint(-1, 2, (32, out_o, in_o), generator=g).numpy().astype(np.int8))
+    return (kw, (1 + 0.5 * torch.randn(32, in_o, generator=g)).cuda(),
+            (scale * torch.randn(32, out_o, generator=g)).cuda())
+
+
+@pytest.mark.parametrize("in_o,out_o,M", [(24, 136, 2048), (64, 172, 17), (64, 172, 1489), (64, 172, 1490),
+                                          (32, 256, 1040), (80, 132, 4096), (84, 132, 300),
+                                          (32, 16, 16385), (32, 16, 32768), (32, 16, 32769), (48, 16, 27264),
+                                          (48, 16, 27297), (40, 16, 16400)])
+def test_hadamard_linear_routes_equal_general(K, in_o, out_o, M):
+    """Layers on both sides of the lines between the wavefront pairs, the
+    workgroup-wide kernel (out_o > 128) and the chunk-parallel one (one output
+    tile): bitwise the general kernel's rows."""
+    g = torch.Generator().manual_seed(in_o * 100 + out_o + M)
+    layer = _layer(K, in_o, out_o, g)
+    x = torch.randn(M, 32 * in_o, generator=g).to(torch.bfloat16).cuda()
+    assert torch.equal(K.hadamard_linear(x, in_o, out_o, *layer), K.hadamard_linear(_off(x), in_o, out_o, *layer))
+
+
+@pytest.mark.parametrize("in_o,out_o,B,T,D", [(24, 24, 3, 21, 24), (64, 24, 1, 130, 8), (20, 16, 2, 2500, 16),
+                                              (32, 16, 1, 20000, 4), (80, 40, 1, 17, 20)])
+def test_hadamard_pair_rope(K, in_o, out_o, B, T, D):
+    """The rotary embedding on the store of layers of several input chunks,
+    against the plain layer's rows turned in float32: ragged rows, head widths
+    and output tiles.  Both round to bf16 once (8 significant bits), by up to 2^-8
+    of a pair's length each."""
+    g = torch.Generator().manual_seed(in_o + out_o + T)
+    layer = _layer(K, in_o, out_o, g)
+    freqs = torch.polar(torch.ones(T, D // 2), torch.randn(T, D // 2, generator=g)).cuda()
+    x = torch.randn(B, T, 32 * in_o, generator=g).to(torch.bfloat16).cuda()
+    y = K.hadamard_linear_rope(x, in_o, out_o, *layer, freqs, D)
+    plain = K.hadamard_linear(x, in_o, out_o, *layer).float().view(B, T, -1, D // 2, 2)
+    turned = torch.view_as_real(torch.view_as_complex(plain) * freqs[None, :, None, :]).reshape(y.shape)
+    size = plain.norm(dim=-1, keepdim=True).expand_as(plain).reshape(y.shape)
+    assert ((y.float() - turned).abs() <= 1.01 * 2.0 ** -7 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("in_o,hid_o,M", [(16, 44, 7168), (16, 44, 7200), (16, 44, 8192), (16, 44, 8193), (8, 24, 12285)])
+def test_hadamard_swiglu_one_round_equals_general(K, in_o, hid_o, M):
+    """One chunk, few output tiles and a row count that nearly fills the
+    one-wavefront kernel's round: bitwise the general kernel's."""
+    g = torch.Generator().manual_seed(in_o + hid_o + M)
+    layers = [_layer(K, in_o, hid_o, g, 0.3) for _ in range(2)]
+    x = torch.randn(M, 32 * in_o, generator=g).to(torch.bfloat16).cuda()
+    assert torch.equal(K.hadamard_swiglu(x, in_o, hid_o, *layers), K.hadamard_swiglu(_off(x), in_o, hid_o, *layers))
 
 
 @pytest.mark.parametrize("in_o,hid_o,M", [(8, 24, 33), (16, 44, 1), (24, 64, 500), (32, 88, 130), (80, 20, 17)])

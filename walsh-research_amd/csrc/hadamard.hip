@@ -2135,7 +2135,7 @@ __global__ __launch_bounds__(kPairThreads * kMlpMaxNt * 2, 3) void hadamard_mlp_
 constexpr int kPairLinMaxKc = 5;
 
 // Linear layers that hadamard_pair_linear_kernel takes (bf16, 8-byte pieces,
-// not the wide kernel's shapes).  Measured us, other kernel -> this one, at
+// not hadamard_wide3_kernel's shapes).  Measured us, other kernel -> this one, at
 // 64 / 1,024 / 6,007 / 16,384 / 65,536 rows, in_o -> out_o:
 //   several chunks and output tiles, always:  24 -> 24  19.5 19.8 23.2 34.5 114
 //     -> 7.8 8.1 13.5 31.5 100;  64 -> 24  33.1 33.6 41.6 94.4 -> 12.7 13.5 23.1 58.0
@@ -2148,8 +2148,21 @@ constexpr int kPairLinMaxKc = 5;
 //     24 -> 16  7.6 7.8 11.7 18.4 61.1 -> 7.8 8.0 11.1 17.7 55.7;  64 -> 16  11.0
 //     11.5 21.6 42.6 -> 12.7 13.3 18.2 46.3
 //   one of each: 16 -> 16  6.4 6.6 9.7 14.9 34.9 -> 6.0 6.1 8.9 14.3 45.2
-static bool pair_linear_shape(int Kc, int Nt, int64_t tiles) {
+// wide: the workgroup-wide kernel (out_o > 128 here) is the other one; it
+// transforms a tile once for eight output tiles, the pairs once for each.  Up
+// to four pairs per CU they are in one round and faster at every shape
+// (80 -> 344 groups' columns, 16 rows 34.3 -> 16.0); past that the smaller of two
+// costs fitted to the measurements (in 0.01 us) decides.  At 2,048 / 8,192 /
+// 32,768 rows, the kernel taken marked:  24 -> 136  26.0 86.9 333 -> 23.5* 60.3* 218*;
+// 32 -> 256  27.1* 88.9* -> 35.3 106;  64 -> 132  34.2* 122 473 -> 38.7 107* 402*;
+// 64 -> 172  34.6* 122* 480* -> 42.7 129 489;  80 -> 344  69.9* 204* -> 87.0 307.
+static bool pair_linear_shape(int Kc, int Nt, int64_t tiles, bool wide) {
     if (Kc > kPairLinMaxKc) return false;
+    if (wide) {
+        const int64_t cus = device_info().cu_count, items = tiles * Nt;
+        const int64_t rounds = ceil_div(tiles * ceil_div(Nt, kWideWaves), cus);
+        return items <= 4 * cus || 900 + 100 * Kc + (65 + 120 * Kc) * items / cus <= 400 + (1250 + 420 * Kc) * rounds;
+    }
     if (Kc == 1) return tiles <= (Nt == 1 ? kPairMaxTilesRows : 512);
     if (Nt == 1) return Kc <= 3 && tiles > 256;
     return true;
@@ -2432,7 +2445,7 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
                 else     { if (one) WALSH_SW_LAUNCH(float, false, false, true); else WALSH_SW_LAUNCH(float, false, false, false); }
             }
 #undef WALSH_SW_LAUNCH
-        } else if (bf16 && vec && !wide3 && pair_linear_shape(Kc, Nt, ceil_div(rows, kTile))) {
+        } else if (bf16 && vec && !wide3 && pair_linear_shape(Kc, Nt, ceil_div(rows, kTile), wide)) {
             launch(hadamard_pair_linear_kernel, dim3((unsigned)(ceil_div(rows, kTile) * Nt)), dim3(kPairThreads),
                    (size_t)16 * 128 * (Kc + 1) + kPairXch, s, a);
         } else if (wide3 && rows <= kSplitRows) {
