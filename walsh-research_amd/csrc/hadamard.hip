@@ -2146,7 +2146,10 @@ constexpr int kPairLinMaxKc = 5;
 //   several chunks, one output tile: the chunk-parallel kernel has the
 //     shorter chain while its pairs fit, and at four chunks keeps it longer:
 //     24 -> 16  7.6 7.8 11.7 18.4 61.1 -> 7.8 8.0 11.1 17.7 55.7;  64 -> 16  11.0
-//     11.5 21.6 42.6 -> 12.7 13.3 18.2 46.3
+//     11.5 21.6 42.6 -> 12.7 13.3 18.2 46.3.  It also runs the tail of a second
+//     round of pairs better (four pairs per CU are a round): 32 -> 16 at 18,000 /
+//     24,576 / 32,768 rows 23.8 26.7 30.3 -> 25 29 34, 48 -> 16 at 18,000 / 24,576 /
+//     30,000 33 40 51 -> 36 42 47 (40 -> 16, a half empty chunk, 32 38 48 -> 31 39 41)
 //   one of each: 16 -> 16  6.4 6.6 9.7 14.9 34.9 -> 6.0 6.1 8.9 14.3 45.2
 // wide: the workgroup-wide kernel (out_o > 128 here) is the other one; it
 // transforms a tile once for eight output tiles, the pairs once for each.  Up
@@ -2156,7 +2159,8 @@ constexpr int kPairLinMaxKc = 5;
 // 32,768 rows, the kernel taken marked:  24 -> 136  26.0 86.9 333 -> 23.5* 60.3* 218*;
 // 32 -> 256  27.1* 88.9* -> 35.3 106;  64 -> 132  34.2* 122 473 -> 38.7 107* 402*;
 // 64 -> 172  34.6* 122* 480* -> 42.7 129 489;  80 -> 344  69.9* 204* -> 87.0 307.
-static bool pair_linear_shape(int Kc, int Nt, int64_t tiles, bool wide) {
+static bool pair_linear_shape(int in_o, int Nt, int64_t tiles, bool wide, bool rope) {
+    const int Kc = (int)ceil_div(in_o, kKChunk);
     if (Kc > kPairLinMaxKc) return false;
     if (wide) {
         const int64_t cus = device_info().cu_count, items = tiles * Nt;
@@ -2164,7 +2168,11 @@ static bool pair_linear_shape(int Kc, int Nt, int64_t tiles, bool wide) {
         return items <= 4 * cus || 900 + 100 * Kc + (65 + 120 * Kc) * items / cus <= 400 + (1250 + 420 * Kc) * rounds;
     }
     if (Kc == 1) return tiles <= (Nt == 1 ? kPairMaxTilesRows : 512);
-    if (Nt == 1) return Kc <= 3 && tiles > 256;
+    if (Nt == 1) {
+        const int64_t slots = 4 * (int64_t)device_info().cu_count;
+        const int64_t tail = rope || tiles <= slots ? 0 : (Kc == 2 ? 2 * slots : (in_o == 3 * kKChunk ? slots * 5 / 3 : 0));
+        return Kc <= 3 && tiles > 256 && tiles > tail;
+    }
     return true;
 }
 
@@ -2445,7 +2453,7 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
                 else     { if (one) WALSH_SW_LAUNCH(float, false, false, true); else WALSH_SW_LAUNCH(float, false, false, false); }
             }
 #undef WALSH_SW_LAUNCH
-        } else if (bf16 && vec && !wide3 && pair_linear_shape(Kc, Nt, ceil_div(rows, kTile), wide)) {
+        } else if (bf16 && vec && !wide3 && pair_linear_shape(base.in_o, Nt, ceil_div(rows, kTile), wide, base.rope != nullptr)) {
             launch(hadamard_pair_linear_kernel, dim3((unsigned)(ceil_div(rows, kTile) * Nt)), dim3(kPairThreads),
                    (size_t)16 * 128 * (Kc + 1) + kPairXch, s, a);
         } else if (wide3 && rows <= kSplitRows) {
