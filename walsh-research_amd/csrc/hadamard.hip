@@ -2429,7 +2429,13 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
         }
         if (grid > cap) grid = cap;
         const dim3 G((unsigned)grid), B(kThreads);
-        if (swiglu && bf16 && vec && Kc <= kPairLinMaxKc) {
+        // One chunk and two or three output tiles: the one-wavefront kernel
+        // where its items nearly fill one round (three per workgroup, two
+        // workgroups per CU); everywhere else the pairs are faster.  At 6,007 /
+        // 8,192 / 9,000 rows, other kernel -> pairs: 16 -> 44  29 29 40 -> 26 31 32 us
+        // (8,192: 1,536 items), 8 -> 24 at 8,192 / 12,288 / 14,000  24 27 34 -> 18 29 31
+        const bool one_round = Kc == 1 && Nt <= 3 && work > resident * 3 * 7 / 8 && work <= resident * 3;
+        if (swiglu && bf16 && vec && Kc <= kPairLinMaxKc && !one_round) {
             HadArgs ua = *ubase;
             ua.x = a.x;
             ua.y = a.y;
@@ -2446,7 +2452,7 @@ static int hadamard_launch(const char *fn, HadArgs base, const HadArgs *ubase, i
 #define WALSH_SW_LAUNCH(T, MMA, V, K1) launch((hadamard_swiglu_kernel<T, MMA, V, K1>), G, B, sw_lds, s, a, ua)
             const bool one = Kc == 1;
             if (bf16) {
-                if (vec) WALSH_SW_LAUNCH(uint16_t, true, true, false);   // more than kPairLinMaxKc chunks
+                if (vec) { if (one) WALSH_SW_LAUNCH(uint16_t, true, true, true); else WALSH_SW_LAUNCH(uint16_t, true, true, false); }
                 else     { if (one) WALSH_SW_LAUNCH(uint16_t, true, false, true); else WALSH_SW_LAUNCH(uint16_t, true, false, false); }
             } else {
                 if (vec) { if (one) WALSH_SW_LAUNCH(float, false, true, true); else WALSH_SW_LAUNCH(float, false, true, false); }
