@@ -1559,6 +1559,11 @@ __global__ __launch_bounds__(64 * kR1Waves) void moe_decode_kernel(const uint16_
 // The tiles are dealt to the workgroups in proportion to the experts' loads
 // (eb_schedule): routed loads differ by a factor of two and more, and the
 // launch lasts as long as its longest workgroup.
+// A workgroup that gets a single tile spreads it over its eight waves instead,
+// a hidden tile of 16 each, and up to W / 2 tiles every tile has a workgroup of
+// its own: whole calls in us against the one thread per hidden unit and with four
+// hidden tiles per wave throughout, 2 experts, 1 / 128 tokens 21 / 29, 33 / 34 to
+// 20 / 22; 16 experts, 6 each 28 / 33, 33 / 34 to 22 / 24.
 // Bound by the float32 matrix rate (512 products of 32 clocks per tile) and
 // the SiLU arithmetic.  Measured at 8,192 tokens x 6 of 16 experts, hidden
 // 128: 74 us (607 us for a thread per hidden unit with dot products from
@@ -1604,15 +1609,21 @@ __device__ __forceinline__ float eb_row_sum16(float v) {
 }
 
 // Deals the experts' 16-pair tiles to W workgroups: expert e gets
-// ceil(tiles_e / T) consecutive workgroups of T tiles each (T a multiple of
-// kEbSlots, such that they fit), starting at start[e]; start[E] of them in
-// all.  Every thread of the workgroup calls it; start and tmp are LDS.
-// Returns T.
-__device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int *start, int *tmp) {
+// ceil(tiles_e / T) consecutive workgroups of T tiles each (T = 1 up to W / 2
+// tiles, else a multiple of kEbSlots, such that they fit), starting at
+// start[e]; start[E] of them in
+// all.  Every thread of the workgroup calls it; start, offs (a copy of
+// offset) and tmp are LDS.  Returns T.
+__device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int *start, int *offs, int *tmp) {
     const int tid = threadIdx.x;
     int tiles = 0;
     if (tid < 128) {
-        tiles = tid < E ? (offset[tid + 1] - offset[tid] + 15) / 16 : 0;
+        if (tid < E) {
+            const int o0 = offset[tid], o1 = offset[tid + 1];
+            tiles = (o1 - o0 + 15) / 16;
+            offs[tid] = o0;
+            if (tid == E - 1) offs[E] = o1;
+        }
         int sum = tiles, top = tiles;
         for (int s = 32; s > 0; s >>= 1) {
             sum += __shfl_xor(sum, s, 64);
@@ -1626,7 +1637,7 @@ __device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int 
     __syncthreads();
     const int total = tmp[0] + tmp[1], top = max(tmp[2], tmp[3]);
     int T = W > E ? (total + W - E - 1) / (W - E) : top;
-    T = max(kEbSlots, (T + kEbSlots - 1) / kEbSlots * kEbSlots);
+    T = total <= W / 2 ? 1 : max(kEbSlots, (T + kEbSlots - 1) / kEbSlots * kEbSlots);
     __syncthreads();
     if (tid < 128) {
         int v = (tiles + T - 1) / T;
@@ -1653,7 +1664,7 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
     // [matrix form][word][lane]: gate, up as [h][d]; down^T as [h][d]; gate^T, up^T as [d][h]
     __shared__ uint32_t words[5][NW][64];
     __shared__ __align__(16) f32x4 sums[3][NHT][2][64];
-    __shared__ int start[kEbMaxE + 1], tmp[4];
+    __shared__ int start[kEbMaxE + 1], offs[kEbMaxE + 1], tmp[4];
     // per wave the transposes, per tile in flight the second half's dx and
     // dw_pair (two buffers)
     struct Work {
@@ -1662,7 +1673,7 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
         float pw[2][kEbSlots][16];
     };
     __shared__ __align__(16) Work work;
-    const int T = eb_schedule(a.offset, a.E, a.W, start, tmp);
+    const int T = eb_schedule(a.offset, a.E, a.W, start, offs, tmp);
     const int wg = (int)blockIdx.x;
     if (wg >= start[a.E]) return;   // workgroup-uniform
     int e = 0;
@@ -1679,49 +1690,20 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), slot = wave & (kEbSlots - 1), half = wave / kEbSlots;
     const int H = a.H, k = a.k;
     // the expert's packed bytes through LDS (the gathers below read single
-    // bytes, from memory a chain of round trips)
+    // bytes, from memory a chain of round trips); requested first, the first
+    // tile's pairs and rows behind them, all in flight before the set-up
     uint8_t *bytes = (uint8_t *)&sums[0][0][0][0];   // gate [H][8], up [H][8], down [32][H/4]
-    for (int i = tid; i < 8 * H; i += kEbThreads) {
-        const uint8_t b0 = a.pg[(int64_t)e * H * 8 + i], b1 = a.pu[(int64_t)e * H * 8 + i],
-                      b2 = a.pd[(int64_t)e * H * 8 + i];
-        bytes[i] = b0;
-        bytes[8 * H + i] = b1;
-        bytes[16 * H + i] = b2;
+    constexpr int kByteIts = (8 * 16 * NHT + kEbThreads - 1) / kEbThreads;
+    uint8_t raw[kByteIts][3];
+#pragma unroll
+    for (int j = 0; j < kByteIts; ++j) {
+        const int i = tid + j * kEbThreads;
+        const int64_t at = (int64_t)e * H * 8 + (i < 8 * H ? i : 0);
+        raw[j][0] = a.pg[at];
+        raw[j][1] = a.pu[at];
+        raw[j][2] = a.pd[at];
     }
-    __syncthreads();
-    for (int i = tid; i < 5 * NW * 64; i += kEbThreads) {
-        const int l = i & 63, w = (i >> 6) % NW, m = i / (64 * NW), lm = l & 15, lq = l >> 4;
-        uint32_t v = 0;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {   // hidden tile 2w + g / 2, depth chunk (or column tile) g % 2
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int hA = 16 * (2 * w + (g >> 1)) + lm, dA = 16 * (g & 1) + 4 * lq + c;   // forms 0, 1, 2
-                const int hB = 16 * (2 * w + (g >> 1)) + 4 * lq + c, dB = 16 * (g & 1) + lm;   // forms 3, 4
-                const int h = m < 3 ? hA : hB, d = m < 3 ? dA : dB;
-                if (h < H) {
-                    const uint32_t b = m == 2 ? packed_bits(bytes + 16 * H + d * (H / 4), h)
-                                              : packed_bits(bytes + (m == 0 || m == 3 ? 0 : 8 * H) + h * 8, d);
-                    v |= b << (14 - 2 * (2 * g + (c >> 1)) + 16 * (c & 1));
-                }
-            }
-        }
-        words[m][w][l] = v;
-    }
-    const float gg = 0.5f * a.gammas[0], gu = 0.5f * a.gammas[1], gd = 0.5f * a.gammas[2];
-    const int p1 = a.offset[e + 1], b0 = a.offset[e] + 16 * T * (wg - start[e]), b1 = min(p1, b0 + 16 * T);
-    __syncthreads();
-    uint32_t cw[5][HW];
-#pragma unroll
-    for (int m = 0; m < 5; ++m)
-#pragma unroll
-        for (int w = 0; w < HW; ++w) cw[m][w] = words[m][half * HW + w][lane];
-
-    f32x4 ag[NH][2], au[NH][2], ad[NH][2];
-#pragma unroll
-    for (int i = 0; i < NH; ++i)
-#pragma unroll
-        for (int c = 0; c < 2; ++c) ag[i][c] = au[i][c] = ad[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int b0 = offs[e] + 16 * T * (wg - start[e]), b1 = min(offs[e + 1], b0 + 16 * T);
 
     // the pair of lane n of the tile at b (-1: none)
     auto pair_of = [&](int b) { return b + n < b1 ? a.list[b + n] : -1; };
@@ -1761,9 +1743,57 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
         return r;
     };
 
-    float *tg = work.tr[wave][0], *tu = work.tr[wave][1];
-    int pid = pair_of(b0 + 16 * slot);
+    // a single tile: its hidden tiles spread over all the waves (one each)
+    const bool spread = b1 - b0 <= 16;
+    int pid = pair_of(spread ? b0 : b0 + 16 * slot);
     Rows r = fetch(pid);
+#pragma unroll
+    for (int j = 0; j < kByteIts; ++j) {
+        const int i = tid + j * kEbThreads;
+        if (i >= 8 * H) continue;
+#pragma unroll
+        for (int m = 0; m < 3; ++m) bytes[8 * m * H + i] = raw[j][m];
+    }
+    __syncthreads();
+    for (int i = tid; i < 5 * NW * 64; i += kEbThreads) {
+        const int l = i & 63, lm = l & 15, lq = l >> 4;
+        const int m = __builtin_amdgcn_readfirstlane(i / (64 * NW)), w = __builtin_amdgcn_readfirstlane((i >> 6) % NW);
+        uint32_t v = 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {   // hidden tile 2w + g / 2, depth chunk (or column tile) g % 2
+            const int h0 = 16 * (2 * w + (g >> 1)), d0 = 16 * (g & 1);
+            auto put = [&](int c, uint32_t b) { v |= b << (14 - 2 * (2 * g + (c >> 1)) + 16 * (c & 1)); };
+            if (m < 2) {          // [h][d]: the four codes are one byte
+                const uint32_t b = h0 + lm < H ? bytes[8 * m * H + (h0 + lm) * 8 + (d0 >> 2) + lq] : 0x55u;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) put(c, code_bits((b >> (6 - 2 * c)) & 3u));
+            } else if (m == 2) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (h0 + lm < H) put(c, packed_bits(bytes + 16 * H + (d0 + 4 * lq + c) * (H / 4), h0 + lm));
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+                    if (h0 + 4 * lq + c < H) put(c, packed_bits(bytes + (m - 3) * 8 * H + (h0 + 4 * lq + c) * 8, d0 + lm));
+            }
+        }
+        words[m][w][l] = v;
+    }
+    const float gg = 0.5f * a.gammas[0], gu = 0.5f * a.gammas[1], gd = 0.5f * a.gammas[2];
+    __syncthreads();
+    uint32_t cw[5][HW];
+#pragma unroll
+    for (int m = 0; m < 5; ++m)
+#pragma unroll
+        for (int w = 0; w < HW; ++w) cw[m][w] = words[m][half * HW + w][lane];
+
+    f32x4 ag[NH][2], au[NH][2], ad[NH][2];
+#pragma unroll
+    for (int i = 0; i < NH; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) ag[i][c] = au[i][c] = ad[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    float *tg = work.tr[wave][0], *tu = work.tr[wave][1];
     // every wave of the workgroup runs every iteration (the barriers below);
     // a slot past the last tile has no pairs and adds zeros
     int it = 0;
@@ -1774,6 +1804,7 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
         const Rows cur = r;
 #pragma unroll
         for (int nt = 0; nt < NH; ++nt) {
+            if (spread && nt != slot) continue;
             // opaque copies: the expansions stay here instead of being hoisted
             // out of the tile loop (160 registers)
             uint32_t w5[5];
@@ -1832,16 +1863,31 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
 #pragma unroll
         for (int j = 0; j < 4; ++j) pw[j] = eb_row_sum16(pw[j]);
         // the second half's sums to the first (two buffers, so one barrier
-        // per iteration orders both the hand-over and the reuse)
-        f32x4 *hdx = &work.dx[it & 1][slot][0][lane];
-        float *hpw = work.pw[it & 1][slot];
-        if (half) {
+        // per iteration orders both the hand-over and the reuse); a spread
+        // tile has one iteration and hands all sums to wave 0 through both
+        f32x4 *hdx = &work.dx[spread ? half : it & 1][slot][0][lane];
+        float *hpw = work.pw[spread ? half : it & 1][slot];
+        if (half || (spread && slot)) {
             hdx[0] = dx[0];
             hdx[64] = dx[1];
             if (n == 0) *(f32x4 *)(hpw + 4 * q) = pw;
         }
         lds_barrier();
-        if (!half) {
+        if (spread ? wave == 0 : !half) {
+            if (spread) {
+                for (int v = 1; v < kEbSlots; ++v) {
+#pragma unroll
+                    for (int mt = 0; mt < 2; ++mt) dx[mt] += work.dx[0][v][mt][lane];
+                    pw += *(const f32x4 *)(work.pw[0][v] + 4 * q);
+                }
+                for (int v = 1; v < kEbSlots; ++v) {
+#pragma unroll
+                    for (int mt = 0; mt < 2; ++mt) dx[mt] += work.dx[1][v][mt][lane];
+                    pw += *(const f32x4 *)(work.pw[1][v] + 4 * q);
+                }
+                hdx = &work.dx[1][0][0][lane];
+                hpw = work.pw[1][0];
+            }
             if (pid >= 0) {
                 float *p = a.dx + (int64_t)(pid / k) * a.ldgx + 32 * e;
 #pragma unroll
@@ -1865,8 +1911,23 @@ __global__ __launch_bounds__(kEbThreads, 2) void moe_experts_bwd_kernel(ExpBwdAr
         }
         pid = next_pid;
     }
-    // the waves' sums in wave order (the two halves hold different units)
-    for (int w = 0; w < kEbSlots; ++w) {
+    // the waves' sums in wave order (the two halves hold different units);
+    // slots that never had a tile hold zeros and are left out
+    const int slots = spread ? 0 : min(kEbSlots, (b1 - b0 + 15) / 16);
+    if (spread) {   // every hidden tile in one wave
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+            if (i == slot) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    sums[0][half * NH + i][c][lane] = ag[i][c];
+                    sums[1][half * NH + i][c][lane] = au[i][c];
+                    sums[2][half * NH + i][c][lane] = ad[i][c];
+                }
+            }
+        __syncthreads();
+    }
+    for (int w = 0; w < slots; ++w) {
         if (slot == w) {
 #pragma unroll
             for (int i = 0; i < NH; ++i)
@@ -1900,8 +1961,8 @@ __global__ __launch_bounds__(256) void moe_experts_bwd_reduce_kernel(const float
                                                                      const int *__restrict__ offset, int W, int E,
                                                                      int H, float *__restrict__ dg,
                                                                      float *__restrict__ du, float *__restrict__ dd) {
-    __shared__ int start[kEbMaxE + 1], tmp[4];
-    eb_schedule(offset, E, W, start, tmp);
+    __shared__ int start[kEbMaxE + 1], offs[kEbMaxE + 1], tmp[4];
+    eb_schedule(offset, E, W, start, offs, tmp);
     const int per = 3 * H * 32, e = (int)blockIdx.y, r = (int)(blockIdx.x * 256 + threadIdx.x);
     if (r >= per) return;
     float v = 0.f;
