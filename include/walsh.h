@@ -53,10 +53,13 @@ const char *walsh_device_arch(void);
  * walsh_timing_end(tags, ms, capacity): stops timing, waits for the timed
  *   kernels and writes up to `capacity` (tag, milliseconds) pairs in launch
  *   order; returns how many were written (negative on error).
+ * walsh_timing_kernel(i): after walsh_timing_end, the symbol of timed launch i
+ *   ("" if there is none), valid until the next walsh_timing_begin.
  * Not thread-safe while timing is on. */
 int walsh_timing_begin(int capacity);
 void walsh_timing_tag(int tag);
 int walsh_timing_end(int *tags, float *ms, int capacity);
+const char *walsh_timing_kernel(int i);
 
 /* ------------------------------------------------------------------ A1 / A11
  * Absmean ternary quantisation.

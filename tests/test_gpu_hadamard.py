@@ -462,6 +462,21 @@ def test_launch_timer_records_kernel_time(K):
     torch.cuda.synchronize()
 
 
+def test_launch_timer_names_the_kernel_that_ran(K):
+    """The label of a timed call is the kernel that the library picked."""
+    from src.model import _hip
+    g = torch.Generator().manual_seed(3)
+    ran = {}
+    for in_o, out_o, M, off in ((16, 16, 64, False), (16, 16, 64, True), (64, 172, 64, False), (64, 172, 8192, False)):
+        layer, x = _layer(K, in_o, out_o, g), torch.randn(M, 32 * in_o, device="cuda").bfloat16()
+        x = _off(x) if off else x
+        with _hip.LaunchTimer() as lt:
+            K.hadamard_linear(x, in_o, out_o, *layer)
+        ran[(in_o, M, off)], = lt.summary()
+    assert list(ran.values()) == ["hadamard_pair_linear_kernel<bf16>", "hadamard_fwd_kernel<bf16>",
+                                  "hadamard_pair_linear_kernel<bf16>", "hadamard_wide_kernel<bf16>"]
+
+
 # --------------------------------------------------------------- head mixer
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])

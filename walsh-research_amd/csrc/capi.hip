@@ -51,7 +51,7 @@ const DeviceInfo &device_info() {
 }
 
 Timing &timing() {
-    static Timing t{false, -1, 0, 0, nullptr, nullptr};
+    static Timing t{false, -1, 0, 0, nullptr, nullptr, nullptr};
     return t;
 }
 
@@ -65,16 +65,20 @@ WALSH_EXPORT int walsh_timing_begin(int capacity) {
         for (int i = 0; i < 2 * t.cap; ++i) (void)hipEventDestroy(t.ev[i]);
         delete[] t.ev;
         delete[] t.tags;
+        delete[] t.names;
         t.ev = new hipEvent_t[2 * capacity];
         t.tags = new int[capacity];
+        t.names = new const char *[capacity]();
         for (int i = 0; i < 2 * capacity; ++i) {
             const hipError_t e = hipEventCreate(&t.ev[i]);
             if (e != hipSuccess) {
                 for (int j = 0; j < i; ++j) (void)hipEventDestroy(t.ev[j]);
                 delete[] t.ev;
                 delete[] t.tags;
+                delete[] t.names;
                 t.ev = nullptr;
                 t.tags = nullptr;
+                t.names = nullptr;
                 t.cap = 0;
                 return check_hip(e, "walsh_timing_begin: hipEventCreate");
             }
@@ -102,6 +106,11 @@ WALSH_EXPORT int walsh_timing_end(int *tags, float *ms, int capacity) {
     }
     t.n = 0;
     return n;
+}
+
+WALSH_EXPORT const char *walsh_timing_kernel(int i) {
+    const walsh::Timing &t = walsh::timing();
+    return i >= 0 && i < t.cap && t.names[i] ? t.names[i] : "";
 }
 
 WALSH_EXPORT int walsh_abi_version(void) { return WALSH_ABI_VERSION; }

@@ -42,6 +42,7 @@ struct Timing {
     int tag, n, cap;
     hipEvent_t *ev;  // 2 * cap events
     int *tags;       // cap
+    const char **names;  // cap: the kernels' symbols
 };
 Timing &timing();
 
@@ -50,6 +51,7 @@ inline void launch(F kernel, dim3 grid, dim3 block, uint32_t lds, hipStream_t s,
     Timing &t = timing();
     if (t.on && t.n < t.cap) {
         hipExtLaunchKernelGGL(kernel, grid, block, lds, s, t.ev[2 * t.n], t.ev[2 * t.n + 1], 0, args...);
+        t.names[t.n] = hipKernelNameRefByPtr((const void *)kernel, s);
         t.tags[t.n++] = t.tag;
     } else {
         hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);

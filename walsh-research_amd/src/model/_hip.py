@@ -6,6 +6,7 @@ missing or no GPU is present, every hot-path op raises.
 """
 import ctypes
 import os
+import re
 
 import torch
 
@@ -28,6 +29,7 @@ SIGNATURES = {
     "walsh_timing_begin": (_I, [_I]),
     "walsh_timing_tag": (None, [_I]),
     "walsh_timing_end": (_I, [_P, _P, _I]),
+    "walsh_timing_kernel": (ctypes.c_char_p, [_I]),
     "walsh_ternary_gamma": (_I, [_P, _I64, _P, _P]),
     "walsh_ternary_quantize": (_I, [_P, _I64, _I64, _P, _P, _P, _P, _P]),
     "walsh_ternary_unpack": (_I, [_P, _I64, _I64, _P, _P]),
@@ -162,7 +164,8 @@ class LaunchTimer:
     kernel's own start/stop timestamps (walsh_timing_begin: the library
     launches through hipExtLaunchKernelGGL with an event pair per launch, on
     the launching stream), labelled with the (kernel, bytes, flops) of the
-    entry-point call that made it.  Used by bench.py for the roofline."""
+    entry-point call that made it; "*" in a kernel label stands for the kernel
+    that the call launched first.  Used by bench.py for the roofline."""
 
     CAPACITY = 1 << 16
 
@@ -188,6 +191,10 @@ class LaunchTimer:
         n = lib().walsh_timing_end(tags, ms, cap)
         if n < 0:
             check(n, "walsh_timing_end")
+        self.kernels = {}
+        for i in reversed(range(n)):
+            m = re.search(r"([a-z][a-z0-9_]*_kernel)", lib().walsh_timing_kernel(i).decode())
+            self.kernels[tags[i]] = re.sub(r"^walsh\d*", "", m.group(1)) if m else "?"
         return [(tags[i], ms[i]) for i in range(n)]
 
     def summary(self):
@@ -200,6 +207,7 @@ class LaunchTimer:
         out = {}
         for tag, ms in per_call.items():
             kname, nbytes, flops = self.meta[tag]
+            kname = kname.replace("*", self.kernels[tag])
             d = out.setdefault(kname, dict(launches=0, ms=0.0, bytes=0, flops=0))
             d["launches"] += 1
             d["ms"] += ms

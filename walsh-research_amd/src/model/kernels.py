@@ -150,58 +150,18 @@ def hadamard_prepare(packed: torch.Tensor, in_o: int, out_o: int) -> torch.Tenso
     return kw
 
 
-# 16-row tiles per layer up to which the library runs the bf16 single-output-tile
-# shapes on wavefront pairs (hadamard_pair_kernel / hadamard_pair_kpar_kernel);
-# 16x16 layers on contiguous 512-value rows switch to the one-wavefront kernel
-# (whole rows through LDS) above PAIR_MAX_TILES_ROWS
-PAIR_MAX_TILES = 2048
-PAIR_MAX_TILES_ROWS = 1024
-
-
-def _whole_rows(in_o, out_o, ldx, dt, ptr):
-    """16x16 bf16 layer on 16-byte aligned rows of 512 contiguous values
-    (outputs allocated contiguous): the library's whole-row variant of the
-    one-wavefront kernel."""
-    return dt == torch.bfloat16 and in_o == 16 and out_o == 16 and ldx == 512 and ptr % 16 == 0
-
-
-def _pair_shape(rows, in_o, out_o, dt, vec, rope=False, whole_rows=False):
-    """The pair kernel the library dispatches for this shape, or None."""
-    limit = PAIR_MAX_TILES_ROWS if whole_rows else PAIR_MAX_TILES
-    tiles, kc, nt = (rows + 15) // 16, (in_o + 15) // 16, (out_o + 15) // 16
-    if dt != torch.bfloat16 or not vec:
-        return None
-    if kc > 1 and nt >= 4 and in_o <= 128 and out_o <= 128:
-        return None
-    if kc <= 5 and (tiles <= (PAIR_MAX_TILES_ROWS if nt == 1 else 512) if kc == 1 else
-                    kc <= 3 and tiles > 256 if nt == 1 else True):
-        return "hadamard_pair_linear_kernel"
-    if out_o > 16 or tiles > limit:
-        return None
-    if in_o <= 16:
-        return "hadamard_pair_kernel"
-    if in_o <= 64 and not rope:
-        return "hadamard_pair_kpar_kernel"
-    return None
-
-
-def _had_meta(rows, in_o, out_o, dt, vec, kc1, swiglu=False, rope=False, whole_rows=False):
+def _had_meta(rows, in_o, out_o, dt, swiglu=False):
+    """(label, bytes, operations) of a call for launch timing; the library's
+    shape rules pick the kernel, whose name takes the label's star."""
     esz = 2 if dt == torch.bfloat16 else 4
     tag = "bf16" if dt == torch.bfloat16 else "f32"
     if swiglu:
-        kname = "hadamard_pair_swiglu_kernel<bf16>" if dt == torch.bfloat16 and vec and in_o <= 80 else \
-            "hadamard_swiglu_kernel<%s,%s>" % (tag, "vec" if vec else "scalar")
         nbytes = rows * 32 * (in_o + out_o) * esz + 2 * 32 * out_o * ((in_o + 3) // 4) + 8 * 32 * (in_o + out_o)
         flops = rows * 2 * (2 * 32 * in_o * out_o + 10 * 32 * (in_o + out_o)) + rows * 32 * out_o * 4
-    else:
-        pair = _pair_shape(rows, in_o, out_o, dt, vec, rope, whole_rows)
-        kname = ("%s<%s>" % (pair, tag)) if pair else \
-            "hadamard_fwd_kernel<%s,%s,%s>" % (tag, "vec" if vec else "scalar", "kc1" if kc1 else "kloop")
-        if whole_rows and not pair:
-            kname = "hadamard_fwd_kernel<bf16,rows>"
-        nbytes = rows * 32 * (in_o + out_o) * esz + 32 * out_o * ((in_o + 3) // 4) + 4 * 32 * (in_o + out_o)
-        flops = rows * (2 * 32 * in_o * out_o + 10 * 32 * (in_o + out_o) + 32 * (in_o + out_o))
-    return kname, nbytes, flops
+        return "*<%s>" % tag, nbytes, flops
+    nbytes = rows * 32 * (in_o + out_o) * esz + 32 * out_o * ((in_o + 3) // 4) + 4 * 32 * (in_o + out_o)
+    flops = rows * (2 * 32 * in_o * out_o + 10 * 32 * (in_o + out_o) + 32 * (in_o + out_o))
+    return "*<%s>" % tag, nbytes, flops
 
 
 def rope_supported(x: torch.Tensor, out_o: int, head_dim: int) -> bool:
@@ -271,13 +231,7 @@ def hadamard_linear_rope(x: torch.Tensor, in_o: int, out_o: int, kweight: torch.
         check_half_range("beta", beta)
     alpha = alpha.detach().float().contiguous()
     beta = beta.detach().float().contiguous()
-    vec = True
-    kc1 = in_o <= 16
-    kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt, vec, kc1, rope=True,
-                                     whole_rows=_whole_rows(in_o, out_o, ldx, dt, xv.data_ptr()))
-    if in_o > 16 and out_o > 48:
-        kname = "hadamard_wide3_kernel<bf16>" if dt == torch.bfloat16 and in_o <= 128 and out_o <= 128 else \
-            "hadamard_wide_kernel<%s>" % ("bf16" if dt == torch.bfloat16 else "f32")
+    kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt)
     _hip.call("walsh_hadamard_linear_rope_fwd", xv.data_ptr(), ldx, rows, in_o, out_o, kweight.data_ptr(),
               alpha.data_ptr(), beta.data_ptr(), table.data_ptr(), T, head_dim, y.data_ptr(), 32 * out_o,
               _hip.dtype_code(dt), _hip.stream(x.device), kernel=kname, nbytes=nbytes, flops=flops)
@@ -346,13 +300,9 @@ def hadamard_linear_multi(x: torch.Tensor, in_o: int, out_o: int, layers, freqs_
         table = torch.view_as_real(freqs_cis[:T].contiguous())
         assert table.shape == (T, head_dim // 2, 2) and table.dtype == torch.float32, "freqs_cis shape"
     arrs = [(ctypes.c_void_p * n)(*v) for v in (kws, als, bes, yps)]
-    kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt, True, in_o <= 16)
+    kname, _, flops = _had_meta(rows, in_o, out_o, dt)
+    kname = "%s,x%d>" % (kname[:-1], n)
     nbytes = rows * 32 * (in_o + n * out_o) * x.element_size()
-    whole = _whole_rows(in_o, out_o, ldx, dt, xv.data_ptr()) and all(o is None for o in outs)
-    pair = dt == torch.bfloat16 and in_o <= 16 and out_o <= 16 and \
-        (rows + 15) // 16 <= (PAIR_MAX_TILES_ROWS if whole else PAIR_MAX_TILES)
-    kname = ("hadamard_pair_kernel<bf16,x%d>" % n) if pair else \
-        "hadamard_fwdn_kernel<%s,x%d%s>" % ("bf16" if dt == torch.bfloat16 else "f32", n, ",rows" if whole else "")
     rope_args = (0 if table is None else table.data_ptr(), T, head_dim or 4, mask, _hip.dtype_code(dt),
                  _hip.stream(x.device))
     if all(o is None for o in outs):
@@ -395,16 +345,7 @@ def hadamard_linear(x: torch.Tensor, in_o: int, out_o: int, kweight: torch.Tenso
     alpha = alpha.detach().float().contiguous()
     beta = beta.detach().float().contiguous()
     assert alpha.numel() == 32 * in_o and beta.numel() == 32 * out_o, "alpha/beta shapes"
-    esz = x.element_size()
-    vec = gsx % 4 == 0 and gsy % 4 == 0 and ldx % 4 == 0 and xv.data_ptr() % (4 * esz) == 0
-    kc1 = in_o <= 16 and (dt == torch.bfloat16 or out_o <= 16)
-    whole = gsx == 16 and gsy == 16 and _whole_rows(in_o, out_o, ldx, dt, xv.data_ptr())
-    kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt, vec, kc1, whole_rows=whole)
-    if vec and in_o > 16 and out_o > 48:
-        if dt == torch.bfloat16 and in_o <= 128 and out_o <= 128:
-            kname = "hadamard_wide3_kernel<bf16>"
-        else:
-            kname = "hadamard_wide_kernel<%s>" % ("bf16" if dt == torch.bfloat16 else "f32")
+    kname, nbytes, flops = _had_meta(rows, in_o, out_o, dt)
     _hip.call("walsh_hadamard_linear_ex_fwd", xv.data_ptr(), ldx, gsx, rows, in_o, out_o, kweight.data_ptr(),
               alpha.data_ptr(), beta.data_ptr(), y.data_ptr(), 32 * gsy, gsy, code, _hip.stream(x.device),
               kernel=kname, nbytes=nbytes, flops=flops)
@@ -427,9 +368,7 @@ def hadamard_swiglu(x: torch.Tensor, in_o: int, hid_o: int, gate, up, gsh: int =
     kg, ag, bg = gate
     ku, au, bu = up
     ag, bg, au, bu = (t.detach().float().contiguous() for t in (ag, bg, au, bu))
-    esz = x.element_size()
-    vec = in_o % 4 == 0 and gsh % 4 == 0 and ldx % 4 == 0 and xv.data_ptr() % (4 * esz) == 0
-    kname, nbytes, flops = _had_meta(rows, in_o, hid_o, dt, vec, True, swiglu=True)
+    kname, nbytes, flops = _had_meta(rows, in_o, hid_o, dt, swiglu=True)
     _hip.call("walsh_hadamard_swiglu_fwd", xv.data_ptr(), ldx, in_o, rows, in_o, hid_o, kg.data_ptr(), ag.data_ptr(),
               bg.data_ptr(), ku.data_ptr(), au.data_ptr(), bu.data_ptr(), h.data_ptr(), 32 * gsh, gsh, code,
               _hip.stream(x.device), kernel=kname, nbytes=nbytes, flops=flops)
@@ -609,6 +548,11 @@ def head_mixer(x: torch.Tensor, kweight: torch.Tensor, beta: torch.Tensor, out: 
               kweight.data_ptr(), b.data_ptr(), y.data_ptr(), y.stride(1), _hip.dtype_code(dt), _hip.stream(x.device),
               kernel="head_mixer<%s>" % ("bf16" if dt == torch.bfloat16 else "f32"), nbytes=nbytes, flops=flops)
     return y
+
+
+# 16-row tiles above which the library runs 16x16 layers on contiguous 512-value
+# rows whole-row instead of on wavefront pairs
+PAIR_MAX_TILES_ROWS = 1024
 
 
 def head_mixer_proj_supported(x: torch.Tensor, rows: int) -> bool:
