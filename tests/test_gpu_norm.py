@@ -83,7 +83,7 @@ def test_rmsnorm_forms():
     assert not norm._fused(x.float()) and not norm._fused(x[:0]) and not norm._fused(x.cpu())
     with torch.autograd.forward_ad.dual_level():
         assert not norm._fused(x)
-    torch.func.vmap(lambda v: norm(v))(x.detach())
+    close((torch.func.vmap(lambda v: norm(v))(x.detach()),), (_plain(norm, x.detach()),))
 
 
 def test_rmsnorm_kernels_capture():
@@ -159,6 +159,17 @@ def test_few_rows_linear_forms():
         assert not FewRowsLinear.takes(x, rows)
     with torch.autocast("cuda", dtype=torch.float16):
         assert not FewRowsLinear.takes(x, rows)
+
+
+def test_few_rows_linear_rule():
+    """Up to 2^18 weights any rows, up to 400 K from 1,024 rows (N <= 32) or 3,072
+    on; never past either."""
+    from src.model.linear import FewRowsLinear
+    for N, K, rows, takes in ((24, 2048, 1, True), (256, 1024, 7, True), (24, 16384, 1023, False), (24, 16384, 1024, True),
+                              (320, 1280, 3071, False), (320, 1280, 3072, True), (1000, 384, 4096, False),
+                              (512, 1024, 8192, False)):
+        x, w = torch.empty(rows, K, device="cuda", dtype=torch.bfloat16), torch.empty(N, K, device="cuda")
+        assert FewRowsLinear.takes(x, w) is takes, (N, K, rows)
 
 
 def test_router_linears_under_hooks():

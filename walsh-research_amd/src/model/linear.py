@@ -6,13 +6,21 @@ import torch.nn.functional as F
 from . import kernels
 from ._common import first_order, plain_eager
 
-# N * K up to which the weight gradient runs on the HIP kernel: the library
-# gives a product with a small output few workgroups.  Kernel against library
-# in us at 64 / 2,048 / 8,192 tokens: 24 x 2,048 6.8 / 9.1 / 14 against 7.5 /
-# 18 / 56; 128 x 512 6.9 / 9.6 / 15 against 7.4 / 22 / 65; 24 x 16,384 7.8 / 18
-# / 47 against 7.5 / 21 / 62; past the line 384 x 1,536 8.5 / 23.5 / 52 against
-# 7.7 / 19 / 56 and 1,024 x 4,096 25 / 61 / 191 against 15 / 34 / 93.
+# Where the weight gradient runs on the HIP kernel: the library gives a product
+# with a small output few workgroups.  Kernel against library in us at 64 / 1,024
+# / 2,048 / 8,192 tokens: 24 x 2,048 6.6 / 7.8 / 8.9 / 14 against 6.9 / 14 / 18 / 55;
+# 128 x 512 6.8 / 8.1 / 9.4 / 14 against 7.3 / 15 / 22 / 65; 256 x 1,024 7.3 / 12.7 / 14
+# / 20 against 6.9 / 13.6 / 18 / 55.  Past 2^18 weights its partial sums count: 24 x
+# 16,384 7.4 / 13.2 / 18 / 47 against 6.9 / 15 / 20 / 62 (at 512 tokens 11.5 against
+# 10.8), 320 x 1,280 7.5 / 16.4 / 20 / 39 against 7.1 / 13.5 / 18 / 56 (at 3,072 21
+# against 25); past the line 1,024 x 4,096 25 / 47 / 61 / 191 against 15 / 27 / 34 / 93.
 MAX_WEIGHTS = 400 * 1024
+ANY_ROWS_WEIGHTS = 2 ** 18
+
+
+def _few_rows(M, N, K) -> bool:
+    return N <= 1024 and (N * K <= ANY_ROWS_WEIGHTS
+                          or (N <= 512 and N * K <= MAX_WEIGHTS and M >= (1024 if N <= 32 else 3072)))
 
 
 class _FewRowsLinearFunction(torch.autograd.Function):
@@ -46,8 +54,8 @@ class FewRowsLinear:
         N, K = w.shape
         return (x.is_cuda and x.dtype == torch.bfloat16 and w.dtype == torch.float32 and w.device == x.device
                 and type(x) is torch.Tensor and type(w) in (torch.Tensor, torch.nn.Parameter) and x.numel() > 0
-                and x.shape[-1] == K and x.is_contiguous() and x.data_ptr() % 16 == 0 and N <= 1024
-                and N * K <= MAX_WEIGHTS and K % 8 == 0 and x.numel() // K * max(N, K) * 2 < 2 ** 31
+                and x.shape[-1] == K and x.is_contiguous() and x.data_ptr() % 16 == 0
+                and _few_rows(x.numel() // K, N, K) and K % 8 == 0 and x.numel() // K * max(N, K) * 2 < 2 ** 31
                 and (not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") == torch.bfloat16)
                 and plain_eager())
 
