@@ -1560,10 +1560,10 @@ __global__ __launch_bounds__(64 * kR1Waves) void moe_decode_kernel(const uint16_
 // (eb_schedule): routed loads differ by a factor of two and more, and the
 // launch lasts as long as its longest workgroup.
 // A workgroup that gets a single tile spreads it over its eight waves instead,
-// a hidden tile of 16 each, and up to W / 2 tiles every tile has a workgroup of
-// its own: whole calls in us against the one thread per hidden unit and with four
-// hidden tiles per wave throughout, 2 experts, 1 / 128 tokens 21 / 29, 33 / 34 to
-// 20 / 22; 16 experts, 6 each 28 / 33, 33 / 34 to 22 / 24.
+// a hidden tile of 16 each, and up to W tiles every tile has a workgroup of its
+// own.  Whole calls in us, one thread per hidden unit / four hidden tiles per wave
+// throughout / now: 2 experts, 1 and 128 tokens 21 29 / 33 34 / 20 22; 16 experts
+// x 6, 1 and 128 tokens 28 33 / 33 34 / 22 24.
 // Bound by the float32 matrix rate (512 products of 32 clocks per tile) and
 // the SiLU arithmetic.  Measured at 8,192 tokens x 6 of 16 experts, hidden
 // 128: 74 us (607 us for a thread per hidden unit with dot products from
@@ -1609,11 +1609,11 @@ __device__ __forceinline__ float eb_row_sum16(float v) {
 }
 
 // Deals the experts' 16-pair tiles to W workgroups: expert e gets
-// ceil(tiles_e / T) consecutive workgroups of T tiles each (T = 1 up to W / 2
-// tiles, else a multiple of kEbSlots, such that they fit), starting at
-// start[e]; start[E] of them in
-// all.  Every thread of the workgroup calls it; start, offs (a copy of
-// offset) and tmp are LDS.  Returns T.
+// ceil(tiles_e / T) consecutive workgroups of T tiles each, starting at
+// start[e]; start[E] of them in all.  T = 1 up to W tiles (16 experts x 6,
+// hidden 128, 193 / 256 tiles: 28 / 32 us, 34 / 35 with T = 4), else a multiple of
+// kEbSlots, such that they fit.  Every thread of the workgroup calls it; start,
+// offs (a copy of offset) and tmp are LDS.  Returns T.
 __device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int *start, int *offs, int *tmp) {
     const int tid = threadIdx.x;
     int tiles = 0;
@@ -1637,7 +1637,7 @@ __device__ __forceinline__ int eb_schedule(const int *offset, int E, int W, int 
     __syncthreads();
     const int total = tmp[0] + tmp[1], top = max(tmp[2], tmp[3]);
     int T = W > E ? (total + W - E - 1) / (W - E) : top;
-    T = total <= W / 2 ? 1 : max(kEbSlots, (T + kEbSlots - 1) / kEbSlots * kEbSlots);
+    T = total <= W ? 1 : max(kEbSlots, (T + kEbSlots - 1) / kEbSlots * kEbSlots);
     __syncthreads();
     if (tid < 128) {
         int v = (tiles + T - 1) / T;
