@@ -27,7 +27,7 @@ MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 
 # kernels allowed to spill (mangled-name fragment -> most spilled VGPRs):
 # backward and fp32 variants off the measured inference path, the n = 8
-# Sinkhorn backward (n <= 4 takes sinkhorn_bwd_lds_kernel), and a few
+# Sinkhorn backward (n <= 4 takes sinkhorn_bwd_quad_kernel), and a few
 # registers in epilogues outside the inner loops
 ALLOWED = {
     "sinkhorn_bwd_kernelILi8E": 244,
