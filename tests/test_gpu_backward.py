@@ -478,13 +478,17 @@ def test_moe_backward_matches_oracle(C, k, T):
 
 
 @pytest.mark.parametrize("M,E,k,H,pad", [(1, 16, 1, 128, 0), (16, 1, 1, 128, 0), (17, 2, 2, 64, 1), (33, 4, 2, 48, 3),
-                                         (530, 16, 6, 128, 4), (1100, 2, 1, 128, 0)])
+                                         (530, 16, 6, 128, 4), (1100, 2, 1, 128, 0), (4096, 1, 1, 16, 0),
+                                         (4097, 1, 1, 16, 3), (2100, 2, 2, 64, 1), (1500, 4, 4, 128, 0),
+                                         (9000, 2, 1, 128, 0)])
 def test_moe_experts_bwd_tiles(K, M, E, k, H, pad):
     """walsh_moe_experts_bwd at the edges of its 16-pair tiles (one pair, a
-    full tile, one more, experts without pairs, several tiles per wavefront),
+    full tile, one more, experts without pairs, several tiles per wavefront; as
+    many tiles as workgroups, a workgroup each, and one tile more),
     hidden sizes on both instantiations and past a tile pair, rows with and
     without 16-byte alignment, against the float64 formulas on the same
-    codes.  Bar: float32 sums of up to 1,100 products, 1e-5."""
+    codes.  Bar: float32 sums of up to 9,000 products of either sign, whose rounding
+    adds up to about 2^-24 sqrt(9,000) = 6e-6 of the result at most: 1e-5."""
     g = torch.Generator().manual_seed(M + H)
     lat = [torch.rand(sh, generator=g) * 2 - 1 for sh in ((E, H, 32), (E, H, 32), (E, 32, H))]
     qs = [K.ternary_quantize(w.cuda(), codes=True, packed=True) for w in lat]
